@@ -2533,24 +2533,29 @@ static void launch_select(const DevBatch &b, const ReadSet &set, int kind, hipSt
     hipLaunchKernelGGL(k_select, dim3(g < 1024u ? (g ? g : 1u) : 1024u), dim3(256), 0, st, b, set, kind);
 }
 
-// one thread per bucket: its line (DevIndex::lines) from starts and the table
+// The bucket lines (DevIndex::lines) from starts and the table, eight lanes a
+// bucket: lane 0 writes the head, lane j > 0 record j - 1. Bound by the lines'
+// own bytes (2^bits x 128): a wave's store covers eight whole lines, where one
+// thread a bucket stored 16 bytes at a 128-byte stride. XX
 __global__ __launch_bounds__(256) void k_bucket_lines(const uint4 *rs, const uint64_t *starts, uint64_t nb,
                                                       uint4 *lines) {
-    const uint64_t bk = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (bk >= nb) return;
-    const uint64_t s = starts[bk], e = starts[bk + 1];
-    const uint64_t size = e - s;
-    uint4 *line = lines + bk * BUCKET_LINE;
-    line[0] = make_uint4((uint32_t)s, (uint32_t)(s >> 32), size < 0xffffffffull ? (uint32_t)size : 0xffffffffu, 0u);
-    for (uint32_t j = 1; j < BUCKET_LINE; j++) {
-        const uint64_t x = s + j - 1;
-        line[j] = x < e ? rs[x] : make_uint4(0u, 0u, 0u, 0u);
+    const uint32_t j = threadIdx.x % BUCKET_LINE;
+    constexpr uint32_t PER_BLOCK = 256 / BUCKET_LINE;
+    for (uint64_t bk = (uint64_t)blockIdx.x * PER_BLOCK + threadIdx.x / BUCKET_LINE; bk < nb;
+         bk += (uint64_t)gridDim.x * PER_BLOCK) {
+        const uint64_t s = starts[bk], size = starts[bk + 1] - s;
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);
+        if (j == 0)
+            v = make_uint4((uint32_t)s, (uint32_t)(s >> 32), size < 0xffffffffull ? (uint32_t)size : 0xffffffffu, 0u);
+        else if (j <= size)
+            v = rs[s + j - 1];
+        lines[bk * BUCKET_LINE + j] = v;
     }
 }
 
 void launch_bucket_lines(const uint4 *rs, const uint64_t *starts, int bits, uint4 *lines, hipStream_t st) {
-    const uint64_t nb = 1ull << bits;
-    hipLaunchKernelGGL(k_bucket_lines, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, st, rs, starts, nb, lines);
+    const uint64_t nb = 1ull << bits, g = nb * BUCKET_LINE / 256;
+    hipLaunchKernelGGL(k_bucket_lines, dim3((unsigned)(g < 65536 ? g : 65536)), dim3(256), 0, st, rs, starts, nb, lines);
 }
 
 void launch_reset_ctl(DevCtl *ctl, hipStream_t st) {
