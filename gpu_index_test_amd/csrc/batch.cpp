@@ -304,7 +304,7 @@ int batch_stage(gis_batch *b, const char *seqs, const uint64_t *offsets, const u
     ensure_input_arrays(b, n);
     b->tot_rs_cap = b->h_rs_off[n];
     b->span = span;
-    ensure<char>(b->seqs, span);
+    ensure<char>(b->seqs, span + SEQ_PAD);
     std::vector<CopyItem> items;
     std::vector<CopyItem> &in = defer ? *defer : items;
     if (span) in.push_back({b->seqs.p, seqs + base, span});
@@ -1015,7 +1015,7 @@ extern "C" int gis_batch_create(gis_ctx *ctx, uint32_t max_reads, uint64_t max_b
     gis_batch *b = batch_new(ctx, nullptr);
     ensure_input_arrays(b, max_reads);
     ensure_read_arrays(b, max_reads);
-    ensure<char>(b->seqs, max_bases);
+    ensure<char>(b->seqs, max_bases + SEQ_PAD);
     *out = b;
     return GIS_OK;
     API_END(ctx)
@@ -1028,7 +1028,7 @@ extern "C" int gis_batch_create_async(gis_ctx *ctx, uint32_t max_reads, uint64_t
     try {
         ensure_input_arrays(b, max_reads);
         ensure_read_arrays(b, max_reads);
-        ensure<char>(b->seqs, max_bases);
+        ensure<char>(b->seqs, max_bases + SEQ_PAD);
     } catch (...) {
         batch_free(b);
         throw;
@@ -1046,7 +1046,7 @@ extern "C" int gis_batch_create_shared(gis_ctx *ctx, uint32_t max_reads, uint64_
     gis_batch *b = batch_new(ctx, share_with->ws);
     b->stream = share_with->stream;
     ensure_input_arrays(b, max_reads);
-    ensure<char>(b->seqs, max_bases);
+    ensure<char>(b->seqs, max_bases + SEQ_PAD);
     *out = b;
     return GIS_OK;
     API_END(ctx)

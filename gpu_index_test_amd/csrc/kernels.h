@@ -140,6 +140,9 @@ __host__ __device__ inline uint32_t span_pack(uint32_t start, uint32_t end) { re
 __host__ __device__ inline uint32_t span_start(uint32_t v) { return v & 0xffffu; }
 __host__ __device__ inline uint32_t span_end(uint32_t v) { return v >> 16; }
 
+// bytes of the sequence array past the last read: the seeding loads four
+// bases at a time
+constexpr int SEQ_PAD = 16;
 constexpr int LMAX_LDS = 320;  // reads up to this length seed from LDS
 constexpr int SEED_WPB = 4;    // waves per block of the seeding kernel
 constexpr int WPB = 4;         // waves per block of the per-read kernels

@@ -39,38 +39,87 @@ struct SeedBufs {
     uint64_t *nmask;    // bit i set when base i is not ACGT
 };
 
-// The passes of the syncmer scan after packing: canonical s-mer hashes,
-// window states, tie replay and compaction, k-mer hashes. CLEAN: the read
-// holds only ACGT bases (a wave-uniform fact), so no window needs the N
-// mask and only the read's first window starts a segment.
-template <bool CLEAN>
+// k-mer hashes over a compacted syncmer list (xxh64 of the canonical k-mer)
+__device__ __forceinline__ void syncmer_hashes(uint32_t nh, const SeedParams &P, const SeedBufs &B,
+                                               uint64_t *out_sy_hash) {
+    for (uint32_t i0 = 0; i0 < nh; i0 += 64) {
+        const uint32_t i = i0 + lane_id();
+        if (i < nh) {
+            const uint64_t hk = xxh64_u64(canonical_code(B.pk, (int)B.sy_pos[i], P.k, P.kmask));
+            B.sy_hash[i] = hk;
+            if (out_sy_hash) out_sy_hash[i] = hk;
+        }
+    }
+    wave_sync();
+}
+
+// canonical s-mer hash at base j (step2/randstrobes.cu:23-32); an s-mer of at
+// most 16 bases is a 32-bit code
+__device__ __forceinline__ uint64_t smer_hash(const SeedBufs &B, int j, const SeedParams &P) {
+    return P.s <= 16 ? xxh64_u64((uint64_t)canonical_code32(B.pk, j, P.s, (uint32_t)P.smask))
+                     : xxh64_u64(canonical_code(B.pk, j, P.s, P.smask));
+}
+
+// The syncmer scan of a read without N, from the high words of the s-mer
+// hashes. A window's state is always a position of its minimum (gis_core.h),
+// so the window is a syncmer when the hash at offset t - 1 lies below its
+// other w - 1 hashes and is none when it lies above their minimum, whatever
+// came before. The high words decide both; where they tie (equal s-mers in
+// one window, or a chance of 2^-32 a window) the answer needs the full hashes
+// and the windows before: the scan returns false, and the read takes
+// syncmer_passes.
+__device__ __forceinline__ bool syncmer_fast(int L, const SeedParams &P, const SeedBufs &B, uint32_t cap,
+                                             uint64_t *out_sy_pos, uint32_t &nsync) {
+    const int lane = (int)lane_id();
+    uint32_t *hi = reinterpret_cast<uint32_t *>(B.sh);
+    const int ns = L - P.s + 1;
+    for (int j0 = 0; j0 < ns; j0 += 64) {
+        const int j = j0 + lane;
+        if (j < ns) hi[j] = (uint32_t)(smer_hash(B, j, P) >> 32);
+    }
+    wave_sync();
+    const int nk = L - P.k + 1, mid = P.t - 1;
+    uint32_t n = 0;
+    for (int p0 = 0; p0 < nk; p0 += 64) {
+        const int p = p0 + lane;
+        bool is_sync = false, tie = false;
+        if (p < nk) {
+            const uint32_t h = hi[p + mid];
+            uint32_t m = 0xffffffffu;
+            if (P.w == 5 && mid == 2) {  // every read-length profile up to 375 bp
+                m = min(min(hi[p], hi[p + 1]), min(hi[p + 3], hi[p + 4]));
+            } else {
+                for (int o = 0; o < P.w; o++)
+                    if (o != mid) m = min(m, hi[p + o]);
+            }
+            is_sync = h < m;
+            tie = h == m;
+        }
+        if (__ballot(tie)) return false;
+        const uint64_t bal = __ballot(is_sync);
+        if (is_sync) {
+            const uint32_t idx = n + mbcnt(bal);
+            if (idx < cap) B.sy_pos[idx] = (uint16_t)p;
+            if (out_sy_pos) out_sy_pos[idx] = (uint64_t)p;
+        }
+        n += (uint32_t)__popcll(bal);
+    }
+    wave_sync();
+    nsync = n;
+    return true;
+}
+
+// The passes of the syncmer scan after packing, for any read: canonical s-mer
+// hashes, window states, tie replay and compaction.
 __device__ __forceinline__ uint32_t syncmer_passes(int L, const SeedParams &P, const SeedBufs &B, uint32_t cap,
-                                                   uint64_t *out_sy_hash, uint64_t *out_sy_pos) {
+                                                   uint64_t *out_sy_pos) {
     const int lane = (int)lane_id();
     const int k = P.k, s = P.s, w = P.w;
 
-    // canonical s-mer hashes, one s-mer per lane (step2/randstrobes.cu:23-32);
-    // an s-mer of at most 16 bases is a 32-bit code
     const int ns = L - s + 1;
-    if (s <= 16) {
-        for (int j0 = 0; j0 < ns; j0 += 64) {
-            const int j = j0 + lane;
-            if (j < ns) {
-                uint64_t h = 0;
-                if (CLEAN || !any_n(B.nmask, j, j + s - 1))
-                    h = xxh64_u64((uint64_t)canonical_code32(B.pk, j, s, (uint32_t)P.smask));
-                B.sh[j] = h;
-            }
-        }
-    } else {
-        for (int j0 = 0; j0 < ns; j0 += 64) {
-            const int j = j0 + lane;
-            if (j < ns) {
-                uint64_t h = 0;
-                if (CLEAN || !any_n(B.nmask, j, j + s - 1)) h = xxh64_u64(canonical_code(B.pk, j, s, P.smask));
-                B.sh[j] = h;
-            }
-        }
+    for (int j0 = 0; j0 < ns; j0 += 64) {
+        const int j = j0 + lane;
+        if (j < ns) B.sh[j] = any_n(B.nmask, j, j + s - 1) ? 0 : smer_hash(B, j, P);
     }
     wave_sync();
 
@@ -80,12 +129,10 @@ __device__ __forceinline__ uint32_t syncmer_passes(int L, const SeedParams &P, c
         const int p = p0 + lane;
         if (p < nk) {
             uint8_t st;
-            if (!CLEAN && any_n(B.nmask, p, p + k - 1)) {
+            if (any_n(B.nmask, p, p + k - 1)) {
                 st = ST_INVALID;
             } else {
-                const bool seg_first =
-                    (p == 0) || (!CLEAN && ((B.nmask[(p - 1) >> 6] >> ((p - 1) & 63)) & 1));
-                // w = k - s + 1 is 5 in every read-length profile up to 375 bp
+                const bool seg_first = (p == 0) || ((B.nmask[(p - 1) >> 6] >> ((p - 1) & 63)) & 1);
                 st = w == 5 ? anchor_state_w<5>(B.sh, p, seg_first) : anchor_state(B.sh, p, w, seg_first);
             }
             B.st[p] = st;
@@ -123,55 +170,92 @@ __device__ __forceinline__ uint32_t syncmer_passes(int L, const SeedParams &P, c
         nsync += (uint32_t)__popcll(bal);
     }
     wave_sync();
-
-    // k-mer hashes over the compacted list (xxh64 of the canonical k-mer)
-    const uint32_t nh = nsync < cap ? nsync : cap;
-    for (uint32_t i0 = 0; i0 < nh; i0 += 64) {
-        const uint32_t i = i0 + (uint32_t)lane;
-        if (i < nh) {
-            const uint64_t hk = xxh64_u64(canonical_code(B.pk, (int)B.sy_pos[i], k, P.kmask));
-            B.sy_hash[i] = hk;
-            if (out_sy_hash) out_sy_hash[i] = hk;
-        }
-    }
-    wave_sync();
     return nsync;
+}
+
+// Four bases at once: the 2-bit codes (nt4 of step2/randstrobes.hpp:22-43), one
+// a byte, and in bad the bytes that are not ACGTU in either case (non-zero).
+// Bits 1 and 2 of a folded letter index the four letters; a byte is a base if
+// it is the letter it indexes, or U where that is T.
+__device__ __forceinline__ uint32_t nt4x4(uint32_t v, uint32_t &bad) {
+    const uint32_t u = v & 0xdfdfdfdfu;
+    const uint32_t idx = (u >> 1) & 0x03030303u;  // A 0, C 1, T and U 2, G 3
+    const uint32_t letter = __builtin_amdgcn_perm(0u, 0x47544341u, idx);
+    const uint32_t is2 = (idx >> 1) & ~idx;  // bit 0 of a byte: index 2
+    bad = (u ^ letter) & ~(is2 & 0x01010101u);
+    return idx ^ ((idx >> 1) & 0x01010101u);
+}
+
+// the four bases 4 i .. 4 i + 3 of a read as loaded together (their last bytes
+// may lie past the read's end: the sequence array has SEQ_PAD bytes after the
+// last read), and the mask of those inside it
+__device__ __forceinline__ uint32_t four_bases(const char *__restrict__ seq, int L, int i, uint32_t &inside) {
+    const int left = L - 4 * i;
+    inside = left >= 4 ? 0xffffffffu : left > 0 ? (1u << (8 * left)) - 1u : 0u;
+    uint32_t v = 0;
+    if (left > 0) __builtin_memcpy(&v, seq + 4 * i, 4);
+    return v;
 }
 
 // Canonical syncmers of one read (SyncmerIterator, step2/randstrobes.cu:18-79),
 // the whole wave working on the same read. The first `cap` syncmers go to
 // B.sy_hash/B.sy_pos (and out_sy_* when given); returns the total count.
+//
+// Bound by VALU issue. Two passes over a read's bases carry it: four bases a
+// lane to pack (150 bases in one pass; one base a lane took three passes and
+// two 32-bit spreads each), and the window test on high words, in one pass
+// with the compaction. 65,536 reads of 150 bp: 101 -> 64 us.
 __device__ __forceinline__ uint32_t seed_syncmers(const char *__restrict__ seq, int L,
                                                   const SeedParams &P, const SeedBufs &B,
                                                   uint32_t cap, uint64_t *out_sy_hash,
                                                   uint64_t *out_sy_pos) {
     const int lane = (int)lane_id();
 
-    // 2-bit packed bases and the N mask from three ballots per 64 bases
-    // (step2/randstrobes.cu:21-22, 70-76)
-    int nch = 0;
-    uint64_t nany = 0;
-    for (int b0 = 0; b0 < L; b0 += 64, nch++) {
-        const int i = b0 + lane;
-        int c = 4;
-        if (i < L) c = nt4((unsigned char)seq[i]);
-        const bool ok = i < L && c < 4;
-        const uint64_t lo = __ballot(ok && (c & 1));
-        const uint64_t hi = __ballot(ok && (c & 2));
-        const uint64_t m = __ballot(i < L && c > 3);
-        nany |= m;
-        if (lane == 0) {
-            B.nmask[b0 >> 6] = m;
-            B.pk[2 * nch] = spread32((uint32_t)lo) | (spread32((uint32_t)hi) << 1);
-        } else if (lane == 1) {
-            B.pk[2 * nch + 1] = spread32((uint32_t)(lo >> 32)) | (spread32((uint32_t)(hi >> 32)) << 1);
-        }
+    // bases packed 2 bits each, four a lane and so 256 a pass: a lane's four
+    // codes are one byte of the packed array. The array is written up to its
+    // pad word, which windows ending in the last word read.
+    const int nch = (L + 63) >> 6, nbytes = 8 * (2 * nch + 1);
+    uint8_t *pkb = reinterpret_cast<uint8_t *>(B.pk);
+    uint32_t any = 0;
+    for (int i0 = 0; i0 < nbytes; i0 += 64) {
+        const int i = i0 + lane;
+        uint32_t inside, bad;
+        const uint32_t v = four_bases(seq, L, i, inside);
+        const uint32_t c = nt4x4(v, bad) & inside;
+        any |= bad & inside;
+        // c0 + 4 c1 + 16 c2 + 64 c3
+        if (i < nbytes) pkb[i] = (uint8_t)__builtin_amdgcn_udot4(c, 0x40100401u, 0u, false);
     }
-    if (lane == 0) B.pk[2 * nch] = 0;  // pad word read by windows ending in the last word
     wave_sync();
-    // the ballots are wave-uniform, so this branch is too
-    return nany == 0 ? syncmer_passes<true>(L, P, B, cap, out_sy_hash, out_sy_pos)
-                     : syncmer_passes<false>(L, P, B, cap, out_sy_hash, out_sy_pos);
+    uint32_t nsync = 0;
+    const bool clean = __ballot(any != 0) == 0;  // wave-uniform
+    if (!(clean && syncmer_fast(L, P, B, cap, out_sy_pos, nsync))) {
+        // the mask of non-ACGT bases (step2/randstrobes.cu:70-76): bit 4 l + b
+        // of 16 lanes' words from the ballots of their byte b
+        for (int i0 = 0; 4 * i0 < L; i0 += 64) {
+            uint32_t inside, bad;
+            const uint32_t v = four_bases(seq, L, i0 + lane, inside);
+            (void)nt4x4(v, bad);
+            bad &= inside;
+            uint64_t m = 0;
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const uint64_t bal = __ballot(((bad >> (8 * q)) & 0xffu) != 0);
+                uint64_t x = lane < 4 ? (bal >> (16 * lane)) & 0xffffull : 0ull;
+                x = (x | (x << 24)) & 0x000000ff000000ffull;
+                x = (x | (x << 12)) & 0x000f000f000f000full;
+                x = (x | (x << 6)) & 0x0303030303030303ull;
+                x = (x | (x << 3)) & 0x1111111111111111ull;
+                m |= x << q;
+            }
+            const int word = i0 / 16 + lane;
+            if (lane < 4 && word < nch) B.nmask[word] = m;
+        }
+        wave_sync();
+        nsync = syncmer_passes(L, P, B, cap, out_sy_pos);
+    }
+    syncmer_hashes(nsync < cap ? nsync : cap, P, B, out_sy_hash);
+    return nsync;
 }
 
 // Randstrobe number j of a read's query list in randstrobes_query order

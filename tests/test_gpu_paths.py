@@ -41,3 +41,43 @@ def test_bucket_lines_of_every_size(ctx, bits):
         assert nams.tobytes() == enams.tobytes()
     idx.ctx.close()
 
+
+
+@pytest.mark.parametrize("profile", [150, 300, 400])
+def test_seeding_pass_edges(ctx, profile):
+    """Read lengths around the seeding's pass sizes (4, 64, 256 bases, the
+    320-base LDS limit), at every alignment of a read's first byte, with every
+    kind of byte (either case, U, IUPAC codes, bytes outside ASCII) and
+    windows with equal s-mers, through randstrobes_query."""
+    rng = np.random.default_rng(profile)
+    acgt = np.frombuffer(b"ACGT", dtype=np.uint8)
+    reads = []
+    for L in list(range(0, 26)) + [62, 63, 64, 65, 127, 128, 129, 150, 151, 252, 253, 254, 255, 256, 257, 258, 259,
+                                   260, 318, 319, 320, 321, 322, 511, 512, 513, 767, 1025]:
+        r = acgt[rng.integers(0, 4, L)]
+        reads.append(r)
+        for byte in (b"N", b"U", b"u", b"t", b"a", b"M", b"!", b"\x00", b"\xc1", b"\xff", b"3", b"\x14"):
+            if L:
+                x = r.copy()
+                x[rng.integers(0, L, 1 + L // 200)] = byte[0]
+                reads.append(x)
+        if L > 40:  # a tandem of period 1 .. 7: tied windows
+            x = r.copy()
+            u = r[: 1 + L % 7]
+            x[5:40] = np.resize(u, 35)
+            reads.append(x)
+    p = G.IndexParameters.from_read_length(profile)
+    op = O.params_from_read_length(profile)
+    ents = [(h, 10 * i, 5) for i, h in enumerate(rng.integers(1, 2 ** 63, 50).tolist())]
+    arr, starts = tiny_index_arrays(ents)
+    idx = G.StrobemerIndex(None, p)
+    idx.upload(arr, starts, 8, 30)
+    s, o, l = G.pack_reads([r.tobytes() for r in reads])
+    off, q = G.randstrobes_batch(idx, s, o, l)
+    soff, sy = G.syncmers_batch(idx, s, o, l)
+    for i, r in enumerate(reads):
+        e = O.randstrobes_query(r.tobytes(), op)
+        assert q[int(off[i]): int(off[i + 1])].tobytes() == e.tobytes(), (i, len(r))
+        e = O.syncmers(r.tobytes(), op)
+        assert sy[int(soff[i]): int(soff[i + 1])].tobytes() == e.tobytes(), (i, len(r))
+    idx.ctx.close()
