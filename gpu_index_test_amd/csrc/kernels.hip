@@ -668,8 +668,6 @@ __device__ __forceinline__ void probe_finish(const DevIndex &ix, Probe &p, int q
         if (!p.found) return;
         p.filtered = eq > ix.filter_cutoff ||
                      (p.key == UINT64_MAX && p.pos + ix.filter_cutoff >= ix.n);
-        if (p.filtered) return;
-        p.run = eq;
         const int qspan = qe - qs;
         int min_diff = 0x7fffffff;
 #pragma unroll
@@ -684,6 +682,9 @@ __device__ __forceinline__ void probe_finish(const DevIndex &ix, Probe &p, int q
                 }
             }
         }
+        // a filtered seed has no hits, but a rescued read may still take its run
+        p.hc = p.filtered ? 0u : p.hc;
+        p.run = p.filtered ? 0u : eq;
         return;
     }
     p.pos = p.e - p.s < 0xffffffffull ? dev_find_in(ix, p.key, p.s, p.e, &p.scan) : dev_find(ix, p.key, &p.scan);

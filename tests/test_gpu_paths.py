@@ -81,3 +81,23 @@ def test_seeding_pass_edges(ctx, profile):
         e = O.syncmers(r.tobytes(), op)
         assert sy[int(soff[i]): int(soff[i + 1])].tobytes() == e.tobytes(), (i, len(r))
     idx.ctx.close()
+
+
+@pytest.mark.parametrize("mode", [G.MODE_PLAIN, G.MODE_FUSED])
+def test_filter_cutoff_inside_a_bucket_line(ctx, mode):
+    """A filter cutoff below seven filters runs that fit a bucket's line; a
+    rescued read takes them all the same (count <= hard cutoff)."""
+    g, lens = G.synth_genome(200_000, n_contigs=2, gc=0.45, repeat_fraction=0.5, n_families=12,
+                             family_len=(400, 1500), copies=(2, 12), divergence=(0.0, 0.005), seed=3)
+    op = O.params_from_read_length(150)
+    built = O.Index.build_arrays(g, lens, op, n_threads=4)
+    oidx = O.Index.wrap(built.randstrobes, built.starts, built.bits, 2, op)
+    idx = G.StrobemerIndex(None, G.IndexParameters.from_read_length(150))
+    idx.upload(built.randstrobes, built.starts, built.bits, 2)
+    s, o, l, _ = G.synth_reads(g, lens, 600, lengths=(100, 150, 250), weights=(1, 1, 1), sub_rate=0.005, seed=4)
+    res = G.find_nams_batch(idx, s, o, l, mode=mode)
+    eo, en, ef, efl = O.map_batch(oidx, s, o, l, 2 * 2, 1000, 4)
+    assert (efl & 1).sum() > 50
+    assert np.array_equal(res.nam_offsets, eo) and res.nams.tobytes() == en.tobytes()
+    assert res.nonrepetitive_fraction.tobytes() == ef.tobytes() and np.array_equal(res.flags & 1, efl & 1)
+    idx.ctx.close()
