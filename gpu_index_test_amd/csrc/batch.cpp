@@ -234,7 +234,9 @@ void ensure_pools(gis_batch *b, uint64_t hit_cap, uint64_t rhit_cap, uint64_t ou
         ensure<WideNam>(b->ws->nam_ws, b->ws->hit_cap);
         ensure<uint64_t>(b->ws->rkeys, 2 * b->ws->rhit_cap);
         ensure<WideNam>(b->ws->rnam_ws, b->ws->rhit_cap);
-        ensure<uint4>(b->ws->gwork, std::max(b->ws->hit_cap, b->ws->rhit_cap) + 64);
+        // a split read of h > SPLIT_MIN hits has at most h / ITEM_HITS + 1 work
+        // items, fewer than h / 128
+        ensure<uint4>(b->ws->gwork, (b->ws->hit_cap + b->ws->rhit_cap) / 128 + 64);
     }
     ensure<gis_nam>(b->ws->nams_out, b->ws->out_cap);
 }
@@ -349,10 +351,10 @@ void enqueue_run(gis_batch *b, int mode, int rescue_mode, uint32_t rcut, uint32_
     b->n_ev = 0;
     b->ev_names.clear();
     mark(b, "start");
-    launch_reset_ctl(d.ctl, st);
     ReadSet set{nullptr, nullptr, n};
     const bool fused = mode == GIS_MODE_FUSED && stop == STOP_NONE;
     if (fused) {
+        launch_reset_ctl(d.ctl, st);
         const gis_fused_config &fc = ctx->fcfg;
         const unsigned grid = fc.blocks_per_cu > 0 ? (unsigned)(ctx->n_cu * fc.blocks_per_cu) : 0u;
         const uint32_t chunk = fc.queue ? (uint32_t)fc.chunk : 0u;
@@ -371,28 +373,22 @@ void enqueue_run(gis_batch *b, int mode, int rescue_mode, uint32_t rcut, uint32_
         mark(b, "fused");
         set = ReadSet{d.spill_ids, &d.ctl->n_spill, n};
     }
-    launch_seed(d, set, sp, b->want_sy ? 1 : 0, b->any_long ? 1 : 0, st);
+    launch_seed(d, set, sp, b->want_sy ? 1 : 0, b->any_long ? 1 : 0, fused ? 0 : 1, st);
     mark(b, "seed");
     if (stop != STOP_SEED) {
         launch_lookup(d, set, ix, rescue_mode, st);
         mark(b, "lookup");
-        launch_hits(d, set, ix, st);
+        launch_hits(d, ix, rcut, hard, st);
         mark(b, "hits");
-        launch_rescue_count(d, set, ix, rcut, hard, st);
-        launch_scan(d.rhit_total, d.rhit_off, n, tmp, st);
-        launch_rescue_hits(d, set, ix, st);
-        mark(b, "rescue");
     }
     if (stop == STOP_NONE) {
-        launch_merge(d, set, 0, st);
+        launch_merge(d, set, st);
         mark(b, "merge");
-        launch_merge(d, set, 1, st);
-        mark(b, "rescue_merge");
-        launch_scan(d.nam_cnt, d.nam_off, n, tmp, st);
-        launch_compact(d, fused ? 1 : 0, st);
+        launch_output(d, fused ? 1 : 0, tmp, b->ws->h_ctl_dev, st);
         mark(b, "output");
+    } else {
+        launch_ctl_to_host(d, b->ws->h_ctl_dev, st);
     }
-    launch_ctl_to_host(d.ctl, b->ws->h_ctl_dev, st);
 }
 
 // size the workspace for this batch's reads (grow-only; cheap when it
@@ -710,20 +706,23 @@ static int copy_hits_out(gis_ctx *ctx, gis_batch *b, uint64_t *out_offsets, gis_
                          uint64_t capacity, uint64_t *n_out) {
     const uint32_t n = b->n_reads;
     std::vector<uint8_t> flags(n);
-    std::vector<uint64_t> ho(n + 1), rho(n + 1);
-    std::vector<uint32_t> hcount(n);
-    if (n) HIP_CHECK(hipMemcpy(flags.data(), b->ws->flags.p, n, hipMemcpyDeviceToHost));
-    if (n) HIP_CHECK(hipMemcpy(hcount.data(), b->ws->hit_total.p, 4ull * n, hipMemcpyDeviceToHost));
-    HIP_CHECK(hipMemcpy(ho.data(), b->ws->hit_off.p, 8ull * (n + 1), hipMemcpyDeviceToHost));
-    HIP_CHECK(hipMemcpy(rho.data(), b->ws->rhit_off.p, 8ull * (n + 1), hipMemcpyDeviceToHost));
-    std::vector<DevHit> h(ho[n]), rh(rho[n]);
-    if (ho[n]) HIP_CHECK(hipMemcpy(h.data(), b->ws->hits.p, sizeof(DevHit) * ho[n], hipMemcpyDeviceToHost));
-    if (rho[n]) HIP_CHECK(hipMemcpy(rh.data(), b->ws->rhits.p, sizeof(DevHit) * rho[n], hipMemcpyDeviceToHost));
+    std::vector<uint64_t> ho(n), rho(n);
+    std::vector<uint32_t> hcount(n), rcount(n);
+    if (n) {
+        HIP_CHECK(hipMemcpy(flags.data(), b->ws->flags.p, n, hipMemcpyDeviceToHost));
+        HIP_CHECK(hipMemcpy(hcount.data(), b->ws->hit_total.p, 4ull * n, hipMemcpyDeviceToHost));
+        HIP_CHECK(hipMemcpy(rcount.data(), b->ws->rhit_total.p, 4ull * n, hipMemcpyDeviceToHost));
+        HIP_CHECK(hipMemcpy(ho.data(), b->ws->hit_off.p, 8ull * n, hipMemcpyDeviceToHost));
+        HIP_CHECK(hipMemcpy(rho.data(), b->ws->rhit_off.p, 8ull * n, hipMemcpyDeviceToHost));
+    }
+    const uint64_t nh = n ? b->ws->h_ctl->tot[0] : 0, nrh = n ? b->ws->h_ctl->tot[1] : 0;
+    std::vector<DevHit> h(nh), rh(nrh);
+    if (nh) HIP_CHECK(hipMemcpy(h.data(), b->ws->hits.p, sizeof(DevHit) * nh, hipMemcpyDeviceToHost));
+    if (nrh) HIP_CHECK(hipMemcpy(rh.data(), b->ws->rhits.p, sizeof(DevHit) * nrh, hipMemcpyDeviceToHost));
     uint64_t total = 0;
     // a read's hits: its region or pool place (hit_off) and count (hit_total);
-    // rescued reads: the scan-placed rescue array
-    for (uint32_t r = 0; r < n; r++)
-        total += (flags[r] & GIS_FLAG_RESCUED) ? rho[r + 1] - rho[r] : hcount[r];
+    // rescued reads: their place in the rescue array
+    for (uint32_t r = 0; r < n; r++) total += (flags[r] & GIS_FLAG_RESCUED) ? rcount[r] : hcount[r];
     if (n_out) *n_out = total;
     if (total > capacity || (total && !out)) return fail(ctx, GIS_ERR_CAPACITY, "hit capacity too small");
     uint64_t o = 0;
@@ -732,7 +731,7 @@ static int copy_hits_out(gis_ctx *ctx, gis_batch *b, uint64_t *out_offsets, gis_
         if (out_offsets) out_offsets[r] = o;
         const bool resc = (flags[r] & GIS_FLAG_RESCUED) != 0;
         const std::vector<DevHit> &src = resc ? rh : h;
-        const uint64_t lo = resc ? rho[r] : ho[r], hi = resc ? rho[r + 1] : ho[r] + hcount[r];
+        const uint64_t lo = resc ? rho[r] : ho[r], hi = lo + (resc ? rcount[r] : hcount[r]);
         // group by (strand, ref) keeping the emission order inside a group
         idx.clear();
         for (uint64_t i = lo; i < hi; i++) idx.push_back(((uint64_t)src[i].ref_strand << 32) | (i - lo));
@@ -849,15 +848,9 @@ static int qrs_run(gis_ctx *ctx, const gis_query_randstrobe *qrs, const uint64_t
         const DevBatch d = make_devbatch(b);
         launch_reset_ctl(d.ctl, st);
         launch_lookup(d, set, ix, rescue ? 2 : 1, st);
-        launch_hits(d, set, ix, st);
-        launch_rescue_count(d, set, ix, rescue_cutoff, hard_cutoff, st);
-        launch_scan(d.rhit_total, d.rhit_off, n, tmp, st);
-        launch_rescue_hits(d, set, ix, st);
-        launch_merge(d, set, 0, st);
-        launch_merge(d, set, 1, st);
-        launch_scan(d.nam_cnt, d.nam_off, n, tmp, st);
-        launch_compact(d, 0, st);
-        launch_ctl_to_host(d.ctl, b->ws->h_ctl_dev, st);
+        launch_hits(d, ix, rescue_cutoff, hard_cutoff, st);
+        launch_merge(d, set, st);
+        launch_output(d, 0, tmp, b->ws->h_ctl_dev, st);
         HIP_CHECK(hipGetLastError());
         HIP_CHECK(hipStreamSynchronize(st));
         b->ws->tot_nams = b->ws->h_ctl->tot[2];

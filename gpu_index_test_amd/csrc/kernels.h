@@ -49,10 +49,12 @@ struct DevCtl {
     unsigned int n_spill;   // reads handed from the fused kernel to the per-stage kernels
     unsigned int overflow;  // OVF_* bits
     unsigned int q_head[2]; // dynamic work-queue heads of the fused kernel's two bins
-    unsigned int n_gwork[2];  // group work items of split reads (normal, rescue merge)
-    unsigned int n_split[2];  // split reads (normal, rescue merge)
+    unsigned int n_gwork;     // group work items of split reads
+    unsigned int n_split;     // split reads
     unsigned int n_sel[3];    // selected reads: rescued, deferred merges, pooled hits
-    unsigned long long hit_pool;  // hits placed in the pool after the per-read regions
+    unsigned int pad_;
+    unsigned long long hit_pool;   // hits placed in the pool after the per-read regions
+    unsigned long long rhit_pool;  // hits of rescued reads
     // totals the host reads with this block: end of the hit pool, rescue
     // hits, NAMs
     unsigned long long tot[3];
@@ -101,10 +103,9 @@ struct DevBatch {
     float *frac;
     uint8_t *flags;
     uint32_t *nam_cnt;
-    uint64_t *hit_off;        // [n+1] the read's hits start here: its own region r * HIT_REGION, or
-                              // (more hits than that) a place in the pool after the regions;
-                              // hit_off[n] = end of the pool
-    uint64_t *rhit_off;       // [n+1] scan of rhit_total
+    uint64_t *hit_off;        // [n] the read's hits start here: its own region r * HIT_REGION, or
+                              // (more hits than that) a place in the pool after the regions
+    uint64_t *rhit_off;       // [n] rescued reads: their hits' place in rhits
     // hit arrays (capacity hit_cap / rhit_cap hits); merge scratch per read r
     // with h hits at hit offset o: keys[2o .. 2o+2h), nam_ws[o .. o+h)
     DevHit *hits;
@@ -159,25 +160,30 @@ constexpr uint32_t BUCKET_LINE = 8;  // uint4 per bucket line
 // launch wrappers (kernels.hip)
 void launch_bucket_lines(const uint4 *rs, const uint64_t *starts, int bits, uint4 *lines, hipStream_t st);
 void launch_reset_ctl(DevCtl *ctl, hipStream_t st);
+// reset: the control block is cleared by the first launch (the seeding does not
+// use it), instead of a launch of its own
 void launch_seed(const DevBatch &b, const ReadSet &set, const SeedParams &sp, int want_syncmers,
-                 int long_reads, hipStream_t st);
+                 int long_reads, int reset, hipStream_t st);
 // rescue_mode: 0 = the caller's decision (nonrepetitive fraction < 0.7 or no
 // hits), 1 = never rescue, 2 = always rescue
 void launch_lookup(const DevBatch &b, const ReadSet &set, const DevIndex &ix, int rescue_mode,
                    hipStream_t st);
-void launch_hits(const DevBatch &b, const ReadSet &set, const DevIndex &ix, hipStream_t st);
-void launch_rescue_count(const DevBatch &b, const ReadSet &set, const DevIndex &ix,
-                         uint32_t rescue_cutoff, uint32_t hard_cutoff, hipStream_t st);
-void launch_rescue_hits(const DevBatch &b, const ReadSet &set, const DevIndex &ix, hipStream_t st);
-void launch_merge(const DevBatch &b, const ReadSet &set, int rescue, hipStream_t st);
+// the hits of the reads the lookup listed: those beyond their region, and those
+// of rescued reads
+void launch_hits(const DevBatch &b, const DevIndex &ix, uint32_t rescue_cutoff, uint32_t hard_cutoff,
+                 hipStream_t st);
+void launch_merge(const DevBatch &b, const ReadSet &set, hipStream_t st);
 // fused kernel over queue[0 .. count); lmax in {160, 320}, wpb in {2, 4, 8};
 // returns false for an unsupported combination
 bool launch_fused(const DevBatch &b, const DevIndex &ix, const SeedParams &sp, uint32_t rescue_cutoff,
                   uint32_t hard_cutoff, const uint32_t *queue, uint32_t count, int lmax, int wpb,
                   unsigned grid, uint32_t chunk, unsigned int *head, hipStream_t st);
-void launch_compact(const DevBatch &b, int fused, hipStream_t st);
-// the control block to pinned host memory (dst: the device's address of it)
-void launch_ctl_to_host(const DevCtl *src, DevCtl *dst, hipStream_t st);
+// NAM offsets and the dense output, and the control block with its totals to
+// pinned host memory (dst: the device's address of it); tmp holds
+// scan_tmp_words(n) u64
+void launch_output(const DevBatch &b, int fused, uint64_t *tmp, DevCtl *dst, hipStream_t st);
+// the control block to pinned host memory after a run that stops before the output
+void launch_ctl_to_host(const DevBatch &b, DevCtl *dst, hipStream_t st);
 void launch_find_flat(const DevIndex &ix, const uint64_t *hashes, uint64_t n, uint64_t *positions,
                       hipStream_t st);
 // exclusive scan of u32 counts into u64 offsets[n+1] (offsets[n] = total);

@@ -8,12 +8,15 @@
 // never changes a read's result.
 //
 // Two forms share the device functions below:
-//  - per-stage: k_seed -> k_lookup -> k_hits -> k_rescue_count ->
-//    k_rescue_hits -> k_merge (normal, rescue), one launch per stage;
+//  - per-stage: k_seed -> k_lookup -> k_hits (reads with many hits, rescued
+//    reads) -> k_merge4 -> k_merge -> k_scan_tiles -> k_compact;
 //  - fused: k_fused runs the whole path of a read in one wave out of LDS and
 //    hands reads that do not fit its LDS budget (long reads, many seeds,
 //    many hits) to the per-stage kernels through the spill list.
-// Both end in a scan of the per-read NAM counts and k_compact.
+// Both end in a scan of the per-read NAM counts and k_compact. A launch that
+// finds nothing to do still takes ~4.5 us of a batch's run, so the passes over
+// few reads share launches, and lists of reads are appended by the kernels that
+// decide them.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -22,6 +25,11 @@
 #include "wave.h"
 
 namespace gis {
+
+// Lists of reads for the passes over few of them, in DevBatch::sel_ids:
+// rescued reads, reads the four-per-wave merge hands on, and reads whose hits
+// go to the pool
+enum { SEL_RESCUED = 0, SEL_DEFERRED = 1, SEL_POOLED = 2 };
 
 // wave-uniform iteration over a ReadSet
 __device__ __forceinline__ uint32_t set_count(const ReadSet &s) { return s.ids ? *s.n_dev : s.n; }
@@ -375,10 +383,17 @@ __device__ __forceinline__ void pin_k20_profile(SeedParams &P) {
 
 static inline bool is_k20_profile(const SeedParams &sp) { return sp.k == 20 && sp.s == 16 && sp.t == 3; }
 
+// the control block cleared by the first threads of one block
+static_assert(sizeof(DevCtl) % 4 == 0 && sizeof(DevCtl) / 4 <= 64, "one word per lane");
+__device__ __forceinline__ void ctl_clear(DevCtl *ctl) {
+    if (threadIdx.x < sizeof(DevCtl) / 4) reinterpret_cast<unsigned *>(ctl)[threadIdx.x] = 0;
+}
+
 template <bool LONG, bool K20>
 __global__ __launch_bounds__(64 * SEED_WPB) __attribute__((amdgpu_waves_per_eu(6))) void k_seed(DevBatch b, ReadSet set, SeedParams P,
-                                                        int want_sy) {
+                                                        int want_sy, int reset) {
     if (K20) pin_k20_profile(P);
+    if (reset && blockIdx.x == 0) ctl_clear(b.ctl);
     __shared__ SeedLds lds[LONG ? 1 : SEED_WPB];
     const int wid = (int)uni32(threadIdx.x >> 6);
     const uint32_t cnt = set_count(set);
@@ -826,53 +841,31 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(6))) v
             uint64_t off = (uint64_t)r * HIT_REGION;
             if (pooled) {
                 off = (uint64_t)b.n_reads * HIT_REGION + atomicAdd(&b.ctl->hit_pool, (unsigned long long)hits);
-                b.sel_ids[2ull * b.n_reads + atomicAdd(&b.ctl->n_sel[2], 1u)] = r;
+                b.sel_ids[2ull * b.n_reads + atomicAdd(&b.ctl->n_sel[SEL_POOLED], 1u)] = r;
             }
             b.hit_off[r] = off;
+            if (rescue) b.sel_ids[atomicAdd(&b.ctl->n_sel[SEL_RESCUED], 1u)] = r;
         }
     }
 }
 
-// end of the hit pool, for the capacity checks of the kernels that follow
-__global__ void k_pool_total(DevBatch b) {
-    if (threadIdx.x == 0) {
-        const uint64_t end = (uint64_t)b.n_reads * HIT_REGION + b.ctl->hit_pool;
-        b.hit_off[b.n_reads] = end;
-        b.ctl->tot[0] = end;
-    }
-}
-
-// write the hits of the reads whose hits did not fit their region into the
-// pool (same walk as k_lookup); runs over the pooled reads' list
-// capacity check of a hit array against the scan total (wave-uniform)
-__device__ __forceinline__ bool over_capacity(const uint64_t *off, uint32_t n, uint64_t cap,
-                                              DevCtl *ctl, unsigned bit) {
-    if (off[n] <= cap) return false;
-    if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&ctl->overflow, bit);
-    return true;
-}
-
-__global__ __launch_bounds__(64 * WPB) void k_hits(DevBatch b, ReadSet set, DevIndex ix) {
+// the hits of a read that did not fit its region, into the pool (same walk as
+// k_lookup)
+__device__ __forceinline__ void pooled_hits(const DevBatch &b, const DevIndex &ix, uint32_t r) {
     const uint32_t lane = lane_id();
-    if (over_capacity(b.hit_off, b.n_reads, b.hit_cap, b.ctl, OVF_HITS)) return;
-    const uint32_t cnt = set_count(set);
-    for (uint32_t w = wave_index(WPB); w < cnt; w += gridDim.x * WPB) {
-        const uint32_t r = set.ids ? sload(set.ids + w) : w;
-        if (sload(b.hit_total + r) == 0) continue;
-        const uint32_t n = sload(b.rs_cnt + r);
-        const uint64_t base = sload(b.rs_off + r);
-        const uint32_t half = sload(b.rs_nfwd + r);
-        DevHit *out = b.hits + sload(b.hit_off + r);
-        uint32_t carry = 0;
-        for (uint32_t i0 = 0; i0 < n; i0 += 64) {
-            const uint32_t i = i0 + lane;
-            const uint32_t hc = i < n ? b.hcnt[base + i] : 0u;
-            const uint32_t ex = wave_excl_scan(hc);
-            if (hc > 0)
-                walk_run(ix, b.pos[base + i], b.rs_hash[base + i], (int)span_start(b.rs_span[base + i]),
-                         (int)span_end(b.rs_span[base + i]), i >= half ? 0x80000000u : 0u, out + carry + ex);
-            carry += wave_sum(hc);
-        }
+    const uint32_t n = sload(b.rs_cnt + r);
+    const uint64_t base = sload(b.rs_off + r);
+    const uint32_t half = sload(b.rs_nfwd + r);
+    DevHit *out = b.hits + sload(b.hit_off + r);
+    uint32_t carry = 0;
+    for (uint32_t i0 = 0; i0 < n; i0 += 64) {
+        const uint32_t i = i0 + lane;
+        const uint32_t hc = i < n ? b.hcnt[base + i] : 0u;
+        const uint32_t incl = wave_incl_scan_dpp(hc);
+        if (hc > 0)
+            walk_run(ix, b.pos[base + i], b.rs_hash[base + i], (int)span_start(b.rs_span[base + i]),
+                     (int)span_end(b.rs_span[base + i]), i >= half ? 0x80000000u : 0u, out + carry + incl - hc);
+        carry += readlane_u32(incl, 63);
     }
 }
 
@@ -890,107 +883,120 @@ __device__ __forceinline__ bool rh_less(uint32_t ca, uint32_t qa, uint32_t ea, u
     return ca < cb || (ca == cb && (qa < qb || (qa == qb && ea < eb)));
 }
 
-__global__ __launch_bounds__(64 * WPB) void k_rescue_count(DevBatch b, ReadSet set, DevIndex ix,
-                                                           uint32_t rescue_cutoff,
-                                                           uint32_t hard_cutoff) {
+// The rescue of one read: counts of its seeds, the taken ones' hits, a place
+// for them in rhits (one atomic per read), and the hits. A read whose hits do
+// not fit rhits is left out (the host grows it to rhit_pool and runs again).
+__device__ __forceinline__ void rescued_hits(const DevBatch &b, const DevIndex &ix, uint32_t r,
+                                             uint32_t rescue_cutoff, uint32_t hard_cutoff) {
     const uint32_t lane = lane_id();
-    const uint32_t cnt = set_count(set);
-    for (uint32_t w = wave_index(WPB); w < cnt; w += gridDim.x * WPB) {
-        const uint32_t r = set.ids ? sload(set.ids + w) : w;
-        if (!(sload(b.flags + r) & GIS_FLAG_RESCUED)) continue;
-        const uint32_t n = sload(b.rs_cnt + r);
-        const uint64_t base = sload(b.rs_off + r);
-        const uint32_t half = sload(b.rs_nfwd + r);
-        for (uint32_t i0 = 0; i0 < n; i0 += 64) {
-            const uint32_t i = i0 + lane;
-            if (i < n) {
-                const uint64_t pos = b.pos[base + i];
-                b.hcnt[base + i] = pos != GIS_NOT_FOUND ? dev_get_count(ix, pos) : 0u;
-            }
+    const uint32_t n = sload(b.rs_cnt + r);
+    const uint64_t base = sload(b.rs_off + r);
+    const uint32_t half = sload(b.rs_nfwd + r);
+    for (uint32_t i0 = 0; i0 < n; i0 += 64) {
+        const uint32_t i = i0 + lane;
+        if (i < n) {
+            const uint64_t pos = b.pos[base + i];
+            b.hcnt[base + i] = pos != GIS_NOT_FOUND ? dev_get_count(ix, pos) : 0u;
         }
-        wave_sync_mem();
-        uint32_t total = 0;
-        for (uint32_t i0 = 0; i0 < n; i0 += 64) {
-            const uint32_t i = i0 + lane;
-            uint32_t rh = 0;
-            bool coop = false;
-            if (i < n) {
-                const uint32_t c = b.hcnt[base + i];
-                bool taken = false;
-                if (c > 0 && c <= hard_cutoff) {
-                    taken = c <= rescue_cutoff;
-                    if (!taken) {
-                        const uint32_t lo = i < half ? 0 : half, hi = i < half ? half : n;
-                        const uint32_t sp = b.rs_span[base + i], qs = span_start(sp), qe = span_end(sp);
-                        uint32_t rank = 0;
-                        for (uint32_t j = lo; j < hi && rank < 5; j++) {
-                            const uint32_t cj = b.hcnt[base + j];
-                            if (cj == 0) continue;
-                            const uint32_t spj = b.rs_span[base + j];
-                            rank += rh_less(cj, span_start(spj), span_end(spj), c, qs, qe) ? 1u : 0u;
-                        }
-                        taken = rank < 5;
+    }
+    wave_sync_mem();
+    uint32_t total = 0;
+    for (uint32_t i0 = 0; i0 < n; i0 += 64) {
+        const uint32_t i = i0 + lane;
+        uint32_t rh = 0;
+        bool coop = false;
+        if (i < n) {
+            const uint32_t c = b.hcnt[base + i];
+            bool taken = false;
+            if (c > 0 && c <= hard_cutoff) {
+                taken = c <= rescue_cutoff;
+                if (!taken) {
+                    const uint32_t lo = i < half ? 0 : half, hi = i < half ? half : n;
+                    const uint32_t sp = b.rs_span[base + i], qs = span_start(sp), qe = span_end(sp);
+                    uint32_t rank = 0;
+                    for (uint32_t j = lo; j < hi && rank < 5; j++) {
+                        const uint32_t cj = b.hcnt[base + j];
+                        if (cj == 0) continue;
+                        const uint32_t spj = b.rs_span[base + j];
+                        rank += rh_less(cj, span_start(spj), span_end(spj), c, qs, qe) ? 1u : 0u;
                     }
+                    taken = rank < 5;
                 }
-                if (taken && c <= WALK_WAVE_MIN)
-                    rh = walk_run(ix, b.pos[base + i], b.rs_hash[base + i], (int)span_start(b.rs_span[base + i]),
-                                  (int)span_end(b.rs_span[base + i]), 0u, nullptr);
-                coop = taken && c > WALK_WAVE_MIN;
             }
-            // long runs: the whole wave walks each one
-            uint64_t cm = __ballot(coop);
-            while (cm) {
-                const uint32_t l = (uint32_t)__builtin_ctzll(cm);
-                cm &= cm - 1;
-                const uint64_t xl = base + i0 + l;
-                const uint32_t k = walk_run_wave(ix, b.pos[xl], b.rs_hash[xl], (int)span_start(b.rs_span[xl]),
-                                                 (int)span_end(b.rs_span[xl]), 0u, nullptr);
-                if (lane == l) rh = k;
-            }
-            if (i < n) b.rcnt[base + i] = rh;
-            total += wave_sum(rh);
+            if (taken && c <= WALK_WAVE_MIN)
+                rh = walk_run(ix, b.pos[base + i], b.rs_hash[base + i], (int)span_start(b.rs_span[base + i]),
+                              (int)span_end(b.rs_span[base + i]), 0u, nullptr);
+            coop = taken && c > WALK_WAVE_MIN;
         }
-        if (lane == 0) b.rhit_total[r] = total;
+        // long runs: the whole wave walks each one
+        uint64_t cm = __ballot(coop);
+        while (cm) {
+            const uint32_t l = (uint32_t)__builtin_ctzll(cm);
+            cm &= cm - 1;
+            const uint64_t xl = base + i0 + l;
+            const uint32_t k = walk_run_wave(ix, b.pos[xl], b.rs_hash[xl], (int)span_start(b.rs_span[xl]),
+                                             (int)span_end(b.rs_span[xl]), 0u, nullptr);
+            if (lane == l) rh = k;
+        }
+        if (i < n) b.rcnt[base + i] = rh;
+        total += wave_sum_dpp(rh);
+    }
+    unsigned long long off = 0;
+    if (lane == 0) {
+        off = atomicAdd(&b.ctl->rhit_pool, (unsigned long long)total);
+        b.rhit_total[r] = total;
+        b.rhit_off[r] = off;
+    }
+    off = uni64(off);
+    if (off + total > b.rhit_cap) {
+        if (lane == 0) atomicOr(&b.ctl->overflow, OVF_RHITS);
+        return;
+    }
+    if (total == 0) return;
+    wave_sync_mem();
+    DevHit *out = b.rhits + off;
+    uint32_t carry = 0;
+    for (uint32_t i0 = 0; i0 < n; i0 += 64) {
+        const uint32_t i = i0 + lane;
+        const uint32_t rh = i < n ? b.rcnt[base + i] : 0u;
+        // runs longer than WALK_WAVE_MIN take the wave walk, as above
+        const bool coop = rh > 0 && b.hcnt[base + i] > WALK_WAVE_MIN;
+        const uint32_t incl = wave_incl_scan_dpp(rh);
+        if (rh > 0 && !coop)
+            walk_run(ix, b.pos[base + i], b.rs_hash[base + i], (int)span_start(b.rs_span[base + i]),
+                     (int)span_end(b.rs_span[base + i]), i >= half ? 0x80000000u : 0u, out + carry + incl - rh);
+        uint64_t cm = __ballot(coop);
+        while (cm) {
+            const uint32_t l = (uint32_t)__builtin_ctzll(cm);
+            cm &= cm - 1;
+            const uint32_t il = i0 + l;
+            const uint64_t xl = base + il;
+            walk_run_wave(ix, b.pos[xl], b.rs_hash[xl], (int)span_start(b.rs_span[xl]), (int)span_end(b.rs_span[xl]),
+                          il >= half ? 0x80000000u : 0u, out + carry + readlane_u32(incl - rh, l));
+        }
+        carry += readlane_u32(incl, 63);
+    }
+}
+
+// the reads that k_lookup listed, one per wave: pooled ones, then rescued ones
+__global__ __launch_bounds__(64 * WPB) void k_hits(DevBatch b, DevIndex ix, uint32_t rescue_cutoff,
+                                                   uint32_t hard_cutoff) {
+    const uint32_t n_pool = sload(&b.ctl->n_sel[SEL_POOLED]), n_resc = sload(&b.ctl->n_sel[SEL_RESCUED]);
+    const bool pool_ok = (uint64_t)b.n_reads * HIT_REGION + sload(&b.ctl->hit_pool) <= b.hit_cap;
+    if (n_pool && !pool_ok && blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&b.ctl->overflow, OVF_HITS);
+    for (uint32_t w = wave_index(WPB); w < n_pool + n_resc; w += gridDim.x * WPB) {
+        if (w >= n_pool)
+            rescued_hits(b, ix, uni32(b.sel_ids[w - n_pool]), rescue_cutoff, hard_cutoff);
+        else if (pool_ok)
+            pooled_hits(b, ix, uni32(b.sel_ids[2ull * b.n_reads + w]));
         wave_sync_mem();
     }
 }
 
-__global__ __launch_bounds__(64 * WPB) void k_rescue_hits(DevBatch b, ReadSet set, DevIndex ix) {
-    const uint32_t lane = lane_id();
-    if (blockIdx.x == 0 && threadIdx.x == 0) b.ctl->tot[1] = b.rhit_off[b.n_reads];
-    if (over_capacity(b.rhit_off, b.n_reads, b.rhit_cap, b.ctl, OVF_RHITS)) return;
-    const uint32_t cnt = set_count(set);
-    for (uint32_t w = wave_index(WPB); w < cnt; w += gridDim.x * WPB) {
-        const uint32_t r = set.ids ? sload(set.ids + w) : w;
-        if (sload(b.rhit_total + r) == 0) continue;
-        const uint32_t n = sload(b.rs_cnt + r);
-        const uint64_t base = sload(b.rs_off + r);
-        const uint32_t half = sload(b.rs_nfwd + r);
-        DevHit *out = b.rhits + sload(b.rhit_off + r);
-        uint32_t carry = 0;
-        for (uint32_t i0 = 0; i0 < n; i0 += 64) {
-            const uint32_t i = i0 + lane;
-            const uint32_t rh = i < n ? b.rcnt[base + i] : 0u;
-            // runs longer than WALK_WAVE_MIN (k_rescue_count left their
-            // lengths in hcnt) take the wave walk, as they did there
-            const bool coop = rh > 0 && b.hcnt[base + i] > WALK_WAVE_MIN;
-            const uint32_t ex = wave_excl_scan(rh);
-            if (rh > 0 && !coop)
-                walk_run(ix, b.pos[base + i], b.rs_hash[base + i], (int)span_start(b.rs_span[base + i]),
-                         (int)span_end(b.rs_span[base + i]), i >= half ? 0x80000000u : 0u, out + carry + ex);
-            uint64_t cm = __ballot(coop);
-            while (cm) {
-                const uint32_t l = (uint32_t)__builtin_ctzll(cm);
-                cm &= cm - 1;
-                const uint32_t il = i0 + l;
-                const uint64_t xl = base + il;
-                walk_run_wave(ix, b.pos[xl], b.rs_hash[xl], (int)span_start(b.rs_span[xl]),
-                              (int)span_end(b.rs_span[xl]), il >= half ? 0x80000000u : 0u,
-                              out + carry + readlane_u32(ex, l));
-            }
-            carry += wave_sum(rh);
-        }
-    }
+// a hit array overflowed (an earlier kernel found it): the host grows it and
+// runs again, and the kernels after the hits leave their work out
+__device__ __forceinline__ bool hits_missing(const DevBatch &b) {
+    return (sload(&b.ctl->overflow) & (OVF_HITS | OVF_RHITS)) != 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -1625,9 +1631,6 @@ struct alignas(8) MergeLds {
     uint64_t keys[MERGE_LDS];
 };
 
-// reads handed from k_merge4 to k_merge (more than 64 hits, or more than
-// 16 NAMs on one strand)
-constexpr uint32_t MERGE_DEFER = 0xfffffffeu;
 // reads whose (strand, ref) groups merge on separate waves (k_merge_groups,
 // then k_merge_split_finish), for reads with more than SPLIT_MIN hits
 constexpr uint32_t MERGE_SPLIT = 0xfffffffdu;
@@ -1642,32 +1645,24 @@ constexpr int GROUP_WIDE_LDS = 1024;
 // chunk bounds of a k_merge_groups wide list (lists up to 32,768 entries)
 constexpr uint32_t GROUP_BOXES = 512;
 
-__global__ __launch_bounds__(64 * WPB) void k_merge(DevBatch b, ReadSet set, int rescue, int only_deferred,
-                                                    int split) {
+// the reads that k_merge4 handed on, one per wave
+__global__ __launch_bounds__(64 * WPB) void k_merge(DevBatch b) {
     __shared__ uint64_t lkeys[WPB][MERGE_LDS];
     __shared__ WideNam lwide[WPB][MERGE_WIDE_LDS];  // the wide list of reads with few enough hits
     const uint32_t lane = lane_id();
     const int wid = (int)uni32(threadIdx.x >> 6);
-    if (rescue ? over_capacity(b.rhit_off, b.n_reads, b.rhit_cap, b.ctl, OVF_RHITS)
-               : over_capacity(b.hit_off, b.n_reads, b.hit_cap, b.ctl, OVF_HITS))
-        return;
-    const uint32_t cnt = set_count(set);
+    if (hits_missing(b)) return;
+    const uint32_t cnt = sload(&b.ctl->n_sel[SEL_DEFERRED]);
     for (uint32_t w = wave_index(WPB); w < cnt; w += gridDim.x * WPB) {
-        const uint32_t r = uni32(set_at(set, w));
-        const bool rescued = (uni32(b.flags[r]) & GIS_FLAG_RESCUED) != 0;
-        if (rescued != (rescue != 0)) continue;
-        if (only_deferred && uni32(b.nam_cnt[r]) != MERGE_DEFER) continue;
+        const uint32_t r = uni32(b.sel_ids[(uint64_t)b.n_reads + w]);
+        const bool rescue = (uni32(b.flags[r]) & GIS_FLAG_RESCUED) != 0;
         const uint64_t hb = uni64(rescue ? b.rhit_off[r] : b.hit_off[r]);
         const uint32_t nh = uni32(rescue ? b.rhit_total[r] : b.hit_total[r]);
-        if (nh == 0) {
-            if (lane == 0) b.nam_cnt[r] = 0;
-            continue;
-        }
         const DevHit *ghits = (rescue ? b.rhits : b.hits) + hb;
         gis_nam *fin = (rescue ? b.rnam_fin : b.nam_fin) + hb;
         uint64_t *gkeys = b.merge_scratch ? (rescue ? b.rkeys : b.keys) + 2 * hb : nullptr;
         WideNam *gwide = b.merge_scratch ? (rescue ? b.rnam_ws : b.nam_ws) + hb : nullptr;
-        if (split && nh > SPLIT_MIN && b.merge_scratch) {
+        if (nh > SPLIT_MIN && b.merge_scratch) {
             // group the hits; each group merges on its own wave
             const uint64_t *ord = group_order(nh, ghits, gkeys, gkeys + nh);
             const uint32_t code = ord == nullptr ? 0u : (ord == gkeys ? 1u : 2u);
@@ -1704,7 +1699,7 @@ __global__ __launch_bounds__(64 * WPB) void k_merge(DevBatch b, ReadSet set, int
             wave_sync_mem();
             {
                 uint32_t at = 0;
-                if (lane == 0) at = atomicAdd(&b.ctl->n_gwork[rescue ? 1 : 0], K);
+                if (lane == 0) at = atomicAdd(&b.ctl->n_gwork, K);
                 at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
                 for (uint32_t g = lane; g < K; g += 64) {
                     const uint32_t gs = (uint32_t)(slots[g] >> 32);
@@ -1712,7 +1707,7 @@ __global__ __launch_bounds__(64 * WPB) void k_merge(DevBatch b, ReadSet set, int
                     b.gwork[at + g] = make_uint4(r, gs, ge, g | (code << 30));
                 }
                 if (lane == 0) {
-                    const uint32_t si = atomicAdd(&b.ctl->n_split[rescue ? 1 : 0], 1u);
+                    const uint32_t si = atomicAdd(&b.ctl->n_split, 1u);
                     b.split_list[si] = make_uint4(r, K, code, 0u);
                     b.nam_cnt[r] = MERGE_SPLIT;
                 }
@@ -1742,14 +1737,15 @@ __global__ __launch_bounds__(64 * WPB) void k_merge(DevBatch b, ReadSet set, int
 // one wave per work item (a run of consecutive groups of a split read): its
 // hits (in grouped order) merge into NAMs at the item's own hit-indexed region
 // of the read's output; the NAM count goes to the read's item slot
-__global__ __launch_bounds__(64) void k_merge_groups(DevBatch b, int rescue) {
+__global__ __launch_bounds__(64) void k_merge_groups(DevBatch b) {
     __shared__ WideNam lwide[GROUP_WIDE_LDS];
     __shared__ ChunkBox lbox[GROUP_BOXES];
     const uint32_t lane = lane_id();
-    const unsigned int cnt = b.ctl->n_gwork[rescue ? 1 : 0];
+    const unsigned int cnt = sload(&b.ctl->n_gwork);
     for (uint32_t w = blockIdx.x; w < cnt; w += gridDim.x) {
         const uint4 it = b.gwork[w];
         const uint32_t r = it.x, gs = it.y, ge = it.z, g = it.w & 0x3fffffffu, code = it.w >> 30;
+        const bool rescue = (b.flags[r] & GIS_FLAG_RESCUED) != 0;
         const uint64_t hb = rescue ? b.rhit_off[r] : b.hit_off[r];
         const uint32_t nh = rescue ? b.rhit_total[r] : b.hit_total[r];
         uint64_t *gkeys = (rescue ? b.rkeys : b.keys) + 2 * hb;
@@ -1769,12 +1765,13 @@ __global__ __launch_bounds__(64) void k_merge_groups(DevBatch b, int rescue) {
 
 // one wave per split read: the groups' NAMs move to consecutive places in
 // group order (canonical order) with nam_id = rank
-__global__ __launch_bounds__(64 * WPB) void k_merge_split_finish(DevBatch b, int rescue) {
+__global__ __launch_bounds__(64 * WPB) void k_merge_split_finish(DevBatch b) {
     const uint32_t lane = lane_id();
-    const unsigned int cnt = b.ctl->n_split[rescue ? 1 : 0];
+    const unsigned int cnt = sload(&b.ctl->n_split);
     for (uint32_t w = blockIdx.x * WPB + (threadIdx.x >> 6); w < cnt; w += gridDim.x * WPB) {
         const uint4 e = b.split_list[w];
         const uint32_t r = e.x, G = e.y, code = e.z;
+        const bool rescue = (b.flags[r] & GIS_FLAG_RESCUED) != 0;
         const uint64_t hb = rescue ? b.rhit_off[r] : b.hit_off[r];
         const uint32_t nh = rescue ? b.rhit_total[r] : b.hit_total[r];
         uint64_t *gkeys = (rescue ? b.rkeys : b.keys) + 2 * hb;
@@ -1815,7 +1812,7 @@ __global__ __launch_bounds__(64 * WPB) void k_merge_split_finish(DevBatch b, int
 // strand's hits end, its NAMs are final: each lane ranks its NAM among the
 // segment's by (ref_id, creation index), which is canonical order within the
 // strand, and writes it. A read with more than 16 NAMs on one strand, or
-// more than 64 hits, is marked MERGE_DEFER for k_merge.
+// more than 64 hits, is listed for k_merge.
 
 constexpr uint32_t SEG = 16;
 constexpr uint32_t RPW = 64 / SEG;
@@ -1837,32 +1834,26 @@ __device__ __forceinline__ void seg_finalize(gis_nam *out, uint32_t base, uint32
     if (on && j < n_open) lane_nam_store(out, base + rank, rsd, o);
 }
 
-__global__ __launch_bounds__(64 * WPB) void k_merge4(DevBatch b, ReadSet set, int rescue) {
+__global__ __launch_bounds__(64 * WPB) void k_merge4(DevBatch b, ReadSet set) {
     __shared__ DevHit lh[WPB][RPW][64];
     const uint32_t lane = lane_id(), seg = lane / SEG, j = lane % SEG;
     const int wid = (int)uni32(threadIdx.x >> 6);
-    if (rescue ? over_capacity(b.rhit_off, b.n_reads, b.rhit_cap, b.ctl, OVF_RHITS)
-               : over_capacity(b.hit_off, b.n_reads, b.hit_cap, b.ctl, OVF_HITS))
-        return;
+    if (hits_missing(b)) return;
     const uint32_t cnt = set_count(set);
     const uint32_t stride = gridDim.x * WPB * RPW;
     for (uint32_t w0 = wave_index(WPB) * RPW; w0 < cnt; w0 += stride) {
         const uint32_t widx = w0 + seg;
-        bool act = widx < cnt;
+        bool act = widx < cnt, defer = false, rescue = false;
         uint32_t r = 0, nh = 0;
         uint64_t hb = 0;
         if (act) {
             r = set_at(set, widx);
-            const bool rescued = (b.flags[r] & GIS_FLAG_RESCUED) != 0;
-            act = rescued == (rescue != 0);
-        }
-        if (act) {
+            rescue = (b.flags[r] & GIS_FLAG_RESCUED) != 0;
             hb = rescue ? b.rhit_off[r] : b.hit_off[r];
             nh = rescue ? b.rhit_total[r] : b.hit_total[r];
-            if (nh == 0 || nh > 64) {
-                if (j == 0) b.nam_cnt[r] = nh == 0 ? 0u : MERGE_DEFER;
-                act = false;
-            }
+            defer = nh > 64;
+            act = nh > 0 && !defer;
+            if (nh == 0 && j == 0) b.nam_cnt[r] = 0u;
         }
         if (act) {
             const DevHit *gh = (rescue ? b.rhits : b.hits) + hb;
@@ -1919,7 +1910,16 @@ __global__ __launch_bounds__(64 * WPB) void k_merge4(DevBatch b, ReadSet set, in
         }
         const bool fin = act && !ovf;
         if (__ballot(fin)) seg_finalize(out, base, j, n_open, rsd_o, o, fin);
-        if (act && j == 0) b.nam_cnt[r] = ovf ? MERGE_DEFER : base + n_open;
+        if (fin && j == 0) b.nam_cnt[r] = base + n_open;
+        // the reads handed on to k_merge
+        defer = (defer || (act && ovf)) && j == 0;
+        const uint64_t dm = __ballot(defer);
+        if (dm) {
+            uint32_t at = 0;
+            if (lane == 0) at = atomicAdd(&b.ctl->n_sel[SEL_DEFERRED], (uint32_t)__popcll(dm));
+            at = uni32(at);
+            if (defer) b.sel_ids[(uint64_t)b.n_reads + at + mbcnt(dm)] = r;
+        }
         wave_sync_mem();
     }
 }
@@ -2349,34 +2349,65 @@ __global__ __launch_bounds__(64 * FWPB) __attribute__((amdgpu_waves_per_eu(6))) 
 // ---------------------------------------------------------------------------
 // dense output: NAMs of read r to nams_out[nam_off[r] ..]
 
+constexpr int SCAN_BLOCK = 256, SCAN_ITEMS = 4, SCAN_TILE = SCAN_BLOCK * SCAN_ITEMS;
 constexpr uint32_t COMPACT_SEG = 16;
 constexpr uint32_t COMPACT_SEG_WORDS = 8 * COMPACT_SEG;  // 11 NAMs of 11 words
 
-__global__ __launch_bounds__(64 * WPB) void k_compact(DevBatch b, int fused) {
-    const uint32_t lane = lane_id();
-    if (blockIdx.x == 0 && threadIdx.x == 0) b.ctl->tot[2] = b.nam_off[b.n_reads];
-    // a hit array overflowed: the merges did not run and the counts are stale
-    if (b.ctl->overflow & (OVF_HITS | OVF_RHITS)) return;
-    if (b.nam_off[b.n_reads] > b.out_cap) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(&b.ctl->overflow, OVF_OUT);
-        return;
+// totals into the control block's copy for the host: lane i holds word i
+__device__ __forceinline__ void ctl_store(const DevBatch &b, DevCtl *dst, uint64_t nams, unsigned overflow) {
+    if (threadIdx.x == 0) {
+        DevCtl c = *b.ctl;
+        c.overflow |= overflow;
+        c.tot[0] = (uint64_t)b.n_reads * HIT_REGION + c.hit_pool;
+        c.tot[1] = c.rhit_pool;
+        c.tot[2] = nams;
+        *dst = c;
     }
+}
+
+// sum of a[0 .. n) over the wave
+__device__ __forceinline__ uint64_t wave_sum_of(const uint64_t *a, uint32_t n) {
+    uint64_t v = 0;
+    for (uint32_t t = lane_id(); t < n; t += 64) v += a[t];
+    for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d, 64);
+    return v;
+}
+
+// NAM offsets and the dense output. nam_off holds each read's offset inside its
+// tile of SCAN_TILE reads and tiles the tiles' NAM counts (k_scan_tiles); each
+// wave adds the counts of the tiles before its reads' own (ntiles > 0), or
+// takes their prefix (ntiles == 0: tiles holds it, nam_off[n] the total). The
+// first block hands the totals to the host.
+__global__ __launch_bounds__(64 * WPB) void k_compact(DevBatch b, int fused, const uint64_t *tiles, uint32_t ntiles,
+                                                      DevCtl *dst) {
+    const uint32_t lane = lane_id();
+    if (blockIdx.x == 0 && threadIdx.x < 64) {
+        const uint64_t total = ntiles ? wave_sum_of(tiles, ntiles) : b.nam_off[b.n_reads];
+        if (lane == 0) b.nam_off[b.n_reads] = total;
+        ctl_store(b, dst, total, total > b.out_cap ? (unsigned)OVF_OUT : 0u);
+    }
+    // the merges did not run and the counts are stale
+    if (hits_missing(b)) return;
     // COMPACT_SEG lanes per read, so that a wave's reads start their loads
     // (count, flags, offsets, then NAMs) together; reads with more than
     // COMPACT_SEG_WORDS words of NAMs (repeats) are copied by the whole wave
     // afterwards, four words per lane in flight
     const uint32_t seg = lane / COMPACT_SEG, j = lane % COMPACT_SEG;
     const uint32_t per_wave = 64 / COMPACT_SEG;
-    for (uint32_t r0 = (blockIdx.x * WPB + (threadIdx.x >> 6)) * per_wave; r0 < b.n_reads;
-         r0 += gridDim.x * WPB * per_wave) {
+    const uint32_t r0 = wave_index(WPB) * per_wave;
+    if (r0 < b.n_reads) {
         const uint32_t r = r0 + seg;
         // the read's count, flags and offsets load together (r clamped to a
         // valid read; lanes past the end copy nothing)
         const uint32_t rr = r < b.n_reads ? r : b.n_reads - 1;
         const uint32_t c0 = b.nam_cnt[rr];
         const uint8_t fl = b.flags[rr];
-        const uint64_t ho = b.hit_off[rr], rho = b.rhit_off[rr], no = b.nam_off[rr];
-        const uint32_t c = r < b.n_reads ? c0 : 0u;
+        const uint64_t ho = b.hit_off[rr], rho = b.rhit_off[rr], in_tile = b.nam_off[rr];
+        // (a wave's reads lie in one tile)
+        const uint32_t tile = r0 / SCAN_TILE;
+        const uint64_t no = in_tile + (ntiles ? wave_sum_of(tiles, tile) : tiles[tile]);
+        if (j == 0 && r < b.n_reads) b.nam_off[r] = no;
+        const uint32_t c = r < b.n_reads && no + c0 <= b.out_cap ? c0 : 0u;
         const gis_nam *srcn;
         if (fused && !(fl & FLAG_SPILL)) srcn = b.nam_slots + (uint64_t)rr * F_NAMCAP;
         else if (fl & GIS_FLAG_RESCUED) srcn = b.rnam_fin + rho;
@@ -2425,54 +2456,7 @@ __global__ __launch_bounds__(64 * WPB) void k_compact(DevBatch b, int fused) {
     }
 }
 
-// Ids of the set's reads that a sparse pass visits, in set order within a
-// block: SEL_RESCUED (rescued reads) or SEL_DEFERRED (normal reads the
-// four-per-wave merge handed on). One atomic per block places a block's ids.
-enum { SEL_RESCUED = 0, SEL_DEFERRED = 1, SEL_POOLED = 2 };
-
-__global__ __launch_bounds__(256) void k_select(DevBatch b, ReadSet set, int kind) {
-    __shared__ uint32_t wcount[4];
-    __shared__ uint32_t block_base;
-    const uint32_t lane = lane_id(), wid = threadIdx.x >> 6;
-    const uint32_t cnt = set_count(set);
-    uint32_t *out = b.sel_ids + (uint64_t)kind * b.n_reads;
-    for (uint32_t base = blockIdx.x * 256u; base < cnt; base += gridDim.x * 256u) {
-        const uint32_t i = base + threadIdx.x;
-        uint32_t r = 0;
-        bool m = false;
-        if (i < cnt) {
-            r = set_at(set, i);
-            const bool rescued = (b.flags[r] & GIS_FLAG_RESCUED) != 0;
-            m = kind == SEL_RESCUED ? rescued : (!rescued && b.nam_cnt[r] == MERGE_DEFER);
-        }
-        const uint64_t bal = __ballot(m);
-        if (lane == 0) wcount[wid] = (uint32_t)__popcll(bal);
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            const uint32_t t = wcount[0] + wcount[1] + wcount[2] + wcount[3];
-            block_base = t ? atomicAdd(&b.ctl->n_sel[kind], t) : 0u;
-        }
-        __syncthreads();
-        uint32_t off = block_base;
-        for (uint32_t w = 0; w < wid; w++) off += wcount[w];
-        if (m) out[off + mbcnt(bal)] = r;
-        __syncthreads();
-    }
-}
-
-__global__ void k_reset_ctl(DevCtl *ctl) {
-    if (threadIdx.x == 0) {
-        ctl->n_spill = 0;
-        ctl->overflow = 0;
-        ctl->q_head[0] = 0;
-        ctl->q_head[1] = 0;
-        ctl->n_gwork[0] = ctl->n_gwork[1] = 0;
-        ctl->n_split[0] = ctl->n_split[1] = 0;
-        ctl->n_sel[0] = ctl->n_sel[1] = ctl->n_sel[2] = 0;
-        ctl->hit_pool = 0;
-        ctl->tot[0] = ctl->tot[1] = ctl->tot[2] = 0;
-    }
-}
+__global__ void k_reset_ctl(DevCtl *ctl) { ctl_clear(ctl); }
 
 // plain lookup over a list of hashes (the microbenchmark gpu_find,
 // gpu_test.cu:186-215, with StrobemerIndex::find semantics)
@@ -2494,8 +2478,6 @@ __global__ void k_find_flat(DevIndex ix, const uint64_t *hashes, uint64_t n, uin
 
 // ---------------------------------------------------------------------------
 // exclusive scan u32 -> u64 offsets[n+1]
-
-constexpr int SCAN_BLOCK = 256, SCAN_ITEMS = 4, SCAN_TILE = SCAN_BLOCK * SCAN_ITEMS;
 
 __device__ __forceinline__ uint64_t block_excl_scan_u64(uint64_t v, uint64_t *lds_w, uint64_t *total) {
     const uint32_t lane = lane_id(), wid = threadIdx.x >> 6;
@@ -2601,21 +2583,11 @@ static inline unsigned grid_for_set(const DevBatch &b, const ReadSet &set, unsig
     return g < 2048u ? g : 2048u;
 }
 
-// the reads a sparse pass visits: the ids k_select wrote
-static inline ReadSet selected(const DevBatch &b, int kind) {
-    return ReadSet{b.sel_ids + (uint64_t)kind * b.n_reads, &b.ctl->n_sel[kind], b.n_reads};
-}
-
 // blocks for a per-read kernel over a selected list (its length is on the
 // device): enough waves to run every heavy read of the list at once
 static inline unsigned grid_selected(const DevBatch &b) {
     const unsigned g = grid_for(b.n_reads, WPB);
     return g < 2048u ? (g ? g : 1u) : 2048u;
-}
-
-static void launch_select(const DevBatch &b, const ReadSet &set, int kind, hipStream_t st) {
-    const unsigned g = grid_for(b.n_reads, 256);
-    hipLaunchKernelGGL(k_select, dim3(g < 1024u ? (g ? g : 1u) : 1024u), dim3(256), 0, st, b, set, kind);
 }
 
 // The bucket lines (DevIndex::lines) from starts and the table, eight lanes a
@@ -2648,15 +2620,18 @@ void launch_reset_ctl(DevCtl *ctl, hipStream_t st) {
 }
 
 void launch_seed(const DevBatch &b, const ReadSet &set, const SeedParams &sp, int want_syncmers,
-                 int long_reads, hipStream_t st) {
-    if (b.n_reads == 0) return;
+                 int long_reads, int reset, hipStream_t st) {
+    if (b.n_reads == 0) {
+        if (reset) launch_reset_ctl(b.ctl, st);
+        return;
+    }
     const unsigned g = grid_for_set(b, set, SEED_WPB);
-    typedef void (*SeedKernel)(DevBatch, ReadSet, SeedParams, int);
+    typedef void (*SeedKernel)(DevBatch, ReadSet, SeedParams, int, int);
     const bool k20 = is_k20_profile(sp);
     const SeedKernel short_k = k20 ? (SeedKernel)k_seed<false, true> : (SeedKernel)k_seed<false, false>;
     const SeedKernel long_k = k20 ? (SeedKernel)k_seed<true, true> : (SeedKernel)k_seed<true, false>;
-    hipLaunchKernelGGL(short_k, dim3(g), dim3(64 * SEED_WPB), 0, st, b, set, sp, want_syncmers);
-    if (long_reads) hipLaunchKernelGGL(long_k, dim3(g), dim3(64 * SEED_WPB), 0, st, b, set, sp, want_syncmers);
+    hipLaunchKernelGGL(short_k, dim3(g), dim3(64 * SEED_WPB), 0, st, b, set, sp, want_syncmers, reset);
+    if (long_reads) hipLaunchKernelGGL(long_k, dim3(g), dim3(64 * SEED_WPB), 0, st, b, set, sp, want_syncmers, 0);
 }
 
 void launch_lookup(const DevBatch &b, const ReadSet &set, const DevIndex &ix, int rescue_mode,
@@ -2666,47 +2641,22 @@ void launch_lookup(const DevBatch &b, const ReadSet &set, const DevIndex &ix, in
                        rescue_mode, set.ids ? 1 : 0);
 }
 
-void launch_hits(const DevBatch &b, const ReadSet &set, const DevIndex &ix, hipStream_t st) {
-    (void)set;
-    hipLaunchKernelGGL(k_pool_total, dim3(1), dim3(64), 0, st, b);
+void launch_hits(const DevBatch &b, const DevIndex &ix, uint32_t rescue_cutoff, uint32_t hard_cutoff,
+                 hipStream_t st) {
     if (b.n_reads == 0) return;
-    hipLaunchKernelGGL(k_hits, dim3(grid_selected(b)), dim3(64 * WPB), 0, st, b, selected(b, SEL_POOLED), ix);
+    hipLaunchKernelGGL(k_hits, dim3(grid_selected(b)), dim3(64 * WPB), 0, st, b, ix, rescue_cutoff, hard_cutoff);
 }
 
-void launch_rescue_count(const DevBatch &b, const ReadSet &set, const DevIndex &ix,
-                         uint32_t rescue_cutoff, uint32_t hard_cutoff, hipStream_t st) {
+// four reads per wave over the set, then the reads it handed on, one per wave,
+// then the (strand, ref) groups of split reads and their finish
+void launch_merge(const DevBatch &b, const ReadSet &set, hipStream_t st) {
     if (b.n_reads == 0) return;
-    launch_select(b, set, SEL_RESCUED, st);
-    hipLaunchKernelGGL(k_rescue_count, dim3(grid_selected(b)), dim3(64 * WPB), 0, st, b,
-                       selected(b, SEL_RESCUED), ix, rescue_cutoff, hard_cutoff);
-}
-
-// (after launch_rescue_count, which selects the rescued reads)
-void launch_rescue_hits(const DevBatch &b, const ReadSet &set, const DevIndex &ix, hipStream_t st) {
-    (void)set;
-    if (b.n_reads == 0) return;
-    hipLaunchKernelGGL(k_rescue_hits, dim3(grid_selected(b)), dim3(64 * WPB), 0, st, b,
-                       selected(b, SEL_RESCUED), ix);
-}
-
-// normal pass: four reads per wave over the set, then the reads it handed
-// on, one per wave; rescue pass: the rescued reads one per wave; then the
-// (strand, ref) groups of split reads and their finish
-void launch_merge(const DevBatch &b, const ReadSet &set, int rescue, hipStream_t st) {
-    if (b.n_reads == 0) return;
-    if (!rescue) {
-        const unsigned g = grid_for_set(b, set, WPB);
-        hipLaunchKernelGGL(k_merge4, dim3((g + RPW - 1) / RPW), dim3(64 * WPB), 0, st, b, set, 0);
-        launch_select(b, set, SEL_DEFERRED, st);
-        hipLaunchKernelGGL(k_merge, dim3(grid_selected(b)), dim3(64 * WPB), 0, st, b,
-                           selected(b, SEL_DEFERRED), 0, 1, 1);
-    } else {
-        hipLaunchKernelGGL(k_merge, dim3(grid_selected(b)), dim3(64 * WPB), 0, st, b,
-                           selected(b, SEL_RESCUED), 1, 0, 1);
-    }
+    const unsigned g = grid_for_set(b, set, WPB);
+    hipLaunchKernelGGL(k_merge4, dim3((g + RPW - 1) / RPW), dim3(64 * WPB), 0, st, b, set);
+    hipLaunchKernelGGL(k_merge, dim3(grid_selected(b)), dim3(64 * WPB), 0, st, b);
     if (b.merge_scratch) {
-        hipLaunchKernelGGL(k_merge_groups, dim3(4096), dim3(64), 0, st, b, rescue);
-        hipLaunchKernelGGL(k_merge_split_finish, dim3(256), dim3(64 * WPB), 0, st, b, rescue);
+        hipLaunchKernelGGL(k_merge_groups, dim3(4096), dim3(64), 0, st, b);
+        hipLaunchKernelGGL(k_merge_split_finish, dim3(256), dim3(64 * WPB), 0, st, b);
     }
 }
 
@@ -2741,23 +2691,35 @@ bool launch_fused(const DevBatch &b, const DevIndex &ix, const SeedParams &sp, u
     return false;
 }
 
-void launch_compact(const DevBatch &b, int fused, hipStream_t st) {
-    if (b.n_reads == 0) return;
-    hipLaunchKernelGGL(k_compact, dim3(grid_for(b.n_reads, WPB * (64 / COMPACT_SEG))), dim3(64 * WPB), 0, st, b,
-                       fused);
-}
-
-// The control block to pinned host memory by one wave's stores, so that the
+// The control block to pinned host memory by a thread's stores, so that the
 // end of a run takes no copy engine (the engines carry the batches' reads and
 // NAMs).
-static_assert(sizeof(DevCtl) % 4 == 0 && sizeof(DevCtl) / 4 <= 64, "one word per lane");
-__global__ void k_ctl_to_host(const DevCtl *__restrict__ src, DevCtl *__restrict__ dst) {
-    const unsigned i = threadIdx.x;
-    if (i < sizeof(DevCtl) / 4) reinterpret_cast<unsigned *>(dst)[i] = reinterpret_cast<const unsigned *>(src)[i];
+__global__ void k_ctl_to_host(DevBatch b, DevCtl *dst) { ctl_store(b, dst, 0, 0u); }
+
+void launch_ctl_to_host(const DevBatch &b, DevCtl *dst, hipStream_t st) {
+    hipLaunchKernelGGL(k_ctl_to_host, dim3(1), dim3(64), 0, st, b, dst);
 }
 
-void launch_ctl_to_host(const DevCtl *src, DevCtl *dst, hipStream_t st) {
-    hipLaunchKernelGGL(k_ctl_to_host, dim3(1), dim3(64), 0, st, src, dst);
+// Up to SCAN_OWN_TILES tiles each wave of k_compact sums the tiles before its
+// own (a load a lane for 64 tiles), which saves the launch that would turn them
+// into a prefix; beyond (1,048,576 reads) that launch is the cheaper way.
+constexpr unsigned SCAN_OWN_TILES = 1024;
+
+void launch_output(const DevBatch &b, int fused, uint64_t *tmp, DevCtl *dst, hipStream_t st) {
+    const uint64_t n = b.n_reads;
+    if (n == 0) {
+        launch_scan(b.nam_cnt, b.nam_off, 0, tmp, st);
+        launch_ctl_to_host(b, dst, st);
+        return;
+    }
+    unsigned tiles = grid_for(n, SCAN_TILE);
+    hipLaunchKernelGGL(k_scan_tiles, dim3(tiles), dim3(SCAN_BLOCK), 0, st, b.nam_cnt, b.nam_off, n, tmp);
+    if (tiles > SCAN_OWN_TILES) {
+        hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_BLOCK), 0, st, tmp, (uint64_t)tiles, b.nam_off, n);
+        tiles = 0;
+    }
+    hipLaunchKernelGGL(k_compact, dim3(grid_for(n, WPB * (64 / COMPACT_SEG))), dim3(64 * WPB), 0, st, b, fused, tmp,
+                       (uint32_t)tiles, dst);
 }
 
 void launch_find_flat(const DevIndex &ix, const uint64_t *hashes, uint64_t n, uint64_t *positions,

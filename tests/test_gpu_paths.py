@@ -101,3 +101,24 @@ def test_filter_cutoff_inside_a_bucket_line(ctx, mode):
     assert np.array_equal(res.nam_offsets, eo) and res.nams.tobytes() == en.tobytes()
     assert res.nonrepetitive_fraction.tobytes() == ef.tobytes() and np.array_equal(res.flags & 1, efl & 1)
     idx.ctx.close()
+
+
+@pytest.mark.parametrize("n", [1, 15, 17, 1023, 1024, 1025, 65537, 1_048_576, 1_048_577])
+def test_output_offsets_over_tiles(ctx, n):
+    """NAM offsets and the dense output around the scan's tile (1024 reads)
+    and the count of tiles each wave sums itself: one mapped read among reads
+    too short to map, again and again, equals that read's NAMs repeated."""
+    g, lens = G.synth_genome(100_000, n_contigs=1, gc=0.45, seed=21)
+    idx = G.StrobemerIndex(None, G.IndexParameters.from_read_length(150))
+    idx.populate_arrays(g, lens)
+    s = g[5000:5150].copy()
+    l = np.full(n, 25, dtype=np.uint32)
+    l[::29] = 150
+    o = np.zeros(n, dtype=np.uint64)
+    one = G.find_nams_batch(idx, s, o[:1], np.array([150], dtype=np.uint32))
+    assert len(one.nams) > 0
+    res = G.find_nams_batch(idx, s, o, l)
+    k = len(range(0, n, 29))
+    assert np.array_equal(np.diff(res.nam_offsets), np.where(l == 150, len(one.nams), 0))
+    assert res.nam_offsets[0] == 0 and res.nams.tobytes() == one.nams.tobytes() * k
+    idx.ctx.close()
