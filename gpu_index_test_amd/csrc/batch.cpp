@@ -53,7 +53,7 @@ static std::vector<DevBuf *> ws_bufs(Workspace *w) {
             &w->hit_total, &w->rhit_total, &w->frac, &w->flags, &w->nam_cnt, &w->hit_off,
             &w->rhit_off, &w->hits, &w->rhits, &w->keys, &w->rkeys, &w->nam_ws, &w->rnam_ws,
             &w->nam_fin, &w->rnam_fin, &w->nam_slots, &w->nam_off, &w->nams_out, &w->scan_tmp,
-            &w->ctl, &w->spill_ids, &w->gwork, &w->split_list, &w->sel_ids};
+            &w->ctl, &w->spill_ids, &w->gwork, &w->split_list, &w->sel_ids, &w->seeds};
 }
 
 static std::vector<DevBuf *> input_bufs(gis_batch *b) {
@@ -375,12 +375,10 @@ void enqueue_run(gis_batch *b, int mode, int rescue_mode, uint32_t rcut, uint32_
     }
     launch_seed(d, set, sp, b->want_sy ? 1 : 0, b->any_long ? 1 : 0, fused ? 0 : 1, st);
     mark(b, "seed");
-    if (stop != STOP_SEED) {
-        launch_lookup(d, set, ix, rescue_mode, st);
-        mark(b, "lookup");
-        launch_hits(d, ix, rcut, hard, st);
-        mark(b, "hits");
-    }
+    launch_lookup(d, set, ix, rescue_mode, st);
+    mark(b, "lookup");
+    launch_hits(d, ix, rcut, hard, st);
+    mark(b, "hits");
     if (stop == STOP_NONE) {
         launch_merge(d, set, st);
         mark(b, "merge");
@@ -582,91 +580,69 @@ gis_map_options opts_or_default(const gis_map_options *opt) {
 
 // ---------------- stage entry points ----------------
 
-extern "C" int gis_syncmers_batch(gis_ctx *ctx, const char *seqs, const uint64_t *offsets,
-                                  const uint32_t *lens, uint32_t n_reads, uint64_t *out_offsets,
-                                  gis_syncmer *out, uint64_t capacity, uint64_t *n_out) {
-    API_BEGIN(ctx)
-    gis_batch *b = scratch_batch(ctx);
-    int rc = batch_upload(b, seqs, offsets, lens, n_reads, true);
-    if (rc) return rc;
-    const gis_map_options o = opts_or_default(nullptr);
-    batch_run(b, o, 0, STOP_SEED);
-    std::vector<uint32_t> cnt(n_reads);
-    if (n_reads) HIP_CHECK(hipMemcpy(cnt.data(), b->ws->sy_cnt.p, 4ull * n_reads, hipMemcpyDeviceToHost));
-    uint64_t total = 0;
-    for (uint32_t r = 0; r < n_reads; r++) total += cnt[r];
-    if (n_out) *n_out = total;
-    if (total > capacity || (total && !out)) return fail(ctx, GIS_ERR_CAPACITY, "syncmer capacity too small");
-    const uint64_t cap = b->h_sy_off[n_reads];
-    std::vector<uint64_t> hh(cap), pp(cap);
-    if (cap) {
-        HIP_CHECK(hipMemcpy(hh.data(), b->ws->sy_hash.p, 8 * cap, hipMemcpyDeviceToHost));
-        HIP_CHECK(hipMemcpy(pp.data(), b->ws->sy_pos.p, 8 * cap, hipMemcpyDeviceToHost));
-    }
-    uint64_t o2 = 0;
-    for (uint32_t r = 0; r < n_reads; r++) {
-        if (out_offsets) out_offsets[r] = o2;
-        for (uint32_t i = 0; i < cnt[r]; i++) {
-            out[o2].hash = hh[b->h_sy_off[r] + i];
-            out[o2].position = pp[b->h_sy_off[r] + i];
-            o2++;
-        }
-    }
-    if (out_offsets) out_offsets[n_reads] = o2;
-    return GIS_OK;
-    API_END(ctx)
-}
+static_assert(sizeof(gis_query_randstrobe) == 24 && sizeof(gis_syncmer) == 16, "the records the device writes");
 
-// randstrobes_query of every read with the given parameters (the index's
-// when params is null); the caller holds the context's lock
-static int randstrobes_of(gis_ctx *ctx, const gis_params *params, const char *seqs, const uint64_t *offsets,
-                          const uint32_t *lens, uint32_t n_reads, uint64_t *out_offsets, gis_query_randstrobe *out,
-                          uint64_t capacity, uint64_t *n_out) {
+// Seeds of every read (query randstrobes, or syncmers) into out, dense and in
+// read order; seeding parameters of the batch's seed_params or the index. The
+// caller holds the context's lock.
+static int seeds_of(gis_ctx *ctx, const gis_params *params, bool syncmers, const char *seqs, const uint64_t *offsets,
+                    const uint32_t *lens, uint32_t n, uint64_t *out_offsets, void *out, uint64_t capacity,
+                    uint64_t *n_out) {
     gis_batch *b = scratch_batch(ctx);
     struct Reset {
         gis_batch *b;
         ~Reset() { b->seed_params = nullptr; }
     } reset{b};
     b->seed_params = params;
-    int rc = batch_upload(b, seqs, offsets, lens, n_reads, false);
-    if (rc) return rc;
-    const gis_map_options o = opts_or_default(nullptr);
-    batch_run(b, o, 0, STOP_SEED);
-    std::vector<uint32_t> cnt(n_reads);
-    if (n_reads) HIP_CHECK(hipMemcpy(cnt.data(), b->ws->rs_cnt.p, 4ull * n_reads, hipMemcpyDeviceToHost));
-    uint64_t total = 0;
-    for (uint32_t r = 0; r < n_reads; r++) total += cnt[r];
+    if (int rc = batch_upload(b, seqs, offsets, lens, n, syncmers)) return rc;
+    Workspace *w = b->ws;
+    ensure_read_arrays(b, n);
+    ensure_slot_arrays(b, b->tot_rs_cap);
+    if (syncmers) {
+        ensure<uint64_t>(w->sy_hash, b->h_sy_off[n]);
+        ensure<uint64_t>(w->sy_pos, b->h_sy_off[n]);
+    }
+    if (b->any_long) ensure<uint8_t>(w->long_scratch, b->h_long_off[n]);
+    w->owner = b;
+    b->ran = false;
+    hipStream_t st = b->stream;
+    const DevBatch d = make_devbatch(b);
+    uint64_t *off = d.nam_off, *tmp = static_cast<uint64_t *>(w->scan_tmp.p);
+    launch_seed(d, ReadSet{nullptr, nullptr, n}, make_seed_params(params ? *params : ctx->ix.params), syncmers ? 1 : 0,
+                b->any_long ? 1 : 0, 0, st);
+    launch_scan(syncmers ? d.sy_cnt : d.rs_cnt, off, n, tmp, st);
+    HIP_CHECK(hipGetLastError());
+    HIP_CHECK(hipMemcpyAsync(&w->h_ctl->tot[2], off + n, 8, hipMemcpyDeviceToHost, st));
+    HIP_CHECK(hipStreamSynchronize(st));
+    const uint64_t total = w->h_ctl->tot[2];
     if (n_out) *n_out = total;
-    if (total > capacity || (total && !out)) return fail(ctx, GIS_ERR_CAPACITY, "randstrobe capacity too small");
-    const uint64_t cap = b->tot_rs_cap;
-    std::vector<uint64_t> hh(cap);
-    std::vector<uint32_t> sp(cap);
-    if (cap) {
-        HIP_CHECK(hipMemcpy(hh.data(), b->ws->rs_hash.p, 8 * cap, hipMemcpyDeviceToHost));
-        HIP_CHECK(hipMemcpy(sp.data(), b->ws->rs_span.p, 4 * cap, hipMemcpyDeviceToHost));
+    if (total > capacity || (total && !out))
+        return fail(ctx, GIS_ERR_CAPACITY, syncmers ? "syncmer capacity too small" : "randstrobe capacity too small");
+    const size_t rec = syncmers ? sizeof(gis_syncmer) : sizeof(gis_query_randstrobe);
+    if (total) {
+        ensure<char>(w->seeds, total * rec);
+        launch_emit_seeds(d, syncmers ? 1 : 0, off, w->seeds.p, st);
+        HIP_CHECK(hipGetLastError());
+        HIP_CHECK(hipMemcpyAsync(out, w->seeds.p, total * rec, hipMemcpyDeviceToHost, st));
     }
-    uint64_t o2 = 0;
-    for (uint32_t r = 0; r < n_reads; r++) {
-        if (out_offsets) out_offsets[r] = o2;
-        const uint64_t base = b->h_rs_off[r];
-        for (uint32_t i = 0; i < cnt[r]; i++) {
-            gis_query_randstrobe q{};
-            q.hash = hh[base + i];
-            q.start = (int32_t)span_start(sp[base + i]);
-            q.end = (int32_t)span_end(sp[base + i]);
-            q.is_reverse = i >= cnt[r] / 2;
-            out[o2++] = q;
-        }
-    }
-    if (out_offsets) out_offsets[n_reads] = o2;
+    if (out_offsets) HIP_CHECK(hipMemcpyAsync(out_offsets, off, 8ull * (n + 1), hipMemcpyDeviceToHost, st));
+    HIP_CHECK(hipStreamSynchronize(st));
     return GIS_OK;
+}
+
+extern "C" int gis_syncmers_batch(gis_ctx *ctx, const char *seqs, const uint64_t *offsets,
+                                  const uint32_t *lens, uint32_t n_reads, uint64_t *out_offsets,
+                                  gis_syncmer *out, uint64_t capacity, uint64_t *n_out) {
+    API_BEGIN(ctx)
+    return seeds_of(ctx, nullptr, true, seqs, offsets, lens, n_reads, out_offsets, out, capacity, n_out);
+    API_END(ctx)
 }
 
 extern "C" int gis_randstrobes_batch(gis_ctx *ctx, const char *seqs, const uint64_t *offsets,
                                      const uint32_t *lens, uint32_t n_reads, uint64_t *out_offsets,
                                      gis_query_randstrobe *out, uint64_t capacity, uint64_t *n_out) {
     API_BEGIN(ctx)
-    return randstrobes_of(ctx, nullptr, seqs, offsets, lens, n_reads, out_offsets, out, capacity, n_out);
+    return seeds_of(ctx, nullptr, false, seqs, offsets, lens, n_reads, out_offsets, out, capacity, n_out);
     API_END(ctx)
 }
 
@@ -681,7 +657,7 @@ extern "C" int gis_randstrobes_params(gis_ctx *ctx, const gis_params *params, co
                         (int)params->q, params->max_dist, &chk) != GIS_OK ||
         chk.t_syncmer != params->t_syncmer || chk.w_min != params->w_min || chk.w_max != params->w_max)
         return fail(ctx, GIS_ERR_BAD_PARAMETER, "invalid index parameters");
-    return randstrobes_of(ctx, params, seqs, offsets, lens, n_reads, out_offsets, out, capacity, n_out);
+    return seeds_of(ctx, params, false, seqs, offsets, lens, n_reads, out_offsets, out, capacity, n_out);
     API_END(ctx)
 }
 

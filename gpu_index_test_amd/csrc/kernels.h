@@ -164,6 +164,9 @@ void launch_reset_ctl(DevCtl *ctl, hipStream_t st);
 // use it), instead of a launch of its own
 void launch_seed(const DevBatch &b, const ReadSet &set, const SeedParams &sp, int want_syncmers,
                  int long_reads, int reset, hipStream_t st);
+// the seeds dense and in read order (gis_query_randstrobe or gis_syncmer records
+// at off[r] of out)
+void launch_emit_seeds(const DevBatch &b, int syncmers, const uint64_t *off, void *out, hipStream_t st);
 // rescue_mode: 0 = the caller's decision (nonrepetitive fraction < 0.7 or no
 // hits), 1 = never rescue, 2 = always rescue
 void launch_lookup(const DevBatch &b, const ReadSet &set, const DevIndex &ix, int rescue_mode,

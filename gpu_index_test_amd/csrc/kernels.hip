@@ -424,6 +424,35 @@ __global__ __launch_bounds__(64 * SEED_WPB) __attribute__((amdgpu_waves_per_eu(6
     }
 }
 
+// The seeds of every read from its slots to their dense place (off: scan of the
+// reads' counts), as the ABI's records: query randstrobes (24 bytes) or
+// syncmers (16 bytes). One wave a read, a lane a 64-bit word, so that the
+// stores are whole lines; a read's slots are several times its seeds, and
+// copying them to the host and packing there took most of the call (20,011
+// reads of 150 bp: 14.9 ms; now bound by the copy of the records).
+__global__ __launch_bounds__(64 * WPB) void k_emit_randstrobes(DevBatch b, const uint64_t *off, uint64_t *out) {
+    for (uint32_t r = wave_index(WPB); r < b.n_reads; r += gridDim.x * WPB) {
+        const uint32_t n = sload(b.rs_cnt + r), half = sload(b.rs_nfwd + r);
+        const uint64_t base = sload(b.rs_off + r);
+        uint64_t *dst = out + 3 * sload(off + r);
+        for (uint32_t w = lane_id(); w < 3 * n; w += 64) {
+            const uint32_t j = w / 3, c = w - 3 * j;
+            const uint32_t sp = b.rs_span[base + j];
+            const uint64_t h = b.rs_hash[base + j];
+            dst[w] = c == 0 ? h : c == 1 ? (uint64_t)span_start(sp) | ((uint64_t)span_end(sp) << 32) : j >= half ? 1u : 0u;
+        }
+    }
+}
+
+__global__ __launch_bounds__(64 * WPB) void k_emit_syncmers(DevBatch b, const uint64_t *off, uint64_t *out) {
+    for (uint32_t r = wave_index(WPB); r < b.n_reads; r += gridDim.x * WPB) {
+        const uint32_t n = sload(b.sy_cnt + r);
+        const uint64_t base = sload(b.sy_off + r);
+        uint64_t *dst = out + 2 * sload(off + r);
+        for (uint32_t w = lane_id(); w < 2 * n; w += 64) dst[w] = (w & 1 ? b.sy_pos : b.sy_hash)[base + (w >> 1)];
+    }
+}
+
 // ---------------------------------------------------------------------------
 // index access (StrobemerIndex, step2/index.hpp:57-147)
 
@@ -2632,6 +2661,13 @@ void launch_seed(const DevBatch &b, const ReadSet &set, const SeedParams &sp, in
     const SeedKernel long_k = k20 ? (SeedKernel)k_seed<true, true> : (SeedKernel)k_seed<true, false>;
     hipLaunchKernelGGL(short_k, dim3(g), dim3(64 * SEED_WPB), 0, st, b, set, sp, want_syncmers, reset);
     if (long_reads) hipLaunchKernelGGL(long_k, dim3(g), dim3(64 * SEED_WPB), 0, st, b, set, sp, want_syncmers, 0);
+}
+
+void launch_emit_seeds(const DevBatch &b, int syncmers, const uint64_t *off, void *out, hipStream_t st) {
+    if (b.n_reads == 0) return;
+    const unsigned g = grid_for(b.n_reads, WPB);
+    hipLaunchKernelGGL(syncmers ? k_emit_syncmers : k_emit_randstrobes, dim3(g), dim3(64 * WPB), 0, st, b, off,
+                       static_cast<uint64_t *>(out));
 }
 
 void launch_lookup(const DevBatch &b, const ReadSet &set, const DevIndex &ix, int rescue_mode,
