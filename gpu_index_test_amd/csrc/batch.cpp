@@ -75,12 +75,16 @@ uint64_t batch_device_bytes(gis_batch *b) {
     return t;
 }
 
+static void graph_drop(gis_batch::GraphEntry &g) {
+    if (g.exec) (void)hipGraphExecDestroy(g.exec);
+    if (g.graph) (void)hipGraphDestroy(g.graph);
+    g.exec = nullptr;
+    g.graph = nullptr;
+}
+
 void batch_trim(gis_batch *b) {
     HIP_CHECK(hipStreamSynchronize(b->stream));
-    for (auto &g : b->graphs) {
-        HIP_CHECK(hipGraphExecDestroy(g.exec));
-        HIP_CHECK(hipGraphDestroy(g.graph));
-    }
+    for (auto &g : b->graphs) graph_drop(g);
     b->graphs.clear();
     for (DevBuf *x : input_bufs(b)) release(*x);
     for (DevBuf *x : ws_bufs(b->ws)) release(*x);
@@ -96,10 +100,7 @@ void batch_free(gis_batch *b) {
     for (DevBuf *x : input_bufs(b)) release(*x);
     for (auto &e : b->ev)
         if (e) (void)hipEventDestroy(e);
-    for (auto &g : b->graphs) {
-        (void)hipGraphExecDestroy(g.exec);
-        (void)hipGraphDestroy(g.graph);
-    }
+    for (auto &g : b->graphs) graph_drop(g);
     if (b->ws) {
         if (b->ws->owner == b) b->ws->owner = nullptr;
         if (b->ws->in_flight == b) b->ws->in_flight = nullptr;
@@ -121,6 +122,82 @@ uint64_t long_bytes(uint64_t L) {
     auto a8 = [](uint64_t x) { return (x + 7) & ~7ULL; };
     return 16 * L + 8 * (L / 64 + 2) + a8(4 * L) + a8(L) + a8(L) + 64;
 }
+
+// Small host calls (at most SMALL_READS reads and SMALL_BYTES of input): inputs
+// go through h_in and one kernel, results through h_out, so a call is its
+// launches and one wait. Larger calls gain more from the copy engines.
+constexpr uint32_t SMALL_READS = 4096;
+constexpr size_t SMALL_BYTES = 1u << 20;
+
+static size_t a16(size_t x) { return (x + 15) & ~(size_t)15; }
+
+// the places of a small call's results in h_out
+struct HostOut {
+    uint64_t *off;
+    float *frac;
+    uint8_t *flags;
+    gis_nam *nams;
+    uint64_t nam_cap;
+    size_t bytes;
+};
+
+static HostOut host_out(gis_batch *b) {
+    const size_t n = b->n_reads;
+    HostOut h;
+    const size_t o_frac = a16(8 * (n + 1)), o_flags = o_frac + a16(4 * n), o_nams = o_flags + a16(n);
+    h.nam_cap = 16 * n + 1024;
+    h.bytes = o_nams + sizeof(gis_nam) * h.nam_cap;
+    uint8_t *p = b->ws->h_out.data();
+    h.off = reinterpret_cast<uint64_t *>(p);
+    h.frac = reinterpret_cast<float *>(p + o_frac);
+    h.flags = p + o_flags;
+    h.nams = reinterpret_cast<gis_nam *>(p + o_nams);
+    return h;
+}
+
+// all of `items` through h_in and one launch on the batch's stream (and the
+// control block cleared, with ctl); the batch's earlier work has been waited for
+static void copy_in_small(gis_batch *b, const std::vector<CopyItem> &items, DevCtl *ctl) {
+    CopyList c{};
+    size_t at = 0;
+    for (const CopyItem &i : items) at += a16(i.bytes);
+    b->h_in.resize(at + 16);
+    at = 0;
+    for (const CopyItem &i : items) {
+        if (!i.bytes) continue;
+        std::memcpy(b->h_in.data() + at, i.src, i.bytes);
+        c.src[c.n] = b->h_in.data() + at;
+        c.dst[c.n] = i.dst;
+        c.bytes[c.n] = (uint32_t)i.bytes;
+        c.block[c.n + 1] = c.block[c.n] + (uint32_t)((i.bytes + CopyList::BLOCK_BYTES - 1) / CopyList::BLOCK_BYTES);
+        c.n++;
+        at += a16(i.bytes);
+    }
+    launch_copy_in(c, ctl, b->stream);
+}
+
+// Enqueue staged inputs; true when they went the small way. The caller's arrays
+// are read until the stream has been waited for.
+static bool copy_in(gis_batch *b, const std::vector<CopyItem> &items) {
+    size_t bytes = 0;
+    for (const CopyItem &i : items) bytes += i.bytes;
+    const bool small = b->n_reads <= SMALL_READS && bytes <= SMALL_BYTES && items.size() <= CopyList::MAX;
+    if (small) copy_in_small(b, items, nullptr);
+    else
+        for (const CopyItem &c : items)
+            HIP_CHECK(hipMemcpyAsync(c.dst, c.src, c.bytes, hipMemcpyHostToDevice, b->stream));
+    return small;
+}
+
+// waits for the stream when a call leaves it early, so that the pinned blocks and
+// the caller's arrays are free
+struct StreamGuard {
+    hipStream_t st;
+    bool armed = true;
+    ~StreamGuard() {
+        if (armed) (void)hipStreamSynchronize(st);
+    }
+};
 
 DevBatch make_devbatch(gis_batch *b) {
     DevBatch d{};
@@ -171,6 +248,14 @@ DevBatch make_devbatch(gis_batch *b) {
     d.long_scratch = static_cast<uint8_t *>(b->ws->long_scratch.p);
     d.ctl = static_cast<DevCtl *>(b->ws->ctl.p);
     d.spill_ids = static_cast<uint32_t *>(b->ws->spill_ids.p);
+    if (b->host_out) {
+        const HostOut h = host_out(b);
+        d.nams_out = h.nams;
+        d.out_cap = h.nam_cap;
+        d.h_off = h.off;
+        d.h_frac = h.frac;
+        d.h_flags = h.flags;
+    }
     return d;
 }
 
@@ -291,6 +376,7 @@ int batch_stage(gis_batch *b, const char *seqs, const uint64_t *offsets, const u
         b->h_long_off[r + 1] = long_at;
     }
     b->n_reads = n;
+    b->host_out = false;
     b->want_sy = want_sy;
     b->n_long = n_long;
     b->queue_ok = want_queue;
@@ -340,7 +426,13 @@ uint32_t rescue_cutoff_of(const gis_ctx *ctx, const gis_map_options &o) {
 }
 
 // The launch sequence of one run, enqueued on the context's stream.
-void enqueue_run(gis_batch *b, int mode, int rescue_mode, uint32_t rcut, uint32_t hard, int stop) {
+// Stage events are recorded only for runs without graphs.
+void enqueue_run(gis_batch *b, const RunOpts &r) {
+    const int mode = r.mode, rescue_mode = r.rescue_mode, stop = r.stop;
+    const uint32_t rcut = r.rcut, hard = r.hard;
+    const auto mark = [&](gis_batch *x, const char *name) {
+        if (!r.graph) gis::mark(x, name);
+    };
     gis_ctx *ctx = b->ctx;
     hipStream_t st = b->stream;
     const DevIndex ix = dev_index(ctx);
@@ -448,12 +540,12 @@ void batch_launch(gis_batch *b, const RunOpts &r) {
                 ++it;
                 continue;
             }
-            HIP_CHECK(hipGraphExecDestroy(it->exec));
-            HIP_CHECK(hipGraphDestroy(it->graph));
+            graph_drop(*it);
             it = b->graphs.erase(it);
         }
     }
     if (r.graph) {
+        bool replay = true;
         const DevBatch key = make_devbatch(b);
         const gis_fused_config &fc = ctx->fcfg;
         const int cfg[11] = {r.mode, r.rescue_mode, (int)r.rcut, (int)r.hard, r.stop,
@@ -468,36 +560,41 @@ void batch_launch(gis_batch *b, const RunOpts &r) {
                 for (auto it = b->graphs.begin(); it != b->graphs.end(); ++it)
                     if (it->used < old->used) old = it;
                 HIP_CHECK(hipStreamSynchronize(st));
-                HIP_CHECK(hipGraphExecDestroy(old->exec));
-                HIP_CHECK(hipGraphDestroy(old->graph));
+                graph_drop(*old);
                 b->graphs.erase(old);
             }
             gis_batch::GraphEntry e{};
             e.key = key;
             e.epoch = ctx->ix.epoch;
             std::memcpy(e.cfg, cfg, sizeof cfg);
+            b->graphs.push_back(e);
+            hit = &b->graphs.back();
+            replay = !b->lazy_graph;
+        }
+        hit->used = ++b->graph_clock;
+        if (replay && !hit->exec) {
+            hipGraph_t g = nullptr;
             HIP_CHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             try {
-                enqueue_run(b, r.mode, r.rescue_mode, r.rcut, r.hard, r.stop);
+                enqueue_run(b, r);
             } catch (...) {
-                hipGraph_t g = nullptr;
                 (void)hipStreamEndCapture(st, &g);
                 if (g) (void)hipGraphDestroy(g);
                 throw;
             }
-            HIP_CHECK(hipStreamEndCapture(st, &e.graph));
-            const hipError_t ie = hipGraphInstantiate(&e.exec, e.graph, nullptr, nullptr, 0);
+            HIP_CHECK(hipStreamEndCapture(st, &g));
+            const hipError_t ie = hipGraphInstantiate(&hit->exec, g, nullptr, nullptr, 0);
             if (ie != hipSuccess) {
-                (void)hipGraphDestroy(e.graph);
+                (void)hipGraphDestroy(g);
+                hit->exec = nullptr;
                 throw HipError{ie, "hipGraphInstantiate"};
             }
-            b->graphs.push_back(e);
-            hit = &b->graphs.back();
+            hit->graph = g;
         }
-        hit->used = ++b->graph_clock;
-        HIP_CHECK(hipGraphLaunch(hit->exec, st));
+        if (replay) HIP_CHECK(hipGraphLaunch(hit->exec, st));
+        else enqueue_run(b, r);
     } else {
-        enqueue_run(b, r.mode, r.rescue_mode, r.rcut, r.hard, r.stop);
+        enqueue_run(b, r);
     }
     HIP_CHECK(hipGetLastError());
 }
@@ -521,6 +618,7 @@ void batch_complete(gis_batch *b, const RunOpts &r) {
         // not final: grow what overflowed now and size the output next time
         if (ovf & (OVF_HITS | OVF_RHITS | OVF_MERGE)) ovf &= ~(unsigned)OVF_OUT;
         if (ovf & OVF_MERGE) b->ws->merge_scratch = true;
+        if (ovf & OVF_OUT) b->host_out = false;  // more NAMs than h_out holds: the large way
         ensure_pools(b, (ovf & OVF_HITS) ? b->ws->h_ctl->tot[0] + b->ws->h_ctl->tot[0] / 8 + 4096 : 0,
                      (ovf & OVF_RHITS) ? b->ws->h_ctl->tot[1] + b->ws->h_ctl->tot[1] / 8 + 4096 : 0,
                      (ovf & OVF_OUT) ? b->ws->tot_nams + b->ws->tot_nams / 8 + 1024 : 0);
@@ -551,6 +649,14 @@ int batch_download(gis_batch *b, gis_nam_out *out) {
         return fail(ctx, GIS_ERR_CAPACITY,
                     "NAM capacity " + std::to_string(out->nam_capacity) + " < " + std::to_string(b->ws->tot_nams));
     hipStream_t st = b->stream;
+    if (b->host_out) {
+        const HostOut h = host_out(b);
+        if (out->nam_offsets) std::memcpy(out->nam_offsets, h.off, 8ull * (n + 1));
+        if (b->ws->tot_nams) std::memcpy(out->nams, h.nams, sizeof(gis_nam) * b->ws->tot_nams);
+        if (out->nonrepetitive_fraction && n) std::memcpy(out->nonrepetitive_fraction, h.frac, 4ull * n);
+        if (out->flags && n) std::memcpy(out->flags, h.flags, n);
+        return GIS_OK;
+    }
     if (out->nam_offsets)
         HIP_CHECK(hipMemcpyAsync(out->nam_offsets, b->ws->nam_off.p, 8ull * (n + 1), hipMemcpyDeviceToHost, st));
     if (b->ws->tot_nams)
@@ -564,7 +670,10 @@ int batch_download(gis_batch *b, gis_nam_out *out) {
 }
 
 gis_batch *scratch_batch(gis_ctx *ctx) {
-    if (!ctx->scratch) ctx->scratch = batch_new(ctx, nullptr);
+    if (!ctx->scratch) {
+        ctx->scratch = batch_new(ctx, nullptr);
+        ctx->scratch->lazy_graph = true;
+    }
     return ctx->scratch;
 }
 
@@ -594,7 +703,8 @@ static int seeds_of(gis_ctx *ctx, const gis_params *params, bool syncmers, const
         ~Reset() { b->seed_params = nullptr; }
     } reset{b};
     b->seed_params = params;
-    if (int rc = batch_upload(b, seqs, offsets, lens, n, syncmers)) return rc;
+    std::vector<CopyItem> items;
+    if (int rc = batch_stage(b, seqs, offsets, lens, n, syncmers, 0, nullptr, &items, false)) return rc;
     Workspace *w = b->ws;
     ensure_read_arrays(b, n);
     ensure_slot_arrays(b, b->tot_rs_cap);
@@ -606,22 +716,45 @@ static int seeds_of(gis_ctx *ctx, const gis_params *params, bool syncmers, const
     w->owner = b;
     b->ran = false;
     hipStream_t st = b->stream;
+    StreamGuard guard{st};
+    const bool small = copy_in(b, items);
     const DevBatch d = make_devbatch(b);
     uint64_t *off = d.nam_off, *tmp = static_cast<uint64_t *>(w->scan_tmp.p);
     launch_seed(d, ReadSet{nullptr, nullptr, n}, make_seed_params(params ? *params : ctx->ix.params), syncmers ? 1 : 0,
                 b->any_long ? 1 : 0, 0, st);
     launch_scan(syncmers ? d.sy_cnt : d.rs_cnt, off, n, tmp, st);
     HIP_CHECK(hipGetLastError());
-    HIP_CHECK(hipMemcpyAsync(&w->h_ctl->tot[2], off + n, 8, hipMemcpyDeviceToHost, st));
-    HIP_CHECK(hipStreamSynchronize(st));
-    const uint64_t total = w->h_ctl->tot[2];
+    const size_t rec = syncmers ? sizeof(gis_syncmer) : sizeof(gis_query_randstrobe);
+    const uint64_t most = syncmers ? b->h_sy_off[n] : b->tot_rs_cap;
+    // a small call's records go straight to pinned memory, as many as its slots
+    // hold at most; a large one's are counted first
+    const bool direct = small && n > 0 && most * rec <= 2 * SMALL_BYTES;
+    uint64_t total = 0;
+    if (direct) {
+        const size_t head = a16(8ull * (n + 1));
+        w->h_out.resize(head + most * rec);
+        uint64_t *h_off = reinterpret_cast<uint64_t *>(w->h_out.data());
+        launch_emit_seeds(d, syncmers ? 1 : 0, off, w->h_out.data() + head, h_off, st);
+        HIP_CHECK(hipGetLastError());
+        HIP_CHECK(hipStreamSynchronize(st));
+        guard.armed = false;
+        total = h_off[n];
+    } else {
+        HIP_CHECK(hipMemcpyAsync(&w->h_ctl->tot[2], off + n, 8, hipMemcpyDeviceToHost, st));
+        HIP_CHECK(hipStreamSynchronize(st));
+        total = w->h_ctl->tot[2];
+    }
     if (n_out) *n_out = total;
     if (total > capacity || (total && !out))
         return fail(ctx, GIS_ERR_CAPACITY, syncmers ? "syncmer capacity too small" : "randstrobe capacity too small");
-    const size_t rec = syncmers ? sizeof(gis_syncmer) : sizeof(gis_query_randstrobe);
+    if (direct) {
+        if (total) std::memcpy(out, w->h_out.data() + a16(8ull * (n + 1)), total * rec);
+        if (out_offsets) std::memcpy(out_offsets, w->h_out.data(), 8ull * (n + 1));
+        return GIS_OK;
+    }
     if (total) {
         ensure<char>(w->seeds, total * rec);
-        launch_emit_seeds(d, syncmers ? 1 : 0, off, w->seeds.p, st);
+        launch_emit_seeds(d, syncmers ? 1 : 0, off, w->seeds.p, nullptr, st);
         HIP_CHECK(hipGetLastError());
         HIP_CHECK(hipMemcpyAsync(out, w->seeds.p, total * rec, hipMemcpyDeviceToHost, st));
     }
@@ -748,9 +881,14 @@ extern "C" int gis_find_nams_batch(gis_ctx *ctx, const char *seqs, const uint64_
     API_BEGIN(ctx)
     const gis_map_options o = opts_or_default(opt);
     gis_batch *b = scratch_batch(ctx);
-    int rc = batch_upload(b, seqs, offsets, lens, n_reads, false);
+    std::vector<CopyItem> items;
+    const int rc = batch_stage(b, seqs, offsets, lens, n_reads, false, 0, nullptr, &items, o.mode == GIS_MODE_FUSED);
     if (rc) return rc;
+    StreamGuard guard{b->stream};
+    b->host_out = copy_in(b, items) && n_reads > 0;
+    if (b->host_out) b->ws->h_out.resize(host_out(b).bytes);
     batch_run(b, o, 0, STOP_NONE);
+    guard.armed = false;
     return batch_download(b, out);
     API_END(ctx)
 }
@@ -765,9 +903,14 @@ static int qrs_run(gis_ctx *ctx, const gis_query_randstrobe *qrs, const uint64_t
     const uint32_t n = n_queries;
     // each read's queries laid out forward strand first, each strand by (start, end, hash)
     const uint64_t total = query_offsets[n];
-    std::vector<uint64_t> hh(total);
-    std::vector<uint32_t> sp(total), cnt(n), nf(n);
-    std::vector<uint64_t> off(n + 1);
+    // the arrays that the seeding would have left, built in pinned memory
+    const size_t o_sp = a16(8 * total), o_cnt = o_sp + a16(4 * total), o_nf = o_cnt + a16(4ull * n),
+                 o_off = o_nf + a16(4ull * n), in_bytes = o_off + 8ull * (n + 1);
+    b->h_in.resize(in_bytes + 16);
+    uint8_t *in = b->h_in.data();
+    uint64_t *hh = reinterpret_cast<uint64_t *>(in), *off = reinterpret_cast<uint64_t *>(in + o_off);
+    uint32_t *sp = reinterpret_cast<uint32_t *>(in + o_sp), *cnt = reinterpret_cast<uint32_t *>(in + o_cnt),
+             *nf = reinterpret_cast<uint32_t *>(in + o_nf);
     std::vector<uint64_t> ord;
     for (uint32_t r = 0; r < n; r++) {
         const uint64_t lo = query_offsets[r], hi = query_offsets[r + 1];
@@ -796,33 +939,47 @@ static int qrs_run(gis_ctx *ctx, const gis_query_randstrobe *qrs, const uint64_t
     b->n_reads = n;
     b->want_sy = false;
     b->any_long = false;
-    b->h_rs_off.assign(off.data(), off.size());
     // the per-read randstrobe offsets are the one input array the stages
     // after seeding read (a fresh context's scratch batch has none yet)
     ensure<uint64_t>(b->rs_off, (size_t)n + 1);
     ensure_read_arrays(b, n);
     ensure_slot_arrays(b, total);
     b->ws->owner = b;
+    b->ran = false;
     ensure_pools(b, (uint64_t)HIT_REGION * n + 16ull * n + 4096, 16ull * n + 4096, 16ull * n + 1024);
     b->tot_rs_cap = total;
+    b->host_out = n > 0 && n <= SMALL_READS && in_bytes <= SMALL_BYTES;
+    if (b->host_out) b->ws->h_out.resize(host_out(b).bytes);
     hipStream_t st = ctx->stream;
-    if (total) {
-        HIP_CHECK(hipMemcpyAsync(b->ws->rs_hash.p, hh.data(), 8 * total, hipMemcpyHostToDevice, st));
-        HIP_CHECK(hipMemcpyAsync(b->ws->rs_span.p, sp.data(), 4 * total, hipMemcpyHostToDevice, st));
+    StreamGuard guard{st};
+    const CopyItem items[] = {{b->ws->rs_hash.p, hh, 8 * total},
+                              {b->ws->rs_span.p, sp, 4 * total},
+                              {b->ws->rs_cnt.p, cnt, 4ull * n},
+                              {b->ws->rs_nfwd.p, nf, 4ull * n},
+                              {b->rs_off.p, off, 8ull * (n + 1)}};
+    const bool small = b->host_out;
+    if (small) {
+        CopyList c{};
+        for (const CopyItem &i : items) {
+            if (!i.bytes) continue;
+            c.src[c.n] = i.src;
+            c.dst[c.n] = i.dst;
+            c.bytes[c.n] = (uint32_t)i.bytes;
+            c.block[c.n + 1] = c.block[c.n] + (uint32_t)((i.bytes + CopyList::BLOCK_BYTES - 1) / CopyList::BLOCK_BYTES);
+            c.n++;
+        }
+        launch_copy_in(c, static_cast<DevCtl *>(b->ws->ctl.p), st);
+    } else {
+        for (const CopyItem &i : items)
+            if (i.bytes) HIP_CHECK(hipMemcpyAsync(i.dst, i.src, i.bytes, hipMemcpyHostToDevice, st));
     }
-    HIP_CHECK(hipMemcpyAsync(b->rs_off.p, off.data(), 8ull * (n + 1), hipMemcpyHostToDevice, st));
-    if (n) {
-        HIP_CHECK(hipMemcpyAsync(b->ws->rs_cnt.p, cnt.data(), 4ull * n, hipMemcpyHostToDevice, st));
-        HIP_CHECK(hipMemcpyAsync(b->ws->rs_nfwd.p, nf.data(), 4ull * n, hipMemcpyHostToDevice, st));
-    }
-    HIP_CHECK(hipStreamSynchronize(st));
     // the stages after seeding, with the rescue decision forced either way
     const DevIndex ix = dev_index(ctx);
     const ReadSet set{nullptr, nullptr, n};
     uint64_t *tmp = static_cast<uint64_t *>(b->ws->scan_tmp.p);
     for (int attempt = 0; attempt < 6; attempt++) {
         const DevBatch d = make_devbatch(b);
-        launch_reset_ctl(d.ctl, st);
+        if (attempt > 0 || !small) launch_reset_ctl(d.ctl, st);
         launch_lookup(d, set, ix, rescue ? 2 : 1, st);
         launch_hits(d, ix, rescue_cutoff, hard_cutoff, st);
         launch_merge(d, set, st);
@@ -835,10 +992,12 @@ static int qrs_run(gis_ctx *ctx, const gis_query_randstrobe *qrs, const uint64_t
         if (attempt == 5) throw HipError{hipErrorOutOfMemory, "batch arrays still too small after regrowth"};
         if (ovf & (OVF_HITS | OVF_RHITS | OVF_MERGE)) ovf &= ~(unsigned)OVF_OUT;
         if (ovf & OVF_MERGE) b->ws->merge_scratch = true;
+        if (ovf & OVF_OUT) b->host_out = false;
         ensure_pools(b, (ovf & OVF_HITS) ? b->ws->h_ctl->tot[0] + 4096 : 0,
                      (ovf & OVF_RHITS) ? b->ws->h_ctl->tot[1] + 4096 : 0,
                      (ovf & OVF_OUT) ? b->ws->tot_nams + 1024 : 0);
     }
+    guard.armed = false;
     b->ran = true;
     return batch_download(b, out);
 }
@@ -862,6 +1021,12 @@ struct QrsCall {
 };
 
 int run_combined(gis_ctx *ctx, std::vector<QrsCall *> &calls) {
+    // a call on its own needs no joined arrays
+    if (calls.size() == 1 && calls[0]->qoff[0] == 0) {
+        QrsCall *c = calls[0];
+        c->rc = qrs_run(ctx, c->qrs, c->qoff, c->n, c->rescue, c->rcut, c->hard, c->out);
+        return c->rc;
+    }
     // one batch: the calls' reads back to back
     uint32_t n = 0;
     uint64_t nq = 0;

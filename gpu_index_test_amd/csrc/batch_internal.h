@@ -94,6 +94,7 @@ struct Workspace {
     DevCtl *h_ctl = nullptr;
     DevCtl *h_ctl_dev = nullptr;
     int refs = 0;
+    Pinned<uint8_t> h_out;        // results of small host calls, written by the kernels
     PairWork *pairs = nullptr;    // the pair step on this workspace's NAMs (pairs.cpp)
 };
 
@@ -118,6 +119,13 @@ struct gis_batch {
     // seeding parameters of a run that needs no index (else the index's)
     const gis_params *seed_params = nullptr;
     gis::Workspace *ws = nullptr;
+    // small host calls: their inputs gathered in pinned memory, and whether the
+    // run writes its results to the workspace's h_out
+    gis::Pinned<uint8_t> h_in;
+    bool host_out = false;
+    // capture a graph only when a launch sequence is met again: calls of ever
+    // new sizes would pay a capture each
+    bool lazy_graph = false;
     int last_mode = GIS_MODE_PLAIN;
     bool last_graph = false;
     bool ran = false;
@@ -130,7 +138,7 @@ struct gis_batch {
         int cfg[11];
         uint64_t epoch;  // the index table the graph was captured against
         hipGraph_t graph;
-        hipGraphExec_t exec;
+        hipGraphExec_t exec;  // null: met once, not captured yet (lazy_graph)
         uint64_t used;
     };
     std::vector<GraphEntry> graphs;

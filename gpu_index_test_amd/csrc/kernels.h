@@ -129,6 +129,11 @@ struct DevBatch {
     uint64_t *nam_off;        // [n+1]
     gis_nam *nams_out;
     uint64_t out_cap;
+    // small host calls: nams_out is pinned host memory, and so are these copies
+    // of nam_off, frac and flags (else null)
+    uint64_t *h_off;
+    float *h_frac;
+    uint8_t *h_flags;
     // long-read scratch for the seeding stage (byte offsets)
     const uint64_t *long_off;
     uint8_t *long_scratch;
@@ -157,7 +162,21 @@ constexpr uint32_t HIT_REGION = 128;
 
 constexpr uint32_t BUCKET_LINE = 8;  // uint4 per bucket line
 
+// Up to MAX small blocks of pinned host memory that one launch copies into device
+// arrays (launch_copy_in). Sources and destinations are 16-byte aligned.
+struct CopyList {
+    static constexpr int MAX = 8;
+    static constexpr uint32_t BLOCK_BYTES = 16384;  // bytes a thread block copies
+    const void *src[MAX];
+    void *dst[MAX];
+    uint32_t bytes[MAX];
+    uint32_t block[MAX + 1];  // first thread block of each item; block[n] = all of them
+    int n;
+};
+
 // launch wrappers (kernels.hip)
+// copies, and with ctl the control block cleared (ctl may be null)
+void launch_copy_in(const CopyList &c, DevCtl *ctl, hipStream_t st);
 void launch_bucket_lines(const uint4 *rs, const uint64_t *starts, int bits, uint4 *lines, hipStream_t st);
 void launch_reset_ctl(DevCtl *ctl, hipStream_t st);
 // reset: the control block is cleared by the first launch (the seeding does not
@@ -165,8 +184,9 @@ void launch_reset_ctl(DevCtl *ctl, hipStream_t st);
 void launch_seed(const DevBatch &b, const ReadSet &set, const SeedParams &sp, int want_syncmers,
                  int long_reads, int reset, hipStream_t st);
 // the seeds dense and in read order (gis_query_randstrobe or gis_syncmer records
-// at off[r] of out)
-void launch_emit_seeds(const DevBatch &b, int syncmers, const uint64_t *off, void *out, hipStream_t st);
+// at off[r] of out); h_off (may be null): a host copy of off
+void launch_emit_seeds(const DevBatch &b, int syncmers, const uint64_t *off, void *out, uint64_t *h_off,
+                       hipStream_t st);
 // rescue_mode: 0 = the caller's decision (nonrepetitive fraction < 0.7 or no
 // hits), 1 = never rescue, 2 = always rescue
 void launch_lookup(const DevBatch &b, const ReadSet &set, const DevIndex &ix, int rescue_mode,

@@ -430,11 +430,20 @@ __global__ __launch_bounds__(64 * SEED_WPB) __attribute__((amdgpu_waves_per_eu(6
 // stores are whole lines; a read's slots are several times its seeds, and
 // copying them to the host and packing there took most of the call (20,011
 // reads of 150 bp: 14.9 ms; now bound by the copy of the records).
-__global__ __launch_bounds__(64 * WPB) void k_emit_randstrobes(DevBatch b, const uint64_t *off, uint64_t *out) {
+__device__ __forceinline__ void emit_offset(const DevBatch &b, const uint64_t *off, uint32_t r, uint64_t o,
+                                            uint64_t *h_off) {
+    h_off[r] = o;
+    if (r + 1 == b.n_reads) h_off[r + 1] = sload(off + r + 1);
+}
+
+__global__ __launch_bounds__(64 * WPB) void k_emit_randstrobes(DevBatch b, const uint64_t *off, uint64_t *out,
+                                                         uint64_t *h_off) {
     for (uint32_t r = wave_index(WPB); r < b.n_reads; r += gridDim.x * WPB) {
         const uint32_t n = sload(b.rs_cnt + r), half = sload(b.rs_nfwd + r);
         const uint64_t base = sload(b.rs_off + r);
-        uint64_t *dst = out + 3 * sload(off + r);
+        const uint64_t o = sload(off + r);
+        uint64_t *dst = out + 3 * o;
+        if (h_off && lane_id() == 0) emit_offset(b, off, r, o, h_off);
         for (uint32_t w = lane_id(); w < 3 * n; w += 64) {
             const uint32_t j = w / 3, c = w - 3 * j;
             const uint32_t sp = b.rs_span[base + j];
@@ -444,11 +453,14 @@ __global__ __launch_bounds__(64 * WPB) void k_emit_randstrobes(DevBatch b, const
     }
 }
 
-__global__ __launch_bounds__(64 * WPB) void k_emit_syncmers(DevBatch b, const uint64_t *off, uint64_t *out) {
+__global__ __launch_bounds__(64 * WPB) void k_emit_syncmers(DevBatch b, const uint64_t *off, uint64_t *out,
+                                                      uint64_t *h_off) {
     for (uint32_t r = wave_index(WPB); r < b.n_reads; r += gridDim.x * WPB) {
         const uint32_t n = sload(b.sy_cnt + r);
         const uint64_t base = sload(b.sy_off + r);
-        uint64_t *dst = out + 2 * sload(off + r);
+        const uint64_t o = sload(off + r);
+        uint64_t *dst = out + 2 * o;
+        if (h_off && lane_id() == 0) emit_offset(b, off, r, o, h_off);
         for (uint32_t w = lane_id(); w < 2 * n; w += 64) dst[w] = (w & 1 ? b.sy_pos : b.sy_hash)[base + (w >> 1)];
     }
 }
@@ -2412,7 +2424,10 @@ __global__ __launch_bounds__(64 * WPB) void k_compact(DevBatch b, int fused, con
     const uint32_t lane = lane_id();
     if (blockIdx.x == 0 && threadIdx.x < 64) {
         const uint64_t total = ntiles ? wave_sum_of(tiles, ntiles) : b.nam_off[b.n_reads];
-        if (lane == 0) b.nam_off[b.n_reads] = total;
+        if (lane == 0) {
+            b.nam_off[b.n_reads] = total;
+            if (b.h_off) b.h_off[b.n_reads] = total;
+        }
         ctl_store(b, dst, total, total > b.out_cap ? (unsigned)OVF_OUT : 0u);
     }
     // the merges did not run and the counts are stale
@@ -2435,7 +2450,14 @@ __global__ __launch_bounds__(64 * WPB) void k_compact(DevBatch b, int fused, con
         // (a wave's reads lie in one tile)
         const uint32_t tile = r0 / SCAN_TILE;
         const uint64_t no = in_tile + (ntiles ? wave_sum_of(tiles, tile) : tiles[tile]);
-        if (j == 0 && r < b.n_reads) b.nam_off[r] = no;
+        if (j == 0 && r < b.n_reads) {
+            b.nam_off[r] = no;
+            if (b.h_off) {
+                b.h_off[r] = no;
+                b.h_frac[r] = b.frac[r];
+                b.h_flags[r] = fl;
+            }
+        }
         const uint32_t c = r < b.n_reads && no + c0 <= b.out_cap ? c0 : 0u;
         const gis_nam *srcn;
         if (fused && !(fl & FLAG_SPILL)) srcn = b.nam_slots + (uint64_t)rr * F_NAMCAP;
@@ -2543,7 +2565,10 @@ __global__ __launch_bounds__(SCAN_BLOCK) void k_scan_tiles(const uint32_t *in, u
         if (base + j < n) out[base + j] = ex;
         ex += v[j];
     }
-    if (threadIdx.x == 0) tile_sums[blockIdx.x] = tot;
+    if (threadIdx.x == 0) {
+        tile_sums[blockIdx.x] = tot;
+        if (gridDim.x == 1) out[n] = tot;
+    }
 }
 
 // single block: exclusive scan of the tile sums in place; out[n] = total
@@ -2644,6 +2669,31 @@ void launch_bucket_lines(const uint4 *rs, const uint64_t *starts, int bits, uint
     hipLaunchKernelGGL(k_bucket_lines, dim3((unsigned)(g < 65536 ? g : 65536)), dim3(256), 0, st, rs, starts, nb, lines);
 }
 
+// The inputs of a small call from one pinned block into their device arrays, read
+// over PCIe by the kernel itself: seven hipMemcpyAsync of a few kilobytes cost
+// 5-10 us each on the host and a blit kernel each on the device.
+__global__ __launch_bounds__(256) void k_copy_in(CopyList c, DevCtl *ctl) {
+    if (ctl && blockIdx.x == 0) ctl_clear(ctl);
+    int i = 0;
+    while (i + 1 < c.n && blockIdx.x >= c.block[i + 1]) i++;
+    if (blockIdx.x >= c.block[c.n]) return;
+    const uint32_t at = (blockIdx.x - c.block[i]) * CopyList::BLOCK_BYTES, bytes = c.bytes[i];
+    const char *src = static_cast<const char *>(c.src[i]);
+    char *dst = static_cast<char *>(c.dst[i]);
+#pragma unroll
+    for (uint32_t u = 0; u < CopyList::BLOCK_BYTES / 4096; u++) {
+        const uint32_t o = at + u * 4096 + threadIdx.x * 16;
+        if (o + 16 <= bytes) *reinterpret_cast<uint4 *>(dst + o) = *reinterpret_cast<const uint4 *>(src + o);
+        else
+            for (uint32_t k = o; k < bytes; k++) dst[k] = src[k];
+    }
+}
+
+void launch_copy_in(const CopyList &c, DevCtl *ctl, hipStream_t st) {
+    const unsigned g = c.block[c.n] ? c.block[c.n] : 1u;
+    hipLaunchKernelGGL(k_copy_in, dim3(g), dim3(256), 0, st, c, ctl);
+}
+
 void launch_reset_ctl(DevCtl *ctl, hipStream_t st) {
     hipLaunchKernelGGL(k_reset_ctl, dim3(1), dim3(64), 0, st, ctl);
 }
@@ -2663,11 +2713,12 @@ void launch_seed(const DevBatch &b, const ReadSet &set, const SeedParams &sp, in
     if (long_reads) hipLaunchKernelGGL(long_k, dim3(g), dim3(64 * SEED_WPB), 0, st, b, set, sp, want_syncmers, 0);
 }
 
-void launch_emit_seeds(const DevBatch &b, int syncmers, const uint64_t *off, void *out, hipStream_t st) {
+void launch_emit_seeds(const DevBatch &b, int syncmers, const uint64_t *off, void *out, uint64_t *h_off,
+                       hipStream_t st) {
     if (b.n_reads == 0) return;
     const unsigned g = grid_for(b.n_reads, WPB);
     hipLaunchKernelGGL(syncmers ? k_emit_syncmers : k_emit_randstrobes, dim3(g), dim3(64 * WPB), 0, st, b, off,
-                       static_cast<uint64_t *>(out));
+                       static_cast<uint64_t *>(out), h_off);
 }
 
 void launch_lookup(const DevBatch &b, const ReadSet &set, const DevIndex &ix, int rescue_mode,
@@ -2770,6 +2821,7 @@ void launch_scan(const uint32_t *in, uint64_t *out, uint64_t n, uint64_t *tmp, h
     const unsigned tiles = grid_for(n ? n : 1, SCAN_TILE);
     if (n > 0 && tiles <= SCAN_FEW_TILES) {
         hipLaunchKernelGGL(k_scan_tiles, dim3(tiles), dim3(SCAN_BLOCK), 0, st, in, out, n, tmp);
+        if (tiles == 1) return;
         hipLaunchKernelGGL(k_scan_add_few, dim3(tiles), dim3(SCAN_BLOCK), 0, st, out, n, tmp, (uint32_t)tiles);
         return;
     }

@@ -122,3 +122,39 @@ def test_output_offsets_over_tiles(ctx, n):
     assert np.array_equal(np.diff(res.nam_offsets), np.where(l == 150, len(one.nams), 0))
     assert res.nam_offsets[0] == 0 and res.nams.tobytes() == one.nams.tobytes() * k
     idx.ctx.close()
+
+
+@pytest.mark.parametrize("mode", [G.MODE_PLAIN, G.MODE_FUSED])
+def test_host_calls_of_any_size(ctx, mode):
+    """Host-buffer calls around the size up to which inputs and results go
+    through pinned memory, empty and single ones, and reads with more NAMs
+    than that way has room for; each size three times (the third replays a
+    captured graph), interleaved with the others."""
+    g, lens = G.synth_genome(300_000, n_contigs=2, gc=0.45, repeat_fraction=0.5, n_families=3,
+                             family_len=(2000, 3000), copies=(40, 50), divergence=(0.0, 0.01), seed=31)
+    idx = G.StrobemerIndex(None, G.IndexParameters.from_read_length(150))
+    idx.populate_arrays(g, lens)
+    oidx = O.Index.build_arrays(g, lens, O.params_from_read_length(150), n_threads=4)
+    cases = []
+    for n in (0, 1, 2, 63, 700, 4095, 4096, 4097, 9000):
+        s, o, l, _ = G.synth_reads(g, lens, n, lengths=(60, 150, 201), weights=(1, 2, 1), sub_rate=0.004, seed=n + 1)
+        cases.append((s, o, l) + (O.map_batch(oidx, s, o, l, 2 * oidx.filter_cutoff, 1000, 4) if n else
+                                  (np.zeros(1, np.uint64), np.zeros(0, G.NAM), np.zeros(0, np.float32), np.zeros(0, np.uint8))))
+    assert any(len(en) > 16 * len(l) + 1024 for _, _, l, _, en, _, _ in cases if 0 < len(l) <= 4096)
+    for _ in range(3):
+        for s, o, l, eo, en, ef, efl in cases:
+            res = G.find_nams_batch(idx, s, o, l, mode=mode)
+            assert np.array_equal(res.nam_offsets, eo) and res.nams.tobytes() == en.tobytes()
+            assert res.nonrepetitive_fraction.tobytes() == ef.tobytes() and np.array_equal(res.flags & 1, efl & 1)
+    # the seeding entry points over the same sizes
+    if mode == G.MODE_PLAIN:
+        op = O.params_from_read_length(150)
+        for s, o, l, *_ in cases:
+            off, q = G.randstrobes_batch(idx, s, o, l)
+            soff, sy = G.syncmers_batch(idx, s, o, l)
+            assert off[0] == 0 and off[-1] == len(q) and soff[0] == 0 and soff[-1] == len(sy)
+            for r in range(0, len(l), 97):
+                read = s[int(o[r]): int(o[r]) + int(l[r])].tobytes()
+                assert q[int(off[r]): int(off[r + 1])].tobytes() == O.randstrobes_query(read, op).tobytes()
+                assert sy[int(soff[r]): int(soff[r + 1])].tobytes() == O.syncmers(read, op).tobytes()
+    idx.ctx.close()
