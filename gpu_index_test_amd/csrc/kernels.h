@@ -27,7 +27,7 @@ struct DevIndex {
 
 // One hit (step2/my_struct.hpp:71-86) with its grouping key:
 // ref_strand = is_rc << 31 | ref_id.
-struct DevHit {
+struct alignas(16) DevHit {
     uint32_t ref_strand;
     int32_t ref_start;
     int32_t ref_end;

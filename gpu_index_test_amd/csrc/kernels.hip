@@ -103,8 +103,8 @@ __device__ __forceinline__ bool syncmer_fast(int L, const SeedParams &P, const S
             is_sync = h < m;
             tie = h == m;
         }
-        if (__ballot(tie)) return false;
-        const uint64_t bal = __ballot(is_sync);
+        if (ballot(tie)) return false;
+        const uint64_t bal = ballot(is_sync);
         if (is_sync) {
             const uint32_t idx = n + mbcnt(bal);
             if (idx < cap) B.sy_pos[idx] = (uint16_t)p;
@@ -169,7 +169,7 @@ __device__ __forceinline__ uint32_t syncmer_passes(int L, const SeedParams &P, c
             }
             is_sync = st == (uint8_t)(P.t - 1);
         }
-        const uint64_t bal = __ballot(is_sync);
+        const uint64_t bal = ballot(is_sync);
         if (is_sync) {
             const uint32_t idx = nsync + mbcnt(bal);
             if (idx < cap) B.sy_pos[idx] = (uint16_t)p;
@@ -236,7 +236,7 @@ __device__ __forceinline__ uint32_t seed_syncmers(const char *__restrict__ seq, 
     }
     wave_sync();
     uint32_t nsync = 0;
-    const bool clean = __ballot(any != 0) == 0;  // wave-uniform
+    const bool clean = ballot(any != 0) == 0;  // wave-uniform
     if (!(clean && syncmer_fast(L, P, B, cap, out_sy_pos, nsync))) {
         // the mask of non-ACGT bases (step2/randstrobes.cu:70-76): bit 4 l + b
         // of 16 lanes' words from the ballots of their byte b
@@ -248,7 +248,7 @@ __device__ __forceinline__ uint32_t seed_syncmers(const char *__restrict__ seq, 
             uint64_t m = 0;
 #pragma unroll
             for (int q = 0; q < 4; q++) {
-                const uint64_t bal = __ballot(((bad >> (8 * q)) & 0xffu) != 0);
+                const uint64_t bal = ballot(((bad >> (8 * q)) & 0xffu) != 0);
                 uint64_t x = lane < 4 ? (bal >> (16 * lane)) & 0xffffull : 0ull;
                 x = (x | (x << 24)) & 0x000000ff000000ffull;
                 x = (x | (x << 12)) & 0x000f000f000f000full;
@@ -607,7 +607,7 @@ __device__ __forceinline__ uint32_t walk_run_wave(const DevIndex &ix, uint64_t p
             in = ((uint64_t)v.x | ((uint64_t)v.y << 32)) == key;
         }
         // equal hashes are contiguous: the run ends at the first other record
-        const uint64_t other = __ballot(!in);
+        const uint64_t other = ballot(!in);
         const uint32_t len = other ? (uint32_t)__builtin_ctzll(other) : 64u;
         const bool valid = lane < len;
         const int rspan = (int)(v.w & 0xffu) + ix.k;
@@ -622,7 +622,7 @@ __device__ __forceinline__ uint32_t walk_run_wave(const DevIndex &ix, uint64_t p
         if (lane == 0) excl = 0x7fffffff;
         excl = carry < excl ? carry : excl;
         const bool keep = valid && d <= excl;
-        const uint64_t km = __ballot(keep);
+        const uint64_t km = ballot(keep);
         if (out && keep) {
             DevHit hh;
             hh.ref_strand = strand_bit | (v.w >> 8);
@@ -970,7 +970,7 @@ __device__ __forceinline__ void rescued_hits(const DevBatch &b, const DevIndex &
             coop = taken && c > WALK_WAVE_MIN;
         }
         // long runs: the whole wave walks each one
-        uint64_t cm = __ballot(coop);
+        uint64_t cm = ballot(coop);
         while (cm) {
             const uint32_t l = (uint32_t)__builtin_ctzll(cm);
             cm &= cm - 1;
@@ -1006,7 +1006,7 @@ __device__ __forceinline__ void rescued_hits(const DevBatch &b, const DevIndex &
         if (rh > 0 && !coop)
             walk_run(ix, b.pos[base + i], b.rs_hash[base + i], (int)span_start(b.rs_span[base + i]),
                      (int)span_end(b.rs_span[base + i]), i >= half ? 0x80000000u : 0u, out + carry + incl - rh);
-        uint64_t cm = __ballot(coop);
+        uint64_t cm = ballot(coop);
         while (cm) {
             const uint32_t l = (uint32_t)__builtin_ctzll(cm);
             cm &= cm - 1;
@@ -1060,19 +1060,6 @@ __device__ __forceinline__ bool hits_missing(const DevBatch &b) {
 // scanned 64 entries at a time (the "wide" form), retiring dead NAMs as the
 // list grows.
 
-__device__ __forceinline__ void bitonic_regs(uint64_t &key) {
-    const uint32_t lane = lane_id();
-    for (uint32_t size = 2; size <= 64; size <<= 1) {
-        for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
-            const uint64_t other = __shfl_xor(key, (int)stride, 64);
-            const bool asc = (lane & size) == 0;
-            const bool lower = (lane & stride) == 0;
-            const uint64_t mn = key < other ? key : other, mx = key < other ? other : key;
-            key = (lower == asc) ? mn : mx;
-        }
-    }
-}
-
 __device__ __forceinline__ void bitonic_mem(uint64_t *keys, uint32_t P) {
     const uint32_t lane = lane_id();
     for (uint32_t size = 2; size <= P; size <<= 1) {
@@ -1106,7 +1093,7 @@ __device__ __forceinline__ uint64_t *radix_sort_groups(uint64_t *src, uint64_t *
             const uint32_t i = i0 + lane;
             const uint32_t d = i < n ? (uint32_t)(src[i] >> shift) & 15u : 16u;
 #pragma unroll
-            for (int v = 0; v < 16; v++) off[v] += (uint32_t)__popcll(__ballot(d == (uint32_t)v));
+            for (int v = 0; v < 16; v++) off[v] += (uint32_t)__popcll(ballot(d == (uint32_t)v));
         }
         uint32_t run = 0;
 #pragma unroll
@@ -1126,7 +1113,7 @@ __device__ __forceinline__ uint64_t *radix_sort_groups(uint64_t *src, uint64_t *
             uint32_t pos = 0;
 #pragma unroll
             for (int v = 0; v < 16; v++) {
-                const uint64_t bal = __ballot(d == (uint32_t)v);
+                const uint64_t bal = ballot(d == (uint32_t)v);
                 if (d == (uint32_t)v) pos = off[v] + mbcnt(bal);
                 off[v] += (uint32_t)__popcll(bal);
             }
@@ -1254,7 +1241,7 @@ __device__ __forceinline__ const uint64_t *group_order(uint32_t nh, const DevHit
             if (i > 0 && hits[i - 1].ref_strand > rsd) unsorted = 1;
         }
     }
-    if (__ballot(unsorted != 0) != 0) {
+    if (ballot(unsorted != 0) != 0) {
         if (nh <= (uint32_t)MERGE_LDS) {
             uint32_t P = 1;
             while (P < nh) P <<= 1;
@@ -1312,19 +1299,157 @@ __device__ __forceinline__ void boxes_rebuild(const WideList &wide, uint32_t nw,
     }
 }
 
+// the NAM list of a strand or group in the lanes of a wave: dead NAMs (query end
+// before qs: they can take no further hit) leave, the others move up in order.
+// Returns the open count; dst of a dead NAM is out[base + cid].
+__device__ __forceinline__ uint32_t retire_lanes(LaneNam &o, int qs, gis_nam *out, uint32_t base, uint32_t grp,
+                                                 uint32_t cap) {
+    const bool keep = o.qe >= qs;
+    const uint64_t km = ballot(keep);
+    const uint32_t nk = (uint32_t)__popcll(km);
+    if (nk == 64) return nk;
+    if (!keep && base + o.cid < cap) lane_nam_store(out, base + o.cid, grp, o);
+    const uint32_t dst = keep ? mbcnt(km) : nk + mbcnt(~km);
+    o.qs = permute_push(o.qs, dst);
+    o.qe = permute_push(o.qe, dst);
+    o.qp = permute_push(o.qp, dst);
+    o.rs = permute_push(o.rs, dst);
+    o.re = permute_push(o.re, dst);
+    o.rp = permute_push(o.rp, dst);
+    o.n = permute_push(o.n, dst);
+    o.cid = (uint32_t)permute_push((int)o.cid, dst);
+    return nk;
+}
+
+// One hit against the NAMs of a wave's lanes: the first of the accepting lanes acc
+// takes it, else the lane `free` (its one bit; lanes from there on accept
+// nothing) opens a NAM with it. Returns the lane's bit, 0 when no lane can: then
+// nothing changed. mk: that bit if it opened one. Masks and selects, no
+// branches: the hit and the masks live in scalar registers.
+__device__ __forceinline__ uint64_t lanes_take(LaneNam &o, uint64_t acc, uint64_t ext, uint64_t free, uint64_t &mk,
+                                               uint32_t cid, int qs, int qe, int rs, int re) {
+    const uint64_t x = acc | free, me = x & (0 - x);
+    mk = me & free;
+    const bool b_me = lane_bit(me), b_mk = lane_bit(mk), b_end = lane_bit(mk | (me & ext));
+    o.qs = b_mk ? qs : o.qs;
+    o.rs = b_mk ? rs : o.rs;
+    o.cid = b_mk ? cid : o.cid;
+    o.qe = b_end ? qe : o.qe;
+    o.re = b_end ? re : o.re;
+    o.qp = b_me ? qs : o.qp;
+    o.rp = b_me ? rs : o.rp;
+    o.n += b_me ? 1 : 0;  // (0 on a free lane)
+    return me;
+}
+
+// Merge of a read's hits in arrival order on one wave, a NAM a lane, without
+// grouping them: NAMs of every group of the current strand share the lanes, and
+// a NAM only accepts hits of its own group, which arrive in (query_start,
+// ref_start) order. A strand's NAMs are ranked by (ref_id, creation) when its
+// hits end. With one group on the strand (a read of one place, the usual case)
+// creation order is the rank, so dead NAMs may leave when the lanes are full.
+// Returns the NAM count (entries at index >= cap are not written), or
+// MERGE_OVERFLOW when a strand needs more than 64 lanes.
+//
+// A lone wave's time is its chain of instructions a hit (one issues every ~8
+// cycles), branches above all: the loop over hits has none but its end and the
+// full-lanes exit (~550 cycles a hit; the group-by-group merge took ~800 with
+// its sort and block tests before it).
+__device__ __forceinline__ uint32_t merge_arrival(const DevHit *hits, uint32_t nh, gis_nam *out, uint32_t cap) {
+    const uint32_t lane = lane_id();
+    const uint4 *hv = reinterpret_cast<const uint4 *>(hits);
+    // forward hits, and whether a strand holds more than one group (against its
+    // first forward and its last reverse hit)
+    uint32_t nf = 0;
+    bool other[2] = {false, false};
+    {
+        const uint32_t h0 = uni32(hv[0].x), hl = uni32(hv[nh ? nh - 1 : 0].x);
+        uint64_t of = 0, orv = 0;
+        for (uint32_t x0 = 0; x0 < nh; x0 += 64) {
+            const bool in = x0 + lane < nh;
+            const uint32_t r = in ? hv[x0 + lane].x : 0xffffffffu;
+            const uint64_t fwd = ballot(r >> 31 == 0);
+            nf += (uint32_t)__popcll(fwd);
+            of |= ballot(r != h0) & fwd;
+            orv |= ballot(in && r != hl) & ~fwd;
+        }
+        other[0] = of != 0;
+        other[1] = orv != 0;
+    }
+    uint32_t base = 0;
+    for (int strand = 0; strand < 2; strand++) {
+        const uint32_t xb = strand ? nf : 0u, xe = strand ? nh : nf;
+        const bool multi = other[strand];
+        LaneNam o{0, 0, 0, 0, 0, 0, 0, 0};
+        uint32_t rsd_o = 0xffffffffu;  // this lane's group (no hit's when the lane is free)
+        uint32_t made = 0;
+        uint64_t free = 1;
+        for (uint32_t x0 = xb; x0 < xe; x0 += 64) {
+            uint4 c = make_uint4(0u, 0u, 0u, 0u);
+            if (x0 + lane < xe) c = hv[x0 + lane];
+            const uint32_t m = xe - x0 < 64 ? xe - x0 : 64;
+            for (uint32_t t = 0;;) {
+                uint32_t rsd = 0;
+                int qs = 0;
+                for (; t < m; t++) {
+                    rsd = readlane_u32(c.x, t);
+                    const uint32_t q = readlane_u32(c.w, t);
+                    const int rs = (int)readlane_u32(c.y, t), re = (int)readlane_u32(c.z, t), qe = (int)(q >> 16);
+                    qs = (int)(q & 0xffffu);
+                    const uint64_t xq = ballot(qe > o.qe), xr = ballot(re > o.re);
+                    const uint64_t acc = ballot(rsd_o == rsd) & ballot(o.qp < qs) & ballot(qs <= o.qe) &
+                                         ballot(o.rp < rs) & ballot(rs <= o.re) & ~(xq ^ xr);
+                    uint64_t mk;
+                    const uint64_t me = lanes_take(o, acc, xq & xr, free, mk, made, qs, qe, rs, re);
+                    rsd_o = lane_bit(mk) ? rsd : rsd_o;
+                    const uint32_t fresh = mk != 0 ? 1u : 0u;
+                    made += fresh;
+                    free <<= fresh;
+                    if (me == 0) break;  // no room: the hit waits
+                }
+                if (t == m) break;
+                if (multi) return MERGE_OVERFLOW;
+                const uint32_t n_open = retire_lanes(o, qs, out, base, rsd, cap);
+                if (n_open == 64) return MERGE_OVERFLOW;
+                rsd_o = lane < n_open ? rsd_o : 0xffffffffu;
+                o.n = lane < n_open ? o.n : 0;
+                free = 1ull << n_open;
+            }
+        }
+        // the strand's NAMs are final
+        uint32_t rank = o.cid;
+        if (multi) {  // nothing was retired: NAM c sits on lane c
+            rank = 0;
+            for (uint32_t q = 0; q < made; q++) {
+                const uint32_t k = readlane_u32(rsd_o, q);
+                rank += (k < rsd_o) | ((k == rsd_o) & (q < lane)) ? 1u : 0u;
+            }
+        }
+        if (o.n > 0 && base + rank < cap) lane_nam_store(out, base + rank, rsd_o, o);
+        base += made;
+    }
+    return base;
+}
+
 // Merge hits order[xb .. xe) (hit indices in grouped order; order nullptr:
-// the hits themselves in order), or, with pre, the xe <= 64 hits already in
-// the chunk registers. NAM c of the k-th group of the range is written at
-// out[(NAMs of the range's earlier groups) + c]; entries at index >= cap are
-// not written. Returns the NAM count, or MERGE_OVERFLOW when a group needs
-// more than 64 open NAMs and there is no wide list.
+// the hits themselves in order). NAM c of the k-th group of the range is
+// written at out[(NAMs of the range's earlier groups) + c]; entries at index
+// >= cap are not written. Returns the NAM count, or MERGE_OVERFLOW when a group
+// needs more than 64 open NAMs and there is no wide list.
 // box (may be nullptr): bounds of up to box_cap chunks of the wide list. A
 // hit can only be accepted by an entry with previous hit start < ref start <=
 // ref end, so the scan for the first accepting entry visits only the chunks
 // whose bounds admit the hit, in order: the same entry as a full scan.
+//
+// The hits go block by block: hits of one group and query start. No NAM can take
+// two of a block (a NAM that takes one gets previous start qs, and so does one
+// that a hit of the block opens), so each meets the NAMs as they were before
+// the block. Their acceptance masks are independent; only the assignment, in
+// hit order (the first accepting NAM that no earlier hit of the block took,
+// else a new one), runs hit by hit, on scalars. A block cut by the end of the
+// 64 hits in registers is two blocks.
 __device__ __forceinline__ uint32_t merge_range(const DevHit *hits, const uint64_t *order, uint32_t xb,
-                                                uint32_t xe, bool pre, uint32_t c_rsd, uint32_t c_rs,
-                                                uint32_t c_re, uint32_t c_q, const WideList wide, gis_nam *out,
+                                                uint32_t xe, const WideList wide, gis_nam *out,
                                                 uint32_t cap, ChunkBox *box = nullptr, uint32_t box_cap = 0) {
     const uint32_t lane = lane_id();
     LaneNam o{0, 0, 0, 0, 0, 0, 0, 0};
@@ -1332,303 +1457,233 @@ __device__ __forceinline__ uint32_t merge_range(const DevHit *hits, const uint64
     bool wide_mode = false;
     uint32_t nw = 0, wide_mark = 0;
     for (uint32_t x0 = xb; x0 < xe; x0 += 64) {
-        if (!pre) {
-            const uint32_t i = x0 + lane;
-            if (i < xe) {
-                const DevHit h = hits[order ? (uint32_t)order[i] : i];
-                c_rsd = h.ref_strand;
-                c_rs = (uint32_t)h.ref_start;
-                c_re = (uint32_t)h.ref_end;
-                c_q = (uint32_t)h.query_start | ((uint32_t)h.query_end << 16);
-            }
-        }
+        uint4 h = make_uint4(0u, 0u, 0u, 0u);
+        if (x0 + lane < xe)
+            h = reinterpret_cast<const uint4 *>(hits)[order ? (uint32_t)order[x0 + lane] : x0 + lane];
+        const uint32_t c_rsd = h.x, c_rs = h.y, c_re = h.z, c_q = h.w;
         const uint32_t m = xe - x0 < 64 ? xe - x0 : 64;
-        uint32_t no_block_until = 0;  // the rest of a block that did not fit goes hit by hit
-        for (uint32_t t = 0; t < m; t++) {
-            const uint32_t rsd = readlane_u32(c_rsd, t);
-            const int rs = (int)readlane_u32(c_rs, t);
-            const int re = (int)readlane_u32(c_re, t);
+        // lanes that start a block, and a group (lane 0 against the last chunk's)
+        const uint32_t p_rsd = (uint32_t)__shfl_up((int)c_rsd, 1, 64), p_q = (uint32_t)__shfl_up((int)c_q, 1, 64);
+        const uint64_t gheads = ballot(c_rsd != (lane ? p_rsd : grp));
+        const uint64_t heads = gheads | ballot(((c_q ^ p_q) & 0xffffu) != 0 || lane == 0);
+        uint32_t singles_until = 0;  // the rest of a block that did not fit the lanes goes hit by hit
+        for (uint32_t t = 0; t < m;) {
             const uint32_t q = readlane_u32(c_q, t);
-            const int qs = (int)(q & 0xffffu), qe = (int)(q >> 16);
-            if (rsd != grp) {
-                if (wide_mode) {
-                    wide_flush(wide, nw, out, base, grp, cap);
-                    wide_mode = false;
-                    nw = 0;
-                } else if (lane < n_open && base + o.cid < cap) {
-                    lane_nam_store(out, base + o.cid, grp, o);
+            const int qs = (int)(q & 0xffffu);
+            const uint64_t next = heads & ~((2ull << t) - 1);
+            uint32_t len = (next ? min((uint32_t)__builtin_ctzll(next), m) : m) - t;
+            if ((gheads >> t) & 1ull) {
+                if (t >= singles_until) {
+                    if (wide_mode) {
+                        wide_flush(wide, nw, out, base, grp, cap);
+                        wide_mode = false;
+                        nw = 0;
+                    } else if (lane < n_open && base + o.cid < cap) {
+                        lane_nam_store(out, base + o.cid, grp, o);
+                    }
+                    base += gcnt;
+                    gcnt = 0;
+                    n_open = 0;
                 }
-                base += gcnt;
-                gcnt = 0;
-                n_open = 0;
-                grp = rsd;
+                grp = readlane_u32(c_rsd, t);
             }
             if (!wide_mode) {
-                // A block of hits with this hit's group and query start: as
-                // in the wide form below, no NAM can take two of them (a NAM
-                // that takes one gets previous start qs, and so does one a
-                // hit of the block opens), so each meets the open NAMs as
-                // they were before the block. Their acceptance ballots are
-                // independent; only the assignment, in hit order (first
-                // accepting NAM not taken by an earlier hit of the block,
-                // else the next new lane), runs hit by hit, on scalars.
-                const uint64_t sm =
-                    __ballot(lane >= t && lane < m && c_rsd == rsd && (c_q & 0xffffu) == (uint32_t)qs);
-                const uint64_t above = sm >> t;
-                const uint32_t len = ~above ? (uint32_t)__builtin_ctzll(~above) : 64u - t;
-                uint32_t n_new = 0;
-                int my_hit = -1;  // the block hit (chunk lane) this lane takes or opens with
-                bool fits = len > 1 && t >= no_block_until;
-                if (fits) {
-                    uint64_t taken = 0;
-                    for (uint32_t i = t; i < t + len; i++) {
-                        const int hrs = (int)readlane_u32(c_rs, i);
-                        const int hre = (int)readlane_u32(c_re, i);
-                        const int hqe = (int)(readlane_u32(c_q, i) >> 16);
-                        bool hext = false;
-                        const bool hacc = lane < n_open && nam_accepts(o.qp, o.qe, o.rp, o.re, qs, hqe, hrs, hre, hext);
-                        const uint64_t avail = __ballot(hacc) & ~taken;
-                        if (!avail && n_open + n_new == 64) {
-                            // a new NAM would not fit the lanes: this block goes hit by hit
-                            fits = false;
-                            no_block_until = t + len;
-                            break;
-                        }
-                        const uint32_t win = avail ? (uint32_t)__builtin_ctzll(avail) : n_open + n_new;
-                        taken |= avail ? (1ull << win) : 0ull;
-                        n_new += avail ? 0u : 1u;
-                        my_hit = lane == win ? (int)i : my_hit;
-                    }
-                }
-                if (fits) {
-                    const int src = my_hit < 0 ? 0 : my_hit;
-                    const int hrs = __shfl((int)c_rs, src, 64), hre = __shfl((int)c_re, src, 64);
-                    const int hqe = (int)((uint32_t)__shfl((int)c_q, src, 64) >> 16);
-                    const bool take = my_hit >= 0 && lane < n_open;
-                    const bool mk = my_hit >= 0 && lane >= n_open;
-                    const bool grow = mk || (take && hqe > o.qe && hre > o.re);
-                    o.qs = mk ? qs : o.qs;
-                    o.rs = mk ? hrs : o.rs;
-                    o.qe = grow ? hqe : o.qe;
-                    o.re = grow ? hre : o.re;
-                    o.qp = take || mk ? qs : o.qp;
-                    o.rp = take || mk ? hrs : o.rp;
-                    o.n = mk ? 1 : o.n + (take ? 1 : 0);
-                    o.cid = mk ? gcnt + (lane - n_open) : o.cid;
-                    n_open += n_new;
-                    gcnt += n_new;
-                    t += len - 1;
-                    continue;
-                }
-                bool ext = false;
-                const bool acc = lane < n_open && nam_accepts(o.qp, o.qe, o.rp, o.re, qs, qe, rs, re, ext);
-                const uint64_t bal = __ballot(acc);
-                if (bal || n_open < 64) {
-                    // the first accepting NAM takes the hit, or, with none, the
-                    // hit opens NAM n_open; predicated updates, no branches
-                    const bool fresh = bal == 0;
-                    const uint32_t win = fresh ? n_open : (uint32_t)__builtin_ctzll(bal);
-                    const bool me = lane == win;
-                    const bool end = me && (fresh || ext);
-                    o.qs = me && fresh ? qs : o.qs;
-                    o.rs = me && fresh ? rs : o.rs;
-                    o.qe = end ? qe : o.qe;
-                    o.re = end ? re : o.re;
-                    o.qp = me ? qs : o.qp;
-                    o.rp = me ? rs : o.rp;
-                    o.n = me ? (fresh ? 1 : o.n + 1) : o.n;
-                    o.cid = me && fresh ? gcnt : o.cid;
-                    n_open += fresh ? 1u : 0u;
-                    gcnt += fresh ? 1u : 0u;
-                    continue;
-                }
-                if (n_open == 64) {
-                    const bool keep = o.qe >= qs;
-                    const uint64_t km = __ballot(keep);
-                    const uint32_t nk = (uint32_t)__popcll(km);
-                    if (nk == 64) {
-                        if (!wide.near && !wide.far) return MERGE_OVERFLOW;
-                        // the group continues on the wide list, in creation order
-                        wput(wide, lane, WideNam{o.qs, o.qe, o.qp, o.rs, o.re, o.rp, (uint32_t)o.n, o.cid});
-                        nw = 64;
-                        wide_mark = 64;
-                        wide_mode = true;
-                        n_open = 0;
-                        if (box && box_cap) {
-                            const int lo = wave_min_i(o.rp), hi = wave_max_i(o.re);
-                            if (lane == 0) box[0] = ChunkBox{lo, hi};
-                        }
+                if (len > 1 && t >= singles_until) {
+                    uint32_t n_new = 0;
+                    int my_hit = -1;  // the block hit (chunk lane) this lane takes or opens with
+                    bool fits = true;
+                    if (n_open == 0) {
+                        n_new = len;  // a group's first block opens a NAM a hit
+                        my_hit = lane < len ? (int)(t + lane) : -1;
                     } else {
-                        if (!keep && base + o.cid < cap) lane_nam_store(out, base + o.cid, grp, o);
-                        const uint32_t dst = keep ? mbcnt(km) : nk + mbcnt(~km);
-                        o.qs = permute_push(o.qs, dst);
-                        o.qe = permute_push(o.qe, dst);
-                        o.qp = permute_push(o.qp, dst);
-                        o.rs = permute_push(o.rs, dst);
-                        o.re = permute_push(o.re, dst);
-                        o.rp = permute_push(o.rp, dst);
-                        o.n = permute_push(o.n, dst);
-                        o.cid = (uint32_t)permute_push((int)o.cid, dst);
-                        n_open = nk;
-                    }
-                }
-                if (!wide_mode) {
-                    if (lane == n_open) o = LaneNam{qs, qe, qs, rs, re, rs, 1, gcnt};
-                    n_open++;
-                    gcnt++;
-                    continue;
-                }
-                // (the hit was accepted by no open NAM: it opens one on the wide list)
-            } else {
-                // Wide form, a block at a time: hit t and the hits after it in
-                // the chunk registers with the same group and query start. A
-                // NAM that takes a hit of the block gets previous start qs and
-                // can take no other, and a NAM opened by one cannot either, so
-                // every hit of the block meets the list as it was before the
-                // block. Hit by hit, each takes the first accepting entry that
-                // has not taken one of the block's hits. Going through the
-                // list's chunks in order and, inside a chunk, through the
-                // block's pending hits in order gives each hit that same entry
-                // (the hits a chunk leaves pending find no acceptor in it, by
-                // induction over the chunks), and a chunk is read once per
-                // block instead of once per hit.
-                const uint64_t sm =
-                    __ballot(lane >= t && lane < m && c_rsd == rsd && (c_q & 0xffffu) == (uint32_t)qs);
-                const uint64_t above = sm >> t;
-                const uint32_t len = ~above ? (uint32_t)__builtin_ctzll(~above) : 64u;
-                uint64_t pend = (len >= 64 ? ~0ull : ((1ull << len) - 1)) << t;
-                const uint32_t nch = (nw + 63) >> 6;
-                const bool boxed = box && nch <= box_cap;
-                const int my_rs = (int)c_rs;
-                for (uint32_t c = 0; c < nch && pend; c++) {
-                    // the pending hits the chunk's bounds admit (all of them
-                    // without bounds); the bounds of the chunk's start hold
-                    // for every entry that has not taken a hit of the block
-                    uint64_t cm = pend;
-                    if (boxed) {
-                        const ChunkBox bx = box[c];
-                        cm = __ballot(((pend >> lane) & 1ull) != 0 && bx.lo < my_rs && my_rs <= bx.hi);
-                    }
-                    if (!cm) continue;
-                    const uint32_t e = c * 64 + lane;
-                    const bool valid = e < nw;
-                    WideNam w{};
-                    if (valid) w = wget(wide, e);
-                    // the admitted hits, in order, take the first accepting
-                    // entry of the chunk that no earlier one took: the
-                    // ballots against the chunk as it was (an entry that
-                    // takes a hit of the block can take no other), the
-                    // assignment on scalars, the updates after
-                    uint64_t taken = 0;
-                    int my_hit = -1;  // the hit (chunk lane) this entry takes
-                    while (cm) {
-                        const uint32_t i = (uint32_t)__builtin_ctzll(cm);
-                        cm &= cm - 1;
-                        const int hrs = (int)readlane_u32(c_rs, i);
-                        const int hre = (int)readlane_u32(c_re, i);
-                        const int hqe = (int)(readlane_u32(c_q, i) >> 16);
-                        bool ext = false;
-                        const bool acc = valid && nam_accepts(w.qp, w.qe, w.rp, w.re, qs, hqe, hrs, hre, ext);
-                        const uint64_t bal = __ballot(acc) & ~taken;
-                        if (bal) {
-                            const uint32_t win = (uint32_t)__builtin_ctzll(bal);
-                            taken |= 1ull << win;
+                        uint64_t taken = 0;
+                        for (uint32_t i = t; i < t + len; i++) {
+                            const int hrs = (int)readlane_u32(c_rs, i);
+                            const int hre = (int)readlane_u32(c_re, i);
+                            const int hqe = (int)(readlane_u32(c_q, i) >> 16);
+                            bool hext = false;
+                            const bool hacc =
+                                lane < n_open && nam_accepts(o.qp, o.qe, o.rp, o.re, qs, hqe, hrs, hre, hext);
+                            const uint64_t avail = ballot(hacc) & ~taken;
+                            if (!avail && n_open + n_new == 64) {
+                                fits = false;
+                                break;
+                            }
+                            const uint32_t win = avail ? (uint32_t)__builtin_ctzll(avail) : n_open + n_new;
+                            taken |= avail ? (1ull << win) : 0ull;
+                            n_new += avail ? 0u : 1u;
                             my_hit = lane == win ? (int)i : my_hit;
-                            pend &= ~(1ull << i);
                         }
                     }
-                    if (taken) {
+                    if (fits) {
                         const int src = my_hit < 0 ? 0 : my_hit;
                         const int hrs = __shfl((int)c_rs, src, 64), hre = __shfl((int)c_re, src, 64);
                         const int hqe = (int)((uint32_t)__shfl((int)c_q, src, 64) >> 16);
-                        const bool tk = my_hit >= 0;
-                        const bool ext = tk && hqe > w.qe && hre > w.re;
-                        if (ext) {
-                            w.qe = hqe;
-                            w.re = hre;
-                        }
-                        if (tk) {
-                            w.qp = qs;
-                            w.rp = hrs;
-                            w.n++;
-                        }
-                        if (boxed) {
-                            const int hi = wave_max_i(ext ? hre : (int)0x80000000);
-                            if (lane == 0 && box[c].hi < hi) box[c].hi = hi;
-                        }
-                        if (tk) wput(wide, e, w);
-                        wave_sync_mem();
+                        const bool take = my_hit >= 0 && lane < n_open;
+                        const bool mk = my_hit >= 0 && lane >= n_open;
+                        const bool grow = mk || (take && hqe > o.qe && hre > o.re);
+                        o.qs = mk ? qs : o.qs;
+                        o.rs = mk ? hrs : o.rs;
+                        o.qe = grow ? hqe : o.qe;
+                        o.re = grow ? hre : o.re;
+                        o.qp = take || mk ? qs : o.qp;
+                        o.rp = take || mk ? hrs : o.rp;
+                        o.n = mk ? 1 : o.n + (take ? 1 : 0);
+                        o.cid = mk ? gcnt + (lane - n_open) : o.cid;
+                        n_open += n_new;
+                        gcnt += n_new;
+                        t += len;
+                        continue;
                     }
+                    singles_until = t + len;
                 }
-                // the hits no entry took open entries, in hit order (lane 0
-                // writes them; the wave syncs before a retirement reads the
-                // list and after the last one)
-                const bool opened = pend != 0;
-                while (pend) {
-                    const uint32_t i = (uint32_t)__builtin_ctzll(pend);
-                    pend &= pend - 1;
+                // one hit
+                const int rs = (int)readlane_u32(c_rs, t), re = (int)readlane_u32(c_re, t), qe = (int)(q >> 16);
+                const uint64_t xq = ballot(qe > o.qe), xr = ballot(re > o.re);
+                uint64_t free = n_open < 64 ? 1ull << n_open : 0ull, mk;
+                const uint64_t acc = (free - 1) & ballot(o.qp < qs) & ballot(qs <= o.qe) & ballot(o.rp < rs) &
+                                     ballot(rs <= o.re) & ~(xq ^ xr);
+                if (acc == 0 && n_open == 64) {
+                    n_open = retire_lanes(o, qs, out, base, grp, cap);
+                    free = n_open < 64 ? 1ull << n_open : 0ull;
+                }
+                if (acc || n_open < 64) {
+                    o.n = lane < n_open ? o.n : 0;
+                    lanes_take(o, acc, xq & xr, free, mk, gcnt, qs, qe, rs, re);
+                    n_open += mk ? 1u : 0u;
+                    gcnt += mk ? 1u : 0u;
+                    t++;
+                    continue;
+                }
+                if (!wide.near && !wide.far) return MERGE_OVERFLOW;
+                // the group continues on the wide list, in creation order, with
+                // this hit and the rest of its block
+                wput(wide, lane, WideNam{o.qs, o.qe, o.qp, o.rs, o.re, o.rp, (uint32_t)o.n, o.cid});
+                nw = 64;
+                wide_mark = 64;
+                wide_mode = true;
+                n_open = 0;
+                singles_until = 0;
+                if (box && box_cap) {
+                    const int lo = wave_min_i(o.rp), hi = wave_max_i(o.re);
+                    if (lane == 0) box[0] = ChunkBox{lo, hi};
+                }
+                wave_sync_mem();
+            }
+            // Wide form: going through the list's chunks in order and, inside a
+            // chunk, through the block's pending hits in order gives each hit
+            // the entry it would take hit by hit (the hits a chunk leaves
+            // pending find no acceptor in it, by induction over the chunks),
+            // and a chunk is read once per block instead of once per hit.
+            uint64_t pend = (len >= 64 ? ~0ull : ((1ull << len) - 1)) << t;
+            const uint32_t nch = (nw + 63) >> 6;
+            const bool boxed = box && nch <= box_cap;
+            const int my_rs = (int)c_rs;
+            for (uint32_t c = 0; c < nch && pend; c++) {
+                // the pending hits the chunk's bounds admit (all of them
+                // without bounds); the bounds of the chunk's start hold
+                // for every entry that has not taken a hit of the block
+                uint64_t cm = pend;
+                if (boxed) {
+                    const ChunkBox bx = box[c];
+                    cm = ballot(bx.lo < my_rs && my_rs <= bx.hi) & pend;
+                }
+                if (!cm) continue;
+                const uint32_t e = c * 64 + lane;
+                const bool valid = e < nw;
+                WideNam w{};
+                if (valid) w = wget(wide, e);
+                uint64_t taken = 0;
+                int my_hit = -1;  // the hit (chunk lane) this entry takes
+                while (cm) {
+                    const uint32_t i = (uint32_t)__builtin_ctzll(cm);
+                    cm &= cm - 1;
                     const int hrs = (int)readlane_u32(c_rs, i);
                     const int hre = (int)readlane_u32(c_re, i);
                     const int hqe = (int)(readlane_u32(c_q, i) >> 16);
-                    if (nw >= 2 * wide_mark) {
+                    bool ext = false;
+                    const bool acc = valid && nam_accepts(w.qp, w.qe, w.rp, w.re, qs, hqe, hrs, hre, ext);
+                    const uint64_t bal = ballot(acc) & ~taken;
+                    if (bal) {
+                        const uint64_t win = bal & (0 - bal);
+                        taken |= win;
+                        my_hit = lane_bit(win) ? (int)i : my_hit;
+                        pend &= ~(1ull << i);
+                    }
+                }
+                if (taken) {
+                    const int src = my_hit < 0 ? 0 : my_hit;
+                    const int hrs = __shfl((int)c_rs, src, 64), hre = __shfl((int)c_re, src, 64);
+                    const int hqe = (int)((uint32_t)__shfl((int)c_q, src, 64) >> 16);
+                    const bool tk = my_hit >= 0;
+                    const bool ext = tk && hqe > w.qe && hre > w.re;
+                    if (ext) {
+                        w.qe = hqe;
+                        w.re = hre;
+                    }
+                    if (tk) {
+                        w.qp = qs;
+                        w.rp = hrs;
+                        w.n++;
+                    }
+                    if (boxed) {
+                        const int hi = wave_max_i(ext ? hre : (int)0x80000000);
+                        if (lane == 0 && box[c].hi < hi) box[c].hi = hi;
+                    }
+                    if (tk) wput(wide, e, w);
+                    wave_sync_mem();
+                }
+            }
+            // the hits no entry took open entries, in hit order, all at once
+            if (pend) {
+                if (nw >= 2 * wide_mark) {
+                    // retire the dead entries (query_end before this block), keeping the order
+                    uint32_t kept = 0;
+                    for (uint32_t c0 = 0; c0 < nw; c0 += 64) {
+                        const uint32_t e = c0 + lane;
+                        WideNam w{};
+                        bool keep = false;
+                        if (e < nw) {
+                            w = wget(wide, e);
+                            keep = w.qe >= qs;
+                            if (!keep && base + w.cid < cap) lane_nam_store(out, base + w.cid, grp, from_wide(w));
+                        }
+                        const uint64_t kb = ballot(keep);
                         wave_sync_mem();
-                        // retire the dead entries (query_end before this hit), keeping the order
-                        uint32_t kept = 0;
-                        for (uint32_t c0 = 0; c0 < nw; c0 += 64) {
-                            const uint32_t e = c0 + lane;
-                            WideNam w{};
-                            bool keep = false;
-                            if (e < nw) {
-                                w = wget(wide, e);
-                                keep = w.qe >= qs;
-                                if (!keep && base + w.cid < cap)
-                                    lane_nam_store(out, base + w.cid, grp, from_wide(w));
-                            }
-                            const uint64_t kb = __ballot(keep);
-                            wave_sync_mem();
-                            if (keep) wput(wide, kept + mbcnt(kb), w);
-                            kept += (uint32_t)__popcll(kb);
-                            wave_sync_mem();
-                        }
-                        nw = kept;
-                        wide_mark = kept > 64 ? kept : 64;
-                        if (box && ((nw + 63) >> 6) <= box_cap) boxes_rebuild(wide, nw, box);
+                        if (keep) wput(wide, kept + mbcnt(kb), w);
+                        kept += (uint32_t)__popcll(kb);
+                        wave_sync_mem();
                     }
-                    if (lane == 0) {
-                        wput(wide, nw, WideNam{qs, hqe, qs, hrs, hre, hrs, 1u, gcnt});
-                        const uint32_t c = nw >> 6;
-                        if (box && c < box_cap && ((nw + 63) >> 6) <= box_cap) {
-                            if ((nw & 63) == 0) {
-                                box[c] = ChunkBox{hrs, hre};
-                            } else {
-                                if (box[c].lo > hrs) box[c].lo = hrs;
-                                if (box[c].hi < hre) box[c].hi = hre;
-                            }
+                    nw = kept;
+                    wide_mark = kept > 64 ? kept : 64;
+                    if (box && ((nw + 63) >> 6) <= box_cap) boxes_rebuild(wide, nw, box);
+                    wave_sync_mem();
+                }
+                const uint32_t k = (uint32_t)__popcll(pend), at = nw + mbcnt(pend);
+                const bool mine = lane_bit(pend);
+                if (mine)
+                    wput(wide, at, WideNam{qs, (int)(c_q >> 16), qs, (int)c_rs, (int)c_re, (int)c_rs, 1u,
+                                           gcnt + mbcnt(pend)});
+                // bounds of the one or two chunks the new entries lie in (only
+                // while every chunk has them)
+                const uint32_t c_last = (nw + k - 1) >> 6;
+                if (box && c_last < box_cap) {
+                    for (uint32_t c = nw >> 6; c <= c_last; c++) {
+                        const bool in = mine && (at >> 6) == c;
+                        const int lo = wave_min_i(in ? (int)c_rs : 0x7fffffff);
+                        const int hi = wave_max_i(in ? (int)c_re : (int)0x80000000);
+                        if (lane == 0) {
+                            const bool begun = c == nw >> 6 && (nw & 63) != 0;
+                            const ChunkBox bx = box[c];
+                            box[c] = ChunkBox{begun ? min(bx.lo, lo) : lo, begun ? max(bx.hi, hi) : hi};
                         }
                     }
-                    nw++;
-                    gcnt++;
                 }
-                if (opened) wave_sync_mem();
-                t += len - 1;
-                continue;
+                nw += k;
+                gcnt += k;
+                wave_sync_mem();
             }
-            if (lane == 0) {
-                wput(wide, nw, WideNam{qs, qe, qs, rs, re, rs, 1u, gcnt});
-                // the new entry's chunk bounds (only while every chunk has them)
-                const uint32_t c = nw >> 6;
-                if (box && c < box_cap && ((nw + 63) >> 6) <= box_cap) {
-                    if ((nw & 63) == 0) {
-                        box[c] = ChunkBox{rs, re};
-                    } else {
-                        if (box[c].lo > rs) box[c].lo = rs;
-                        if (box[c].hi < re) box[c].hi = re;
-                    }
-                }
-            }
-            nw++;
-            gcnt++;
-            wave_sync_mem();
+            t += len;
         }
     }
     if (wide_mode) wide_flush(wide, nw, out, base, grp, cap);
@@ -1636,40 +1691,8 @@ __device__ __forceinline__ uint32_t merge_range(const DevHit *hits, const uint64
     return base + gcnt;
 }
 
-// Merge the nh hits of a read into NAMs written to out[0 .. total) in
-// canonical order (entries at index >= cap are not written). keys: scratch
-// of the next power of two >= nh entries when nh <= MERGE_LDS (bitonic
-// grouping), else of nh entries with keys_alt another nh (radix grouping).
-// wide: a list of nh entries for groups with more than 64 open NAMs, or
-// nullptr (then such a read returns MERGE_OVERFLOW).
-__device__ __forceinline__ uint32_t merge_wave(uint32_t nh, const DevHit *hits, uint64_t *keys,
-                                               uint64_t *keys_alt, WideNam *wide, gis_nam *out,
-                                               uint32_t cap) {
-    const uint32_t lane = lane_id();
-    if (nh > 64) return merge_range(hits, group_order(nh, hits, keys, keys_alt), 0, nh, false, 0, 0, 0, 0,
-                                    wide_in(wide), out, cap);
-    DevHit h{};
-    if (lane < nh) h = hits[lane];
-    const uint32_t rsd = lane < nh ? h.ref_strand : 0xffffffffu;
-    const uint32_t prev = __shfl_up(rsd, 1, 64);
-    const bool uns = __ballot(lane > 0 && lane < nh && prev > rsd) != 0;
-    uint32_t c_rsd = rsd, c_rs = (uint32_t)h.ref_start, c_re = (uint32_t)h.ref_end;
-    uint32_t c_q = (uint32_t)h.query_start | ((uint32_t)h.query_end << 16);
-    if (uns) {
-        uint64_t key = lane < nh ? (((uint64_t)rsd << 32) | lane) : UINT64_MAX;
-        bitonic_regs(key);
-        const int src = (int)((uint32_t)key & 63u);
-        c_rsd = (uint32_t)__shfl((int)c_rsd, src, 64);
-        c_rs = (uint32_t)__shfl((int)c_rs, src, 64);
-        c_re = (uint32_t)__shfl((int)c_re, src, 64);
-        c_q = (uint32_t)__shfl((int)c_q, src, 64);
-    }
-    return merge_range(hits, nullptr, 0, nh, true, c_rsd, c_rs, c_re, c_q, wide_in(wide), out, cap);
-}
-
-struct alignas(8) MergeLds {
+struct MergeLds {
     DevHit hits[MERGE_LDS];
-    uint64_t keys[MERGE_LDS];
 };
 
 // reads whose (strand, ref) groups merge on separate waves (k_merge_groups,
@@ -1679,8 +1702,10 @@ constexpr uint32_t SPLIT_MIN = 512;
 // hits of one k_merge_groups work item: consecutive small groups of a split
 // read merge on one wave
 constexpr uint32_t ITEM_HITS = 384;
-// wide lists in LDS: per wave of k_merge for reads of at most this many
-// hits, and per group of k_merge_groups (one wave per block)
+// reads of up to this many hits are tried in arrival order first
+constexpr uint32_t ARRIVAL_MAX = 512;
+// entries of a wide list that lie in LDS: per wave of k_merge, and per group of
+// k_merge_groups (one wave per block)
 constexpr int MERGE_WIDE_LDS = 256;
 constexpr int GROUP_WIDE_LDS = 1024;
 // chunk bounds of a k_merge_groups wide list (lists up to 32,768 entries)
@@ -1716,7 +1741,7 @@ __global__ __launch_bounds__(64 * WPB) void k_merge(DevBatch b) {
                     const uint32_t cur = ghits[ord ? (uint32_t)ord[i] : i].ref_strand;
                     head = i == 0 || ghits[ord ? (uint32_t)ord[i - 1] : i - 1].ref_strand != cur;
                 }
-                const uint64_t bal = __ballot(head);
+                const uint64_t bal = ballot(head);
                 if (head) slots[G + mbcnt(bal)] = (uint64_t)i << 32;
                 G += (uint32_t)__popcll(bal);
             }
@@ -1756,12 +1781,14 @@ __global__ __launch_bounds__(64 * WPB) void k_merge(DevBatch b) {
                 continue;
             }
         }
-        uint32_t total = MERGE_OVERFLOW;
-        if (nh <= (uint32_t)MERGE_WIDE_LDS) gwide = lwide[wid];  // NAMs <= hits fit
-        if (nh <= (uint32_t)MERGE_LDS)
-            total = merge_wave(nh, ghits, lkeys[wid], nullptr, gwide, fin, nh);
-        else if (b.merge_scratch)
-            total = merge_wave(nh, ghits, gkeys, gkeys + nh, gwide, fin, nh);
+        uint32_t total = nh <= ARRIVAL_MAX ? merge_arrival(ghits, nh, fin, nh) : MERGE_OVERFLOW;
+        if (total == MERGE_OVERFLOW && (nh <= (uint32_t)MERGE_LDS || b.merge_scratch)) {
+            // more than 64 NAMs at once: group by group, with a wide list (NAMs <= hits)
+            const uint64_t *ord = nh <= (uint32_t)MERGE_LDS ? group_order(nh, ghits, lkeys[wid], nullptr)
+                                                            : group_order(nh, ghits, gkeys, gkeys + nh);
+            const WideList wl{(LdsWideNam *)lwide[wid], gwide, (uint32_t)MERGE_WIDE_LDS};
+            total = merge_range(ghits, ord, 0, nh, wl, fin, nh);
+        }
         if (total == MERGE_OVERFLOW) {
             // needs the global scratch, which this run does not have yet
             if (lane == 0) {
@@ -1798,7 +1825,7 @@ __global__ __launch_bounds__(64) void k_merge_groups(DevBatch b) {
         WideNam *far = (rescue ? b.rnam_ws : b.nam_ws) + hb + gs;
         gis_nam *out = (rescue ? b.rnam_fin : b.nam_fin) + hb + gs;
         const WideList wl{(LdsWideNam *)lwide, far, (uint32_t)GROUP_WIDE_LDS};
-        const uint32_t c = merge_range(ghits, ord, gs, ge, false, 0, 0, 0, 0, wl, out, ge - gs, lbox, GROUP_BOXES);
+        const uint32_t c = merge_range(ghits, ord, gs, ge, wl, out, ge - gs, lbox, GROUP_BOXES);
         if (lane == 0) slots[g] = ((uint64_t)gs << 32) | c;
         wave_sync_mem();
     }
@@ -1852,27 +1879,85 @@ __global__ __launch_bounds__(64 * WPB) void k_merge_split_finish(DevBatch b) {
 // and a hit nobody accepts opens a NAM in the segment's next lane. When a
 // strand's hits end, its NAMs are final: each lane ranks its NAM among the
 // segment's by (ref_id, creation index), which is canonical order within the
-// strand, and writes it. A read with more than 16 NAMs on one strand, or
-// more than 64 hits, is listed for k_merge.
+// strand, and writes it. A read with more than 16 NAMs on one strand is merged
+// again by the whole wave (merge_arrival; 64 hits make at most 64 NAMs), and a
+// read of more than 64 hits is listed for k_merge.
 
 constexpr uint32_t SEG = 16;
 constexpr uint32_t RPW = 64 / SEG;
 
-__device__ __forceinline__ void seg_finalize(gis_nam *out, uint32_t base, uint32_t j, uint32_t n_open,
-                                             uint32_t rsd, const LaneNam &o, bool on) {
-    // rank by (ref_id, creation index) among the segment's open lanes. A
-    // segment is one DPP row of 16 lanes: rotating the row by 1..15 shows
-    // each lane every other lane's key. Creation indices are below 16, so
-    // no key is all ones, which marks the lanes beyond n_open.
-    const uint32_t key = ((rsd & 0x7fffffffu) << 8) | (o.cid & 0xffu);
-    const int kv = (int)(j < n_open ? key : 0xffffffffu);
+// The NAMs of the segments for which `on` holds (those of their lanes that took
+// hits) at out + base, ranked by (ref_id, creation index = lane). A segment is
+// one DPP row of 16 lanes: rotating the row by 1..15 shows each lane every
+// other lane's key. Lanes are below 16, so no key is all ones, which marks the
+// free lanes.
+__device__ __forceinline__ void seg_finalize(gis_nam *out, uint32_t base, uint32_t j, uint32_t rsd, const LaneNam &o,
+                                             bool on) {
+    const uint32_t key = ((rsd & 0x7fffffffu) << 8) | j;
+    const int kv = (int)(o.n > 0 ? key : 0xffffffffu);
     uint32_t rank = 0;
-#define GIS_ROW_ROR(r) rank += (uint32_t)__builtin_amdgcn_update_dpp(0, kv, 0x120 + (r), 0xf, 0xf, false) < key ? 1u : 0u
+#define GIS_ROW_ROR(r) rank += (uint32_t)__builtin_amdgcn_mov_dpp(kv, 0x120 + (r), 0xf, 0xf, true) < key ? 1u : 0u
     GIS_ROW_ROR(1); GIS_ROW_ROR(2); GIS_ROW_ROR(3); GIS_ROW_ROR(4); GIS_ROW_ROR(5);
     GIS_ROW_ROR(6); GIS_ROW_ROR(7); GIS_ROW_ROR(8); GIS_ROW_ROR(9); GIS_ROW_ROR(10);
     GIS_ROW_ROR(11); GIS_ROW_ROR(12); GIS_ROW_ROR(13); GIS_ROW_ROR(14); GIS_ROW_ROR(15);
 #undef GIS_ROW_ROR
-    if (on && j < n_open) lane_nam_store(out, base + rank, rsd, o);
+    if (on && o.n > 0) lane_nam_store(out, base + rank, rsd, o);
+}
+
+// The hits of one strand of each segment's read (cnt of them from hits on, in
+// LDS) merged into the segment's lanes. Returns the read's hits that found a
+// lane (fewer than cnt: the strand needs more than 16 NAMs).
+__device__ __forceinline__ uint32_t seg_merge(const DevHit *hits, uint32_t cnt, LaneNam &o, uint32_t &rsd_o) {
+    constexpr uint64_t FIRST = 0x0001000100010001ull;  // lane 0 of each row
+    uint64_t free = FIRST;  // the lane of each row that opens the next NAM (none when the row is full)
+    const uint32_t most = wave_max_dpp(cnt), last = cnt ? cnt - 1 : 0;
+    for (uint32_t t = 0; t < most; t++) {
+        const uint4 h = reinterpret_cast<const uint4 *>(hits)[min(t, last)];
+        const int rs = (int)h.y, re = (int)h.z, qs = (int)(h.w & 0xffffu), qe = (int)(h.w >> 16);
+        const uint64_t xq = ballot(qe > o.qe), xr = ballot(re > o.re);
+        const uint64_t acc = ballot(rsd_o == h.x) & ballot(o.qp < qs) & ballot(qs <= o.qe) & ballot(o.rp < rs) &
+                             ballot(rs <= o.re) & ~(xq ^ xr);
+        // the first accepting lane of the segment takes the hit; else the
+        // segment's free lane opens a NAM with it
+        const uint64_t me = first_of_rows((acc | free) & ballot(t < cnt)), mk = me & free;
+        const bool b_mk = lane_bit(mk), b_end = lane_bit(mk | (me & xq & xr)), b_me = lane_bit(me);
+        free = (free ^ mk) | ((mk << 1) & ~FIRST);
+        o.qs = b_mk ? qs : o.qs;
+        o.rs = b_mk ? rs : o.rs;
+        rsd_o = b_mk ? h.x : rsd_o;
+        o.qe = b_end ? qe : o.qe;
+        o.re = b_end ? re : o.re;
+        o.qp = b_me ? qs : o.qp;
+        o.rp = b_me ? rs : o.rp;
+        o.n += b_me ? 1 : 0;
+    }
+    return row_sum((uint32_t)o.n);
+}
+
+// The four reads of a wave: hits points at this lane's read's hits in LDS (at
+// least one may be read), nh and nf at their count and the count of forward
+// ones, out at its NAMs. Returns the read's NAM count, or MERGE_OVERFLOW when a
+// strand needs more than 16.
+//
+// Bound by VALU issue, so what can be a mask is one, on the scalar unit: the
+// acceptance tests, the first accepting or else the free lane of each row, the
+// free lanes. A lane's creation index is its place in the row. The two strands
+// are independent: each read's longer one goes first, so that the wave's steps
+// are the longest of four long strands plus the longest of four short ones,
+// without a strand switch inside, and the NAMs are ranked and written twice a
+// wave and not at every read's own switch. 65,536 reads of 23 hits: 51 -> 38 us.
+__device__ __forceinline__ uint32_t merge_segments(const DevHit *hits, uint32_t nh, uint32_t nf, gis_nam *out) {
+    const uint32_t j = lane_id() % SEG, nr = nh - nf;
+    const bool rev = nr > nf;  // the reverse strand first
+    LaneNam oa{0, 0, 0, 0, 0, 0, 0, 0}, ob{0, 0, 0, 0, 0, 0, 0, 0};
+    uint32_t ra = 0xffffffffu, rb = 0xffffffffu;  // the lanes' groups
+    uint32_t took = seg_merge(hits + (rev ? nf : 0u), rev ? nr : nf, oa, ra);
+    took += seg_merge(hits + (rev || nr == 0 ? 0u : nf), rev ? nf : nr, ob, rb);
+    const uint32_t ma = row_sum(oa.n > 0 ? 1u : 0u), mb = row_sum(ob.n > 0 ? 1u : 0u);
+    const bool ok = took == nh;
+    seg_finalize(out, rev ? mb : 0u, j, ra, oa, ok);
+    seg_finalize(out, rev ? 0u : ma, j, rb, ob, ok);
+    return ok ? ma + mb : MERGE_OVERFLOW;
 }
 
 __global__ __launch_bounds__(64 * WPB) void k_merge4(DevBatch b, ReadSet set) {
@@ -1884,77 +1969,46 @@ __global__ __launch_bounds__(64 * WPB) void k_merge4(DevBatch b, ReadSet set) {
     const uint32_t stride = gridDim.x * WPB * RPW;
     for (uint32_t w0 = wave_index(WPB) * RPW; w0 < cnt; w0 += stride) {
         const uint32_t widx = w0 + seg;
-        bool act = widx < cnt, defer = false, rescue = false;
+        const bool act = widx < cnt;
         uint32_t r = 0, nh = 0;
         uint64_t hb = 0;
+        bool rescue = false;
         if (act) {
             r = set_at(set, widx);
             rescue = (b.flags[r] & GIS_FLAG_RESCUED) != 0;
             hb = rescue ? b.rhit_off[r] : b.hit_off[r];
             nh = rescue ? b.rhit_total[r] : b.hit_total[r];
-            defer = nh > 64;
-            act = nh > 0 && !defer;
-            if (nh == 0 && j == 0) b.nam_cnt[r] = 0u;
         }
-        if (act) {
-            const DevHit *gh = (rescue ? b.rhits : b.hits) + hb;
-            for (uint32_t k = j; k < nh; k += SEG) lh[wid][seg][k] = gh[k];
+        const bool many = nh > 64;
+        if (many) nh = 0;
+        const DevHit *gh = (rescue ? b.rhits : b.hits) + hb;
+        uint32_t fwd = 0;
+        for (uint32_t k = j; k < nh; k += SEG) {
+            const uint4 h = reinterpret_cast<const uint4 *>(gh)[k];
+            reinterpret_cast<uint4 *>(lh[wid][seg])[k] = h;
+            fwd += (h.x >> 31) ^ 1u;
         }
+        const uint32_t nf = row_sum(fwd);
         wave_sync_mem();
         gis_nam *out = (rescue ? b.rnam_fin : b.nam_fin) + hb;
-        LaneNam o{0, 0, 0, 0, 0, 0, 0, 0};
-        uint32_t rsd_o = 0;        // this lane's NAM group
-        uint32_t n_open = 0;       // NAMs of the segment on the current strand
-        uint32_t strand = 0, base = 0;
-        bool ovf = false;
-        const uint32_t maxh = wave_max_dpp(act ? nh : 0u);
-        for (uint32_t t = 0; t < maxh; t++) {
-            const bool valid = act && !ovf && t < nh;
-            DevHit h{};
-            if (valid) h = lh[wid][seg][t];
-            const uint32_t hs = h.ref_strand >> 31;
-            // the strand changes: the segment's forward NAMs are final
-            const bool sw = valid && hs != strand;
-            if (__ballot(sw)) {
-                seg_finalize(out, base, j, n_open, rsd_o, o, sw);
-                if (sw) {
-                    base += n_open;
-                    n_open = 0;
-                    strand = hs;
-                }
-            }
-            const int qs = h.query_start, qe = h.query_end, rs = h.ref_start, re = h.ref_end;
-            bool ext = false;
-            const bool acc = valid & (j < n_open) & (rsd_o == h.ref_strand) &
-                             nam_accepts(o.qp, o.qe, o.rp, o.re, qs, qe, rs, re, ext);
-            const uint64_t bal = __ballot(acc);
-            const uint32_t mine = (uint32_t)(bal >> (seg * SEG)) & ((1u << SEG) - 1u);
-            // the first accepting lane of the segment takes the hit; else the
-            // hit opens a NAM in the segment's next lane (selects, no branches)
-            const bool take = (mine != 0u) & (j == (uint32_t)__builtin_ctz(mine | 0x10000u));
-            const bool opens = valid & (mine == 0u);
-            const bool full = n_open == SEG;
-            const bool mk = opens & !full & (j == n_open);
-            o.qe = (take & ext) ? qe : o.qe;
-            o.re = (take & ext) ? re : o.re;
-            o.qp = (take | mk) ? qs : o.qp;
-            o.rp = (take | mk) ? rs : o.rp;
-            o.n = mk ? 1 : o.n + (take ? 1 : 0);
-            o.qs = mk ? qs : o.qs;
-            o.rs = mk ? rs : o.rs;
-            o.qe = mk ? qe : o.qe;
-            o.re = mk ? re : o.re;
-            o.cid = mk ? n_open : o.cid;
-            rsd_o = mk ? h.ref_strand : rsd_o;
-            ovf = ovf | (opens & full);
-            n_open += (opens & !full) ? 1u : 0u;
+        const uint32_t total = merge_segments(lh[wid][seg], nh, nf, out);
+        const bool ovf = total == MERGE_OVERFLOW;
+        if (act && j == 0 && !many && !ovf) b.nam_cnt[r] = total;
+        // a read with more than 16 NAMs on a strand has the whole wave
+        uint64_t redo = ballot(ovf && j == 0);
+        while (redo) {
+            const uint32_t l = (uint32_t)__builtin_ctzll(redo);
+            redo &= redo - 1;
+            const uint32_t nl = readlane_u32(nh, l);
+            gis_nam *ol = reinterpret_cast<gis_nam *>(
+                (uint64_t)readlane_u32((uint32_t)(uintptr_t)out, l) |
+                ((uint64_t)readlane_u32((uint32_t)((uintptr_t)out >> 32), l) << 32));
+            const uint32_t all = merge_arrival(lh[wid][l / SEG], nl, ol, nl);
+            if (lane == l) b.nam_cnt[r] = all;
         }
-        const bool fin = act && !ovf;
-        if (__ballot(fin)) seg_finalize(out, base, j, n_open, rsd_o, o, fin);
-        if (fin && j == 0) b.nam_cnt[r] = base + n_open;
         // the reads handed on to k_merge
-        defer = (defer || (act && ovf)) && j == 0;
-        const uint64_t dm = __ballot(defer);
+        const bool defer = many && j == 0;
+        const uint64_t dm = ballot(defer);
         if (dm) {
             uint32_t at = 0;
             if (lane == 0) at = atomicAdd(&b.ctl->n_sel[SEL_DEFERRED], (uint32_t)__popcll(dm));
@@ -1992,7 +2046,7 @@ struct alignas(8) FusedSeedLds {
 };
 
 template <int LMAX>
-union alignas(8) FusedLds {
+union alignas(16) FusedLds {
     FusedSeedLds<LMAX> seed;
     MergeLds merge;
 };
@@ -2064,7 +2118,7 @@ __device__ __forceinline__ void fused_wave_walks(const DevIndex &ix, bool mine, 
                                                  uint32_t qs, uint32_t qe, uint32_t strand_bit, uint32_t &kept,
                                                  DevHit *out, uint32_t at) {
     const uint32_t lane = lane_id();
-    uint64_t m = __ballot(mine);
+    uint64_t m = ballot(mine);
     while (m) {
         const uint32_t l = (uint32_t)__builtin_ctzll(m);
         m &= m - 1;
@@ -2085,12 +2139,13 @@ __device__ __forceinline__ void fused_wave_walks(const DevIndex &ix, bool mine, 
 template <int LMAX>
 __device__ __forceinline__ void fused_read(const DevBatch &b, const DevIndex &ix, const SeedParams &P,
                                            FusedLds<LMAX> &S, uint32_t r, uint32_t rescue_cutoff,
-                                           uint32_t hard_cutoff, DevHit *stash, uint32_t &stashed) {
+                                           uint32_t hard_cutoff, DevHit *stash, uint32_t &stashed,
+                                           uint32_t &stashed_fwd) {
     stashed = 0;
     const uint32_t lane = lane_id();
     const int L = (int)sload(b.read_len + r);
     bool spill = L > LMAX;
-    uint32_t nh = 0, n_fwd = 0;
+    uint32_t nh = 0, n_fwd = 0, nh_fwd = 0;
     bool rescue = false;
     float frac = 1.0f;
     if (!spill) {
@@ -2142,6 +2197,7 @@ __device__ __forceinline__ void fused_read(const DevBatch &b, const DevIndex &ix
                 // fetched, a second slot's lines read again
                 const uint32_t ia = wave_incl_scan_dpp(ha), ib = nq > 64 ? wave_incl_scan_dpp(hb) : 0u;
                 const uint32_t tot_a = readlane_u32(ia, 63);
+                nh_fwd = n_fwd ? readlane_u32(ia, n_fwd - 1) : 0u;
                 nh = tot_a + readlane_u32(ib, 63);
                 spill = nh > (uint32_t)MERGE_LDS;
                 if (!spill) {
@@ -2189,6 +2245,7 @@ __device__ __forceinline__ void fused_read(const DevBatch &b, const DevIndex &ix
                 // hits into LDS in query order: forward seeds, then reverse ones
                 const uint32_t ia = wave_incl_scan_dpp(ha), ib = nq > 64 ? wave_incl_scan_dpp(hb) : 0u;
                 const uint32_t tot_a = readlane_u32(ia, 63);
+                nh_fwd = n_fwd ? readlane_u32(ia, n_fwd - 1) : 0u;
                 nh = tot_a + readlane_u32(ib, 63);
                 spill = nh > (uint32_t)MERGE_LDS;
                 if (!spill) {
@@ -2227,12 +2284,11 @@ __device__ __forceinline__ void fused_read(const DevBatch &b, const DevIndex &ix
             b.rhit_total[r] = 0;
         }
         stashed = nh;
+        stashed_fwd = nh_fwd;
         return;
     }
     uint32_t total = 0;
-    if (nh > 0)
-        total = merge_wave(nh, S.merge.hits, S.merge.keys, nullptr, nullptr,
-                           b.nam_slots + (uint64_t)r * F_NAMCAP, (uint32_t)F_NAMCAP);
+    if (nh > 0) total = merge_arrival(S.merge.hits, nh, b.nam_slots + (uint64_t)r * F_NAMCAP, (uint32_t)F_NAMCAP);
     if (total > (uint32_t)F_NAMCAP) {  // includes MERGE_OVERFLOW
         spill_read(b, r);
         return;
@@ -2250,78 +2306,29 @@ __device__ __forceinline__ void fused_read(const DevBatch &b, const DevIndex &ix
 // The merge of up to four stashed reads (read k's hits in stash[k] for
 // k < 3, the fourth read's in slot3) on one wave, 16 lanes a read, as
 // k_merge4 merges them. A read a strand of which needs more than 16 NAMs is
-// then merged alone from its stash (merge_wave), and spilled if its NAMs
-// exceed F_NAMCAP.
-// meta: the reads' ids (0..3) and hit counts (4..7), in LDS.
+// then merged alone from its stash, and spilled if its NAMs exceed F_NAMCAP.
+// meta: the reads' ids (0..3), hit counts (4..7) and forward hits (8..11), in
+// LDS.
 __device__ __forceinline__ void fused_quad_merge(const DevBatch &b, DevHit (*stash)[64], DevHit *slot3, uint32_t qn,
                                                  const uint32_t *meta) {
     const uint32_t lane = lane_id(), seg = lane / SEG, j = lane % SEG;
     const bool act = seg < qn;
-    const uint32_t r = meta[seg];
-    const uint32_t nh = act ? meta[4 + seg] : 0u;
+    const uint32_t r = meta[seg], nh = act ? meta[4 + seg] : 0u, nf = act ? meta[8 + seg] : 0u;
     const DevHit *mine = seg < 3 ? stash[seg] : slot3;
-    gis_nam *out = b.nam_slots + (uint64_t)r * F_NAMCAP;
-    LaneNam o{0, 0, 0, 0, 0, 0, 0, 0};
-    uint32_t rsd_o = 0, n_open = 0, strand = 0, base = 0;
-    bool ovf = false;
-    const uint32_t maxh = wave_max_dpp(nh);
-    for (uint32_t t = 0; t < maxh; t++) {
-        const bool valid = act && !ovf && t < nh;
-        DevHit h{};
-        if (valid) h = mine[t];
-        const uint32_t hs = h.ref_strand >> 31;
-        const bool sw = valid && hs != strand;
-        if (__ballot(sw)) {
-            seg_finalize(out, base, j, n_open, rsd_o, o, sw);
-            if (sw) {
-                base += n_open;
-                n_open = 0;
-                strand = hs;
-            }
-        }
-        const int qs = h.query_start, qe = h.query_end, rs = h.ref_start, re = h.ref_end;
-        bool ext = false;
-        const bool acc = valid & (j < n_open) & (rsd_o == h.ref_strand) &
-                         nam_accepts(o.qp, o.qe, o.rp, o.re, qs, qe, rs, re, ext);
-        const uint64_t bal = __ballot(acc);
-        const uint32_t mine = (uint32_t)(bal >> (seg * SEG)) & ((1u << SEG) - 1u);
-        // as in k_merge4: the first accepting lane takes the hit, else it
-        // opens a NAM in the segment's next lane (selects, no branches)
-        const bool take = (mine != 0u) & (j == (uint32_t)__builtin_ctz(mine | 0x10000u));
-        const bool opens = valid & (mine == 0u);
-        const bool full = n_open == SEG;
-        const bool mk = opens & !full & (j == n_open);
-        o.qe = (take & ext) ? qe : o.qe;
-        o.re = (take & ext) ? re : o.re;
-        o.qp = (take | mk) ? qs : o.qp;
-        o.rp = (take | mk) ? rs : o.rp;
-        o.n = mk ? 1 : o.n + (take ? 1 : 0);
-        o.qs = mk ? qs : o.qs;
-        o.rs = mk ? rs : o.rs;
-        o.qe = mk ? qe : o.qe;
-        o.re = mk ? re : o.re;
-        o.cid = mk ? n_open : o.cid;
-        rsd_o = mk ? h.ref_strand : rsd_o;
-        ovf = ovf | (opens & full);
-        n_open += (opens & !full) ? 1u : 0u;
-    }
-    const bool fin = act && !ovf;
-    if (__ballot(fin)) seg_finalize(out, base, j, n_open, rsd_o, o, fin);
-    if (fin && j == 0) b.nam_cnt[r] = base + n_open;
+    const uint32_t total = merge_segments(mine, nh, nf, b.nam_slots + (uint64_t)r * F_NAMCAP);
+    if (act && j == 0 && total != MERGE_OVERFLOW) b.nam_cnt[r] = total;
+    uint64_t redo = ballot(act && j == 0 && total == MERGE_OVERFLOW);
     wave_sync_mem();
-    uint64_t redo = __ballot(act && ovf && j == 0);
     while (redo) {
         const uint32_t l = (uint32_t)__builtin_ctzll(redo);
         redo &= redo - 1;
         const uint32_t rk = readlane_u32(r, l), nk = readlane_u32(nh, l);
-        const uint32_t total =
-            merge_wave(nk, l / SEG < 3 ? stash[l / SEG] : slot3, nullptr, nullptr, nullptr,
-                       b.nam_slots + (uint64_t)rk * F_NAMCAP,
-                       (uint32_t)F_NAMCAP);
-        if (total > (uint32_t)F_NAMCAP) {
+        const uint32_t all = merge_arrival(l / SEG < 3 ? stash[l / SEG] : slot3, nk,
+                                           b.nam_slots + (uint64_t)rk * F_NAMCAP, (uint32_t)F_NAMCAP);
+        if (all > (uint32_t)F_NAMCAP) {
             spill_read(b, rk);
         } else {
-            if (lane == 0) b.nam_cnt[rk] = total;
+            if (lane == 0) b.nam_cnt[rk] = all;
             wave_sync_mem();
         }
     }
@@ -2339,7 +2346,7 @@ __global__ __launch_bounds__(64 * FWPB) __attribute__((amdgpu_waves_per_eu(6))) 
     if (K20) pin_k20_profile(P);
     __shared__ FusedLds<LMAX> lds[FWPB];
     __shared__ DevHit qstash[FWPB][3][64];
-    __shared__ uint32_t qmeta[FWPB][8];
+    __shared__ uint32_t qmeta[FWPB][12];
     const int wid = (int)uni32(threadIdx.x >> 6);
     FusedLds<LMAX> &S = lds[wid];
     DevHit(*stash)[64] = qstash[wid];
@@ -2367,13 +2374,14 @@ __global__ __launch_bounds__(64 * FWPB) __attribute__((amdgpu_waves_per_eu(6))) 
         if (have) {
             const uint32_t r = sload(queue + w);
             w += chunk == 0 ? gridDim.x * FWPB : 1u;
-            uint32_t nh = 0;
+            uint32_t nh = 0, nf = 0;
             DevHit *slot = qn < 3 ? stash[qn] : S.merge.hits;
-            fused_read<LMAX>(b, ix, P, S, r, rescue_cutoff, hard_cutoff, alone ? nullptr : slot, nh);
+            fused_read<LMAX>(b, ix, P, S, r, rescue_cutoff, hard_cutoff, alone ? nullptr : slot, nh, nf);
             if (nh) {
                 if (lane_id() == 0) {
                     meta[qn] = r;
                     meta[4 + qn] = nh;
+                    meta[8 + qn] = nf;
                 }
                 wave_sync_mem();
                 qn++;
@@ -2482,7 +2490,7 @@ __global__ __launch_bounds__(64 * WPB) void k_compact(DevBatch b, int fused, con
                 if (i < words) dst[i] = v[u];
             }
         }
-        uint64_t bigs = __ballot(big && j == 0);
+        uint64_t bigs = ballot(big && j == 0);
         while (bigs) {
             const uint32_t l = (uint32_t)__builtin_ctzll(bigs);
             bigs &= bigs - 1;

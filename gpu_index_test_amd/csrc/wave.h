@@ -102,8 +102,30 @@ __device__ __forceinline__ uint32_t wave_max_dpp(uint32_t x) {
     return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
 }
 
+// The lanes for which p holds, straight from the comparison's mask (__ballot
+// takes an int and compares again), and a mask's own bit on each lane. Every
+// lane must be active.
+__device__ __forceinline__ uint64_t ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+__device__ __forceinline__ bool lane_bit(uint64_t m) { return __builtin_amdgcn_inverse_ballot_w64(m); }
+
 // lanes for which p holds
-__device__ __forceinline__ uint32_t wave_count(bool p) { return (uint32_t)__popcll(__ballot(p)); }
+__device__ __forceinline__ uint32_t wave_count(bool p) { return (uint32_t)__popcll(ballot(p)); }
+
+// the lowest lane of each row of 16 that m holds, for all four rows at once on the
+// scalar unit (a row's top bit, set before the subtraction, keeps its borrow
+// inside the row)
+__device__ __forceinline__ uint64_t first_of_rows(uint64_t m) {
+    return m & ~((m | 0x8000800080008000ull) - 0x0001000100010001ull);
+}
+
+// sum of x over each row of 16 lanes, on every lane of the row
+__device__ __forceinline__ uint32_t row_sum(uint32_t x) {
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, true);   // row_shr:1
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, true);   // row_shr:2
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, true);   // row_shr:4
+    x += (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, true);   // row_shr:8
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x15f, 0xf, 0xf, false);  // row_newbcast:15
+}
 
 __device__ __forceinline__ uint32_t readlane_u32(uint32_t v, uint32_t l) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l);

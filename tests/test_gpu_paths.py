@@ -158,3 +158,54 @@ def test_host_calls_of_any_size(ctx, mode):
                 assert q[int(off[r]): int(off[r + 1])].tobytes() == O.randstrobes_query(read, op).tobytes()
                 assert sy[int(soff[r]): int(soff[r + 1])].tobytes() == O.syncmers(read, op).tobytes()
     idx.ctx.close()
+
+
+@pytest.mark.parametrize("hits", [1, 15, 16, 17, 33, 63, 64, 65, 66, 127, 128, 129, 255, 256, 257, 400, 512, 513, 700])
+@pytest.mark.parametrize("refs", [1, 3])
+def test_merge_path_edges(ctx, hits, refs):
+    """Merges around the limits of their ways (16 and 64 NAMs a strand, 64,
+    128, 256 and 512 hits): a strand of hits that each open a NAM, one of hits
+    on a few diagonals, and runs of equal query starts, on one and on several
+    references and split between the strands in several ways, against the
+    oracle."""
+    rng = np.random.default_rng(100 * hits + refs)
+    ents, reads, used = [], [], set()
+
+    def query(starts, style, rev):
+        q = np.zeros(len(starts), dtype=O.QUERY_RANDSTROBE)
+        q["start"], q["end"], q["is_reverse"] = starts, starts + rng.integers(20, 60, len(starts)), rev
+        for i in range(len(q)):
+            h = int(rng.integers(1 << 50, 1 << 63))
+            assert h not in used
+            used.add(h)
+            q["hash"][i] = h
+            s = int(starts[i])
+            if style == "apart":       # a NAM a hit
+                pos = [2_000_000 - 300 * i]
+            elif style == "diagonals":  # mostly extended or contained, four diagonals
+                pos = [50_000 + s + int(rng.choice([0, 0, 0, 7, 200, 5000]))]
+            else:                      # a tandem: several hits of one query start
+                pos = sorted(set((70_000 + s + 11 * rng.integers(0, 40, 6)).tolist()))
+            for p in pos:
+                ents.append((h, p, int(rng.integers(0, refs)) << 8 | int(rng.integers(0, 40))))
+        return q
+
+    for style in ("apart", "diagonals", "tandem"):
+        per = 5 if style == "tandem" else 1
+        for cut in (0, 1, hits // 2, hits):
+            n = max(1, hits // per)
+            f = min(n, cut // per)
+            starts = np.arange(n, dtype=np.int64) * 5
+            reads.append(np.concatenate([query(starts[:f], style, 0), query(starts[f:], style, 1)]))
+    arr, starts = tiny_index_arrays(ents, 12)
+    op = O.params_from_read_length(150)
+    oidx = O.Index.wrap(arr, starts, 12, 30, op)
+    idx = G.StrobemerIndex(None, G.IndexParameters.from_read_length(150))
+    idx.upload(arr, starts, 12, 30)
+    res = G._qrs_call(idx, reads, 0, 0, 1000)
+    resc = G._qrs_call(idx, reads, 1, 60, 1000)
+    for r, q in enumerate(reads):
+        _, exp, _ = O.find_nams(oidx, q, canonical=True)
+        assert res.read_nams(r).tobytes() == exp.tobytes(), r
+        assert resc.read_nams(r).tobytes() == O.find_nams_rescue(oidx, q, 60, 1000, canonical=True).tobytes(), r
+    idx.ctx.close()
