@@ -1079,54 +1079,6 @@ __device__ __forceinline__ void bitonic_mem(uint64_t *keys, uint32_t P) {
     }
 }
 
-// Stable wave radix sort of n keys (group << 32 | hit index) by the group
-// field, 4 bits a pass over key_bits bits; src and alt hold n entries each.
-// Returns the buffer that holds the sorted keys.
-__device__ __forceinline__ uint64_t *radix_sort_groups(uint64_t *src, uint64_t *alt, uint32_t n,
-                                                       uint32_t key_bits) {
-    const uint32_t lane = lane_id();
-    for (uint32_t shift = 32; shift < 32 + key_bits; shift += 4) {
-        uint32_t off[16];
-#pragma unroll
-        for (int v = 0; v < 16; v++) off[v] = 0;
-        for (uint32_t i0 = 0; i0 < n; i0 += 64) {
-            const uint32_t i = i0 + lane;
-            const uint32_t d = i < n ? (uint32_t)(src[i] >> shift) & 15u : 16u;
-#pragma unroll
-            for (int v = 0; v < 16; v++) off[v] += (uint32_t)__popcll(ballot(d == (uint32_t)v));
-        }
-        uint32_t run = 0;
-#pragma unroll
-        for (int v = 0; v < 16; v++) {
-            const uint32_t c = off[v];
-            off[v] = run;
-            run += c;
-        }
-        for (uint32_t i0 = 0; i0 < n; i0 += 64) {
-            const uint32_t i = i0 + lane;
-            uint64_t key = 0;
-            uint32_t d = 16u;
-            if (i < n) {
-                key = src[i];
-                d = (uint32_t)(key >> shift) & 15u;
-            }
-            uint32_t pos = 0;
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                const uint64_t bal = ballot(d == (uint32_t)v);
-                if (d == (uint32_t)v) pos = off[v] + mbcnt(bal);
-                off[v] += (uint32_t)__popcll(bal);
-            }
-            if (i < n) alt[pos] = key;
-        }
-        wave_sync_mem();
-        uint64_t *t = src;
-        src = alt;
-        alt = t;
-    }
-    return src;
-}
-
 constexpr uint32_t MERGE_OVERFLOW = 0xffffffffu;
 
 struct LaneNam {
@@ -1225,45 +1177,111 @@ __device__ __forceinline__ void wide_flush(const WideList &wide, uint32_t nw, gi
     }
 }
 
-// Grouped order of nh > 64 hits: nullptr when they already are in (strand,
-// ref) order, else keys (bitonic in keys, nh <= MERGE_LDS) or one of keys /
-// keys_alt (stable radix sort) holding group << 32 | hit index.
-__device__ __forceinline__ const uint64_t *group_order(uint32_t nh, const DevHit *hits, uint64_t *keys,
-                                                      uint64_t *keys_alt) {
+// items loaded ahead per lane by the passes over a read's hits: a lone wave's
+// time in them is the latency of its loads
+constexpr uint32_t AHEAD = 4;
+
+// One stable pass of group_order's radix sort by the 8-bit digit at `shift` of
+// the group: from the hits themselves (src == nullptr) or from keys (group << 32
+// | hit index). bins: 256 words of LDS.
+template <typename Load>
+__device__ __forceinline__ void radix_pass(uint32_t n, uint32_t shift, Load load, uint64_t *dst, uint32_t *bins) {
     const uint32_t lane = lane_id();
-    const uint64_t *order = nullptr;
-    uint32_t unsorted = 0, max_ref = 0;
+    for (uint32_t u = lane; u < 256; u += 64) bins[u] = 0;
+    wave_sync();
+    for (uint32_t i0 = 0; i0 < n; i0 += 64 * AHEAD) {
+        uint64_t k[AHEAD];
+#pragma unroll
+        for (uint32_t u = 0; u < AHEAD; u++) {
+            const uint32_t i = i0 + 64 * u + lane;
+            k[u] = load(i < n ? i : n - 1);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < AHEAD; u++)
+            if (i0 + 64 * u + lane < n) atomicAdd(&bins[(uint32_t)(k[u] >> (32 + shift)) & 255u], 1u);
+    }
+    wave_sync();
+    // exclusive prefix over the bins, four a lane
+    const uint32_t b0 = bins[4 * lane], b1 = bins[4 * lane + 1], b2 = bins[4 * lane + 2], b3 = bins[4 * lane + 3];
+    const uint32_t t = b0 + b1 + b2 + b3, at = wave_incl_scan_dpp(t) - t;
+    wave_sync();
+    bins[4 * lane] = at;
+    bins[4 * lane + 1] = at + b0;
+    bins[4 * lane + 2] = at + b0 + b1;
+    bins[4 * lane + 3] = at + b0 + b1 + b2;
+    wave_sync();
+    for (uint32_t i0 = 0; i0 < n; i0 += 64 * AHEAD) {
+        uint64_t k[AHEAD];
+#pragma unroll
+        for (uint32_t u = 0; u < AHEAD; u++) {
+            const uint32_t i = i0 + 64 * u + lane;
+            k[u] = load(i < n ? i : n - 1);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < AHEAD; u++) {
+            const bool in = i0 + 64 * u + lane < n;
+            const uint32_t d = (uint32_t)(k[u] >> (32 + shift)) & 255u;
+            // the 64 keys digit by digit: a read's hits lie in few groups
+            uint32_t pos = 0;
+            uint64_t left = ballot(in);
+            while (left) {
+                const uint32_t l = (uint32_t)__builtin_ctzll(left), dl = readlane_u32(d, l);
+                const uint64_t m = ballot(in && d == dl);
+                const uint32_t at_d = bins[dl];
+                if (d == dl) pos = at_d + mbcnt(m);
+                wave_sync();
+                if (lane == l) bins[dl] = at_d + (uint32_t)__popcll(m);
+                wave_sync();
+                left &= ~m;
+            }
+            if (in) dst[pos] = k[u];
+        }
+    }
+    wave_sync_mem();
+}
+
+// Grouped order of nh hits: nullptr when they already are in (strand, ref)
+// order, else keys (bitonic in keys, nh <= MERGE_LDS) or one of keys /
+// keys_alt (stable radix sort) holding group << 32 | hit index. bins: 256 words
+// of LDS for nh > MERGE_LDS.
+__device__ __forceinline__ const uint64_t *group_order(uint32_t nh, const DevHit *hits, uint64_t *keys,
+                                                      uint64_t *keys_alt, uint32_t *bins) {
+    const uint32_t lane = lane_id();
+    const uint4 *hv = reinterpret_cast<const uint4 *>(hits);
+    uint32_t max_ref = 0;
+    bool unsorted = false;
+#pragma unroll 4
     for (uint32_t i0 = 0; i0 < nh; i0 += 64) {
         const uint32_t i = i0 + lane;
-        if (i < nh) {
-            const uint32_t rsd = hits[i].ref_strand;
-            max_ref = max_ref > (rsd & 0x7fffffffu) ? max_ref : (rsd & 0x7fffffffu);
-            if (i > 0 && hits[i - 1].ref_strand > rsd) unsorted = 1;
-        }
+        const uint32_t rsd = hv[i < nh ? i : nh - 1].x, before = hv[i < nh ? (i ? i - 1 : 0) : nh - 1].x;
+        max_ref = max(max_ref, rsd & 0x7fffffffu);
+        unsorted |= before > rsd;
     }
-    if (ballot(unsorted != 0) != 0) {
-        if (nh <= (uint32_t)MERGE_LDS) {
-            uint32_t P = 1;
-            while (P < nh) P <<= 1;
-            for (uint32_t i = lane; i < P; i += 64)
-                keys[i] = i < nh ? (((uint64_t)hits[i].ref_strand << 32) | i) : UINT64_MAX;
-            wave_sync_mem();
-            bitonic_mem(keys, P);
-            order = keys;
-        } else {
-            // compact group key: strand above the bits of the largest ref_id
-            const uint32_t mr = wave_max(max_ref);
-            const uint32_t rbits = mr ? 32u - (uint32_t)__builtin_clz(mr) : 0u;
-            for (uint32_t i = lane; i < nh; i += 64) {
-                const uint32_t rsd = hits[i].ref_strand;
-                const uint64_t g = ((uint64_t)(rsd >> 31) << rbits) | (rsd & 0x7fffffffu);
-                keys[i] = (g << 32) | i;
-            }
-            wave_sync_mem();
-            order = radix_sort_groups(keys, keys_alt, nh, rbits + 1);
-        }
+    if (ballot(unsorted) == 0) return nullptr;
+    if (nh <= (uint32_t)MERGE_LDS) {
+        uint32_t P = 1;
+        while (P < nh) P <<= 1;
+        for (uint32_t i = lane; i < P; i += 64) keys[i] = i < nh ? (((uint64_t)hv[i].x << 32) | i) : UINT64_MAX;
+        wave_sync_mem();
+        bitonic_mem(keys, P);
+        return keys;
     }
-    return order;
+    // compact group key: strand above the bits of the largest ref_id. The first
+    // pass reads the hits, a read on few references needs no other.
+    const uint32_t mr = wave_max_dpp(max_ref);
+    const uint32_t rbits = mr ? 32u - (uint32_t)__builtin_clz(mr) : 0u;
+    radix_pass(nh, 0, [&](uint32_t i) {
+        const uint32_t x = hv[i].x;
+        return (((uint64_t)(x >> 31) << rbits | (x & 0x7fffffffu)) << 32) | i;
+    }, keys, bins);
+    uint64_t *src = keys, *alt = keys_alt;
+    for (uint32_t shift = 8; shift < rbits + 1; shift += 8) {
+        const uint64_t *from = src;
+        radix_pass(nh, shift, [&](uint32_t i) { return from[i]; }, alt, bins);
+        alt = src;
+        src = const_cast<uint64_t *>(from == keys ? keys_alt : keys);
+    }
+    return src;
 }
 
 // Reference-interval bounds of one 64-entry chunk of the wide list: every
@@ -1273,15 +1291,20 @@ struct ChunkBox {
     int lo, hi;
 };
 
-__device__ __forceinline__ int wave_min_i(int v) {
-    for (int d = 32; d >= 1; d >>= 1) v = min(v, __shfl_xor(v, d, 64));
-    return v;
+// wave minimum and maximum by DPP row shifts and broadcasts (wave_incl_scan_dpp);
+// lanes a step does not reach keep the identity
+__device__ __forceinline__ int wave_max_i(int v) {
+    constexpr int LOW = (int)0x80000000;
+    v = max(v, __builtin_amdgcn_update_dpp(LOW, v, 0x111, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(LOW, v, 0x112, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(LOW, v, 0x114, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(LOW, v, 0x118, 0xf, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(LOW, v, 0x142, 0xa, 0xf, false));
+    v = max(v, __builtin_amdgcn_update_dpp(LOW, v, 0x143, 0xc, 0xf, false));
+    return __builtin_amdgcn_readlane(v, 63);
 }
 
-__device__ __forceinline__ int wave_max_i(int v) {
-    for (int d = 32; d >= 1; d >>= 1) v = max(v, __shfl_xor(v, d, 64));
-    return v;
-}
+__device__ __forceinline__ int wave_min_i(int v) { return ~wave_max_i(~v); }
 
 // bounds of the wide list's chunks c0 .. (all of them when c0 == 0)
 __device__ __forceinline__ void boxes_rebuild(const WideList &wide, uint32_t nw, ChunkBox *box) {
@@ -1342,6 +1365,8 @@ __device__ __forceinline__ uint64_t lanes_take(LaneNam &o, uint64_t acc, uint64_
     return me;
 }
 
+constexpr uint32_t ARRIVAL_BLOCK = 4;
+
 // Merge of a read's hits in arrival order on one wave, a NAM a lane, without
 // grouping them: NAMs of every group of the current strand share the lanes, and
 // a NAM only accepts hits of its own group, which arrive in (query_start,
@@ -1349,12 +1374,15 @@ __device__ __forceinline__ uint64_t lanes_take(LaneNam &o, uint64_t acc, uint64_
 // hits end. With one group on the strand (a read of one place, the usual case)
 // creation order is the rank, so dead NAMs may leave when the lanes are full.
 // Returns the NAM count (entries at index >= cap are not written), or
-// MERGE_OVERFLOW when a strand needs more than 64 lanes.
+// MERGE_OVERFLOW when a strand needs more than 64 lanes, or, with BLOCKS, when
+// the hits come in blocks of ARRIVAL_BLOCK or more equal query starts on
+// average (repeats): merge_range takes a block at a time.
 //
 // A lone wave's time is its chain of instructions a hit (one issues every ~8
 // cycles), branches above all: the loop over hits has none but its end and the
 // full-lanes exit (~550 cycles a hit; the group-by-group merge took ~800 with
 // its sort and block tests before it).
+template <bool BLOCKS = false>
 __device__ __forceinline__ uint32_t merge_arrival(const DevHit *hits, uint32_t nh, gis_nam *out, uint32_t cap) {
     const uint32_t lane = lane_id();
     const uint4 *hv = reinterpret_cast<const uint4 *>(hits);
@@ -1365,9 +1393,15 @@ __device__ __forceinline__ uint32_t merge_arrival(const DevHit *hits, uint32_t n
     {
         const uint32_t h0 = uni32(hv[0].x), hl = uni32(hv[nh ? nh - 1 : 0].x);
         uint64_t of = 0, orv = 0;
+        uint32_t blocks = 0;
         for (uint32_t x0 = 0; x0 < nh; x0 += 64) {
             const bool in = x0 + lane < nh;
             const uint32_t r = in ? hv[x0 + lane].x : 0xffffffffu;
+            if (BLOCKS) {
+                const uint32_t q = in ? hv[x0 + lane].w & 0xffffu : 0u;
+                const uint32_t pq = (uint32_t)__shfl_up((int)q, 1, 64);
+                blocks += wave_count(in && (lane == 0 || q != pq));
+            }
             const uint64_t fwd = ballot(r >> 31 == 0);
             nf += (uint32_t)__popcll(fwd);
             of |= ballot(r != h0) & fwd;
@@ -1375,6 +1409,7 @@ __device__ __forceinline__ uint32_t merge_arrival(const DevHit *hits, uint32_t n
         }
         other[0] = of != 0;
         other[1] = orv != 0;
+        if (BLOCKS && nh >= ARRIVAL_BLOCK * blocks) return MERGE_OVERFLOW;
     }
     uint32_t base = 0;
     for (int strand = 0; strand < 2; strand++) {
@@ -1431,6 +1466,72 @@ __device__ __forceinline__ uint32_t merge_arrival(const DevHit *hits, uint32_t n
     return base;
 }
 
+// LDS of one wave's block matching: the 64 hits in its registers (ref start, ref
+// end, query end), and who holds them
+struct alignas(16) BlockLds {
+    int4 h[64];
+    uint32_t hold[64];
+};
+
+// The hits that the lanes' NAMs (those of `can`) take of a block: hits [t, t +
+// len) of B, ref starts ascending, less those not in cm. Hit by hit, each takes
+// the first accepting NAM that no earlier hit of the block took. All hits rank
+// the NAMs alike (by lane) and all NAMs the hits (by order), so that assignment
+// is also the one where each NAM, in lane order, takes the first accepting hit
+// that is left, and the only stable one: NAMs propose to their first accepting
+// hit, a hit holds its lowest lane, and a NAM that is turned down goes on to its
+// next. A NAM's candidates are the hits with ref start in (o_rp, o_re], found by
+// binary search. Returns this lane's hit or -1; took: the hits taken.
+//
+// A tandem repeat's block has hundreds of hits and NAMs, each NAM with a handful
+// of candidates. The hit-by-hit loop took ~25 instructions a hit for every chunk
+// of NAMs; this is ~150 for a chunk and 64 hits, most of them waiting for LDS,
+// so the candidates are read four at a time.
+__device__ __forceinline__ int match_block(BlockLds &B, uint32_t t, uint32_t len, uint64_t cm, bool can, int o_qe,
+                                           int o_rp, int o_re, uint64_t &took) {
+    const uint32_t lane = lane_id(), end = t + len;
+    uint32_t i = t, n = len;  // the first hit with ref start above o_rp
+    while (n > 0) {
+        const uint32_t half = n >> 1;
+        const bool up = B.h[i + half].x <= o_rp;
+        i = up ? i + half + 1 : i;
+        n = up ? n - half - 1 : half;
+    }
+    uint64_t mask = 0;
+    bool more = can && i < end;
+    while (ballot(more)) {
+        int4 h[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; u++) h[u] = B.h[min(i + u, end - 1)];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; u++) {
+            more = more && i < end && h[u].x <= o_re;
+            if (more && ((h[u].z > o_qe) == (h[u].y > o_re))) mask |= 1ull << i;
+            i++;
+        }
+        more = more && i < end;
+    }
+    mask &= cm;
+    B.hold[lane] = 0xffffffffu;
+    wave_sync();
+    int p;
+    for (;;) {
+        p = mask ? (int)__builtin_ctzll(mask) : -1;
+        if (p >= 0) atomicMin(&B.hold[p], lane);
+        wave_sync();
+        const bool down = p >= 0 && B.hold[p] != lane;
+        if (ballot(down) == 0) break;
+        if (down) mask &= mask - 1;
+        wave_sync();
+    }
+    took = ballot(B.hold[lane] != 0xffffffffu);
+    wave_sync();
+    return p;
+}
+
+// blocks of fewer hits go hit by hit
+constexpr uint32_t MATCH_MIN = 8;
+
 // Merge hits order[xb .. xe) (hit indices in grouped order; order nullptr:
 // the hits themselves in order). NAM c of the k-th group of the range is
 // written at out[(NAMs of the range's earlier groups) + c]; entries at index
@@ -1450,28 +1551,53 @@ __device__ __forceinline__ uint32_t merge_arrival(const DevHit *hits, uint32_t n
 // 64 hits in registers is two blocks.
 __device__ __forceinline__ uint32_t merge_range(const DevHit *hits, const uint64_t *order, uint32_t xb,
                                                 uint32_t xe, const WideList wide, gis_nam *out,
-                                                uint32_t cap, ChunkBox *box = nullptr, uint32_t box_cap = 0) {
+                                                uint32_t cap, BlockLds &B, ChunkBox *box = nullptr,
+                                                uint32_t box_cap = 0) {
     const uint32_t lane = lane_id();
     LaneNam o{0, 0, 0, 0, 0, 0, 0, 0};
     uint32_t n_open = 0, grp = 0xffffffffu, base = 0, gcnt = 0;
     bool wide_mode = false;
     uint32_t nw = 0, wide_mark = 0;
+    // the next 64 hits load while these merge (their place in the grouped order
+    // was read one step before)
+    const uint4 *hv = reinterpret_cast<const uint4 *>(hits);
+    const auto place = [&](uint32_t x) {
+        const uint32_t i = min(x + lane, xe - 1);
+        return order ? (uint32_t)order[i] : i;
+    };
+    uint32_t at_next = 0;
+    uint4 h_next = make_uint4(0u, 0u, 0u, 0u);
+    if (xb < xe) {
+        h_next = hv[place(xb)];
+        at_next = place(xb + 64);
+    }
     for (uint32_t x0 = xb; x0 < xe; x0 += 64) {
-        uint4 h = make_uint4(0u, 0u, 0u, 0u);
-        if (x0 + lane < xe)
-            h = reinterpret_cast<const uint4 *>(hits)[order ? (uint32_t)order[x0 + lane] : x0 + lane];
+        const uint4 h = h_next;
+        if (x0 + 64 < xe) {
+            h_next = hv[at_next];
+            at_next = place(x0 + 128);
+        }
         const uint32_t c_rsd = h.x, c_rs = h.y, c_re = h.z, c_q = h.w;
         const uint32_t m = xe - x0 < 64 ? xe - x0 : 64;
         // lanes that start a block, and a group (lane 0 against the last chunk's)
         const uint32_t p_rsd = (uint32_t)__shfl_up((int)c_rsd, 1, 64), p_q = (uint32_t)__shfl_up((int)c_q, 1, 64);
         const uint64_t gheads = ballot(c_rsd != (lane ? p_rsd : grp));
         const uint64_t heads = gheads | ballot(((c_q ^ p_q) & 0xffffu) != 0 || lane == 0);
+        // hits whose ref start lies below the one before them in their block (a
+        // block of one seed has none)
+        const int p_rs = __shfl_up((int)c_rs, 1, 64);
+        const uint64_t falls = ballot((int)c_rs < p_rs) & ~heads;
+        wave_sync();
+        B.h[lane] = make_int4((int)c_rs, (int)c_re, (int)(c_q >> 16), 0);
+        wave_sync();
         uint32_t singles_until = 0;  // the rest of a block that did not fit the lanes goes hit by hit
         for (uint32_t t = 0; t < m;) {
             const uint32_t q = readlane_u32(c_q, t);
             const int qs = (int)(q & 0xffffu);
             const uint64_t next = heads & ~((2ull << t) - 1);
-            uint32_t len = (next ? min((uint32_t)__builtin_ctzll(next), m) : m) - t;
+            const uint32_t len = (next ? min((uint32_t)__builtin_ctzll(next), m) : m) - t;
+            const uint64_t block = (len >= 64 ? ~0ull : ((1ull << len) - 1)) << t;
+            const bool match = len >= MATCH_MIN && (falls & block) == 0;
             if ((gheads >> t) & 1ull) {
                 if (t >= singles_until) {
                     if (wide_mode) {
@@ -1495,6 +1621,20 @@ __device__ __forceinline__ uint32_t merge_range(const DevHit *hits, const uint64
                     if (n_open == 0) {
                         n_new = len;  // a group's first block opens a NAM a hit
                         my_hit = lane < len ? (int)(t + lane) : -1;
+                    } else if (match) {
+                        uint64_t took;
+                        my_hit = match_block(B, t, len, block, lane < n_open && o.qp < qs && qs <= o.qe, o.qe, o.rp,
+                                             o.re, took);
+                        const uint64_t opens = block & ~took;
+                        n_new = (uint32_t)__popcll(opens);
+                        fits = n_open + n_new <= 64;
+                        // the k-th hit that opens a NAM goes to lane n_open + k
+                        if (fits && n_new) {
+                            if (lane_bit(opens)) B.hold[n_open + mbcnt(opens)] = lane;
+                            wave_sync();
+                            if (lane >= n_open && lane < n_open + n_new) my_hit = (int)B.hold[lane];
+                            wave_sync();
+                        }
                     } else {
                         uint64_t taken = 0;
                         for (uint32_t i = t; i < t + len; i++) {
@@ -1517,8 +1657,8 @@ __device__ __forceinline__ uint32_t merge_range(const DevHit *hits, const uint64
                     }
                     if (fits) {
                         const int src = my_hit < 0 ? 0 : my_hit;
-                        const int hrs = __shfl((int)c_rs, src, 64), hre = __shfl((int)c_re, src, 64);
-                        const int hqe = (int)((uint32_t)__shfl((int)c_q, src, 64) >> 16);
+                        const int4 hh = B.h[src];
+                        const int hrs = hh.x, hre = hh.y, hqe = hh.z;
                         const bool take = my_hit >= 0 && lane < n_open;
                         const bool mk = my_hit >= 0 && lane >= n_open;
                         const bool grow = mk || (take && hqe > o.qe && hre > o.re);
@@ -1575,7 +1715,7 @@ __device__ __forceinline__ uint32_t merge_range(const DevHit *hits, const uint64
             // the entry it would take hit by hit (the hits a chunk leaves
             // pending find no acceptor in it, by induction over the chunks),
             // and a chunk is read once per block instead of once per hit.
-            uint64_t pend = (len >= 64 ? ~0ull : ((1ull << len) - 1)) << t;
+            uint64_t pend = block;
             const uint32_t nch = (nw + 63) >> 6;
             const bool boxed = box && nch <= box_cap;
             const int my_rs = (int)c_rs;
@@ -1595,6 +1735,11 @@ __device__ __forceinline__ uint32_t merge_range(const DevHit *hits, const uint64
                 if (valid) w = wget(wide, e);
                 uint64_t taken = 0;
                 int my_hit = -1;  // the hit (chunk lane) this entry takes
+                if (match) {
+                    my_hit = match_block(B, t, len, cm, valid && w.qp < qs && qs <= w.qe, w.qe, w.rp, w.re, taken);
+                    pend &= ~taken;
+                    cm = 0;
+                }
                 while (cm) {
                     const uint32_t i = (uint32_t)__builtin_ctzll(cm);
                     cm &= cm - 1;
@@ -1613,8 +1758,8 @@ __device__ __forceinline__ uint32_t merge_range(const DevHit *hits, const uint64
                 }
                 if (taken) {
                     const int src = my_hit < 0 ? 0 : my_hit;
-                    const int hrs = __shfl((int)c_rs, src, 64), hre = __shfl((int)c_re, src, 64);
-                    const int hqe = (int)((uint32_t)__shfl((int)c_q, src, 64) >> 16);
+                    const int4 hh = B.h[src];
+                    const int hrs = hh.x, hre = hh.y, hqe = hh.z;
                     const bool tk = my_hit >= 0;
                     const bool ext = tk && hqe > w.qe && hre > w.re;
                     if (ext) {
@@ -1706,15 +1851,16 @@ constexpr uint32_t ITEM_HITS = 384;
 constexpr uint32_t ARRIVAL_MAX = 512;
 // entries of a wide list that lie in LDS: per wave of k_merge, and per group of
 // k_merge_groups (one wave per block)
-constexpr int MERGE_WIDE_LDS = 256;
-constexpr int GROUP_WIDE_LDS = 1024;
-// chunk bounds of a k_merge_groups wide list (lists up to 32,768 entries)
-constexpr uint32_t GROUP_BOXES = 512;
+constexpr int MERGE_WIDE_LDS = 128;
+constexpr int GROUP_WIDE_LDS = 512;
+// chunk bounds of a k_merge_groups wide list (lists up to 8,192 entries)
+constexpr uint32_t GROUP_BOXES = 128;
 
 // the reads that k_merge4 handed on, one per wave
 __global__ __launch_bounds__(64 * WPB) void k_merge(DevBatch b) {
     __shared__ uint64_t lkeys[WPB][MERGE_LDS];
     __shared__ WideNam lwide[WPB][MERGE_WIDE_LDS];  // the wide list of reads with few enough hits
+    __shared__ BlockLds lblock[WPB];
     const uint32_t lane = lane_id();
     const int wid = (int)uni32(threadIdx.x >> 6);
     if (hits_missing(b)) return;
@@ -1730,7 +1876,8 @@ __global__ __launch_bounds__(64 * WPB) void k_merge(DevBatch b) {
         WideNam *gwide = b.merge_scratch ? (rescue ? b.rnam_ws : b.nam_ws) + hb : nullptr;
         if (nh > SPLIT_MIN && b.merge_scratch) {
             // group the hits; each group merges on its own wave
-            const uint64_t *ord = group_order(nh, ghits, gkeys, gkeys + nh);
+            uint32_t *bins = reinterpret_cast<uint32_t *>(lkeys[wid]);
+            const uint64_t *ord = group_order(nh, ghits, gkeys, gkeys + nh, bins);
             const uint32_t code = ord == nullptr ? 0u : (ord == gkeys ? 1u : 2u);
             uint64_t *slots = code == 1u ? gkeys + nh : gkeys;
             uint32_t G = 0;
@@ -1738,8 +1885,9 @@ __global__ __launch_bounds__(64 * WPB) void k_merge(DevBatch b) {
                 const uint32_t i = i0 + lane;
                 bool head = false;
                 if (i < nh) {
-                    const uint32_t cur = ghits[ord ? (uint32_t)ord[i] : i].ref_strand;
-                    head = i == 0 || ghits[ord ? (uint32_t)ord[i - 1] : i - 1].ref_strand != cur;
+                    // (keys hold the group above the index)
+                    const uint32_t cur = ord ? (uint32_t)(ord[i] >> 32) : ghits[i].ref_strand;
+                    head = i == 0 || (ord ? (uint32_t)(ord[i - 1] >> 32) : ghits[i - 1].ref_strand) != cur;
                 }
                 const uint64_t bal = ballot(head);
                 if (head) slots[G + mbcnt(bal)] = (uint64_t)i << 32;
@@ -1781,13 +1929,14 @@ __global__ __launch_bounds__(64 * WPB) void k_merge(DevBatch b) {
                 continue;
             }
         }
-        uint32_t total = nh <= ARRIVAL_MAX ? merge_arrival(ghits, nh, fin, nh) : MERGE_OVERFLOW;
+        uint32_t total = nh <= ARRIVAL_MAX ? merge_arrival<true>(ghits, nh, fin, nh) : MERGE_OVERFLOW;
         if (total == MERGE_OVERFLOW && (nh <= (uint32_t)MERGE_LDS || b.merge_scratch)) {
             // more than 64 NAMs at once: group by group, with a wide list (NAMs <= hits)
-            const uint64_t *ord = nh <= (uint32_t)MERGE_LDS ? group_order(nh, ghits, lkeys[wid], nullptr)
-                                                            : group_order(nh, ghits, gkeys, gkeys + nh);
+            const bool lds = nh <= (uint32_t)MERGE_LDS;
+            const uint64_t *ord = group_order(nh, ghits, lds ? lkeys[wid] : gkeys, lds ? nullptr : gkeys + nh,
+                                              reinterpret_cast<uint32_t *>(lkeys[wid]));
             const WideList wl{(LdsWideNam *)lwide[wid], gwide, (uint32_t)MERGE_WIDE_LDS};
-            total = merge_range(ghits, ord, 0, nh, wl, fin, nh);
+            total = merge_range(ghits, ord, 0, nh, wl, fin, nh, lblock[wid]);
         }
         if (total == MERGE_OVERFLOW) {
             // needs the global scratch, which this run does not have yet
@@ -1808,6 +1957,7 @@ __global__ __launch_bounds__(64 * WPB) void k_merge(DevBatch b) {
 __global__ __launch_bounds__(64) void k_merge_groups(DevBatch b) {
     __shared__ WideNam lwide[GROUP_WIDE_LDS];
     __shared__ ChunkBox lbox[GROUP_BOXES];
+    __shared__ BlockLds lblock;
     const uint32_t lane = lane_id();
     const unsigned int cnt = sload(&b.ctl->n_gwork);
     for (uint32_t w = blockIdx.x; w < cnt; w += gridDim.x) {
@@ -1825,7 +1975,7 @@ __global__ __launch_bounds__(64) void k_merge_groups(DevBatch b) {
         WideNam *far = (rescue ? b.rnam_ws : b.nam_ws) + hb + gs;
         gis_nam *out = (rescue ? b.rnam_fin : b.nam_fin) + hb + gs;
         const WideList wl{(LdsWideNam *)lwide, far, (uint32_t)GROUP_WIDE_LDS};
-        const uint32_t c = merge_range(ghits, ord, gs, ge, wl, out, ge - gs, lbox, GROUP_BOXES);
+        const uint32_t c = merge_range(ghits, ord, gs, ge, wl, out, ge - gs, lblock, lbox, GROUP_BOXES);
         if (lane == 0) slots[g] = ((uint64_t)gs << 32) | c;
         wave_sync_mem();
     }
