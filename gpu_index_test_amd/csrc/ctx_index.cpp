@@ -149,15 +149,15 @@ extern "C" int gis_index_build(gis_ctx *ctx, const char *const *seqs, const uint
     uint64_t n = 0;
     uint64_t hist[RUN_BINS] = {};
     try {
-        uint4 *recs = nullptr;
-        device_seed_reference(seqs, lens, n_refs, *params, &recs, &n, ctx->stream);
-        ix.rs.p = recs;
-        ix.rs.bytes = std::max<uint64_t>(n, 1) * sizeof(gis_ref_randstrobe);
+        BuildArena arena(build_estimate(total, *params));
+        const RefSeeds seeds = device_seed_reference(seqs, lens, n_refs, *params, true, arena, ctx->stream);
+        n = seeds.n;
+        uint4 *rs = ensure<uint4>(ix.rs, n);
         ensure<uint64_t>(ix.starts, (1ull << bits) + 1);
-        device_sort_records(static_cast<uint4 *>(ix.rs.p), n, ctx->stream);
-        device_finish_index(static_cast<const uint4 *>(ix.rs.p), n, bits, static_cast<uint64_t *>(ix.starts.p),
-                            hist, ctx->stream);
+        device_sort_records(seeds, rs, arena, ctx->stream);
+        device_finish_index(rs, n, bits, static_cast<uint64_t *>(ix.starts.p), hist, arena, ctx->stream);
     } catch (const BuildError &e) {
+        (void)hipStreamSynchronize(ctx->stream);
         throw HipError{e.e, e.what};
     }
     HostIndex st;
@@ -187,22 +187,18 @@ extern "C" int gis_reference_randstrobes(gis_ctx *ctx, const char *const *seqs, 
     uint64_t total = 0;
     for (uint32_t j = 0; j < n_refs; j++) total += lens[j];
     if (total == 0) return GIS_OK;
-    uint4 *recs = nullptr;
-    uint64_t n = 0;
     try {
-        device_seed_reference(seqs, lens, n_refs, *params, &recs, &n, ctx->stream);
+        BuildArena arena(build_estimate(total, *params));
+        const RefSeeds seeds = device_seed_reference(seqs, lens, n_refs, *params, false, arena, ctx->stream);
+        const uint64_t n = seeds.n;
+        *n_out = n;
+        if (n > capacity || (n && !out))
+            return fail(ctx, GIS_ERR_CAPACITY,
+                        "record capacity " + std::to_string(capacity) + " < " + std::to_string(n));
+        if (n) HIP_CHECK(hipMemcpy(out, seeds.recs, n * sizeof(gis_ref_randstrobe), hipMemcpyDeviceToHost));
     } catch (const BuildError &e) {
         throw HipError{e.e, e.what};
     }
-    DevBuf keep{recs, n * sizeof(gis_ref_randstrobe)};
-    *n_out = n;
-    if (n > capacity || (n && !out)) {
-        release(keep);
-        return fail(ctx, GIS_ERR_CAPACITY, "record capacity " + std::to_string(capacity) + " < " + std::to_string(n));
-    }
-    const hipError_t e = n ? hipMemcpy(out, recs, n * sizeof(gis_ref_randstrobe), hipMemcpyDeviceToHost) : hipSuccess;
-    release(keep);
-    HIP_CHECK(e);
     return GIS_OK;
     API_END(ctx)
 }

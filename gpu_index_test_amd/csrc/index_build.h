@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <vector>
+
 #include "../../include/gis.h"
 
 namespace gis {
@@ -15,16 +17,52 @@ struct BuildError {
     const char *what;
 };
 
+// Device memory of one build, freed with it: pieces cut from a few large blocks.
+// An allocation and its release cost ~180 us together, more than most of the
+// build's kernels on a bacterial genome, so the first block is sized for the
+// whole build and a second one is taken only where the estimate falls short.
+class BuildArena {
+  public:
+    explicit BuildArena(uint64_t estimate) : next_(estimate) {}
+    ~BuildArena();
+    BuildArena(const BuildArena &) = delete;
+    BuildArena &operator=(const BuildArena &) = delete;
+    void *bytes(uint64_t n);
+    template <typename T>
+    T *get(uint64_t n) {
+        return static_cast<T *>(bytes(n * sizeof(T)));
+    }
+
+  private:
+    std::vector<void *> blocks_;
+    char *at_ = nullptr;
+    uint64_t left_ = 0, next_;
+};
+
+// device memory of a whole build of `bases` bases (a randstrobe in every k - s +
+// 1 bases or so): sequence, windows, syncmers, records twice for the sort
+uint64_t build_estimate(uint64_t bases, const gis_params &p);
+
 // The RefRandstrobe records of every contig (RandstrobeGenerator over each
 // contig, step2/randstrobes.cu:161-190, step2/index.cu:246-311), seeded on
 // the device in (contig, position) order; contigs shorter than w_max get
-// zero records in their slots. *out is a device array of *n_out records
-// from hipMalloc, owned by the caller.
-void device_seed_reference(const char *const *seqs, const uint64_t *lens, uint32_t n_refs, const gis_params &p,
-                           uint4 **out, uint64_t *n_out, hipStream_t st);
-// sort n RefRandstrobe records (16 B: u64 hash, u32 position, u32 packed) in
-// place by (hash, position, packed); allocates and frees its own buffers
-void device_sort_records(uint4 *rs, uint64_t n, hipStream_t st);
+// zero records in their slots. The arrays are the arena's.
+struct RefSeeds {
+    uint64_t n = 0;
+    uint64_t *hash = nullptr;  // split form: hashes, and position << 32 | packed
+    uint64_t *sec = nullptr;
+    uint4 *recs = nullptr;     // else: records
+    // sorting by the position bits alone (below 2^pos_bits) leaves records of
+    // equal hash and position in the order of their packed word: they come in
+    // contig order, one a contig and position. Zero records break that.
+    int pos_bits = 0;
+    bool zeros = false;
+};
+RefSeeds device_seed_reference(const char *const *seqs, const uint64_t *lens, uint32_t n_refs, const gis_params &p,
+                               bool split, BuildArena &arena, hipStream_t st);
+// the records of a split RefSeeds sorted by (hash, position, packed) into rs (n
+// records); the seeds' arrays are used up
+void device_sort_records(const RefSeeds &s, uint4 *rs, BuildArena &arena, hipStream_t st);
 // checks a resident table and its starts: null if the lookups can trust
 // them, else what is wrong (unsorted records, or bucket starts that do not
 // match the records' top hash bits)
@@ -32,6 +70,6 @@ const char *device_validate_index(const uint4 *rs, uint64_t n, const uint64_t *s
 // bucket starts (2^bits + 1 entries) and the run-length histogram of a
 // sorted table; hist_out receives RUN_BINS host counters
 void device_finish_index(const uint4 *rs, uint64_t n, int bits, uint64_t *starts, uint64_t *hist_out,
-                         hipStream_t st);
+                         BuildArena &arena, hipStream_t st);
 
 }  // namespace gis

@@ -181,19 +181,6 @@ __device__ __forceinline__ uint32_t syncmer_passes(int L, const SeedParams &P, c
     return nsync;
 }
 
-// Four bases at once: the 2-bit codes (nt4 of step2/randstrobes.hpp:22-43), one
-// a byte, and in bad the bytes that are not ACGTU in either case (non-zero).
-// Bits 1 and 2 of a folded letter index the four letters; a byte is a base if
-// it is the letter it indexes, or U where that is T.
-__device__ __forceinline__ uint32_t nt4x4(uint32_t v, uint32_t &bad) {
-    const uint32_t u = v & 0xdfdfdfdfu;
-    const uint32_t idx = (u >> 1) & 0x03030303u;  // A 0, C 1, T and U 2, G 3
-    const uint32_t letter = __builtin_amdgcn_perm(0u, 0x47544341u, idx);
-    const uint32_t is2 = (idx >> 1) & ~idx;  // bit 0 of a byte: index 2
-    bad = (u ^ letter) & ~(is2 & 0x01010101u);
-    return idx ^ ((idx >> 1) & 0x01010101u);
-}
-
 // the four bases 4 i .. 4 i + 3 of a read as loaded together (their last bytes
 // may lie past the read's end: the sequence array has SEQ_PAD bytes after the
 // last read), and the mask of those inside it
@@ -231,8 +218,7 @@ __device__ __forceinline__ uint32_t seed_syncmers(const char *__restrict__ seq, 
         const uint32_t v = four_bases(seq, L, i, inside);
         const uint32_t c = nt4x4(v, bad) & inside;
         any |= bad & inside;
-        // c0 + 4 c1 + 16 c2 + 64 c3
-        if (i < nbytes) pkb[i] = (uint8_t)__builtin_amdgcn_udot4(c, 0x40100401u, 0u, false);
+        if (i < nbytes) pkb[i] = (uint8_t)pack4(c);
     }
     wave_sync();
     uint32_t nsync = 0;

@@ -7,17 +7,17 @@
 // boundary acts as an N run: no window spans two contigs and the first
 // window after a boundary starts a segment. The scan runs as passes over
 // the whole genome, each a grid over positions:
-//   1. bases packed 2 bits each, with a mask of non-ACGT bases (ballots);
-//   2. the canonical s-mer hash at every position;
-//   3. the state of every k-mer window that needs no history (segment
+//   1. bases packed 2 bits each, with a mask of non-ACGT bases, sixteen a lane;
+//   2. a tile of k-mer windows a block: the canonical s-mer hashes in LDS, and
+//      from them the state of every window that needs no history (segment
 //      starts and windows with a unique minimum below ~0, gis_core.h);
-//   4. each maximal run of windows with tied minima replayed from the known
-//      window before it by one lane (slide, gis_core.h) -- tied runs are
-//      rare and short except in tandem repeats, and a run's replay is
-//      sequential in the reference too;
-//   5. syncmer positions compacted per 4096-window tile (scan of tile
+//   3. each maximal run of windows with tied minima replayed from the known
+//      window before it by one lane (slide, gis_core.h), its hashes computed
+//      again -- tied runs are rare and short except in tandem repeats, and a
+//      run's replay is sequential in the reference too;
+//   4. syncmer positions compacted per 4096-window tile (scan of tile
 //      counts), then the canonical k-mer hash of each syncmer;
-//   6. per contig, the range of its syncmers; then one lane per syncmer
+//   5. per contig, the range of its syncmers; then one lane per syncmer
 //      picks its partner among the next w_min..w_max syncmers of the contig
 //      within max_dist (the smallest popcount((h_i ^ h_j) & q), earliest on
 //      ties) and writes its record. A contig's last w_min syncmers start no
@@ -40,23 +40,6 @@ namespace {
 
 constexpr int TILE_THREADS = 256, TILE_WIN = 16, TILE = TILE_THREADS * TILE_WIN;
 
-struct Dev {
-    void *p = nullptr;
-    ~Dev() {
-        if (p) (void)hipFree(p);
-    }
-};
-
-template <typename T>
-T *dalloc(Dev &d, uint64_t n) {
-    const hipError_t e = hipMalloc(&d.p, std::max<uint64_t>(n, 1) * sizeof(T));
-    if (e != hipSuccess) {
-        d.p = nullptr;
-        throw BuildError{e, "hipMalloc (reference seeding)"};
-    }
-    return static_cast<T *>(d.p);
-}
-
 void check(hipError_t e, const char *what) {
     if (e != hipSuccess) throw BuildError{e, what};
 }
@@ -69,88 +52,178 @@ unsigned grid(uint64_t items, unsigned per_block) {
 #define GRID_STRIDE(i, n) \
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < (n); i += (uint64_t)gridDim.x * blockDim.x)
 
-// 1. one wave per 64 bases: pk[2w], pk[2w+1] and nmask[w]
-__global__ void k_ref_pack(const char *__restrict__ seq, uint64_t T, uint64_t nwords, uint64_t *__restrict__ pk,
-                           uint64_t *__restrict__ nmask) {
-    const uint32_t lane = lane_id();
-    const uint64_t waves = (uint64_t)gridDim.x * (blockDim.x / 64);
-    for (uint64_t w = (uint64_t)blockIdx.x * (blockDim.x / 64) + threadIdx.x / 64; w < nwords; w += waves) {
-        const uint64_t i = w * 64 + lane;
-        int c = 4;
-        if (i < T) c = nt4((unsigned char)seq[i]);
-        const bool ok = i < T && c < 4;
-        const uint64_t lo = __ballot(ok && (c & 1));
-        const uint64_t hi = __ballot(ok && (c & 2));
-        const uint64_t m = __ballot(!ok);  // past the end reads as N
-        if (lane == 0) {
-            nmask[w] = m;
-            pk[2 * w] = spread32((uint32_t)lo) | (spread32((uint32_t)hi) << 1);
-        } else if (lane == 1) {
-            pk[2 * w + 1] = spread32((uint32_t)(lo >> 32)) | (spread32((uint32_t)(hi >> 32)) << 1);
+// 1. sixteen bases a lane: a 32-bit word of packed bases and 16 bits of the N
+// mask; past the end reads as N
+__global__ __launch_bounds__(256) void k_ref_pack(const uint4 *__restrict__ seq, uint64_t T, uint64_t n16,
+                                                  uint32_t *__restrict__ pk, uint16_t *__restrict__ nmask) {
+    GRID_STRIDE(w, n16) {
+        const uint64_t first = 16 * w;
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);
+        if (first < T) v = seq[w];  // (the array is padded to 16 bytes)
+        const uint32_t in[4] = {v.x, v.y, v.z, v.w};
+        uint32_t p = 0, n = 0;
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            uint32_t bad;
+            p |= pack4(nt4x4(in[u], bad)) << (8 * u);
+#pragma unroll
+            for (int q = 0; q < 4; q++) n |= (bad >> (8 * q) & 0xffu) != 0 ? 1u << (4 * u + q) : 0u;
         }
+        if (first + 16 > T) n |= first >= T ? 0xffffu : 0xffffu << (T - first) & 0xffffu;
+        pk[w] = p;
+        nmask[w] = (uint16_t)n;
     }
 }
 
-// 2. canonical s-mer hash per s-mer start (0 where it holds a non-ACGT base:
-// such windows are invalid)
-__global__ void k_ref_smer(const uint64_t *__restrict__ pk, const uint64_t *__restrict__ nmask, uint64_t ns,
-                           SeedParams P, uint64_t *__restrict__ sh) {
-    GRID_STRIDE(j, ns) {
+// the 'N' after each contig
+__global__ void k_ref_separators(char *__restrict__ seq, const uint64_t *__restrict__ cstart, uint32_t n_refs) {
+    GRID_STRIDE(c, n_refs) seq[cstart[c + 1] - 1] = 'N';
+}
+
+// canonical s-mer hash at base j
+__device__ __forceinline__ uint64_t smer_hash(const uint64_t *pk, uint64_t j, const SeedParams &P) {
+    return xxh64_u64(canonical_code(pk, j, P.s, P.smask));
+}
+
+// 2. window states that need no history, WIN windows a block. The s-mer hashes
+// stay in LDS, high words apart: they decide a window unless two of them tie.
+// The hashes' 64-bit products bound it. (20.0 M windows: 77 us; a pass that wrote
+// the hashes and one that read five of them a window took 88 us each and 160 MB.)
+// S16: s <= 16, an s-mer's code is one 32-bit word.
+constexpr int WIN = 2048, WIN_MAX_W = 32;
+
+template <bool S16>
+__global__ __launch_bounds__(256) void k_ref_windows(const uint64_t *__restrict__ pk,
+                                                     const uint64_t *__restrict__ nmask, uint64_t ns, uint64_t nk,
+                                                     SeedParams P, uint8_t *__restrict__ st) {
+    __shared__ uint32_t hi[WIN + WIN_MAX_W], lo[WIN + WIN_MAX_W];
+    const uint64_t p0 = (uint64_t)blockIdx.x * WIN;
+    const uint64_t *bpk = pk + p0 / 32;
+    const int bns = ns > p0 ? (int)std::min<uint64_t>(ns - p0, WIN + WIN_MAX_W) : 0;
+    // (s-mers with a non-ACGT base lie in invalid windows only)
+    for (int i = threadIdx.x; i < WIN + P.w - 1; i += 256) {
         uint64_t h = 0;
-        if (!any_n(nmask, j, j + (uint64_t)P.s - 1)) h = xxh64_u64(canonical_code(pk, j, P.s, P.smask));
-        sh[j] = h;
+        if (i < bns)
+            h = xxh64_u64(S16 ? canonical_code32(bpk, i, P.s, (uint32_t)P.smask)
+                              : canonical_code(bpk, i, P.s, P.smask));
+        hi[i] = (uint32_t)(h >> 32);
+        lo[i] = (uint32_t)h;
     }
-}
-
-// 3. window states that need no history
-__global__ void k_ref_anchor(const uint64_t *__restrict__ nmask, const uint64_t *__restrict__ sh, uint64_t nk,
-                             SeedParams P, uint8_t *__restrict__ st) {
-    GRID_STRIDE(p, nk) {
+    __syncthreads();
+    for (int i = threadIdx.x; i < WIN; i += 256) {
+        const uint64_t p = p0 + i;
+        if (p >= nk) break;
         uint8_t s;
         if (any_n(nmask, p, p + (uint64_t)P.k - 1)) {
             s = ST_INVALID;
         } else {
-            const bool seg_first = p == 0 || ((nmask[(p - 1) >> 6] >> ((p - 1) & 63)) & 1);
-            s = P.w == 5 ? anchor_state_w<5>(sh, p, seg_first) : anchor_state(sh + p, 0, P.w, seg_first);
+            uint32_t m = hi[i];
+            int at = 0, eq = 1;
+            for (int o = 1; o < P.w; o++) {
+                const uint32_t v = hi[i + o];
+                eq = v < m ? 1 : eq + (v == m ? 1 : 0);
+                at = v < m ? o : at;
+                m = min(m, v);
+            }
+            s = (uint8_t)at;
+            if (eq > 1) {  // the full hashes decide
+                uint64_t mv = UINT64_MAX;
+                int first = 0, ties = 0;
+                for (int o = 0; o < P.w; o++) {
+                    const uint64_t v = ((uint64_t)hi[i + o] << 32) | lo[i + o];
+                    if (v < mv) { mv = v; first = o; ties = 1; }
+                    else if (v == mv) ties++;
+                }
+                const bool seg_first = p == 0 || ((nmask[(p - 1) >> 6] >> ((p - 1) & 63)) & 1);
+                if (seg_first) s = mv == UINT64_MAX ? ST_NONE : (uint8_t)first;
+                else s = ties == 1 && mv != UINT64_MAX ? (uint8_t)first : ST_UNKNOWN;
+            } else if (m == 0xffffffffu && lo[i + at] == 0xffffffffu) {
+                // a minimum of ~0 (one window of one s-mer)
+                const bool seg_first = p == 0 || ((nmask[(p - 1) >> 6] >> ((p - 1) & 63)) & 1);
+                s = seg_first ? ST_NONE : ST_UNKNOWN;
+            }
         }
         st[p] = s;
     }
 }
 
-// 4. each run of tied windows replayed from the known window before it (a
+// 3. each run of tied windows replayed from the known window before it (a
 // run never starts a segment: a segment's first window is an anchor). The
 // resolved states go to st2, so that st, which decides where runs start,
 // never changes under the other lanes.
-__global__ void k_ref_resolve(const uint64_t *__restrict__ sh, const uint8_t *__restrict__ st, uint64_t nk,
-                              SeedParams P, uint8_t *__restrict__ st2) {
-    GRID_STRIDE(p, nk) {
-        if (p == 0 || st[p] != ST_UNKNOWN || st[p - 1] == ST_UNKNOWN) continue;
-        uint8_t r = st[p - 1];
-        for (uint64_t x = p; x < nk && st[x] == ST_UNKNOWN; x++) {
-            r = slide(r, sh + (x - 1), 1, P.w);
-            st2[x] = r;
+__global__ void k_ref_resolve(const uint64_t *__restrict__ pk,
+                              const uint8_t *__restrict__ st, uint64_t nk, SeedParams P,
+                              uint8_t *__restrict__ st2) {
+    // sixteen windows a lane: unknown ones are rare
+    GRID_STRIDE(g, (nk + 15) / 16) {
+        const uint4 v = reinterpret_cast<const uint4 *>(st)[g];  // (padded)
+        const uint32_t u4 = 0x01010101u * ST_UNKNOWN, w[4] = {v.x ^ u4, v.y ^ u4, v.z ^ u4, v.w ^ u4};
+        bool any = false;
+#pragma unroll
+        for (int q = 0; q < 4; q++) any |= ((w[q] - 0x01010101u) & ~w[q] & 0x80808080u) != 0;
+        if (!any) continue;
+        for (uint64_t p = std::max<uint64_t>(16 * g, 1); p < std::min(16 * g + 16, nk); p++) {
+            if (st[p] != ST_UNKNOWN || st[p - 1] == ST_UNKNOWN) continue;
+            // slide (gis_core.h) with the tracked hash kept; no base of these
+            // windows is an N
+            uint8_t r = st[p - 1];
+            uint64_t tracked = r == ST_NONE ? UINT64_MAX : smer_hash(pk, p - 1 + r, P);
+            for (uint64_t x = p; x < nk && st[x] == ST_UNKNOWN; x++) {
+                const uint64_t v = smer_hash(pk, x + P.w - 1, P);
+                if (r == 0) {  // left the window: its rightmost minimum
+                    r = (uint8_t)(P.w - 1);
+                    tracked = v;
+                    for (int o = P.w - 2; o >= 0; o--) {
+                        const uint64_t c = smer_hash(pk, x + o, P);
+                        if (c < tracked) { tracked = c; r = (uint8_t)o; }
+                    }
+                } else if (v < tracked) {
+                    r = (uint8_t)(P.w - 1);
+                    tracked = v;
+                } else if (r != ST_NONE) {
+                    r--;
+                }
+                st2[x] = r;
+            }
         }
     }
 }
 
-__device__ __forceinline__ bool is_syncmer(const uint8_t *st, const uint8_t *st2, uint64_t p, int t) {
-    uint8_t s = st[p];
-    if (s == ST_UNKNOWN) s = st2[p];
-    return s == (uint8_t)(t - 1);
+// which of the TILE_WIN windows from base on (a multiple of it) are syncmers
+static_assert(TILE_WIN == 16, "one 16-byte load of states");
+__device__ __forceinline__ uint32_t sync_flags(const uint8_t *st, const uint8_t *st2, uint64_t base, uint64_t nk,
+                                               int t) {
+    if (base >= nk) return 0;
+    const uint4 v = *reinterpret_cast<const uint4 *>(st + base);  // (padded)
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    const uint32_t want = (uint32_t)(t - 1);
+    uint32_t f = 0, unknown = 0;
+#pragma unroll
+    for (int u = 0; u < TILE_WIN; u++) {
+        const uint32_t s = w[u / 4] >> (8 * (u % 4)) & 0xffu;
+        f |= s == want ? 1u << u : 0u;
+        unknown |= s == ST_UNKNOWN ? 1u << u : 0u;
+    }
+    if (base + TILE_WIN > nk) {
+        const uint32_t in = (1u << (nk - base)) - 1u;
+        f &= in;
+        unknown &= in;
+    }
+    while (unknown) {
+        const uint32_t u = (uint32_t)__builtin_ctz(unknown);
+        unknown &= unknown - 1;
+        if (st2[base + u] == (uint8_t)want) f |= 1u << u;
+    }
+    return f;
 }
 
-// 5a. syncmers per tile of TILE windows
+// 4a. syncmers per tile of TILE windows
 __global__ __launch_bounds__(TILE_THREADS) void k_ref_sync_count(const uint8_t *__restrict__ st,
                                                                  const uint8_t *__restrict__ st2, uint64_t nk,
                                                                  int t, uint32_t *__restrict__ cnt) {
     __shared__ uint32_t part[TILE_THREADS / 64];
     const uint64_t base = (uint64_t)blockIdx.x * TILE + (uint64_t)threadIdx.x * TILE_WIN;
-    uint32_t c = 0;
-    for (int u = 0; u < TILE_WIN; u++) {
-        const uint64_t p = base + u;
-        if (p < nk && is_syncmer(st, st2, p, t)) c++;
-    }
-    c = wave_sum(c);
+    const uint32_t c = wave_sum((uint32_t)__popc(sync_flags(st, st2, base, nk, t)));
     if (lane_id() == 0) part[threadIdx.x / 64] = c;
     __syncthreads();
     if (threadIdx.x == 0) {
@@ -160,19 +233,14 @@ __global__ __launch_bounds__(TILE_THREADS) void k_ref_sync_count(const uint8_t *
     }
 }
 
-// 5b. syncmer positions in order: tile offset + rank inside the tile
+// 4b. syncmer positions in order: tile offset + rank inside the tile
 __global__ __launch_bounds__(TILE_THREADS) void k_ref_sync_write(const uint8_t *__restrict__ st,
                                                                  const uint8_t *__restrict__ st2, uint64_t nk,
                                                                  int t, const uint64_t *__restrict__ tile_off,
                                                                  uint64_t *__restrict__ sy_pos) {
     __shared__ uint32_t part[TILE_THREADS / 64];
     const uint64_t base = (uint64_t)blockIdx.x * TILE + (uint64_t)threadIdx.x * TILE_WIN;
-    uint32_t flags = 0;
-    for (int u = 0; u < TILE_WIN; u++) {
-        const uint64_t p = base + u;
-        if (p < nk && is_syncmer(st, st2, p, t)) flags |= 1u << u;
-    }
-    const uint32_t c = (uint32_t)__popc(flags);
+    const uint32_t flags = sync_flags(st, st2, base, nk, t), c = (uint32_t)__popc(flags);
     const uint32_t ex = wave_excl_scan(c);
     const uint32_t wtot = wave_sum(c);
     const uint32_t wid = threadIdx.x / 64;
@@ -185,13 +253,13 @@ __global__ __launch_bounds__(TILE_THREADS) void k_ref_sync_write(const uint8_t *
         if ((flags >> u) & 1u) sy_pos[at++] = base + u;
 }
 
-// 5c. canonical k-mer hash of each syncmer
+// 4c. canonical k-mer hash of each syncmer
 __global__ void k_ref_sync_hash(const uint64_t *__restrict__ pk, const uint64_t *__restrict__ sy_pos, uint64_t n,
                                 SeedParams P, uint64_t *__restrict__ sy_hash) {
     GRID_STRIDE(i, n) sy_hash[i] = xxh64_u64(canonical_code(pk, sy_pos[i], P.k, P.kmask));
 }
 
-// 6a. first syncmer of each contig (and n at the end): lower bound of the
+// 5a. first syncmer of each contig (and n at the end): lower bound of the
 // contig's first base among the syncmer positions
 __global__ void k_ref_contig_syncmers(const uint64_t *__restrict__ sy_pos, uint64_t n,
                                       const uint64_t *__restrict__ cstart, uint32_t n_refs,
@@ -212,12 +280,13 @@ __global__ void k_ref_contig_syncmers(const uint64_t *__restrict__ sy_pos, uint6
     }
 }
 
-// 6b. the randstrobe of each syncmer that starts one
+// 5b. the randstrobe of each syncmer that starts one
 __global__ void k_ref_randstrobes(const uint64_t *__restrict__ sy_pos, const uint64_t *__restrict__ sy_hash,
                                   uint64_t n, const uint64_t *__restrict__ sy_start,
                                   const uint64_t *__restrict__ rs_start, const uint64_t *__restrict__ cstart,
                                   const uint8_t *__restrict__ is_short, uint32_t n_refs, SeedParams P,
-                                  uint4 *__restrict__ out) {
+                                  uint4 *__restrict__ out, uint64_t *__restrict__ o_hash,
+                                  uint64_t *__restrict__ o_sec) {
     GRID_STRIDE(i, n) {
         // the contig: last c with sy_start[c] <= i
         uint32_t lo = 0, hi = n_refs;  // sy_start[lo] <= i < sy_start[hi]
@@ -232,7 +301,8 @@ __global__ void k_ref_randstrobes(const uint64_t *__restrict__ sy_pos, const uin
         if (i + P.w_min > last) continue;  // fewer than w_min syncmers follow
         const uint64_t o = rs_start[c] + (i - first);
         if (is_short[c]) {
-            out[o] = make_uint4(0u, 0u, 0u, 0u);
+            if (out) out[o] = make_uint4(0u, 0u, 0u, 0u);
+            else o_hash[o] = o_sec[o] = 0;
             continue;
         }
         const uint64_t hi_ = sy_hash[i], pi = sy_pos[i];
@@ -254,63 +324,69 @@ __global__ void k_ref_randstrobes(const uint64_t *__restrict__ sy_pos, const uin
         const uint64_t hash = hi_ + bh;
         const uint32_t pos = (uint32_t)(pi - cstart[c]);
         const uint32_t packed = (c << 8) + (uint32_t)(sy_pos[best] - pi);
-        out[o] = make_uint4((uint32_t)hash, (uint32_t)(hash >> 32), pos, packed);
+        if (out) {
+            out[o] = make_uint4((uint32_t)hash, (uint32_t)(hash >> 32), pos, packed);
+        } else {
+            o_hash[o] = hash;
+            o_sec[o] = ((uint64_t)pos << 32) | packed;
+        }
     }
 }
 
 }  // namespace
 
-void device_seed_reference(const char *const *seqs, const uint64_t *lens, uint32_t n_refs, const gis_params &gp,
-                           uint4 **out, uint64_t *n_out, hipStream_t st) {
-    *out = nullptr;
-    *n_out = 0;
+RefSeeds device_seed_reference(const char *const *seqs, const uint64_t *lens, uint32_t n_refs, const gis_params &gp,
+                               bool split, BuildArena &arena, hipStream_t st) {
+    RefSeeds out;
     const SeedParams P = make_seed_params(gp);
     // contig c at cstart[c], one 'N' after each; cstart[n_refs] = T
     std::vector<uint64_t> cstart(n_refs + 1);
-    uint64_t T = 0;
+    uint64_t T = 0, longest = 0;
     for (uint32_t c = 0; c < n_refs; c++) {
         cstart[c] = T;
         T += lens[c] + 1;
+        longest = std::max(longest, lens[c]);
     }
     cstart[n_refs] = T;
+    // (all host arrays here outlive the copies: the stream is waited for before
+    // they go, also on the way out of an error)
+    struct Drain {
+        hipStream_t st;
+        ~Drain() { (void)hipStreamSynchronize(st); }
+    } drain{st};
     const uint64_t nwords = (T + 63) / 64;
-    Dev d_seq, d_pk, d_nm, d_sh, d_st, d_st2, d_cnt, d_toff, d_tmp, d_pos, d_hash, d_cs, d_sys, d_rss, d_short;
-    char *seq = dalloc<char>(d_seq, T);
-    for (uint32_t c = 0; c < n_refs; c++) {
-        if (lens[c]) check(hipMemcpyAsync(seq + cstart[c], seqs[c], lens[c], hipMemcpyHostToDevice, st), "genome upload");
-        check(hipMemsetAsync(seq + cstart[c] + lens[c], 'N', 1, st), "contig separator");
-    }
-    // two pad words: canonical_code reads the word after a window's first
-    uint64_t *pk = dalloc<uint64_t>(d_pk, 2 * nwords + 2);
-    uint64_t *nm = dalloc<uint64_t>(d_nm, nwords + 1);
-    check(hipMemsetAsync(pk + 2 * nwords, 0, 16, st), "pad");
-    check(hipMemsetAsync(nm + nwords, 0xff, 8, st), "pad");
-    hipLaunchKernelGGL(k_ref_pack, dim3(grid(nwords, 4)), dim3(256), 0, st, seq, T, nwords, pk, nm);
+    char *seq = arena.get<char>(T + 16);
+    uint64_t *cs = arena.get<uint64_t>(n_refs + 1);
+    check(hipMemcpyAsync(cs, cstart.data(), 8ull * (n_refs + 1), hipMemcpyHostToDevice, st), "contig starts");
+    for (uint32_t c = 0; c < n_refs; c++)
+        if (lens[c])
+            check(hipMemcpyAsync(seq + cstart[c], seqs[c], lens[c], hipMemcpyHostToDevice, st), "genome upload");
+    hipLaunchKernelGGL(k_ref_separators, dim3(grid(n_refs, 256)), dim3(256), 0, st, seq, cs, n_refs);
+    // pad words: canonical_code reads the word after a window's first, any_n the
+    // last one's
+    uint64_t *pk = arena.get<uint64_t>(2 * nwords + 2);
+    uint64_t *nm = arena.get<uint64_t>(nwords + 1);
+    const uint64_t n16 = 4 * nwords + 4;
+    hipLaunchKernelGGL(k_ref_pack, dim3(grid(n16, 256)), dim3(256), 0, st, reinterpret_cast<const uint4 *>(seq), T,
+                       n16, reinterpret_cast<uint32_t *>(pk), reinterpret_cast<uint16_t *>(nm));
     check(hipGetLastError(), "k_ref_pack");
-    check(hipStreamSynchronize(st), "k_ref_pack");
-    (void)hipFree(d_seq.p);
-    d_seq.p = nullptr;
 
     const uint64_t ns = T >= (uint64_t)P.s ? T - P.s + 1 : 0;
     const uint64_t nk = T >= (uint64_t)P.k ? T - P.k + 1 : 0;
-    if (nk == 0) return;
-    uint64_t *sh = dalloc<uint64_t>(d_sh, ns);
-    uint8_t *stt = dalloc<uint8_t>(d_st, nk);
-    uint8_t *st2 = dalloc<uint8_t>(d_st2, nk);
-    hipLaunchKernelGGL(k_ref_smer, dim3(grid(ns, 256)), dim3(256), 0, st, pk, nm, ns, P, sh);
-    check(hipGetLastError(), "k_ref_smer");
-    hipLaunchKernelGGL(k_ref_anchor, dim3(grid(nk, 256)), dim3(256), 0, st, nm, sh, nk, P, stt);
-    check(hipGetLastError(), "k_ref_anchor");
-    hipLaunchKernelGGL(k_ref_resolve, dim3(grid(nk, 256)), dim3(256), 0, st, sh, stt, nk, P, st2);
+    if (nk == 0) return out;
+    if (P.w > WIN_MAX_W) throw BuildError{hipErrorInvalidValue, "windows of more than 32 s-mers"};
+    uint8_t *stt = arena.get<uint8_t>(nk + 16);
+    uint8_t *st2 = arena.get<uint8_t>(nk + 16);
+    hipLaunchKernelGGL(P.s <= 16 ? k_ref_windows<true> : k_ref_windows<false>, dim3((unsigned)((nk + WIN - 1) / WIN)), dim3(256), 0, st, pk, nm, ns, nk, P,
+                       stt);
+    check(hipGetLastError(), "k_ref_windows");
+    hipLaunchKernelGGL(k_ref_resolve, dim3(grid((nk + 15) / 16, 256)), dim3(256), 0, st, pk, stt, nk, P, st2);
     check(hipGetLastError(), "k_ref_resolve");
-    check(hipStreamSynchronize(st), "window states");
-    (void)hipFree(d_sh.p);
-    d_sh.p = nullptr;
 
     const uint64_t ntiles = (nk + TILE - 1) / TILE;
-    uint32_t *cnt = dalloc<uint32_t>(d_cnt, ntiles);
-    uint64_t *toff = dalloc<uint64_t>(d_toff, ntiles + 1);
-    uint64_t *tmp = dalloc<uint64_t>(d_tmp, scan_tmp_words(ntiles) + 8);
+    uint32_t *cnt = arena.get<uint32_t>(ntiles);
+    uint64_t *toff = arena.get<uint64_t>(ntiles + 1);
+    uint64_t *tmp = arena.get<uint64_t>(scan_tmp_words(ntiles) + 8);
     hipLaunchKernelGGL(k_ref_sync_count, dim3((unsigned)ntiles), dim3(TILE_THREADS), 0, st, stt, st2, nk, P.t, cnt);
     check(hipGetLastError(), "k_ref_sync_count");
     launch_scan(cnt, toff, ntiles, tmp, st);
@@ -318,18 +394,16 @@ void device_seed_reference(const char *const *seqs, const uint64_t *lens, uint32
     uint64_t nsy = 0;
     check(hipMemcpyAsync(&nsy, toff + ntiles, 8, hipMemcpyDeviceToHost, st), "syncmer count");
     check(hipStreamSynchronize(st), "syncmer count");
-    uint64_t *pos = dalloc<uint64_t>(d_pos, nsy);
+    uint64_t *pos = arena.get<uint64_t>(nsy);
     hipLaunchKernelGGL(k_ref_sync_write, dim3((unsigned)ntiles), dim3(TILE_THREADS), 0, st, stt, st2, nk, P.t, toff,
                        pos);
     check(hipGetLastError(), "k_ref_sync_write");
-    uint64_t *hsh = dalloc<uint64_t>(d_hash, nsy);
+    uint64_t *hsh = arena.get<uint64_t>(nsy);
     hipLaunchKernelGGL(k_ref_sync_hash, dim3(grid(nsy, 256)), dim3(256), 0, st, pk, pos, nsy, P, hsh);
     check(hipGetLastError(), "k_ref_sync_hash");
 
     // per contig: syncmer range, randstrobe slots, short contigs
-    uint64_t *cs = dalloc<uint64_t>(d_cs, n_refs + 1);
-    uint64_t *sys = dalloc<uint64_t>(d_sys, n_refs + 1);
-    check(hipMemcpyAsync(cs, cstart.data(), 8ull * (n_refs + 1), hipMemcpyHostToDevice, st), "contig starts");
+    uint64_t *sys = arena.get<uint64_t>(n_refs + 1);
     hipLaunchKernelGGL(k_ref_contig_syncmers, dim3(grid(n_refs + 1, 256)), dim3(256), 0, st, pos, nsy, cs, n_refs,
                        sys);
     check(hipGetLastError(), "k_ref_contig_syncmers");
@@ -341,26 +415,30 @@ void device_seed_reference(const char *const *seqs, const uint64_t *lens, uint32
     for (uint32_t c = 0; c < n_refs; c++) {
         rs_start[c] = total;
         const uint64_t nc = sy_start[c + 1] - sy_start[c];
-        total += nc > gp.w_min ? nc - gp.w_min : 0;
+        const uint64_t nr = nc > gp.w_min ? nc - gp.w_min : 0;
+        total += nr;
         is_short[c] = lens[c] < gp.w_max ? 1 : 0;
+        out.zeros |= is_short[c] && nr > 0;
     }
     rs_start[n_refs] = total;
-    uint64_t *rss = dalloc<uint64_t>(d_rss, n_refs + 1);
-    uint8_t *shrt = dalloc<uint8_t>(d_short, n_refs);
+    uint64_t *rss = arena.get<uint64_t>(n_refs + 1);
+    uint8_t *shrt = arena.get<uint8_t>(n_refs);
     check(hipMemcpyAsync(rss, rs_start.data(), 8ull * (n_refs + 1), hipMemcpyHostToDevice, st), "slot starts");
     check(hipMemcpyAsync(shrt, is_short.data(), n_refs, hipMemcpyHostToDevice, st), "short contigs");
-    uint4 *recs = nullptr;
-    check(hipMalloc(&recs, std::max<uint64_t>(total, 1) * sizeof(uint4)), "hipMalloc (records)");
-    hipLaunchKernelGGL(k_ref_randstrobes, dim3(grid(nsy, 256)), dim3(256), 0, st, pos, hsh, nsy, sys, rss, cs, shrt,
-                       n_refs, P, recs);
-    const hipError_t e = hipGetLastError();
-    const hipError_t e2 = hipStreamSynchronize(st);
-    if (e != hipSuccess || e2 != hipSuccess) {
-        (void)hipFree(recs);
-        throw BuildError{e != hipSuccess ? e : e2, "k_ref_randstrobes"};
+    out.n = total;
+    // one contig's positions ascend
+    out.pos_bits = n_refs > 1 && longest > 1 ? 64 - __builtin_clzll(longest - 1) : 0;
+    if (split) {
+        out.hash = arena.get<uint64_t>(total);
+        out.sec = arena.get<uint64_t>(total);
+    } else {
+        out.recs = arena.get<uint4>(total);
     }
-    *out = recs;
-    *n_out = total;
+    hipLaunchKernelGGL(k_ref_randstrobes, dim3(grid(nsy, 256)), dim3(256), 0, st, pos, hsh, nsy, sys, rss, cs, shrt,
+                       n_refs, P, out.recs, out.hash, out.sec);
+    check(hipGetLastError(), "k_ref_randstrobes");
+    check(hipStreamSynchronize(st), "k_ref_randstrobes");
+    return out;
 }
 
 }  // namespace gis

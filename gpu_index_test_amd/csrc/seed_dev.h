@@ -24,16 +24,21 @@ __device__ __forceinline__ bool any_n(const uint64_t *nm, I a, I b) {
     return (m1 | m2) != 0;
 }
 
-// bit m of v to bit 2m
-__device__ __forceinline__ uint64_t spread32(uint32_t v) {
-    uint64_t x = v;
-    x = (x | (x << 16)) & 0x0000FFFF0000FFFFULL;
-    x = (x | (x << 8)) & 0x00FF00FF00FF00FFULL;
-    x = (x | (x << 4)) & 0x0F0F0F0F0F0F0F0FULL;
-    x = (x | (x << 2)) & 0x3333333333333333ULL;
-    x = (x | (x << 1)) & 0x5555555555555555ULL;
-    return x;
+// Four bases at once: the 2-bit codes (nt4 of step2/randstrobes.hpp:22-43), one
+// a byte, and in bad the bytes that are not ACGTU in either case (non-zero).
+// Bits 1 and 2 of a folded letter index the four letters; a byte is a base if
+// it is the letter it indexes, or U where that is T.
+__device__ __forceinline__ uint32_t nt4x4(uint32_t v, uint32_t &bad) {
+    const uint32_t u = v & 0xdfdfdfdfu;
+    const uint32_t idx = (u >> 1) & 0x03030303u;  // A 0, C 1, T and U 2, G 3
+    const uint32_t letter = __builtin_amdgcn_perm(0u, 0x47544341u, idx);
+    const uint32_t is2 = (idx >> 1) & ~idx;  // bit 0 of a byte: index 2
+    bad = (u ^ letter) & ~(is2 & 0x01010101u);
+    return idx ^ ((idx >> 1) & 0x01010101u);
 }
+
+// four codes of nt4x4 as one byte, the first base lowest
+__device__ __forceinline__ uint32_t pack4(uint32_t c) { return __builtin_amdgcn_udot4(c, 0x40100401u, 0u, false); }
 
 // the 2-bit groups of x in reverse order
 __device__ __forceinline__ uint64_t rev_pairs(uint64_t x) {

@@ -209,3 +209,31 @@ def test_merge_path_edges(ctx, hits, refs):
         assert res.read_nams(r).tobytes() == exp.tobytes(), r
         assert resc.read_nams(r).tobytes() == O.find_nams_rescue(oidx, q, 60, 1000, canonical=True).tobytes(), r
     idx.ctx.close()
+
+
+@pytest.mark.parametrize("profile", [50, 150, 400])
+@pytest.mark.parametrize("lens", [[60_000], [30_000, 20_000, 12_345, 4096], [25_000, 8, 24, 31, 300, 25_000, 1]])
+def test_index_build_edges(ctx, profile, lens):
+    """One and several contigs, equal sequence at equal positions of several
+    contigs, contigs too short for a randstrobe, runs of tied s-mers, N runs
+    and lengths off every tile."""
+    rng = np.random.default_rng(len(lens) + profile)
+    lens = np.array(lens, dtype=np.uint64)
+    g = rng.choice(np.frombuffer(b"ACGT", dtype=np.uint8), size=int(lens.sum()))
+    at = np.concatenate([[0], np.cumsum(lens)]).astype(np.int64)
+    for c in range(len(lens)):
+        if lens[c] > 20_000:
+            s = g[at[c]:at[c + 1]]
+            s[:4000] = g[:4000]
+            s[5000:5400] = ord("A")
+            s[6000:6600] = np.frombuffer(b"AC" * 300, dtype=np.uint8)
+            s[7000:7150] = ord("N")
+            s[8000:8100] = np.frombuffer(b"acgtN" * 20, dtype=np.uint8)
+            s[-25:] = ord("T")
+    idx = G.StrobemerIndex(None, G.IndexParameters.from_read_length(profile))
+    idx.populate_arrays(g, lens)
+    oidx = O.Index.build_arrays(g, lens, O.params_from_read_length(profile), n_threads=4)
+    assert idx.randstrobes.tobytes() == oidx.randstrobes.tobytes()
+    assert np.array_equal(idx.randstrobe_start_indices, oidx.starts)
+    assert idx.filter_cutoff == oidx.filter_cutoff
+    idx.ctx.close()
