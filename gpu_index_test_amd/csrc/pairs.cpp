@@ -2,10 +2,12 @@
 //
 // A pair step is one sequence of launches on the batch's stream: reference
 // order, pair types, per-type lists and, with GIS_PAIRS_JOINT, the joint NAM
-// pairs. The joint entries are placed by a scan of per-pair upper bounds, so
-// the host reads that total once to size the entry array; a second
-// synchronisation at the end reads the type counts, the entry total and the
-// error bits.
+// pairs. The joint entries are placed by bounds that follow from the list
+// offsets, so nothing is read back in between; the last kernel writes the type
+// counts, the entry total and the error bits to pinned memory, read after one
+// synchronisation. The compacted entries have the room of earlier steps or one
+// NAM's worth of entries; where the total is larger, the compaction alone runs
+// again.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -22,8 +24,8 @@ namespace gis {
 
 struct PairWork {
     DevBuf in_off, in_nams;  // lists uploaded by gis_pairs_from_nams
-    DevBuf ord, types, drop, mapq, tcnt, tpos, tids, ttot, jbound, jboff, jtmp, jcnt, joff, jout, err, scan_tmp;
-    uint64_t *h = nullptr;  // pinned: [0..5] type starts, [6] joint bound total, [7] joint total, [8] error bits
+    DevBuf ord, types, drop, mapq, tcnt, tpos, tids, jtmp, jcnt, joff, jout, err, scan_tmp;
+    uint64_t *h = nullptr;  // pinned: [0..5] type starts, [6] joint total, [7] error bits
     const void *owner = nullptr;  // the batch (or context) whose lists the results belong to
     const uint64_t *dev_off = nullptr;
     uint32_t n_pairs = 0;
@@ -35,8 +37,8 @@ struct PairWork {
 void pairwork_free(PairWork *w) {
     if (!w) return;
     DevBuf *all[] = {&w->in_off, &w->in_nams, &w->ord,  &w->types, &w->drop, &w->mapq,
-                     &w->tcnt,   &w->tpos,    &w->tids, &w->ttot,  &w->jbound, &w->jboff,
-                     &w->jtmp,   &w->jcnt,    &w->joff, &w->jout,  &w->err,  &w->scan_tmp};
+                     &w->tcnt,   &w->tpos,    &w->tids, &w->jtmp,  &w->jcnt, &w->joff,
+                     &w->jout,   &w->err,     &w->scan_tmp};
     for (DevBuf *x : all) release(*x);
     if (w->h) (void)hipHostFree(w->h);
     delete w;
@@ -78,7 +80,6 @@ static int pairs_run(gis_ctx *ctx, PairWork &w, hipStream_t st, const uint64_t *
     P.tcnt = ensure<uint32_t>(w.tcnt, 5 * nb);
     P.tpos = ensure<uint64_t>(w.tpos, 5 * nb + 1);
     P.tids = ensure<uint32_t>(w.tids, n_pairs);
-    P.ttot = ensure<uint64_t>(w.ttot, 6);
     P.nblk = (uint32_t)nb;
     P.err = ensure<unsigned>(w.err, 1);
     P.dropoff = pp.dropoff_threshold;
@@ -86,38 +87,39 @@ static int pairs_run(gis_ctx *ctx, PairWork &w, hipStream_t st, const uint64_t *
     P.sigma = pp.sigma;
     P.max_tries = pp.max_tries;
     P.joint = (pp.flags & GIS_PAIRS_JOINT) ? 1 : 0;
+    uint64_t *h = w.h;
+    P.totals = h;
     if (P.joint) {
-        P.jbound = ensure<uint32_t>(w.jbound, n_pairs);
-        P.jboff = ensure<uint64_t>(w.jboff, n_pairs + 1ull);
+        P.jtmp = ensure<gis_nam_pair>(w.jtmp, n_nams + (uint64_t)n_pairs * (2ull * P.max_tries + 1));
         P.jcnt = ensure<uint32_t>(w.jcnt, n_pairs);
         P.joff = ensure<uint64_t>(w.joff, n_pairs + 1ull);
+        P.jout = ensure<gis_nam_pair>(w.jout, n_nams);
+        P.jout_cap = w.jout.bytes / sizeof(gis_nam_pair);
     }
     uint64_t *tmp = ensure<uint64_t>(w.scan_tmp, scan_tmp_words(std::max<uint64_t>(5 * nb, n_pairs)));
     w.owner = nullptr;
     HIP_CHECK(hipMemsetAsync(P.err, 0, sizeof(unsigned), st));
     launch_pairs_classify(P, tmp, st);
-    uint64_t *h = w.h;
-    if (P.joint) {
-        HIP_CHECK(hipMemcpyAsync(&h[6], P.jboff + n_pairs, 8, hipMemcpyDeviceToHost, st));
-        HIP_CHECK(hipStreamSynchronize(st));
-        const uint64_t bound = h[6];
-        P.jtmp = ensure<gis_nam_pair>(w.jtmp, bound);
-        P.jout = ensure<gis_nam_pair>(w.jout, bound);
-        launch_pairs_joint(P, tmp, st);
-        HIP_CHECK(hipMemcpyAsync(&h[7], P.joff + n_pairs, 8, hipMemcpyDeviceToHost, st));
-    }
-    HIP_CHECK(hipMemcpyAsync(h, P.ttot, 6 * sizeof(uint64_t), hipMemcpyDeviceToHost, st));
-    unsigned *herr = reinterpret_cast<unsigned *>(&h[8]);
-    HIP_CHECK(hipMemcpyAsync(herr, P.err, sizeof(unsigned), hipMemcpyDeviceToHost, st));
+    if (P.joint) launch_pairs_joint(P, tmp, st);
+    launch_pairs_totals(P, st);
+    HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipStreamSynchronize(st));
-    if (*herr & PAIR_ERR_DUPLICATE)
+    if (P.joint && h[6] > P.jout_cap) {
+        P.jout = ensure<gis_nam_pair>(w.jout, h[6]);
+        P.jout_cap = h[6];
+        launch_pairs_joint_compact(P, st);
+        HIP_CHECK(hipGetLastError());
+        HIP_CHECK(hipStreamSynchronize(st));
+    }
+    const unsigned err = (unsigned)h[7];
+    if (err & PAIR_ERR_DUPLICATE)
         return fail(ctx, GIS_ERR_BAD_PARAMETER,
                     "a NAM list holds two NAMs with the same (is_rc, ref_id, query_start, ref_start)");
-    if (*herr & PAIR_ERR_JOINT) return fail(ctx, GIS_ERR_STATE, "joint NAM pairs exceeded their bound");
+    if (err & PAIR_ERR_JOINT) return fail(ctx, GIS_ERR_STATE, "joint NAM pairs exceeded their bound");
     for (int t = 0; t < 5; t++) w.type_counts[t] = (uint32_t)(h[t + 1] - h[t]);
     w.n_pairs = n_pairs;
     w.n_nams = n_nams;
-    w.n_joint = P.joint ? h[7] : 0;
+    w.n_joint = h[6];
     w.joint = P.joint != 0;
     w.dev_off = off;
     return GIS_OK;

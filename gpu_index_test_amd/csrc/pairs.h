@@ -27,14 +27,13 @@ struct PairDev {
     uint32_t *tcnt;       // [5 * nblk] per block type counts, type-major
     const uint64_t *tpos; // [5 * nblk + 1] their exclusive scan
     uint32_t *tids;       // [n] pair ids grouped by type
-    uint64_t *ttot;       // [6] type starts in tids and the total
     uint32_t nblk;
-    uint32_t *jbound;     // [n] upper bound of a pair's joint entries
-    const uint64_t *jboff;// [n+1]
-    gis_nam_pair *jtmp;   // entries at jboff
+    gis_nam_pair *jtmp;   // entries at joint_place()
     uint32_t *jcnt;       // [n]
     const uint64_t *joff; // [n+1]
     gis_nam_pair *jout;   // entries at joff
+    uint64_t jout_cap;    // its room; a larger total leaves it as it is
+    uint64_t *totals;     // [8], pinned host words: type starts in tids and their total, joint total, err
     unsigned *err;        // PAIR_ERR_* bits
     float dropoff, mu, sigma;
     int max_tries;
@@ -46,10 +45,13 @@ enum : unsigned { PAIR_ERR_DUPLICATE = 1, PAIR_ERR_JOINT = 2 };
 constexpr unsigned PAIR_BLOCK = 256;
 
 size_t pair_blocks(uint32_t n_pairs);
-// reference order, types, dropoff, MAPQ, type lists and the joint-entry
-// bounds (and their scan into jboff)
+// reference order, types, dropoff, MAPQ and type lists
 void launch_pairs_classify(const PairDev &P, uint64_t *scan_tmp, hipStream_t st);
 // joint NAM pairs into jtmp, their counts scanned into joff, compacted into jout
 void launch_pairs_joint(const PairDev &P, uint64_t *scan_tmp, hipStream_t st);
+// the compaction again, with more room at jout
+void launch_pairs_joint_compact(const PairDev &P, hipStream_t st);
+// the step's totals and error bits to the host
+void launch_pairs_totals(const PairDev &P, hipStream_t st);
 
 }  // namespace gis

@@ -127,6 +127,36 @@ __device__ __forceinline__ uint32_t row_sum(uint32_t x) {
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x15f, 0xf, 0xf, false);  // row_newbcast:15
 }
 
+// or of x over each row of 16 lanes, on every lane of the row
+__device__ __forceinline__ uint32_t row_or(uint32_t x) {
+    x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x111, 0xf, 0xf, true);   // row_shr:1
+    x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x112, 0xf, 0xf, true);   // row_shr:2
+    x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x114, 0xf, 0xf, true);   // row_shr:4
+    x |= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x118, 0xf, 0xf, true);   // row_shr:8
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)x, 0x15f, 0xf, 0xf, false);  // row_newbcast:15
+}
+
+// signed maximum over the lanes up to each one (inclusive), over those before it,
+// and over the wave; every lane active
+__device__ __forceinline__ int wave_incl_max(int x) {
+    constexpr int least = (int)0x80000000;
+    x = max(x, __builtin_amdgcn_update_dpp(least, x, 0x111, 0xf, 0xf, false));  // row_shr:1
+    x = max(x, __builtin_amdgcn_update_dpp(least, x, 0x112, 0xf, 0xf, false));  // row_shr:2
+    x = max(x, __builtin_amdgcn_update_dpp(least, x, 0x114, 0xf, 0xf, false));  // row_shr:4
+    x = max(x, __builtin_amdgcn_update_dpp(least, x, 0x118, 0xf, 0xf, false));  // row_shr:8
+    x = max(x, __builtin_amdgcn_update_dpp(least, x, 0x142, 0xa, 0xf, false));  // row_bcast:15
+    return max(x, __builtin_amdgcn_update_dpp(least, x, 0x143, 0xc, 0xf, false));  // row_bcast:31
+}
+__device__ __forceinline__ int wave_excl_max(int x) {
+    return __builtin_amdgcn_update_dpp((int)0x80000000, wave_incl_max(x), 0x138, 0xf, 0xf, false);  // wave_shr:1
+}
+__device__ __forceinline__ int wave_imax(int x) { return __builtin_amdgcn_readlane(wave_incl_max(x), 63); }
+
+__device__ __forceinline__ uint64_t readlane_u64(uint64_t v, uint32_t l) {
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), (int)l) << 32 |
+           (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)v, (int)l);
+}
+
 __device__ __forceinline__ uint32_t readlane_u32(uint32_t v, uint32_t l) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l);
 }

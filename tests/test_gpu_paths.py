@@ -5,6 +5,8 @@ import pytest
 import gpu_index_test_amd as G
 from oracle import oracle_lib as O
 from tests.helpers import tiny_index_arrays
+from tests.test_gpu_pairs import _compare, _flatten, _proper_rich_pair
+from tests.test_pairs_oracle import rand_list
 
 pytestmark = pytest.mark.gpu
 
@@ -237,3 +239,26 @@ def test_index_build_edges(ctx, profile, lens):
     assert np.array_equal(idx.randstrobe_start_indices, oidx.starts)
     assert idx.filter_cutoff == oidx.filter_cutoff
     idx.ctx.close()
+
+
+@pytest.mark.parametrize("max_tries", [1, 20, 31, 32, 64])
+def test_pair_list_edges(ctx, max_tries):
+    """List lengths around the lanes of a row, of a wave and of a pass over a
+    pair's cells; many and few proper cells, equal scores, equal entries."""
+    rng = np.random.default_rng(max_tries)
+    sizes = [0, 1, 2, 3, 7, 8, 9, 15, 16, 17, 31, 32, 33, 63, 64, 65, 100]
+    m1, m2 = [], []
+    for a in sizes:
+        for b in sizes:
+            if (a + b) % 2:
+                x, y = _proper_rich_pair(rng, max(a, b, 1))
+                x["score"], y["score"] = x["score"] // 30, y["score"] // 30
+                x, y = x[:a], y[:b]
+            else:
+                x, y = rand_list(rng, a, 2), rand_list(rng, b, 2)
+            m1.append(x[rng.permutation(len(x))])
+            m2.append(y[rng.permutation(len(y))])
+    offs, flat = _flatten(m1 + m2)
+    n = len(m1)
+    _compare(G.pairs_from_nams(ctx, offs, flat, n, max_tries=max_tries),
+             O.pairs_batch(offs, flat, n, max_tries=max_tries), offs)
