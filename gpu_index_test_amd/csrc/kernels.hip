@@ -1277,21 +1277,6 @@ struct ChunkBox {
     int lo, hi;
 };
 
-// wave minimum and maximum by DPP row shifts and broadcasts (wave_incl_scan_dpp);
-// lanes a step does not reach keep the identity
-__device__ __forceinline__ int wave_max_i(int v) {
-    constexpr int LOW = (int)0x80000000;
-    v = max(v, __builtin_amdgcn_update_dpp(LOW, v, 0x111, 0xf, 0xf, false));
-    v = max(v, __builtin_amdgcn_update_dpp(LOW, v, 0x112, 0xf, 0xf, false));
-    v = max(v, __builtin_amdgcn_update_dpp(LOW, v, 0x114, 0xf, 0xf, false));
-    v = max(v, __builtin_amdgcn_update_dpp(LOW, v, 0x118, 0xf, 0xf, false));
-    v = max(v, __builtin_amdgcn_update_dpp(LOW, v, 0x142, 0xa, 0xf, false));
-    v = max(v, __builtin_amdgcn_update_dpp(LOW, v, 0x143, 0xc, 0xf, false));
-    return __builtin_amdgcn_readlane(v, 63);
-}
-
-__device__ __forceinline__ int wave_min_i(int v) { return ~wave_max_i(~v); }
-
 // bounds of the wide list's chunks c0 .. (all of them when c0 == 0)
 __device__ __forceinline__ void boxes_rebuild(const WideList &wide, uint32_t nw, ChunkBox *box) {
     for (uint32_t c = 0; c * 64 < nw; c++) {
@@ -1302,8 +1287,8 @@ __device__ __forceinline__ void boxes_rebuild(const WideList &wide, uint32_t nw,
             lo = w.rp;
             hi = w.re;
         }
-        lo = wave_min_i(lo);
-        hi = wave_max_i(hi);
+        lo = wave_imin(lo);
+        hi = wave_imax(hi);
         if (lane_id() == 0) box[c] = ChunkBox{lo, hi};
     }
 }
@@ -1351,23 +1336,60 @@ __device__ __forceinline__ uint64_t lanes_take(LaneNam &o, uint64_t acc, uint64_
     return me;
 }
 
+// The hits after hit t of the 64 in a wave's lanes (c, m of them) that the NAM on
+// lane w, which took hit t, takes one after the other: with no live NAM of its
+// group on a lower lane it is the first to accept each of them as long as it does.
+// A hit of the run sees the one before it as the previous hit and the ends' maxima
+// so far as the NAM's ends (a hit raises both or neither), so one prefix maximum
+// tests the 64 at once. Returns the last hit taken (t if none is).
+__device__ __forceinline__ uint32_t take_run(LaneNam &o, uint32_t w, const uint4 &c, uint32_t t, uint32_t m) {
+    const uint32_t lane = lane_id();
+    const int qs = (int)(c.w & 0xffffu), rs = (int)c.y;
+    const uint64_t after = ~0ull << t;  // t and the hits after it
+    const uint64_t from = after & (after - 1);
+    const bool in = lane_bit(from);
+    const int qe_t = __builtin_amdgcn_readlane(o.qe, (int)w), re_t = __builtin_amdgcn_readlane(o.re, (int)w);
+    const int qe = in ? (int)(c.w >> 16) : qe_t, re = in ? (int)c.z : re_t;
+    const int hq = wave_incl_max(qe), hr = wave_incl_max(re);
+    auto before = [](int v) { return __builtin_amdgcn_update_dpp(0, v, 0x138, 0xf, 0xf, false); };  // wave_shr:1
+    const int pq = before(hq), pr = before(hr);
+    const uint64_t ok = ballot((uint32_t)before((int)c.x) == c.x) & ballot(before(qs) < qs) & ballot(qs <= pq) &
+                        ballot(before(rs) < rs) & ballot(rs <= pr) & ~(ballot(qe > pq) ^ ballot(re > pr));
+    const uint64_t stop = (~ok & from) | (m < 64 ? ~0ull << m : 0ull);
+    const uint32_t last = (stop ? (uint32_t)__builtin_ctzll(stop) : 64u) - 1;
+    const bool me = lane == w;
+    o.qe = me ? __builtin_amdgcn_readlane(hq, (int)last) : o.qe;
+    o.re = me ? __builtin_amdgcn_readlane(hr, (int)last) : o.re;
+    o.qp = me ? __builtin_amdgcn_readlane(qs, (int)last) : o.qp;
+    o.rp = me ? __builtin_amdgcn_readlane(rs, (int)last) : o.rp;
+    o.n += me ? (int)(last - t) : 0;
+    return last;
+}
+
 constexpr uint32_t ARRIVAL_BLOCK = 4;
+// a strand of more groups than this and more NAMs than lanes is merge_range's
+constexpr uint32_t ARRIVAL_GROUPS = 16;
 
 // Merge of a read's hits in arrival order on one wave, a NAM a lane, without
 // grouping them: NAMs of every group of the current strand share the lanes, and
 // a NAM only accepts hits of its own group, which arrive in (query_start,
 // ref_start) order. A strand's NAMs are ranked by (ref_id, creation) when its
 // hits end. With one group on the strand (a read of one place, the usual case)
-// creation order is the rank, so dead NAMs may leave when the lanes are full.
+// creation order is the rank, so dead NAMs may leave when the lanes are full. With
+// more, a strand that fills the lanes goes again, one group after the other.
 // Returns the NAM count (entries at index >= cap are not written), or
-// MERGE_OVERFLOW when a strand needs more than 64 lanes, or, with BLOCKS, when
-// the hits come in blocks of ARRIVAL_BLOCK or more equal query starts on
+// MERGE_OVERFLOW when a group needs more than 64 lanes (or such a strand has more
+// than ARRIVAL_GROUPS groups), or, with BLOCKS, when the hits come in blocks of ARRIVAL_BLOCK or more equal query starts on
 // average (repeats): merge_range takes a block at a time.
 //
 // A lone wave's time is its chain of instructions a hit (one issues every ~8
-// cycles), branches above all: the loop over hits has none but its end and the
-// full-lanes exit (~550 cycles a hit; the group-by-group merge took ~800 with
-// its sort and block tests before it).
+// cycles), branches above all: the loop over hits has none but its end, the
+// full-lanes exit and the run's (~550 cycles a hit; the group-by-group merge took
+// ~800 with its sort and block tests before it). Most hits come in runs that one
+// NAM takes (of a long read's 128 hits, 78 in two runs, take_run). 8191 reads of
+// 400 to 2500 bp, 4230 of them here: k_merge 240 us before, 196 with the runs
+// (then the time of three reads with more NAMs than lanes on several references,
+// which went to merge_range), 74 with those taken group by group.
 template <bool BLOCKS = false>
 __device__ __forceinline__ uint32_t merge_arrival(const DevHit *hits, uint32_t nh, gis_nam *out, uint32_t cap) {
     const uint32_t lane = lane_id();
@@ -1380,18 +1402,29 @@ __device__ __forceinline__ uint32_t merge_arrival(const DevHit *hits, uint32_t n
         const uint32_t h0 = uni32(hv[0].x), hl = uni32(hv[nh ? nh - 1 : 0].x);
         uint64_t of = 0, orv = 0;
         uint32_t blocks = 0;
-        for (uint32_t x0 = 0; x0 < nh; x0 += 64) {
-            const bool in = x0 + lane < nh;
-            const uint32_t r = in ? hv[x0 + lane].x : 0xffffffffu;
-            if (BLOCKS) {
-                const uint32_t q = in ? hv[x0 + lane].w & 0xffffu : 0u;
-                const uint32_t pq = (uint32_t)__shfl_up((int)q, 1, 64);
-                blocks += wave_count(in && (lane == 0 || q != pq));
+        for (uint32_t y0 = 0; y0 < nh; y0 += 256) {
+            // (four loads in flight: a lone wave waits for each)
+            uint32_t r4[4], w4[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; u++) {
+                const uint32_t x = y0 + 64 * u + lane;
+                r4[u] = x < nh ? hv[x].x : 0xffffffffu;
+                w4[u] = BLOCKS && x < nh ? hv[x].w & 0xffffu : 0u;
             }
-            const uint64_t fwd = ballot(r >> 31 == 0);
-            nf += (uint32_t)__popcll(fwd);
-            of |= ballot(r != h0) & fwd;
-            orv |= ballot(in && r != hl) & ~fwd;
+#pragma unroll
+            for (uint32_t u = 0; u < 4; u++) {
+                const uint32_t x0 = y0 + 64 * u;
+                if (x0 >= nh) break;
+                const bool in = x0 + lane < nh;
+                if (BLOCKS) {
+                    const uint32_t pq = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)w4[u], 0x138, 0xf, 0xf, false);
+                    blocks += wave_count(in && (lane == 0 || w4[u] != pq));
+                }
+                const uint64_t fwd = ballot(r4[u] >> 31 == 0);
+                nf += (uint32_t)__popcll(fwd);
+                of |= ballot(r4[u] != h0) & fwd;
+                orv |= ballot(in && r4[u] != hl) & ~fwd;
+            }
         }
         other[0] = of != 0;
         other[1] = orv != 0;
@@ -1400,54 +1433,93 @@ __device__ __forceinline__ uint32_t merge_arrival(const DevHit *hits, uint32_t n
     uint32_t base = 0;
     for (int strand = 0; strand < 2; strand++) {
         const uint32_t xb = strand ? nf : 0u, xe = strand ? nh : nf;
-        const bool multi = other[strand];
-        LaneNam o{0, 0, 0, 0, 0, 0, 0, 0};
-        uint32_t rsd_o = 0xffffffffu;  // this lane's group (no hit's when the lane is free)
-        uint32_t made = 0;
-        uint64_t free = 1;
-        for (uint32_t x0 = xb; x0 < xe; x0 += 64) {
-            uint4 c = make_uint4(0u, 0u, 0u, 0u);
-            if (x0 + lane < xe) c = hv[x0 + lane];
-            const uint32_t m = xe - x0 < 64 ? xe - x0 : 64;
-            for (uint32_t t = 0;;) {
-                uint32_t rsd = 0;
-                int qs = 0;
-                for (; t < m; t++) {
-                    rsd = readlane_u32(c.x, t);
-                    const uint32_t q = readlane_u32(c.w, t);
-                    const int rs = (int)readlane_u32(c.y, t), re = (int)readlane_u32(c.z, t), qe = (int)(q >> 16);
-                    qs = (int)(q & 0xffffu);
-                    const uint64_t xq = ballot(qe > o.qe), xr = ballot(re > o.re);
-                    const uint64_t acc = ballot(rsd_o == rsd) & ballot(o.qp < qs) & ballot(qs <= o.qe) &
-                                         ballot(o.rp < rs) & ballot(rs <= o.re) & ~(xq ^ xr);
-                    uint64_t mk;
-                    const uint64_t me = lanes_take(o, acc, xq & xr, free, mk, made, qs, qe, rs, re);
-                    rsd_o = lane_bit(mk) ? rsd : rsd_o;
-                    const uint32_t fresh = mk != 0 ? 1u : 0u;
-                    made += fresh;
-                    free <<= fresh;
-                    if (me == 0) break;  // no room: the hit waits
+        bool multi = other[strand];
+        // the group whose hits alone are taken (`each`), and how many there were
+        bool each = false;
+        uint32_t grp = 0, n_grp = 0;
+        for (;;) {
+            LaneNam o{0, 0, 0, 0, 0, 0, 0, 0};
+            uint32_t rsd_o = 0xffffffffu;  // this lane's group (no hit's when the lane is free)
+            uint32_t made = 0;
+            uint64_t free = 1;
+            uint32_t after = 0xffffffffu;  // the least group above grp
+            bool full = false;
+            uint4 next = make_uint4(0u, 0u, 0u, 0u);
+            if (xb + lane < xe) next = hv[xb + lane];
+            for (uint32_t x0 = xb; x0 < xe && !full; x0 += 64) {
+                const uint4 c = next;
+                if (x0 + 64 + lane < xe) next = hv[x0 + 64 + lane];
+                const uint32_t m = xe - x0 < 64 ? xe - x0 : 64;
+                uint64_t todo = ~0ull >> (64 - m);
+                if (each) {
+                    if (lane < m && c.x > grp) after = min(after, c.x);
+                    todo &= ballot(c.x == grp);
                 }
-                if (t == m) break;
-                if (multi) return MERGE_OVERFLOW;
-                const uint32_t n_open = retire_lanes(o, qs, out, base, rsd, cap);
-                if (n_open == 64) return MERGE_OVERFLOW;
-                rsd_o = lane < n_open ? rsd_o : 0xffffffffu;
-                o.n = lane < n_open ? o.n : 0;
-                free = 1ull << n_open;
+                while (todo) {
+                    uint32_t rsd = 0;
+                    int qs = 0;
+                    uint64_t me;
+                    do {
+                        const uint32_t t = (uint32_t)__builtin_ctzll(todo);
+                        rsd = readlane_u32(c.x, t);
+                        const uint32_t q = readlane_u32(c.w, t);
+                        const int rs = (int)readlane_u32(c.y, t), re = (int)readlane_u32(c.z, t), qe = (int)(q >> 16);
+                        qs = (int)(q & 0xffffu);
+                        const uint64_t xq = ballot(qe > o.qe), xr = ballot(re > o.re);
+                        const uint64_t live = ballot(rsd_o == rsd) & ballot(qs <= o.qe);
+                        const uint64_t acc =
+                            live & ballot(o.qp < qs) & ballot(o.rp < rs) & ballot(rs <= o.re) & ~(xq ^ xr);
+                        uint64_t mk;
+                        me = lanes_take(o, acc, xq & xr, free, mk, made, qs, qe, rs, re);
+                        rsd_o = lane_bit(mk) ? rsd : rsd_o;
+                        const uint32_t fresh = mk != 0 ? 1u : 0u;
+                        made += fresh;
+                        free <<= fresh;
+                        if (me == 0) break;  // no room: the hit waits
+                        todo &= todo - 1;
+                        // taken by the first live NAM
+                        if (me == (live & (0 - live)))
+                            todo &= ~0ull << 1 << take_run(o, (uint32_t)__builtin_ctzll(me), c, t, m);
+                    } while (todo);
+                    if (me != 0) break;
+                    if (multi) {
+                        full = true;
+                        break;
+                    }
+                    const uint32_t n_open = retire_lanes(o, qs, out, base, rsd, cap);
+                    if (n_open == 64) return MERGE_OVERFLOW;
+                    rsd_o = lane < n_open ? rsd_o : 0xffffffffu;
+                    o.n = lane < n_open ? o.n : 0;
+                    free = 1ull << n_open;
+                }
             }
-        }
-        // the strand's NAMs are final
-        uint32_t rank = o.cid;
-        if (multi) {  // nothing was retired: NAM c sits on lane c
-            rank = 0;
-            for (uint32_t q = 0; q < made; q++) {
-                const uint32_t k = readlane_u32(rsd_o, q);
-                rank += (k < rsd_o) | ((k == rsd_o) & (q < lane)) ? 1u : 0u;
+            if (full) {
+                // more NAMs than lanes, of several groups: the groups one by one
+                // (nothing of the strand is written yet), least one first
+                uint32_t least = 0xffffffffu;
+                for (uint32_t x = xb + lane; x < xe; x += 64) least = min(least, hv[x].x);
+                multi = false;
+                each = true;
+                grp = wave_umin(least);
+                n_grp = 1;
+                continue;
             }
+            // the NAMs are final
+            uint32_t rank = o.cid;
+            if (multi) {  // nothing was retired: NAM c sits on lane c
+                rank = 0;
+                for (uint32_t q = 0; q < made; q++) {
+                    const uint32_t k = readlane_u32(rsd_o, q);
+                    rank += (k < rsd_o) | ((k == rsd_o) & (q < lane)) ? 1u : 0u;
+                }
+            }
+            if (o.n > 0 && base + rank < cap) lane_nam_store(out, base + rank, rsd_o, o);
+            base += made;
+            if (!each) break;
+            grp = wave_umin(after);
+            if (grp == 0xffffffffu) break;
+            if (++n_grp > ARRIVAL_GROUPS) return MERGE_OVERFLOW;
         }
-        if (o.n > 0 && base + rank < cap) lane_nam_store(out, base + rank, rsd_o, o);
-        base += made;
     }
     return base;
 }
@@ -1691,7 +1763,7 @@ __device__ __forceinline__ uint32_t merge_range(const DevHit *hits, const uint64
                 n_open = 0;
                 singles_until = 0;
                 if (box && box_cap) {
-                    const int lo = wave_min_i(o.rp), hi = wave_max_i(o.re);
+                    const int lo = wave_imin(o.rp), hi = wave_imax(o.re);
                     if (lane == 0) box[0] = ChunkBox{lo, hi};
                 }
                 wave_sync_mem();
@@ -1758,7 +1830,7 @@ __device__ __forceinline__ uint32_t merge_range(const DevHit *hits, const uint64
                         w.n++;
                     }
                     if (boxed) {
-                        const int hi = wave_max_i(ext ? hre : (int)0x80000000);
+                        const int hi = wave_imax(ext ? hre : (int)0x80000000);
                         if (lane == 0 && box[c].hi < hi) box[c].hi = hi;
                     }
                     if (tk) wput(wide, e, w);
@@ -1801,8 +1873,8 @@ __device__ __forceinline__ uint32_t merge_range(const DevHit *hits, const uint64
                 if (box && c_last < box_cap) {
                     for (uint32_t c = nw >> 6; c <= c_last; c++) {
                         const bool in = mine && (at >> 6) == c;
-                        const int lo = wave_min_i(in ? (int)c_rs : 0x7fffffff);
-                        const int hi = wave_max_i(in ? (int)c_re : (int)0x80000000);
+                        const int lo = wave_imin(in ? (int)c_rs : 0x7fffffff);
+                        const int hi = wave_imax(in ? (int)c_re : (int)0x80000000);
                         if (lane == 0) {
                             const bool begun = c == nw >> 6 && (nw & 63) != 0;
                             const ChunkBox bx = box[c];
@@ -1842,16 +1914,17 @@ constexpr int GROUP_WIDE_LDS = 512;
 // chunk bounds of a k_merge_groups wide list (lists up to 8,192 entries)
 constexpr uint32_t GROUP_BOXES = 128;
 
-// the reads that k_merge4 handed on, one per wave
-__global__ __launch_bounds__(64 * WPB) void k_merge(DevBatch b) {
-    __shared__ uint64_t lkeys[WPB][MERGE_LDS];
-    __shared__ WideNam lwide[WPB][MERGE_WIDE_LDS];  // the wide list of reads with few enough hits
-    __shared__ BlockLds lblock[WPB];
+// the reads that k_merge4 handed on, one per wave, and one wave per block: waves
+// take very different times, and a block holds its LDS (for groups and wide lists)
+// until its slowest is done
+__global__ __launch_bounds__(64) void k_merge(DevBatch b) {
+    __shared__ uint64_t lkeys[MERGE_LDS];
+    __shared__ WideNam lwide[MERGE_WIDE_LDS];  // the wide list of reads with few enough hits
+    __shared__ BlockLds lblock;
     const uint32_t lane = lane_id();
-    const int wid = (int)uni32(threadIdx.x >> 6);
     if (hits_missing(b)) return;
     const uint32_t cnt = sload(&b.ctl->n_sel[SEL_DEFERRED]);
-    for (uint32_t w = wave_index(WPB); w < cnt; w += gridDim.x * WPB) {
+    for (uint32_t w = blockIdx.x; w < cnt; w += gridDim.x) {
         const uint32_t r = uni32(b.sel_ids[(uint64_t)b.n_reads + w]);
         const bool rescue = (uni32(b.flags[r]) & GIS_FLAG_RESCUED) != 0;
         const uint64_t hb = uni64(rescue ? b.rhit_off[r] : b.hit_off[r]);
@@ -1862,7 +1935,7 @@ __global__ __launch_bounds__(64 * WPB) void k_merge(DevBatch b) {
         WideNam *gwide = b.merge_scratch ? (rescue ? b.rnam_ws : b.nam_ws) + hb : nullptr;
         if (nh > SPLIT_MIN && b.merge_scratch) {
             // group the hits; each group merges on its own wave
-            uint32_t *bins = reinterpret_cast<uint32_t *>(lkeys[wid]);
+            uint32_t *bins = reinterpret_cast<uint32_t *>(lkeys);
             const uint64_t *ord = group_order(nh, ghits, gkeys, gkeys + nh, bins);
             const uint32_t code = ord == nullptr ? 0u : (ord == gkeys ? 1u : 2u);
             uint64_t *slots = code == 1u ? gkeys + nh : gkeys;
@@ -1919,10 +1992,10 @@ __global__ __launch_bounds__(64 * WPB) void k_merge(DevBatch b) {
         if (total == MERGE_OVERFLOW && (nh <= (uint32_t)MERGE_LDS || b.merge_scratch)) {
             // more than 64 NAMs at once: group by group, with a wide list (NAMs <= hits)
             const bool lds = nh <= (uint32_t)MERGE_LDS;
-            const uint64_t *ord = group_order(nh, ghits, lds ? lkeys[wid] : gkeys, lds ? nullptr : gkeys + nh,
-                                              reinterpret_cast<uint32_t *>(lkeys[wid]));
-            const WideList wl{(LdsWideNam *)lwide[wid], gwide, (uint32_t)MERGE_WIDE_LDS};
-            total = merge_range(ghits, ord, 0, nh, wl, fin, nh, lblock[wid]);
+            const uint64_t *ord = group_order(nh, ghits, lds ? lkeys : gkeys, lds ? nullptr : gkeys + nh,
+                                              reinterpret_cast<uint32_t *>(lkeys));
+            const WideList wl{(LdsWideNam *)lwide, gwide, (uint32_t)MERGE_WIDE_LDS};
+            total = merge_range(ghits, ord, 0, nh, wl, fin, nh, lblock);
         }
         if (total == MERGE_OVERFLOW) {
             // needs the global scratch, which this run does not have yet
@@ -2885,7 +2958,7 @@ void launch_merge(const DevBatch &b, const ReadSet &set, hipStream_t st) {
     if (b.n_reads == 0) return;
     const unsigned g = grid_for_set(b, set, WPB);
     hipLaunchKernelGGL(k_merge4, dim3((g + RPW - 1) / RPW), dim3(64 * WPB), 0, st, b, set);
-    hipLaunchKernelGGL(k_merge, dim3(grid_selected(b)), dim3(64 * WPB), 0, st, b);
+    hipLaunchKernelGGL(k_merge, dim3(grid_selected(b) * WPB), dim3(64), 0, st, b);
     if (b.merge_scratch) {
         hipLaunchKernelGGL(k_merge_groups, dim3(4096), dim3(64), 0, st, b);
         hipLaunchKernelGGL(k_merge_split_finish, dim3(256), dim3(64 * WPB), 0, st, b);

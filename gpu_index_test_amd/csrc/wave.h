@@ -151,6 +151,11 @@ __device__ __forceinline__ int wave_excl_max(int x) {
     return __builtin_amdgcn_update_dpp((int)0x80000000, wave_incl_max(x), 0x138, 0xf, 0xf, false);  // wave_shr:1
 }
 __device__ __forceinline__ int wave_imax(int x) { return __builtin_amdgcn_readlane(wave_incl_max(x), 63); }
+__device__ __forceinline__ int wave_imin(int x) { return ~wave_imax(~x); }
+
+__device__ __forceinline__ uint32_t wave_umin(uint32_t x) {
+    return (uint32_t)wave_imin((int)(x ^ 0x80000000u)) ^ 0x80000000u;
+}
 
 __device__ __forceinline__ uint64_t readlane_u64(uint64_t v, uint32_t l) {
     return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(v >> 32), (int)l) << 32 |
