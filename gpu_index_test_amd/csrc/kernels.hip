@@ -42,7 +42,7 @@ struct SeedBufs {
     uint64_t *pk;       // bases 2 bits each, LSB first: base i at bits 2(i%32) of pk[i/32]
     uint8_t *st;        // per k-mer window: anchor state / ST_UNKNOWN / ST_INVALID
     uint64_t *sh;       // canonical s-mer hash per s-mer start
-    uint64_t *sy_hash;  // syncmer list
+    uint64_t *sy_hash;  // syncmer list (written when sh is done with: may be the same memory)
     uint16_t *sy_pos;   // read positions fit 16 bits (reads are at most 65535 bp)
     uint64_t *nmask;    // bit i set when base i is not ACGT
 };
@@ -192,6 +192,25 @@ __device__ __forceinline__ uint32_t four_bases(const char *__restrict__ seq, int
     return v;
 }
 
+// A read's bases packed 2 bits each, four a lane and so 256 a pass: a lane's four
+// codes are one byte of the packed array, which is written up to its pad word
+// (windows ending in the last word read it). True if every base is ACGT.
+__device__ __forceinline__ bool pack_bases(const char *__restrict__ seq, int L, uint64_t *pk) {
+    const int nch = (L + 63) >> 6, nbytes = 8 * (2 * nch + 1);
+    uint8_t *pkb = reinterpret_cast<uint8_t *>(pk);
+    uint32_t any = 0;
+    for (int i0 = 0; i0 < nbytes; i0 += 64) {
+        const int i = i0 + (int)lane_id();
+        uint32_t inside, bad;
+        const uint32_t v = four_bases(seq, L, i, inside);
+        const uint32_t c = nt4x4(v, bad) & inside;
+        any |= bad & inside;
+        if (i < nbytes) pkb[i] = (uint8_t)pack4(c);
+    }
+    wave_sync();
+    return ballot(any != 0) == 0;
+}
+
 // Canonical syncmers of one read (SyncmerIterator, step2/randstrobes.cu:18-79),
 // the whole wave working on the same read. The first `cap` syncmers go to
 // B.sy_hash/B.sy_pos (and out_sy_* when given); returns the total count.
@@ -205,24 +224,9 @@ __device__ __forceinline__ uint32_t seed_syncmers(const char *__restrict__ seq, 
                                                   uint32_t cap, uint64_t *out_sy_hash,
                                                   uint64_t *out_sy_pos) {
     const int lane = (int)lane_id();
-
-    // bases packed 2 bits each, four a lane and so 256 a pass: a lane's four
-    // codes are one byte of the packed array. The array is written up to its
-    // pad word, which windows ending in the last word read.
-    const int nch = (L + 63) >> 6, nbytes = 8 * (2 * nch + 1);
-    uint8_t *pkb = reinterpret_cast<uint8_t *>(B.pk);
-    uint32_t any = 0;
-    for (int i0 = 0; i0 < nbytes; i0 += 64) {
-        const int i = i0 + lane;
-        uint32_t inside, bad;
-        const uint32_t v = four_bases(seq, L, i, inside);
-        const uint32_t c = nt4x4(v, bad) & inside;
-        any |= bad & inside;
-        if (i < nbytes) pkb[i] = (uint8_t)pack4(c);
-    }
-    wave_sync();
+    const int nch = (L + 63) >> 6;
+    const bool clean = pack_bases(seq, L, B.pk);
     uint32_t nsync = 0;
-    const bool clean = ballot(any != 0) == 0;  // wave-uniform
     if (!(clean && syncmer_fast(L, P, B, cap, out_sy_pos, nsync))) {
         // the mask of non-ACGT bases (step2/randstrobes.cu:70-76): bit 4 l + b
         // of 16 lanes' words from the ballots of their byte b
@@ -250,6 +254,101 @@ __device__ __forceinline__ uint32_t seed_syncmers(const char *__restrict__ seq, 
     }
     syncmer_hashes(nsync < cap ? nsync : cap, P, B, out_sy_hash);
     return nsync;
+}
+
+// LDS of a wave that seeds a long read, and the reads it holds: of up to
+// LONG_LDS_BASES bases with up to LONG_LDS_SYNC syncmers (one in k - s + 1 bases on
+// average: 2200 to 3100 bases). Six waves a SIMD fit.
+constexpr int LONG_LDS_BASES = 4096;
+constexpr uint32_t LONG_LDS_SYNC = 448;
+constexpr int LONG_RING = 128;
+
+struct alignas(8) LongLds {
+    uint64_t sy_hash[LONG_LDS_SYNC];
+    uint64_t pk[2 * (LONG_LDS_BASES / 64) + 1];
+    uint32_t hi[LONG_RING], lo[LONG_RING];
+    uint16_t sy_pos[LONG_LDS_SYNC];
+};
+
+// the hashes in the ring by s-mer start (the last 64 to 128 of them)
+struct RingHash {
+    const LongLds &S;
+    __device__ __forceinline__ uint64_t operator[](int j) const {
+        return (uint64_t)S.hi[j % LONG_RING] << 32 | S.lo[j % LONG_RING];
+    }
+};
+
+// whether the hash in the middle of the window at p is below (true) or equal to
+// (tie) the others' minimum, by high words; W > 0: the window's width
+template <int W>
+__device__ __forceinline__ bool ring_test(const LongLds &S, int p, int w, int mid, bool &tie) {
+    const uint32_t h = S.hi[(p + mid) % LONG_RING];
+    uint32_t m = 0xffffffffu;
+#pragma unroll
+    for (int o = 0; o < (W ? W : w); o++) {
+        const uint32_t v = S.hi[(p + o) % LONG_RING];
+        m = o == mid ? m : min(m, v);
+    }
+    tie = h == m;
+    return h < m;
+}
+
+// The canonical syncmers of a long read from LDS, as syncmer_fast finds them: the
+// windows are tested as their last s-mer is hashed, so that the hashes live in a
+// ring. A tied window is replayed from the nearest one before it whose state needs
+// no history, as syncmer_passes does, while the ring holds that. False if it does
+// not, or if the read does not fit or has a base other than ACGT: then it takes
+// the passes in global scratch. (8191 reads of 400 to 2500 bp: 91 us; with every pass
+// in global scratch 179 us, the latency of the longest reads' chains.)
+__device__ __forceinline__ bool long_syncmers(const char *__restrict__ seq, int L, const SeedParams &P, LongLds &S,
+                                              const SeedBufs &B, uint64_t *out_sy_pos, uint32_t &nsync) {
+    if (L > LONG_LDS_BASES || !pack_bases(seq, L, S.pk)) return false;
+    const int lane = (int)lane_id(), ns = L - P.s + 1, mid = P.t - 1;
+    uint32_t n = 0;
+    for (int j0 = 0; j0 < ns; j0 += 64) {
+        const int j = j0 + lane, p = j - (P.w - 1);
+        if (j < ns) {
+            const uint64_t h = smer_hash(B, j, P);
+            S.hi[j % LONG_RING] = (uint32_t)(h >> 32);
+            S.lo[j % LONG_RING] = (uint32_t)h;
+        }
+        wave_sync();
+        const bool in = j < ns && p >= 0;
+        bool is_sync = false, tie = false;
+        if (in) {  // (5 and 7 are the widths of the read-length profiles)
+            if (P.w == 5) is_sync = ring_test<5>(S, p, 5, mid, tie);
+            else if (P.w == 7) is_sync = ring_test<7>(S, p, 7, mid, tie);
+            else is_sync = ring_test<0>(S, p, P.w, mid, tie);
+        }
+        if (ballot(tie)) {
+            bool lost = false;
+            if (tie) {
+                const RingHash H{S};
+                const int oldest = max(0, j0 - 64);
+                int q = p;
+                uint8_t r = anchor_state(H, q, P.w, q == 0);
+                while (r == ST_UNKNOWN && q > oldest) {
+                    q--;
+                    r = anchor_state(H, q, P.w, q == 0);
+                }
+                lost = r == ST_UNKNOWN;
+                if (!lost)
+                    for (int x = q + 1; x <= p; x++) r = slide(r, H, x, P.w);
+                is_sync = r == (uint8_t)mid;
+            }
+            if (ballot(lost)) return false;
+        }
+        const uint64_t bal = ballot(is_sync);
+        if (is_sync) {
+            const uint32_t idx = n + mbcnt(bal);
+            if (idx < LONG_LDS_SYNC) S.sy_pos[idx] = (uint16_t)p;
+            if (out_sy_pos) out_sy_pos[idx] = (uint64_t)p;
+        }
+        n += (uint32_t)__popcll(bal);
+        wave_sync();
+    }
+    nsync = n;
+    return n <= LONG_LDS_SYNC;
 }
 
 // Randstrobe number j of a read's query list in randstrobes_query order
@@ -307,14 +406,11 @@ __device__ __forceinline__ Rs1 randstrobe_one(const SeedBufs &B, uint32_t n, uin
     return o;
 }
 
-// randstrobes_query order: forward (strobe1 ascending) then reverse complement,
-// one randstrobe per lane
-__device__ __forceinline__ uint32_t seed_one(const char *__restrict__ seq, int L, const SeedParams &P,
-                                             const SeedBufs &B, uint64_t *out_sy_hash,
-                                             uint64_t *out_sy_pos, uint64_t *rs_hash,
-                                             uint32_t *rs_span,
-                                             uint32_t *n_sync_out) {
-    const uint32_t n = seed_syncmers(seq, L, P, B, 0xffffffffu, out_sy_hash, out_sy_pos);
+// a read's randstrobes from its n syncmers, in randstrobes_query order: forward
+// (strobe1 ascending) then reverse complement, one randstrobe per lane. Returns
+// their count.
+__device__ __forceinline__ uint32_t seed_randstrobes(uint32_t n, int L, const SeedParams &P, const SeedBufs &B,
+                                                     uint64_t *rs_hash, uint32_t *rs_span) {
     const uint32_t n_fwd = ((uint32_t)L >= P.w_max && n > P.w_min) ? n - P.w_min : 0;
     const uint32_t nrs = 2 * n_fwd;
     for (uint32_t j0 = 0; j0 < nrs; j0 += 64) {
@@ -325,13 +421,11 @@ __device__ __forceinline__ uint32_t seed_one(const char *__restrict__ seq, int L
             rs_span[j] = span_pack(o.s, o.e);
         }
     }
-    *n_sync_out = n;
     return nrs;
 }
 
 struct alignas(8) SeedLds {
-    uint64_t sh[LMAX_LDS];
-    uint64_t sy_hash[LMAX_LDS];
+    uint64_t sh[LMAX_LDS];  // then the syncmers' hashes
     uint64_t nmask[LMAX_LDS / 64 + 2];
     uint64_t pk[2 * (LMAX_LDS / 64) + 1];
     uint16_t sy_pos[LMAX_LDS];
@@ -375,32 +469,47 @@ __device__ __forceinline__ void ctl_clear(DevCtl *ctl) {
     if (threadIdx.x < sizeof(DevCtl) / 4) reinterpret_cast<unsigned *>(ctl)[threadIdx.x] = 0;
 }
 
+// (long reads' lengths differ: a block would hold four waves' LDS until its
+// longest read is done)
+static constexpr int seed_wpb(bool long_reads) { return long_reads ? 1 : SEED_WPB; }
+
 template <bool LONG, bool K20>
-__global__ __launch_bounds__(64 * SEED_WPB) __attribute__((amdgpu_waves_per_eu(6))) void k_seed(DevBatch b, ReadSet set, SeedParams P,
+__global__ __launch_bounds__(64 * seed_wpb(LONG)) __attribute__((amdgpu_waves_per_eu(LONG ? 6 : 8))) void k_seed(DevBatch b, ReadSet set, SeedParams P,
                                                         int want_sy, int reset) {
     if (K20) pin_k20_profile(P);
     if (reset && blockIdx.x == 0) ctl_clear(b.ctl);
-    __shared__ SeedLds lds[LONG ? 1 : SEED_WPB];
+    constexpr int W = seed_wpb(LONG);
+    __shared__ SeedLds lds[LONG ? 1 : W];
+    __shared__ LongLds long_lds[LONG ? W : 1];
     const int wid = (int)uni32(threadIdx.x >> 6);
     const uint32_t cnt = set_count(set);
-    for (uint32_t w = wave_index(SEED_WPB); w < cnt; w += gridDim.x * SEED_WPB) {
+    for (uint32_t w = wave_index(W); w < cnt; w += gridDim.x * W) {
         const uint32_t r = set.ids ? sload(set.ids + w) : w;
         const int L = (int)sload(b.read_len + r);
         if ((L > LMAX_LDS) != LONG) continue;
-        SeedBufs B;
-        if (LONG) {
-            B = long_bufs(b.long_scratch + sload(b.long_off + r), (uint64_t)L);
-        } else {
-            SeedLds &S = lds[wid];
-            B = SeedBufs{S.pk, S.st, S.sh, S.sy_hash, S.sy_pos, S.nmask};
-        }
         const uint64_t so = want_sy ? sload(b.sy_off + r) : 0;
         uint64_t *osh = want_sy ? b.sy_hash + so : nullptr;
         uint64_t *osp = want_sy ? b.sy_pos + so : nullptr;
         const uint64_t ro = sload(b.rs_off + r);
-        uint32_t nsync = 0;
-        const uint32_t nrs = seed_one(b.seqs + sload(b.read_off + r), L, P, B, osh, osp, b.rs_hash + ro,
-                                      b.rs_span + ro, &nsync);
+        const char *seq = b.seqs + sload(b.read_off + r);
+        uint32_t nsync = 0, nrs = 0;
+        if (LONG) {
+            LongLds &S = long_lds[wid];
+            const SeedBufs B{S.pk, nullptr, nullptr, S.sy_hash, S.sy_pos, nullptr};
+            if (long_syncmers(seq, L, P, S, B, osp, nsync)) {
+                syncmer_hashes(nsync, P, B, osh);
+                nrs = seed_randstrobes(nsync, L, P, B, b.rs_hash + ro, b.rs_span + ro);
+            } else {
+                const SeedBufs G = long_bufs(b.long_scratch + sload(b.long_off + r), (uint64_t)L);
+                nsync = seed_syncmers(seq, L, P, G, 0xffffffffu, osh, osp);
+                nrs = seed_randstrobes(nsync, L, P, G, b.rs_hash + ro, b.rs_span + ro);
+            }
+        } else {
+            SeedLds &S = lds[wid];
+            const SeedBufs B{S.pk, S.st, S.sh, S.sh, S.sy_pos, S.nmask};
+            nsync = seed_syncmers(seq, L, P, B, 0xffffffffu, osh, osp);
+            nrs = seed_randstrobes(nsync, L, P, B, b.rs_hash + ro, b.rs_span + ro);
+        }
         if (lane_id() == 0) {
             b.rs_cnt[r] = nrs;
             b.rs_nfwd[r] = nrs / 2;
@@ -2243,12 +2352,12 @@ __global__ __launch_bounds__(64 * WPB) void k_merge4(DevBatch b, ReadSet set) {
 // grabs `chunk` entries at a time from a counter in the control block).
 
 constexpr int F_SYCAP = 96;
+static_assert(F_SYCAP <= 160, "the syncmer hashes take the s-mer hashes' place");
 
 template <int LMAX>
 struct alignas(8) FusedSeedLds {
-    uint64_t sh[LMAX];
+    uint64_t sh[LMAX];  // then the syncmers' hashes
     uint64_t nmask[LMAX / 64 + 2];
-    uint64_t sy_hash[F_SYCAP];
     uint64_t pk[2 * ((LMAX + 63) / 64) + 1];
     uint16_t sy_pos[F_SYCAP];
     uint8_t st[LMAX];
@@ -2358,7 +2467,7 @@ __device__ __forceinline__ void fused_read(const DevBatch &b, const DevIndex &ix
     bool rescue = false;
     float frac = 1.0f;
     if (!spill) {
-        SeedBufs B{S.seed.pk, S.seed.st, S.seed.sh, S.seed.sy_hash, S.seed.sy_pos, S.seed.nmask};
+        SeedBufs B{S.seed.pk, S.seed.st, S.seed.sh, S.seed.sh, S.seed.sy_pos, S.seed.nmask};
         const uint32_t n = seed_syncmers(b.seqs + sload(b.read_off + r), L, P, B, F_SYCAP, nullptr, nullptr);
         n_fwd = ((uint32_t)L >= P.w_max && n > P.w_min) ? n - P.w_min : 0;
         spill = n > (uint32_t)F_SYCAP || n_fwd > 64;
@@ -2928,7 +3037,7 @@ void launch_seed(const DevBatch &b, const ReadSet &set, const SeedParams &sp, in
     const SeedKernel short_k = k20 ? (SeedKernel)k_seed<false, true> : (SeedKernel)k_seed<false, false>;
     const SeedKernel long_k = k20 ? (SeedKernel)k_seed<true, true> : (SeedKernel)k_seed<true, false>;
     hipLaunchKernelGGL(short_k, dim3(g), dim3(64 * SEED_WPB), 0, st, b, set, sp, want_syncmers, reset);
-    if (long_reads) hipLaunchKernelGGL(long_k, dim3(g), dim3(64 * SEED_WPB), 0, st, b, set, sp, want_syncmers, 0);
+    if (long_reads) hipLaunchKernelGGL(long_k, dim3(g * SEED_WPB), dim3(64), 0, st, b, set, sp, want_syncmers, 0);
 }
 
 void launch_emit_seeds(const DevBatch &b, int syncmers, const uint64_t *off, void *out, uint64_t *h_off,

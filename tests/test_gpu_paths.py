@@ -48,14 +48,14 @@ def test_bucket_lines_of_every_size(ctx, bits):
 @pytest.mark.parametrize("profile", [150, 300, 400])
 def test_seeding_pass_edges(ctx, profile):
     """Read lengths around the seeding's pass sizes (4, 64, 256 bases, the
-    320-base LDS limit), at every alignment of a read's first byte, with every
+    320-base and 4096-base LDS limits, more and fewer than 448 syncmers), at every alignment of a read's first byte, with every
     kind of byte (either case, U, IUPAC codes, bytes outside ASCII) and
     windows with equal s-mers, through randstrobes_query."""
     rng = np.random.default_rng(profile)
     acgt = np.frombuffer(b"ACGT", dtype=np.uint8)
     reads = []
     for L in list(range(0, 26)) + [62, 63, 64, 65, 127, 128, 129, 150, 151, 252, 253, 254, 255, 256, 257, 258, 259,
-                                   260, 318, 319, 320, 321, 322, 511, 512, 513, 767, 1025]:
+                                   260, 318, 319, 320, 321, 322, 511, 512, 513, 767, 1025, 2600, 4000, 4096, 4097]:
         r = acgt[rng.integers(0, 4, L)]
         reads.append(r)
         for byte in (b"N", b"U", b"u", b"t", b"a", b"M", b"!", b"\x00", b"\xc1", b"\xff", b"3", b"\x14"):
