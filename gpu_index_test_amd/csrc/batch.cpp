@@ -236,6 +236,7 @@ DevBatch make_devbatch(gis_batch *b) {
     d.rnam_ws = static_cast<WideNam *>(b->ws->rnam_ws.p);
     d.merge_scratch = b->ws->merge_scratch ? 1u : 0u;
     d.gwork = static_cast<uint4 *>(b->ws->gwork.p);
+    d.gwork_cap = (uint32_t)std::min<uint64_t>(b->ws->gwork.bytes / sizeof(uint4), UINT32_MAX);
     d.split_list = static_cast<uint4 *>(b->ws->split_list.p);
     d.sel_ids = static_cast<uint32_t *>(b->ws->sel_ids.p);
     d.nam_fin = static_cast<gis_nam *>(b->ws->nam_fin.p);
@@ -319,9 +320,9 @@ void ensure_pools(gis_batch *b, uint64_t hit_cap, uint64_t rhit_cap, uint64_t ou
         ensure<WideNam>(b->ws->nam_ws, b->ws->hit_cap);
         ensure<uint64_t>(b->ws->rkeys, 2 * b->ws->rhit_cap);
         ensure<WideNam>(b->ws->rnam_ws, b->ws->rhit_cap);
-        // a split read of h > SPLIT_MIN hits has at most h / ITEM_HITS + 1 work
-        // items, fewer than h / 128
-        ensure<uint4>(b->ws->gwork, (b->ws->hit_cap + b->ws->rhit_cap) / 128 + 64);
+        // a split read of h > 64 hits has at most h / ITEM_HITS + 1 work items,
+        // fewer than h / 48
+        ensure<uint4>(b->ws->gwork, (b->ws->hit_cap + b->ws->rhit_cap) / 48 + 64);
     }
     ensure<gis_nam>(b->ws->nams_out, b->ws->out_cap);
 }

@@ -49,10 +49,9 @@ struct DevCtl {
     unsigned int n_spill;   // reads handed from the fused kernel to the per-stage kernels
     unsigned int overflow;  // OVF_* bits
     unsigned int q_head[2]; // dynamic work-queue heads of the fused kernel's two bins
-    unsigned int n_gwork;     // group work items of split reads
+    unsigned int n_gwork[2];  // group work items of split reads: long ones, others
     unsigned int n_split;     // split reads
     unsigned int n_sel[3];    // selected reads: rescued, deferred merges, pooled hits
-    unsigned int pad_;
     unsigned long long hit_pool;   // hits placed in the pool after the per-read regions
     unsigned long long rhit_pool;  // hits of rescued reads
     // totals the host reads with this block: end of the hit pool, rescue
@@ -118,6 +117,7 @@ struct DevBatch {
     // gwork items {read, first, end, group | order code << 30}, split list
     // entries {read, groups, order code, 0}
     uint4 *gwork;
+    uint32_t gwork_cap;       // long items from the front, the others from the back
     uint4 *split_list;
     // ids of the reads of the sparse passes: rescued at [0, n), deferred
     // merges at [n, 2n), reads whose hits go to the pool at [2n, 3n)

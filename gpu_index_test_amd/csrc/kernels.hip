@@ -646,32 +646,41 @@ __device__ __forceinline__ uint32_t dev_get_count(const DevIndex &ix, uint64_t p
 // keep entry e iff |query span - ref span| <= the running minimum. Counts the
 // kept hits, and writes them when out != nullptr; *run receives the run's
 // length.
+// AHEAD: records loaded together (the walk waits for each load; the lookup's runs,
+// of buckets beyond the line, are short)
+template <uint32_t AHEAD = 4>
 __device__ __forceinline__ uint32_t walk_run(const DevIndex &ix, uint64_t pos, uint64_t key,
                                              int qs, int qe, uint32_t strand_bit, DevHit *out,
                                              uint32_t *run = nullptr) {
     const int qspan = qe - qs;
     int min_diff = 0x7fffffff;
     uint32_t c = 0, rec = 0;
-    for (uint64_t x = pos; x < ix.n; x++) {
-        const uint4 v = ix.rs[x];
-        const uint64_t h = (uint64_t)v.x | ((uint64_t)v.y << 32);
-        if (h != key) break;
-        rec++;
-        const int rspan = (int)(v.w & 0xffu) + ix.k;
-        int d = qspan - rspan;
-        d = d < 0 ? -d : d;
-        if (d <= min_diff) {
-            if (out) {
-                DevHit hh;
-                hh.ref_strand = strand_bit | (v.w >> 8);
-                hh.ref_start = (int32_t)v.z;
-                hh.ref_end = (int32_t)v.z + rspan;
-                hh.query_start = (uint16_t)qs;
-                hh.query_end = (uint16_t)qe;
-                out[c] = hh;
+    bool in = pos < ix.n;
+    for (uint64_t x = pos; in; x += AHEAD) {
+        uint4 v[AHEAD];
+#pragma unroll
+        for (uint32_t u = 0; u < AHEAD; u++) v[u] = ix.rs[x + u < ix.n ? x + u : ix.n - 1];
+#pragma unroll
+        for (uint32_t u = 0; u < AHEAD; u++) {
+            in = in && x + u < ix.n && ((uint64_t)v[u].x | ((uint64_t)v[u].y << 32)) == key;
+            if (!in) break;
+            rec++;
+            const int rspan = (int)(v[u].w & 0xffu) + ix.k;
+            int d = qspan - rspan;
+            d = d < 0 ? -d : d;
+            if (d <= min_diff) {
+                if (out) {
+                    DevHit hh;
+                    hh.ref_strand = strand_bit | (v[u].w >> 8);
+                    hh.ref_start = (int32_t)v[u].z;
+                    hh.ref_end = (int32_t)v[u].z + rspan;
+                    hh.query_start = (uint16_t)qs;
+                    hh.query_end = (uint16_t)qe;
+                    out[c] = hh;
+                }
+                c++;
+                min_diff = d;
             }
-            c++;
-            min_diff = d;
         }
     }
     if (run) *run = rec;
@@ -686,6 +695,9 @@ __device__ __forceinline__ uint32_t walk_run(const DevIndex &ix, uint64_t pos, u
 // same on every lane) and writes the kept hits in run order when out !=
 // nullptr. Every lane calls it with the same arguments.
 constexpr uint32_t WALK_WAVE_MIN = 32;  // runs longer than this take the wave walk
+// kept hits above which pooled_hits gives a seed the wave: a lane's walk is a wait
+// for memory every AHEAD records, the wave's one every 64
+constexpr uint32_t WALK_LANE_MAX = 8;
 
 __device__ __forceinline__ uint32_t walk_run_wave(const DevIndex &ix, uint64_t pos, uint64_t key, int qs, int qe,
                                                   uint32_t strand_bit, DevHit *out) {
@@ -693,14 +705,13 @@ __device__ __forceinline__ uint32_t walk_run_wave(const DevIndex &ix, uint64_t p
     const int qspan = qe - qs;
     int carry = 0x7fffffff;
     uint32_t kept = 0;
+    // (the next records are loaded while these are looked at)
+    uint4 next = ix.rs[pos + lane < ix.n ? pos + lane : ix.n - 1];
     for (uint64_t x0 = pos; x0 < ix.n; x0 += 64) {
+        const uint4 v = next;
         const uint64_t x = x0 + lane;
-        uint4 v = make_uint4(0u, 0u, 0u, 0u);
-        bool in = false;
-        if (x < ix.n) {
-            v = ix.rs[x];
-            in = ((uint64_t)v.x | ((uint64_t)v.y << 32)) == key;
-        }
+        next = ix.rs[x + 64 < ix.n ? x + 64 : ix.n - 1];
+        const bool in = x < ix.n && ((uint64_t)v.x | ((uint64_t)v.y << 32)) == key;
         // equal hashes are contiguous: the run ends at the first other record
         const uint64_t other = ballot(!in);
         const uint32_t len = other ? (uint32_t)__builtin_ctzll(other) : 64u;
@@ -708,13 +719,8 @@ __device__ __forceinline__ uint32_t walk_run_wave(const DevIndex &ix, uint64_t p
         const int rspan = (int)(v.w & 0xffu) + ix.k;
         int d = qspan - rspan;
         d = d < 0 ? -d : d;
-        int incl = valid ? d : 0x7fffffff;
-        for (int sh = 1; sh < 64; sh <<= 1) {
-            const int y = __shfl_up(incl, sh, 64);
-            if (lane >= (uint32_t)sh) incl = y < incl ? y : incl;
-        }
-        int excl = __shfl_up(incl, 1, 64);
-        if (lane == 0) excl = 0x7fffffff;
+        const int incl = ~wave_incl_max(~(valid ? d : 0x7fffffff));
+        int excl = __builtin_amdgcn_update_dpp(0x7fffffff, incl, 0x138, 0xf, 0xf, false);  // wave_shr:1
         excl = carry < excl ? carry : excl;
         const bool keep = valid && d <= excl;
         const uint64_t km = ballot(keep);
@@ -843,14 +849,14 @@ __device__ __forceinline__ void probe_finish(const DevIndex &ix, Probe &p, int q
     if (!p.found) return;
     p.filtered = dev_filtered(ix, p.pos, p.key);
     if (p.filtered) return;
-    p.hc = walk_run(ix, p.pos, p.key, qs, qe, 0u, nullptr, &p.run);
+    p.hc = walk_run<1>(ix, p.pos, p.key, qs, qe, 0u, nullptr, &p.run);
 }
 
 // the kept hits of a probe, in run order
 __device__ __forceinline__ void probe_emit(const DevIndex &ix, const Probe &p, int qs, int qe,
                                            uint32_t strand_bit, DevHit *out) {
     if (!probe_small(p)) {
-        walk_run(ix, p.pos, p.key, qs, qe, strand_bit, out);
+        walk_run<1>(ix, p.pos, p.key, qs, qe, strand_bit, out);
         return;
     }
     uint32_t c = 0;
@@ -998,9 +1004,16 @@ __device__ __forceinline__ void pooled_hits(const DevBatch &b, const DevIndex &i
         const uint32_t i = i0 + lane;
         const uint32_t hc = i < n ? b.hcnt[base + i] : 0u;
         const uint32_t incl = wave_incl_scan_dpp(hc);
-        if (hc > 0)
+        if (hc > 0 && hc <= WALK_LANE_MAX)
             walk_run(ix, b.pos[base + i], b.rs_hash[base + i], (int)span_start(b.rs_span[base + i]),
                      (int)span_end(b.rs_span[base + i]), i >= half ? 0x80000000u : 0u, out + carry + incl - hc);
+        // long runs: the whole wave walks each one
+        for (uint64_t cm = ballot(hc > WALK_LANE_MAX); cm; cm &= cm - 1) {
+            const uint32_t l = (uint32_t)__builtin_ctzll(cm), il = i0 + l;
+            const uint64_t xl = base + il;
+            walk_run_wave(ix, b.pos[xl], b.rs_hash[xl], (int)span_start(b.rs_span[xl]), (int)span_end(b.rs_span[xl]),
+                          il >= half ? 0x80000000u : 0u, out + carry + readlane_u32(incl - hc, l));
+        }
         carry += readlane_u32(incl, 63);
     }
 }
@@ -1274,29 +1287,28 @@ __device__ __forceinline__ void wide_flush(const WideList &wide, uint32_t nw, gi
 
 // items loaded ahead per lane by the passes over a read's hits: a lone wave's
 // time in them is the latency of its loads
-constexpr uint32_t AHEAD = 4;
+constexpr uint32_t AHEAD = 8;
 
-// One stable pass of group_order's radix sort by the 8-bit digit at `shift` of
-// the group: from the hits themselves (src == nullptr) or from keys (group << 32
-// | hit index). bins: 256 words of LDS.
-template <typename Load>
-__device__ __forceinline__ void radix_pass(uint32_t n, uint32_t shift, Load load, uint64_t *dst, uint32_t *bins) {
-    const uint32_t lane = lane_id();
-    for (uint32_t u = lane; u < 256; u += 64) bins[u] = 0;
-    wave_sync();
+// f(i, item i) for the n items of a read that load gives, AHEAD chunks of 64 at a
+// time; lanes beyond the end get the last item, with i >= n
+template <typename T, typename Load, typename F>
+__device__ __forceinline__ void each_ahead(uint32_t n, Load load, F f) {
     for (uint32_t i0 = 0; i0 < n; i0 += 64 * AHEAD) {
-        uint64_t k[AHEAD];
+        T v[AHEAD];
 #pragma unroll
         for (uint32_t u = 0; u < AHEAD; u++) {
-            const uint32_t i = i0 + 64 * u + lane;
-            k[u] = load(i < n ? i : n - 1);
+            const uint32_t i = i0 + 64 * u + lane_id();
+            v[u] = load(i < n ? i : n - 1);
         }
 #pragma unroll
-        for (uint32_t u = 0; u < AHEAD; u++)
-            if (i0 + 64 * u + lane < n) atomicAdd(&bins[(uint32_t)(k[u] >> (32 + shift)) & 255u], 1u);
+        for (uint32_t u = 0; u < AHEAD; u++) f(i0 + 64 * u + lane_id(), v[u]);
     }
+}
+
+// counts to exclusive prefixes over 256 bins, four a lane
+__device__ __forceinline__ void bins_prefix(uint32_t *bins) {
+    const uint32_t lane = lane_id();
     wave_sync();
-    // exclusive prefix over the bins, four a lane
     const uint32_t b0 = bins[4 * lane], b1 = bins[4 * lane + 1], b2 = bins[4 * lane + 2], b3 = bins[4 * lane + 3];
     const uint32_t t = b0 + b1 + b2 + b3, at = wave_incl_scan_dpp(t) - t;
     wave_sync();
@@ -1305,76 +1317,109 @@ __device__ __forceinline__ void radix_pass(uint32_t n, uint32_t shift, Load load
     bins[4 * lane + 2] = at + b0 + b1;
     bins[4 * lane + 3] = at + b0 + b1 + b2;
     wave_sync();
-    for (uint32_t i0 = 0; i0 < n; i0 += 64 * AHEAD) {
-        uint64_t k[AHEAD];
+}
+
+// The n keys (group << 32 | hit index) that load gives to dst, stable by the digit
+// that digit(key) gives; bins: the digits' places, afterwards their ends.
+template <typename Load, typename Digit>
+__device__ __forceinline__ void radix_scatter(uint32_t n, Load load, Digit digit, uint64_t *dst, uint32_t *bins) {
+    each_ahead<uint64_t>(n, load, [&](uint32_t i, uint64_t k) {
+        const bool in = i < n;
+        const uint32_t d = digit(k);
+        // the lanes of the same digit, a ballot a bit (digit by digit took a trip
+        // to LDS for each of up to 48 groups)
+        uint64_t peers = ballot(in);
 #pragma unroll
-        for (uint32_t u = 0; u < AHEAD; u++) {
-            const uint32_t i = i0 + 64 * u + lane;
-            k[u] = load(i < n ? i : n - 1);
+        for (uint32_t bit = 0; bit < 8; bit++) {
+            const uint64_t m = ballot((d >> bit) & 1u);
+            peers &= (d >> bit) & 1u ? m : ~m;
         }
-#pragma unroll
-        for (uint32_t u = 0; u < AHEAD; u++) {
-            const bool in = i0 + 64 * u + lane < n;
-            const uint32_t d = (uint32_t)(k[u] >> (32 + shift)) & 255u;
-            // the 64 keys digit by digit: a read's hits lie in few groups
-            uint32_t pos = 0;
-            uint64_t left = ballot(in);
-            while (left) {
-                const uint32_t l = (uint32_t)__builtin_ctzll(left), dl = readlane_u32(d, l);
-                const uint64_t m = ballot(in && d == dl);
-                const uint32_t at_d = bins[dl];
-                if (d == dl) pos = at_d + mbcnt(m);
-                wave_sync();
-                if (lane == l) bins[dl] = at_d + (uint32_t)__popcll(m);
-                wave_sync();
-                left &= ~m;
-            }
-            if (in) dst[pos] = k[u];
-        }
-    }
+        const uint32_t rank = mbcnt(peers);
+        uint32_t pos = 0;
+        if (in) pos = bins[d] + rank;
+        wave_sync();
+        if (in && rank == 0) bins[d] = pos + (uint32_t)__popcll(peers);
+        wave_sync();
+        if (in) dst[pos] = k;
+    });
     wave_sync_mem();
 }
 
 // Grouped order of nh hits: nullptr when they already are in (strand, ref)
-// order, else keys (bitonic in keys, nh <= MERGE_LDS) or one of keys /
-// keys_alt (stable radix sort) holding group << 32 | hit index. bins: 256 words
-// of LDS for nh > MERGE_LDS.
+// order, else keys (bitonic in keys, nh <= MERGE_LDS and no keys_alt) or one of
+// keys / keys_alt (stable radix sort) holding group << 32 | hit index. bins: 256
+// words of LDS (the bitonic sort's keys may lie there). binned: the groups are
+// the bins, which hold their ends in the order.
+//
+// A wave's time here is that of its passes over the hits. The first counts the
+// groups of a read on references below 128 as it looks for the largest one, so
+// that those need one more, the scatter; others sort compact group keys by 8 bits
+// a pass. (A read of 5810 hits alone kept k_merge at 119 us; now 76.)
 __device__ __forceinline__ const uint64_t *group_order(uint32_t nh, const DevHit *hits, uint64_t *keys,
-                                                      uint64_t *keys_alt, uint32_t *bins) {
+                                                      uint64_t *keys_alt, uint32_t *bins, bool &binned) {
     const uint32_t lane = lane_id();
     const uint4 *hv = reinterpret_cast<const uint4 *>(hits);
-    uint32_t max_ref = 0;
+    for (uint32_t u = lane; u < 256; u += 64) bins[u] = 0;
+    wave_sync();
+    uint32_t max_ref = 0, last = 0;
     bool unsorted = false;
-#pragma unroll 4
-    for (uint32_t i0 = 0; i0 < nh; i0 += 64) {
-        const uint32_t i = i0 + lane;
-        const uint32_t rsd = hv[i < nh ? i : nh - 1].x, before = hv[i < nh ? (i ? i - 1 : 0) : nh - 1].x;
+    each_ahead<uint32_t>(nh, [&](uint32_t i) { return hv[i].x; }, [&](uint32_t i, uint32_t rsd) {
+        const uint32_t before = (uint32_t)__builtin_amdgcn_update_dpp((int)last, (int)rsd, 0x138, 0xf, 0xf, false);
+        last = readlane_u32(rsd, 63);
         max_ref = max(max_ref, rsd & 0x7fffffffu);
         unsorted |= before > rsd;
+        if (i < nh) atomicAdd(&bins[rsd >> 31 << 7 | (rsd & 127u)], 1u);
+    });
+    const uint32_t mr = wave_max_dpp(max_ref);
+    binned = mr < 128;
+    if (ballot(unsorted) == 0) {
+        bins_prefix(bins);  // each bin's start: its end is the next one's
+        uint32_t e[4];
+        for (uint32_t u = 0; u < 4; u++) e[u] = 4 * lane + u < 255 ? bins[4 * lane + u + 1] : nh;
+        wave_sync();
+        for (uint32_t u = 0; u < 4; u++) bins[4 * lane + u] = e[u];
+        wave_sync();
+        return nullptr;
     }
-    if (ballot(unsorted) == 0) return nullptr;
-    if (nh <= (uint32_t)MERGE_LDS) {
+    if (nh <= (uint32_t)MERGE_LDS && !keys_alt) {
         uint32_t P = 1;
         while (P < nh) P <<= 1;
+        wave_sync();
         for (uint32_t i = lane; i < P; i += 64) keys[i] = i < nh ? (((uint64_t)hv[i].x << 32) | i) : UINT64_MAX;
         wave_sync_mem();
         bitonic_mem(keys, P);
+        binned = false;
         return keys;
     }
-    // compact group key: strand above the bits of the largest ref_id. The first
-    // pass reads the hits, a read on few references needs no other.
-    const uint32_t mr = wave_max_dpp(max_ref);
-    const uint32_t rbits = mr ? 32u - (uint32_t)__builtin_clz(mr) : 0u;
-    radix_pass(nh, 0, [&](uint32_t i) {
-        const uint32_t x = hv[i].x;
-        return (((uint64_t)(x >> 31) << rbits | (x & 0x7fffffffu)) << 32) | i;
-    }, keys, bins);
-    uint64_t *src = keys, *alt = keys_alt;
-    for (uint32_t shift = 8; shift < rbits + 1; shift += 8) {
-        const uint64_t *from = src;
-        radix_pass(nh, shift, [&](uint32_t i) { return from[i]; }, alt, bins);
-        alt = src;
-        src = const_cast<uint64_t *>(from == keys ? keys_alt : keys);
+    if (binned) {
+        bins_prefix(bins);
+        radix_scatter(nh, [&](uint32_t i) {
+            const uint32_t x = hv[i].x;
+            return (uint64_t)(x >> 31 << 7 | x) << 32 | i;
+        }, [](uint64_t k) { return (uint32_t)(k >> 32) & 255u; }, keys, bins);
+        return keys;
+    }
+    // compact group key: strand above the bits of the largest ref_id; the first
+    // pass makes it from the hits
+    const uint32_t rbits = 32u - (uint32_t)__builtin_clz(mr);
+    const uint64_t *src = nullptr;
+    uint64_t *dst = keys;
+    for (uint32_t shift = 0; shift < rbits + 1; shift += 8) {
+        auto load = [&](uint32_t i) {
+            if (src) return src[i];
+            const uint32_t x = hv[i].x;
+            return (((uint64_t)(x >> 31) << rbits | (x & 0x7fffffffu)) << 32) | i;
+        };
+        auto digit = [&](uint64_t k) { return (uint32_t)(k >> (32 + shift)) & 255u; };
+        for (uint32_t u = lane; u < 256; u += 64) bins[u] = 0;
+        wave_sync();
+        each_ahead<uint64_t>(nh, load, [&](uint32_t i, uint64_t k) {
+            if (i < nh) atomicAdd(&bins[digit(k)], 1u);
+        });
+        bins_prefix(bins);
+        radix_scatter(nh, load, digit, dst, bins);
+        src = dst;
+        dst = dst == keys ? keys_alt : keys;
     }
     return src;
 }
@@ -1476,8 +1521,9 @@ __device__ __forceinline__ uint32_t take_run(LaneNam &o, uint32_t w, const uint4
 }
 
 constexpr uint32_t ARRIVAL_BLOCK = 4;
-// a strand of more groups than this and more NAMs than lanes is merge_range's
-constexpr uint32_t ARRIVAL_GROUPS = 16;
+// a strand of more groups than this and more NAMs than lanes is merge_range's (reads
+// in repeats)
+constexpr uint32_t ARRIVAL_GROUPS = 8;
 
 // Merge of a read's hits in arrival order on one wave, a NAM a lane, without
 // grouping them: NAMs of every group of the current strand share the lanes, and
@@ -1592,6 +1638,12 @@ __device__ __forceinline__ uint32_t merge_arrival(const DevHit *hits, uint32_t n
                     } while (todo);
                     if (me != 0) break;
                     if (multi) {
+                        // (its groups so far)
+                        uint64_t nams = ~0ull;
+                        uint32_t k = 0;
+                        for (; nams && k <= ARRIVAL_GROUPS; k++)
+                            nams &= ~ballot(rsd_o == readlane_u32(rsd_o, (uint32_t)__builtin_ctzll(nams)));
+                        if (k > ARRIVAL_GROUPS) return MERGE_OVERFLOW;
                         full = true;
                         break;
                     }
@@ -2007,10 +2059,13 @@ struct MergeLds {
     DevHit hits[MERGE_LDS];
 };
 
-// reads whose (strand, ref) groups merge on separate waves (k_merge_groups,
-// then k_merge_split_finish), for reads with more than SPLIT_MIN hits
+// reads whose (strand, ref) groups merge on waves of their own (k_merge_groups,
+// then k_merge_split_finish): those that do not merge in arrival order. k_merge
+// only groups them, so that its few long merges and those of k_merge_groups run
+// side by side (100 003 reads of a repeat-rich genome: k_merge 185 us with the
+// merges of up to 512 hits, now 76; k_merge_groups, as long as its largest group
+// of 1590 hits, 219 us before and after, with long items first)
 constexpr uint32_t MERGE_SPLIT = 0xfffffffdu;
-constexpr uint32_t SPLIT_MIN = 512;
 // hits of one k_merge_groups work item: consecutive small groups of a split
 // read merge on one wave
 constexpr uint32_t ITEM_HITS = 384;
@@ -2041,52 +2096,69 @@ __global__ __launch_bounds__(64) void k_merge(DevBatch b) {
         const DevHit *ghits = (rescue ? b.rhits : b.hits) + hb;
         gis_nam *fin = (rescue ? b.rnam_fin : b.nam_fin) + hb;
         uint64_t *gkeys = b.merge_scratch ? (rescue ? b.rkeys : b.keys) + 2 * hb : nullptr;
-        WideNam *gwide = b.merge_scratch ? (rescue ? b.rnam_ws : b.nam_ws) + hb : nullptr;
-        if (nh > SPLIT_MIN && b.merge_scratch) {
-            // group the hits; each group merges on its own wave
+        uint32_t total = nh <= ARRIVAL_MAX ? merge_arrival<true>(ghits, nh, fin, nh) : MERGE_OVERFLOW;
+        if (total == MERGE_OVERFLOW && b.merge_scratch) {
+            // group the hits; k_merge_groups merges them, a large group a wave
             uint32_t *bins = reinterpret_cast<uint32_t *>(lkeys);
-            const uint64_t *ord = group_order(nh, ghits, gkeys, gkeys + nh, bins);
+            bool binned;
+            const uint64_t *ord = group_order(nh, ghits, gkeys, gkeys + nh, bins, binned);
             const uint32_t code = ord == nullptr ? 0u : (ord == gkeys ? 1u : 2u);
             uint64_t *slots = code == 1u ? gkeys + nh : gkeys;
-            uint32_t G = 0;
-            for (uint32_t i0 = 0; i0 < nh; i0 += 64) {
-                const uint32_t i = i0 + lane;
-                bool head = false;
-                if (i < nh) {
-                    // (keys hold the group above the index)
-                    const uint32_t cur = ord ? (uint32_t)(ord[i] >> 32) : ghits[i].ref_strand;
-                    head = i == 0 || (ord ? (uint32_t)(ord[i - 1] >> 32) : ghits[i - 1].ref_strand) != cur;
+            // work items: runs of consecutive groups of at least ITEM_HITS hits (a
+            // larger group is an item of its own); each item's start goes to
+            // slots[item], which later holds its NAM count
+            uint32_t K = 0, cur = 0;
+            // start: of a lane's group where head, growing with the lane
+            auto cut = [&](uint64_t heads, uint32_t start) {
+                for (;;) {
+                    heads &= ballot(start >= cur + ITEM_HITS);
+                    if (!heads) break;
+                    if (lane == 0) slots[K] = (uint64_t)cur << 32;
+                    K++;
+                    cur = readlane_u32(start, (uint32_t)__builtin_ctzll(heads));
                 }
-                const uint64_t bal = ballot(head);
-                if (head) slots[G + mbcnt(bal)] = (uint64_t)i << 32;
-                G += (uint32_t)__popcll(bal);
-            }
-            wave_sync_mem();
-            // work items: runs of consecutive groups of at least ITEM_HITS
-            // hits (a larger group is an item of its own); each item's start
-            // goes to slots[item], which later holds its NAM count
-            uint32_t K = 0;
-            if (lane == 0) {
-                uint32_t cur = 0;
-                for (uint32_t g = 1; g < G; g++) {
-                    const uint32_t st = (uint32_t)(slots[g] >> 32);
-                    if (st - cur >= ITEM_HITS) {
-                        slots[K++] = (uint64_t)cur << 32;  // K < g: heads not read yet stay intact
-                        cur = st;
-                    }
+            };
+            if (binned) {
+                uint32_t done = 0;
+                for (uint32_t d0 = 0; d0 < 256; d0 += 64) {
+                    const uint32_t end = bins[d0 + lane];
+                    const uint32_t start = (uint32_t)__builtin_amdgcn_update_dpp((int)done, (int)end, 0x138, 0xf, 0xf, false);
+                    done = readlane_u32(end, 63);
+                    cut(ballot(end > start), start);
                 }
-                slots[K++] = (uint64_t)cur << 32;
+            } else {
+                uint32_t before = 0;
+                each_ahead<uint32_t>(nh, [&](uint32_t i) {
+                    return ord ? (uint32_t)(ord[i] >> 32) : ghits[i].ref_strand;  // (the group above the index)
+                }, [&](uint32_t i, uint32_t grp) {
+                    const uint32_t prev =
+                        (uint32_t)__builtin_amdgcn_update_dpp((int)before, (int)grp, 0x138, 0xf, 0xf, false);
+                    before = readlane_u32(grp, 63);
+                    cut(ballot(i > 0 && i < nh && prev != grp), i);
+                });
             }
-            K = (uint32_t)__builtin_amdgcn_readfirstlane((int)K);
+            if (lane == 0) slots[K] = (uint64_t)cur << 32;
+            K++;
             wave_sync_mem();
             {
-                uint32_t at = 0;
-                if (lane == 0) at = atomicAdd(&b.ctl->n_gwork, K);
-                at = (uint32_t)__builtin_amdgcn_readfirstlane((int)at);
-                for (uint32_t g = lane; g < K; g += 64) {
-                    const uint32_t gs = (uint32_t)(slots[g] >> 32);
-                    const uint32_t ge = g + 1 < K ? (uint32_t)(slots[g + 1] >> 32) : nh;
-                    b.gwork[at + g] = make_uint4(r, gs, ge, g | (code << 30));
+                // long items from the list's front, the others from its back
+                for (uint32_t g0 = 0; g0 < K; g0 += 64) {
+                    const uint32_t g = g0 + lane;
+                    uint32_t gs = 0, ge = 0;
+                    if (g < K) {
+                        gs = (uint32_t)(slots[g] >> 32);
+                        ge = g + 1 < K ? (uint32_t)(slots[g + 1] >> 32) : nh;
+                    }
+                    const uint64_t lm = ballot(ge - gs >= 2 * ITEM_HITS), sm = ballot(g < K) & ~lm;
+                    uint32_t at_l = 0, at_s = 0;
+                    if (lane == 0) {
+                        if (lm) at_l = atomicAdd(&b.ctl->n_gwork[0], (uint32_t)__popcll(lm));
+                        if (sm) at_s = atomicAdd(&b.ctl->n_gwork[1], (uint32_t)__popcll(sm));
+                    }
+                    at_l = uni32(at_l) + mbcnt(lm);
+                    at_s = uni32(at_s) + mbcnt(sm);
+                    if (g < K)
+                        b.gwork[lane_bit(lm) ? at_l : b.gwork_cap - 1 - at_s] = make_uint4(r, gs, ge, g | (code << 30));
                 }
                 if (lane == 0) {
                     const uint32_t si = atomicAdd(&b.ctl->n_split, 1u);
@@ -2097,13 +2169,11 @@ __global__ __launch_bounds__(64) void k_merge(DevBatch b) {
                 continue;
             }
         }
-        uint32_t total = nh <= ARRIVAL_MAX ? merge_arrival<true>(ghits, nh, fin, nh) : MERGE_OVERFLOW;
-        if (total == MERGE_OVERFLOW && (nh <= (uint32_t)MERGE_LDS || b.merge_scratch)) {
-            // more than 64 NAMs at once: group by group, with a wide list (NAMs <= hits)
-            const bool lds = nh <= (uint32_t)MERGE_LDS;
-            const uint64_t *ord = group_order(nh, ghits, lds ? lkeys : gkeys, lds ? nullptr : gkeys + nh,
-                                              reinterpret_cast<uint32_t *>(lkeys));
-            const WideList wl{(LdsWideNam *)lwide, gwide, (uint32_t)MERGE_WIDE_LDS};
+        if (total == MERGE_OVERFLOW && nh <= (uint32_t)MERGE_LDS) {
+            // no scratch (yet): here, group by group, with a wide list (NAMs <= hits)
+            bool binned;
+            const uint64_t *ord = group_order(nh, ghits, lkeys, nullptr, reinterpret_cast<uint32_t *>(lkeys), binned);
+            const WideList wl{(LdsWideNam *)lwide, nullptr, (uint32_t)MERGE_WIDE_LDS};
             total = merge_range(ghits, ord, 0, nh, wl, fin, nh, lblock);
         }
         if (total == MERGE_OVERFLOW) {
@@ -2127,9 +2197,10 @@ __global__ __launch_bounds__(64) void k_merge_groups(DevBatch b) {
     __shared__ ChunkBox lbox[GROUP_BOXES];
     __shared__ BlockLds lblock;
     const uint32_t lane = lane_id();
-    const unsigned int cnt = sload(&b.ctl->n_gwork);
+    // (long items first: the kernel is as long as the last of them)
+    const uint32_t n_long = sload(&b.ctl->n_gwork[0]), cnt = n_long + sload(&b.ctl->n_gwork[1]);
     for (uint32_t w = blockIdx.x; w < cnt; w += gridDim.x) {
-        const uint4 it = b.gwork[w];
+        const uint4 it = b.gwork[w < n_long ? w : b.gwork_cap - 1 - (w - n_long)];
         const uint32_t r = it.x, gs = it.y, ge = it.z, g = it.w & 0x3fffffffu, code = it.w >> 30;
         const bool rescue = (b.flags[r] & GIS_FLAG_RESCUED) != 0;
         const uint64_t hb = rescue ? b.rhit_off[r] : b.hit_off[r];
@@ -2163,23 +2234,51 @@ __global__ __launch_bounds__(64 * WPB) void k_merge_split_finish(DevBatch b) {
         uint64_t *gkeys = (rescue ? b.rkeys : b.keys) + 2 * hb;
         const uint64_t *slots = code == 1u ? gkeys + nh : gkeys;
         gis_nam *fin = (rescue ? b.rnam_fin : b.nam_fin) + hb;
-        uint32_t base = 0;
-        for (uint32_t g = 0; g < G; g++) {
-            const uint64_t sg = slots[g];
-            const uint32_t gs = (uint32_t)(sg >> 32), c = (uint32_t)sg;
-            // base <= gs: every NAM moves towards the front, chunk by chunk
-            for (uint32_t c0 = 0; c0 < c; c0 += 64) {
-                const uint32_t k = c0 + lane;
-                gis_nam x{};
-                if (k < c) x = fin[gs + k];
-                wave_sync_mem();
-                if (k < c) {
-                    x.nam_id = (int32_t)(base + k);
-                    fin[base + k] = x;
-                }
-                wave_sync_mem();
+        // base <= gs: every NAM moves towards the front, and nothing is moved onto
+        // what a later step reads, so each step's 128 NAMs are loaded before the
+        // one before it stores (a lone wave waits for its loads); the first item's
+        // are in place
+        const uint64_t some = lane < G ? slots[lane] : 0;
+        auto slot = [&](uint32_t g) { return g < 64 ? readlane_u64(some, g) : uni64(slots[g]); };
+        uint32_t g = 0, c0 = 0, base = (uint32_t)slot(0);
+        uint32_t gs = 0, c = 0;
+        auto step = [&](gis_nam (&x)[2]) {  // loads the next step's; false at the end
+            c0 += 128;
+            while (c0 >= c) {
+                base += g > 0 ? c : 0;
+                if (++g >= G) return false;
+                const uint64_t sg = slot(g);
+                gs = (uint32_t)(sg >> 32);
+                c = (uint32_t)sg;
+                c0 = 0;
+                if (c) break;
             }
-            base += c;
+#pragma unroll
+            for (uint32_t u = 0; u < 2; u++)
+                if (c0 + 64 * u + lane < c) x[u] = fin[gs + c0 + 64 * u + lane];
+            return true;
+        };
+        auto store = [&](gis_nam (&x)[2], uint32_t at, uint32_t n) {
+            wave_sync_mem();
+#pragma unroll
+            for (uint32_t u = 0; u < 2; u++) {
+                const uint32_t k = 64 * u + lane;
+                if (k < n) {
+                    x[u].nam_id = (int32_t)(at + k);
+                    fin[at + k] = x[u];
+                }
+            }
+        };
+        gis_nam x[2], y[2];
+        bool more = step(x);
+        while (more) {
+            const uint32_t at = base + c0, n = min(128u, c - c0);
+            more = step(y);
+            store(x, at, n);
+            if (!more) break;
+            const uint32_t at2 = base + c0, n2 = min(128u, c - c0);
+            more = step(x);
+            store(y, at2, n2);
         }
         if (lane == 0) b.nam_cnt[r] = base;
         wave_sync_mem();

@@ -163,7 +163,7 @@ def test_host_calls_of_any_size(ctx, mode):
 
 
 @pytest.mark.parametrize("hits", [1, 15, 16, 17, 33, 63, 64, 65, 66, 127, 128, 129, 255, 256, 257, 400, 512, 513, 700])
-@pytest.mark.parametrize("refs", [1, 3, 20])
+@pytest.mark.parametrize("refs", [1, 3, 20, 300])
 def test_merge_path_edges(ctx, hits, refs):
     """Merges around the limits of their ways (16 and 64 NAMs a strand, 64,
     128, 256 and 512 hits): a strand of hits that each open a NAM, one of hits
