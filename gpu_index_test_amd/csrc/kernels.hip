@@ -117,6 +117,31 @@ __device__ __forceinline__ bool syncmer_fast(int L, const SeedParams &P, const S
     return true;
 }
 
+// What window p does to the state before it (slide, gis_core.h), w <= 7: nibble r is
+// the state after state r, nibble 7 and value 7 stand for NONE. st: the window's
+// state if it needs no history.
+__device__ __forceinline__ uint32_t window_map(const uint64_t *h, int p, int w, uint8_t st) {
+    if (st != ST_UNKNOWN) return 0x11111111u * (st < (uint8_t)w ? st : 7u);
+    const uint64_t v = h[p + w - 1];
+    uint32_t best = (uint32_t)w - 1;
+    uint64_t bv = v;
+    for (int o = w - 2; o >= 0; o--) {
+        const uint64_t c = h[p + o];
+        if (c < bv) { bv = c; best = (uint32_t)o; }
+    }
+    uint32_t m = best | (v < UINT64_MAX ? (uint32_t)w - 1 : 7u) << 28;
+    for (int r = 1; r < w; r++) m |= (v < h[p - 1 + r] ? (uint32_t)w - 1 : (uint32_t)r - 1) << (4 * r);
+    return m;
+}
+
+// the map `first` and then `then`
+__device__ __forceinline__ uint32_t map_after(uint32_t then, uint32_t first) {
+    uint32_t m = 0;
+#pragma unroll
+    for (int r = 0; r < 8; r++) m |= (then >> (4 * (first >> (4 * r) & 7u)) & 7u) << (4 * r);
+    return m;
+}
+
 // The passes of the syncmer scan after packing, for any read: canonical s-mer
 // hashes, window states, tie replay and compaction.
 __device__ __forceinline__ uint32_t syncmer_passes(int L, const SeedParams &P, const SeedBufs &B, uint32_t cap,
@@ -152,23 +177,34 @@ __device__ __forceinline__ uint32_t syncmer_passes(int L, const SeedParams &P, c
     // positions; a window is a syncmer when its minimum sits at offset t-1
     // (step2/randstrobes.cu:64-69)
     uint32_t nsync = 0;
+    uint32_t carry = 7;  // the state of the window before the 64 (w <= 7)
     for (int p0 = 0; p0 < nk; p0 += 64) {
         const int p = p0 + lane;
-        bool is_sync = false;
-        if (p < nk) {
-            uint8_t st = B.st[p];
-            if (st == ST_UNKNOWN) {
-                // window p-1 is valid and in the same segment; walk back to the
-                // segment's nearest anchor (the segment's first window is one)
-                int q = p - 1;
-                while (q > 0 && B.st[q] == ST_UNKNOWN) q--;
-                uint8_t r = B.st[q];
-                if (r != ST_NONE && r >= (uint8_t)w) r = ST_NONE;  // cannot happen; keeps indexing in range
-                for (int x = q + 1; x <= p; x++) r = slide(r, B.sh, x, w);
-                st = r;
+        uint8_t st = p < nk ? B.st[p] : ST_INVALID;
+        const bool tied = ballot(st == ST_UNKNOWN) != 0;
+        if (tied && w <= 7) {
+            // a tandem repeat ties window after window: the windows' maps
+            // composed over the lanes give every state at once. (Each lane
+            // walking back by itself was the last waves' time: 100 003 reads of
+            // a repeat-rich genome 158 us, now 104.)
+            uint32_t m = window_map(B.sh, p, w, st);
+            for (int d = 1; d < 64; d <<= 1) {
+                const uint32_t before = (uint32_t)__shfl_up((int)m, d, 64);
+                if (lane >= d) m = map_after(m, before);
             }
-            is_sync = st == (uint8_t)(P.t - 1);
+            st = (uint8_t)(m >> (4 * carry) & 7u);
+        } else if (st == ST_UNKNOWN) {
+            // window p-1 is valid and in the same segment; walk back to the
+            // segment's nearest anchor (the segment's first window is one)
+            int q = p - 1;
+            while (q > 0 && B.st[q] == ST_UNKNOWN) q--;
+            uint8_t r = B.st[q];
+            if (r != ST_NONE && r >= (uint8_t)w) r = ST_NONE;  // cannot happen; keeps indexing in range
+            for (int x = q + 1; x <= p; x++) r = slide(r, B.sh, x, w);
+            st = r;
         }
+        const bool is_sync = p < nk && st == (uint8_t)(P.t - 1);
+        carry = readlane_u32(st < (uint8_t)w ? st : 7u, 63);
         const uint64_t bal = ballot(is_sync);
         if (is_sync) {
             const uint32_t idx = nsync + mbcnt(bal);
