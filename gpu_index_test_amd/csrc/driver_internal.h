@@ -68,13 +68,29 @@ struct DevIndexStore {
     uint64_t epoch = 0;
 };
 
-// free the resident table (before another is loaded)
+// the resident table is no longer one (before another is loaded): no run still
+// reads it, and its memory is the next table's
 inline void drop_table(DevIndexStore &ix) {
+    (void)hipDeviceSynchronize();
     ix.loaded = false;
+    ix.epoch++;
+}
+
+// room for n elements of a table: the memory of the one before, unless that is too
+// small or more than twice as large (an allocation and its release cost ~180 us
+// together, three of them a fifth of a bacterial index's build)
+template <typename T>
+T *table_room(DevBuf &b, size_t n) {
+    const size_t need = std::max<size_t>(n, 1) * sizeof(T);
+    if (b.bytes < need || b.bytes / 2 > need) release(b);
+    return ensure<T>(b, n);
+}
+
+// the table's memory back (a load failed)
+inline void release_table(DevIndexStore &ix) {
     release(ix.rs);
     release(ix.starts);
     release(ix.lines);
-    ix.epoch++;
 }
 
 inline int fail(gis_ctx *ctx, int code, const std::string &msg);
@@ -92,6 +108,7 @@ struct gis_ctx {
     std::recursive_mutex mu;
     std::string err;
     gis::DevIndexStore ix;
+    gis::DevBuf build_mem;  // a build's device memory, kept for the next one if it is not large
     gis_batch *scratch = nullptr;  // batch reused by the host-buffer entry points
     int n_cu = 256;                // compute units of the device (persistent grids)
     gis_fused_config fcfg{4, 1, 0, 0, 8};

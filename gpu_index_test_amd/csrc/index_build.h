@@ -17,13 +17,17 @@ struct BuildError {
     const char *what;
 };
 
-// Device memory of one build, freed with it: pieces cut from a few large blocks.
-// An allocation and its release cost ~180 us together, more than most of the
-// build's kernels on a bacterial genome, so the first block is sized for the
-// whole build and a second one is taken only where the estimate falls short.
+// Device memory of one build: pieces cut from a few large blocks. An allocation
+// and its release cost ~180 us together for a small block and ~600 us for the 400
+// MB that 20 Mbp of reference take, so the first block is sized for the whole
+// build, a second one is taken only where the estimate falls short, and the first
+// one stays with the context (kept) for its next build if it is at most KEEP_MAX:
+// a larger reference's build takes far longer than that. The others go with the
+// arena.
 class BuildArena {
   public:
-    explicit BuildArena(uint64_t estimate) : next_(estimate) {}
+    static constexpr uint64_t KEEP_MAX = 512ull << 20;
+    BuildArena(uint64_t estimate, void *&kept, uint64_t &kept_bytes);
     ~BuildArena();
     BuildArena(const BuildArena &) = delete;
     BuildArena &operator=(const BuildArena &) = delete;
@@ -37,6 +41,8 @@ class BuildArena {
     std::vector<void *> blocks_;
     char *at_ = nullptr;
     uint64_t left_ = 0, next_;
+    void *&kept_;
+    uint64_t &kept_bytes_;
 };
 
 // device memory of a whole build of `bases` bases (a randstrobe in every k - s +

@@ -214,11 +214,11 @@ def test_merge_path_edges(ctx, hits, refs):
 
 
 @pytest.mark.parametrize("profile", [50, 150, 400])
-@pytest.mark.parametrize("lens", [[60_000], [30_000, 20_000, 12_345, 4096], [25_000, 8, 24, 31, 300, 25_000, 1]])
+@pytest.mark.parametrize("lens", [[60_000], [30_000, 20_000, 12_345, 4096], [25_000, 8, 24, 31, 300, 25_000, 1], [45_000, 5000]])
 def test_index_build_edges(ctx, profile, lens):
     """One and several contigs, equal sequence at equal positions of several
-    contigs, contigs too short for a randstrobe, runs of tied s-mers, N runs
-    and lengths off every tile."""
+    contigs, contigs too short for a randstrobe, runs of tied s-mers, N runs,
+    lengths off every tile and hashes of thousands of records."""
     rng = np.random.default_rng(len(lens) + profile)
     lens = np.array(lens, dtype=np.uint64)
     g = rng.choice(np.frombuffer(b"ACGT", dtype=np.uint8), size=int(lens.sum()))
@@ -232,6 +232,8 @@ def test_index_build_edges(ctx, profile, lens):
             s[7000:7150] = ord("N")
             s[8000:8100] = np.frombuffer(b"acgtN" * 20, dtype=np.uint8)
             s[-25:] = ord("T")
+    if lens[0] == 45_000:
+        g[:45_000] = np.resize(g[:11], 45_000)
     idx = G.StrobemerIndex(None, G.IndexParameters.from_read_length(profile))
     idx.populate_arrays(g, lens)
     oidx = O.Index.build_arrays(g, lens, O.params_from_read_length(profile), n_threads=4)
