@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "batch_internal.h"
+#include "host_copy.h"
 
 using namespace gis;
 
@@ -658,14 +659,10 @@ int batch_download(gis_batch *b, gis_nam_out *out) {
         if (out->flags && n) std::memcpy(out->flags, h.flags, n);
         return GIS_OK;
     }
-    if (out->nam_offsets)
-        HIP_CHECK(hipMemcpyAsync(out->nam_offsets, b->ws->nam_off.p, 8ull * (n + 1), hipMemcpyDeviceToHost, st));
-    if (b->ws->tot_nams)
-        HIP_CHECK(hipMemcpyAsync(out->nams, b->ws->nams_out.p, sizeof(gis_nam) * b->ws->tot_nams,
-                                 hipMemcpyDeviceToHost, st));
-    if (out->nonrepetitive_fraction && n)
-        HIP_CHECK(hipMemcpyAsync(out->nonrepetitive_fraction, b->ws->frac.p, 4ull * n, hipMemcpyDeviceToHost, st));
-    if (out->flags && n) HIP_CHECK(hipMemcpyAsync(out->flags, b->ws->flags.p, n, hipMemcpyDeviceToHost, st));
+    if (out->nam_offsets) copy_to_host(ctx, out->nam_offsets, b->ws->nam_off.p, 8ull * (n + 1), st);
+    if (b->ws->tot_nams) copy_to_host(ctx, out->nams, b->ws->nams_out.p, sizeof(gis_nam) * b->ws->tot_nams, st);
+    if (out->nonrepetitive_fraction) copy_to_host(ctx, out->nonrepetitive_fraction, b->ws->frac.p, 4ull * n, st);
+    if (out->flags) copy_to_host(ctx, out->flags, b->ws->flags.p, n, st);
     HIP_CHECK(hipStreamSynchronize(st));
     return GIS_OK;
 }
@@ -757,9 +754,9 @@ static int seeds_of(gis_ctx *ctx, const gis_params *params, bool syncmers, const
         ensure<char>(w->seeds, total * rec);
         launch_emit_seeds(d, syncmers ? 1 : 0, off, w->seeds.p, nullptr, st);
         HIP_CHECK(hipGetLastError());
-        HIP_CHECK(hipMemcpyAsync(out, w->seeds.p, total * rec, hipMemcpyDeviceToHost, st));
+        copy_to_host(ctx, out, w->seeds.p, total * rec, st);
     }
-    if (out_offsets) HIP_CHECK(hipMemcpyAsync(out_offsets, off, 8ull * (n + 1), hipMemcpyDeviceToHost, st));
+    if (out_offsets) copy_to_host(ctx, out_offsets, off, 8ull * (n + 1), st);
     HIP_CHECK(hipStreamSynchronize(st));
     return GIS_OK;
 }
@@ -800,13 +797,19 @@ extern "C" int gis_lookup_batch(gis_ctx *ctx, const uint64_t *hashes, uint64_t n
     if (!ctx->ix.loaded) return fail(ctx, GIS_ERR_STATE, "no index loaded");
     if (n && (!hashes || !positions)) return fail(ctx, GIS_ERR_BAD_PARAMETER, "null argument");
     if (n == 0) return GIS_OK;
+    // (overlapping arrays: all keys are read before a position is written)
+    const bool apart = positions + n <= hashes || hashes + n <= positions;
+    if (apart && !pinned_array(hashes) && !pinned_array(positions)) {
+        lookup_through_host(ctx, hashes, n, positions, ctx->stream);
+        return GIS_OK;
+    }
     gis_batch *b = scratch_batch(ctx);
     uint64_t *dh = ensure<uint64_t>(b->ws->rs_hash, n);
     uint64_t *dp = ensure<uint64_t>(b->ws->pos, n);
     HIP_CHECK(hipMemcpyAsync(dh, hashes, 8 * n, hipMemcpyHostToDevice, ctx->stream));
     launch_find_flat(dev_index(ctx), dh, n, dp, ctx->stream);
     HIP_CHECK(hipGetLastError());
-    HIP_CHECK(hipMemcpyAsync(positions, dp, 8 * n, hipMemcpyDeviceToHost, ctx->stream));
+    copy_to_host(ctx, positions, dp, 8 * n, ctx->stream);
     HIP_CHECK(hipStreamSynchronize(ctx->stream));
     return GIS_OK;
     API_END(ctx)

@@ -11,6 +11,7 @@
 #include <vector>
 
 #include "driver_internal.h"
+#include "host_copy.h"
 #include "index_build.h"
 #include "index_host.h"
 
@@ -115,6 +116,8 @@ extern "C" void gis_ctx_destroy(gis_ctx *ctx) {
         release(ctx->ix.starts);
         release(ctx->ix.lines);
         release(ctx->build_mem);
+        hostcopy_free(ctx->host_copy);
+        ctx->host_copy = nullptr;
         (void)hipStreamDestroy(ctx->stream);
     }
     delete ctx;
@@ -361,11 +364,8 @@ extern "C" int gis_index_download(gis_ctx *ctx, gis_ref_randstrobe *randstrobes,
     // (in stream order: a pinned array then takes them at the link's rate, 1.1 ms
     // for 64 MB, where hipMemcpy took 2.1 ms)
     if (randstrobes && ix.n)
-        HIP_CHECK(hipMemcpyAsync(randstrobes, ix.rs.p, ix.n * sizeof(gis_ref_randstrobe), hipMemcpyDeviceToHost,
-                                 ctx->stream));
-    if (starts)
-        HIP_CHECK(hipMemcpyAsync(starts, ix.starts.p, ((1ULL << ix.bits) + 1) * 8, hipMemcpyDeviceToHost,
-                                 ctx->stream));
+        copy_to_host(ctx, randstrobes, ix.rs.p, ix.n * sizeof(gis_ref_randstrobe), ctx->stream);
+    if (starts) copy_to_host(ctx, starts, ix.starts.p, ((1ULL << ix.bits) + 1) * 8, ctx->stream);
     HIP_CHECK(hipStreamSynchronize(ctx->stream));
     return GIS_OK;
     API_END(ctx)

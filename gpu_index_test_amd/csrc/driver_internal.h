@@ -99,6 +99,7 @@ inline int fail(gis_ctx *ctx, int code, const std::string &msg);
 struct PairWork;
 void pairwork_free(PairWork *w);
 struct DmaEngines;
+struct HostCopy;
 
 }  // namespace gis
 
@@ -118,6 +119,7 @@ struct gis_ctx {
     std::vector<gis_batch *> lanes;
     // the copy engines those lanes drive directly (stream.cpp), found on first use
     gis::DmaEngines *dma = nullptr;
+    gis::HostCopy *host_copy = nullptr;  // pinned chunks of copies of pageable arrays (host_copy.h)
     // concurrent gis_find_nams_qrs calls waiting to be run together
     std::mutex comb_mu;
     std::condition_variable comb_cv;

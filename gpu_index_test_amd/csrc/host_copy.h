@@ -1,0 +1,28 @@
+// Copies from HBM to a caller's arrays, in stream order. A pageable array of some
+// size goes through pinned chunks of the context, emptied on the host while the next
+// ones cross the link; the runtime's own way pins the array for each copy (20 MB of
+// seeds: 1.44 ms, now 0.82; for arrays that the device reads it measured no worse
+// than chunks, and stays). The caller holds the context's lock.
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stddef.h>
+#include <stdint.h>
+
+struct gis_ctx;
+
+namespace gis {
+
+struct HostCopy;
+void hostcopy_free(HostCopy *h);
+// dst is complete when the stream is, or already on return (pageable)
+void copy_to_host(gis_ctx *ctx, void *dst, const void *src, size_t n, hipStream_t st);
+
+// positions of keys, both pageable: the lookup reads its keys from the pinned chunks
+// and writes their positions over them, across the link and while other chunks are
+// filled and emptied on the host (10^6 keys: 790 us with a copy each way, now 440)
+void lookup_through_host(gis_ctx *ctx, const uint64_t *keys, uint64_t n, uint64_t *positions, hipStream_t st);
+
+bool pinned_array(const void *p);
+
+}  // namespace gis

@@ -207,6 +207,7 @@ bool launch_fused(const DevBatch &b, const DevIndex &ix, const SeedParams &sp, u
 void launch_output(const DevBatch &b, int fused, uint64_t *tmp, DevCtl *dst, hipStream_t st);
 // the control block to pinned host memory after a run that stops before the output
 void launch_ctl_to_host(const DevBatch &b, DevCtl *dst, hipStream_t st);
+void launch_copy_out(const void *src, void *dst, uint64_t n, hipStream_t st);
 void launch_find_flat(const DevIndex &ix, const uint64_t *hashes, uint64_t n, uint64_t *positions,
                       hipStream_t st);
 // exclusive scan of u32 counts into u64 offsets[n+1] (offsets[n] = total);

@@ -264,3 +264,26 @@ def test_pair_list_edges(ctx, max_tries):
     n = len(m1)
     _compare(G.pairs_from_nams(ctx, offs, flat, n, max_tries=max_tries),
              O.pairs_batch(offs, flat, n, max_tries=max_tries), offs)
+
+
+@pytest.mark.parametrize("n", [1, 65_535, 65_536, 131_071, 131_072, 131_073, 400_000, 1_300_000])
+def test_lookups_of_any_size(ctx, n):
+    """Key counts around the chunks that pageable arrays go through, from and to
+    pageable and pinned arrays."""
+    rng = np.random.default_rng(n)
+    ents = [(h, 10 * i, 5) for i, h in enumerate(rng.integers(1, 2 ** 63, 500).tolist())]
+    arr, starts = tiny_index_arrays(ents)
+    oidx = O.Index.wrap(arr, starts, 8, 30, O.params_from_read_length(150))
+    idx = G.StrobemerIndex(None, G.IndexParameters.from_read_length(150))
+    idx.upload(arr, starts, 8, 30)
+    pool = np.concatenate([arr["hash"], rng.integers(0, 2 ** 64, 500, dtype=np.uint64)])
+    exp = np.array([oidx.find(int(k)) for k in pool], dtype=np.uint64)
+    at = rng.integers(0, len(pool), n)
+    keys = pool[at]
+    assert np.array_equal(idx.find_many(keys), exp[at])
+    pk, po = G.pinned_copy(keys), G.pinned_empty(n, np.uint64)
+    for k, o in ((pk, np.empty(n, np.uint64)), (keys, po), (pk, po)):
+        o[:] = 7
+        idx.ctx.check(idx.ctx.L.gis_lookup_batch(idx.ctx.h, k.ctypes.data, n, o.ctypes.data))
+        assert np.array_equal(o, exp[at])
+    idx.ctx.close()
