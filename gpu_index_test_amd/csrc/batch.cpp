@@ -403,8 +403,9 @@ int batch_stage(gis_batch *b, const char *seqs, const uint64_t *offsets, const u
         in.push_back({b->read_len.p, lens, 4ull * n});
     }
     in.push_back({b->rs_off.p, b->h_rs_off.data(), 8ull * (n + 1)});
-    in.push_back({b->sy_off.p, b->h_sy_off.data(), 8ull * (n + 1)});
-    in.push_back({b->long_off.p, b->h_long_off.data(), 8ull * (n + 1)});
+    // (read by the seeding for these alone)
+    if (want_sy) in.push_back({b->sy_off.p, b->h_sy_off.data(), 8ull * (n + 1)});
+    if (b->any_long) in.push_back({b->long_off.p, b->h_long_off.data(), 8ull * (n + 1)});
     if (n && want_queue) in.push_back({b->queue.p, b->h_queue.data(), 4ull * n});
     b->ran = false;
     if (defer) return GIS_OK;

@@ -186,6 +186,7 @@ struct StreamJob {
     // 0 .. i-1, known once batch i-1 has counted its own
     uint64_t next = 0;  // the batch whose first NAM's place is `base`
     uint64_t base = 0;
+    uint64_t ran = 0;  // of the first batch of each lane, those whose run is over
     bool failed = false;
     int code = GIS_OK;
     std::string msg;
@@ -229,8 +230,24 @@ void lane_main(StreamJob &J, gis_batch *b, uint32_t lane, uint32_t lanes) {
             hipStream_t st = b->stream;
             run_copies(E, true, in, sig, have_sig, st);
             const RunOpts r = run_opts(b, J.opt, 0, STOP_NONE);
+            // The lanes start together, and runs that share the device end
+            // together: the way back, which bounds the pass, would wait for
+            // all of them (four lanes of 65,536 reads: the first results after
+            // 1.7 ms). So their first runs go one after the other.
+            if (i < lanes) {
+                std::unique_lock<std::mutex> lk(J.m);
+                J.cv.wait(lk, [&] { return J.failed || J.ran == i; });
+                if (J.failed) break;
+            }
             batch_launch(b, r);
             batch_complete(b, r);  // regrowth reruns included
+            if (i < lanes) {
+                {
+                    std::lock_guard<std::mutex> lk(J.m);
+                    J.ran = i + 1;
+                }
+                J.cv.notify_all();
+            }
             const uint64_t tot = b->ws->tot_nams;
             uint64_t mine = 0;
             {
