@@ -655,7 +655,6 @@ __device__ __forceinline__ bool rank_nams(const gis_nam *L, uint32_t c, uint8_t 
     const CmpNam n = cmp_nam(L, lane < c ? (int32_t)lane : -1);
     const CmpKey k = cmp_key(n);
     uint32_t rank = 0;
-#pragma unroll 2
     for (uint32_t q = 0; q <= c; q++) rank += cmp_less(readlane_key(k, q), k) ? 1u : 0u;
     if (lane <= c) ranks[lane] = (uint8_t)rank;
     return ballot(n.score != n.score) != 0;
