@@ -922,7 +922,7 @@ __device__ __forceinline__ void probe_emit(const DevIndex &ix, const Probe &p, i
 // Write traffic is part of this kernel's bound, so a one-pass read (at most
 // 64 randstrobes) keeps its per-randstrobe results (position, kept-hit count)
 // in registers and stores them only when a later kernel reads them: when the
-// read is rescued (k_rescue_count, k_rescue_hits) or its hits go to the pool
+// read is rescued (k_hits) or its hits go to the pool
 // (k_hits). Longer reads, and the fused kernel's spilled reads, store them
 // in every pass. Wave sums and scans use DPP (52 VGPRs).
 __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(6))) void k_lookup(
