@@ -104,7 +104,10 @@ void batch_free(gis_batch *b) {
     for (auto &g : b->graphs) graph_drop(g);
     if (b->ws) {
         if (b->ws->owner == b) b->ws->owner = nullptr;
-        if (b->ws->in_flight == b) b->ws->in_flight = nullptr;
+        if (b->ws->in_flight == b) {
+            b->ws->in_flight = nullptr;
+            b->ctx->launched--;
+        }
         if (--b->ws->refs == 0) workspace_release(b->ws);
     }
     delete b;
@@ -443,12 +446,15 @@ void enqueue_run(gis_batch *b, const RunOpts &r) {
     const DevBatch d = make_devbatch(b);
     const uint32_t n = b->n_reads;
     uint64_t *tmp = static_cast<uint64_t *>(b->ws->scan_tmp.p);
-    b->n_ev = 0;
-    b->ev_names.clear();
-    mark(b, "start");
+    const bool front = r.part != PART_BACK, back = r.part != PART_FRONT;
+    if (front) {
+        b->n_ev = 0;
+        b->ev_names.clear();
+        mark(b, "start");
+    }
     ReadSet set{nullptr, nullptr, n};
     const bool fused = mode == GIS_MODE_FUSED && stop == STOP_NONE;
-    if (fused) {
+    if (fused && front) {
         launch_reset_ctl(d.ctl, st);
         const gis_fused_config &fc = ctx->fcfg;
         const unsigned grid = fc.blocks_per_cu > 0 ? (unsigned)(ctx->n_cu * fc.blocks_per_cu) : 0u;
@@ -466,12 +472,15 @@ void enqueue_run(gis_batch *b, const RunOpts &r) {
         }
         if (!ok) throw HipError{hipErrorInvalidValue, "unsupported fused configuration"};
         mark(b, "fused");
-        set = ReadSet{d.spill_ids, &d.ctl->n_spill, n};
     }
-    launch_seed(d, set, sp, b->want_sy ? 1 : 0, b->any_long ? 1 : 0, fused ? 0 : 1, st);
-    mark(b, "seed");
-    launch_lookup(d, set, ix, rescue_mode, st);
-    mark(b, "lookup");
+    if (fused) set = ReadSet{d.spill_ids, &d.ctl->n_spill, n};
+    if (fused ? back : front) {
+        launch_seed(d, set, sp, b->want_sy ? 1 : 0, b->any_long ? 1 : 0, fused ? 0 : 1, st);
+        mark(b, "seed");
+        launch_lookup(d, set, ix, rescue_mode, st);
+        mark(b, "lookup");
+    }
+    if (!back) return;
     launch_hits(d, ix, rcut, hard, st);
     mark(b, "hits");
     if (stop == STOP_NONE) {
@@ -518,47 +527,22 @@ RunOpts run_opts(const gis_batch *b, const gis_map_options &o, int rescue_mode, 
     return r;
 }
 
-// Enqueue one run on the batch's stream. With r.graph the launch sequence is
-// captured once per configuration (buffers, mode, cutoffs, fused launch
-// configuration) and replayed; a batch keeps the graphs of its last 8
-// configurations.
-void batch_launch(gis_batch *b, const RunOpts &r) {
+// the launches of r (or of its part), by its captured graph where it has one
+static void launch_part(gis_batch *b, const RunOpts &r) {
     gis_ctx *ctx = b->ctx;
     hipStream_t st = b->stream;
-    prepare_workspace(b);
-    b->ws->owner = b;
-    b->ran = false;
-    if (r.mode == GIS_MODE_FUSED && r.stop == STOP_NONE) {
-        if (!b->queue_ok) throw HipError{hipErrorInvalidValue, "fused run of reads staged without the work queue"};
-        ensure<gis_nam>(b->ws->nam_slots, (size_t)b->n_reads * F_NAMCAP);
-    }
-    // graphs captured against a table that has since been dropped hold its
-    // freed addresses and old parameters: never replay them
-    bool stale = false;
-    for (const auto &g : b->graphs) stale |= g.epoch != ctx->ix.epoch;
-    if (stale) {
-        HIP_CHECK(hipStreamSynchronize(st));
-        for (auto it = b->graphs.begin(); it != b->graphs.end();) {
-            if (it->epoch == ctx->ix.epoch) {
-                ++it;
-                continue;
-            }
-            graph_drop(*it);
-            it = b->graphs.erase(it);
-        }
-    }
     if (r.graph) {
         bool replay = true;
         const DevBatch key = make_devbatch(b);
         const gis_fused_config &fc = ctx->fcfg;
-        const int cfg[11] = {r.mode, r.rescue_mode, (int)r.rcut, (int)r.hard, r.stop,
+        const int cfg[12] = {r.mode, r.rescue_mode, (int)r.rcut, (int)r.hard, r.stop,
                              (b->want_sy ? 1 : 0) | (b->any_long ? 2 : 0), fc.waves_per_block,
-                             fc.length_split, fc.chunk, fc.blocks_per_cu, (int)b->n_long};
+                             fc.length_split, fc.chunk, fc.blocks_per_cu, (int)b->n_long, r.part};
         gis_batch::GraphEntry *hit = nullptr;
         for (auto &g : b->graphs)
             if (std::memcmp(&key, &g.key, sizeof key) == 0 && std::memcmp(cfg, g.cfg, sizeof cfg) == 0) hit = &g;
         if (!hit) {
-            if (b->graphs.size() >= 8) {
+            if (b->graphs.size() >= 16) {
                 auto old = b->graphs.begin();
                 for (auto it = b->graphs.begin(); it != b->graphs.end(); ++it)
                     if (it->used < old->used) old = it;
@@ -600,6 +584,62 @@ void batch_launch(gis_batch *b, const RunOpts &r) {
         enqueue_run(b, r);
     }
     HIP_CHECK(hipGetLastError());
+}
+
+// Enqueue one run on the batch's stream. With r.graph the launch sequence is
+// captured once per configuration (buffers, mode, cutoffs, fused launch
+// configuration) and replayed; a batch keeps the graphs of its last 8
+// configurations, in two parts each at most.
+//
+// in_turn (a burst: runs launched on streams of their own onto an idle device, none
+// waited for yet): a large batch starts after the front of the one before it, that
+// is its seeding and lookup or its fused kernels. Launched together they would
+// share the device from their first kernel and end together, and the first one's
+// copies back could not run beside the others' kernels. (Three batches of 65,536
+// reads of 150 bp and their results: 1797 us, side by side 2046.) Later launches
+// find the runs out of step already, and side by side their phases fill the device
+// better: 4 lanes without copies took 321 M reads/s against 291 M with turns kept
+// throughout. A batch of fewer than TURN_READS does not fill the device and runs
+// beside the others as it did.
+constexpr uint32_t TURN_READS = 16384;
+void batch_launch(gis_batch *b, const RunOpts &r, bool in_turn) {
+    gis_ctx *ctx = b->ctx;
+    hipStream_t st = b->stream;
+    prepare_workspace(b);
+    b->ws->owner = b;
+    b->ran = false;
+    if (r.mode == GIS_MODE_FUSED && r.stop == STOP_NONE) {
+        if (!b->queue_ok) throw HipError{hipErrorInvalidValue, "fused run of reads staged without the work queue"};
+        ensure<gis_nam>(b->ws->nam_slots, (size_t)b->n_reads * F_NAMCAP);
+    }
+    // graphs captured against a table that has since been dropped hold its
+    // freed addresses and old parameters: never replay them
+    bool stale = false;
+    for (const auto &g : b->graphs) stale |= g.epoch != ctx->ix.epoch;
+    if (stale) {
+        HIP_CHECK(hipStreamSynchronize(st));
+        for (auto it = b->graphs.begin(); it != b->graphs.end();) {
+            if (it->epoch == ctx->ix.epoch) {
+                ++it;
+                continue;
+            }
+            graph_drop(*it);
+            it = b->graphs.erase(it);
+        }
+    }
+    if (!in_turn || b->n_reads < TURN_READS || st == ctx->stream) {
+        launch_part(b, r);
+        return;
+    }
+    if (!ctx->turn_ev) HIP_CHECK(hipEventCreateWithFlags(&ctx->turn_ev, hipEventDisableTiming));
+    if (ctx->turn_st && ctx->turn_st != st) HIP_CHECK(hipStreamWaitEvent(st, ctx->turn_ev, 0));
+    RunOpts p = r;
+    p.part = PART_FRONT;
+    launch_part(b, p);
+    HIP_CHECK(hipEventRecord(ctx->turn_ev, st));
+    ctx->turn_st = st;
+    p.part = PART_BACK;
+    launch_part(b, p);
 }
 
 bool batch_ready(const gis_batch *b) { return hipStreamQuery(b->stream) == hipSuccess; }
@@ -1228,8 +1268,13 @@ extern "C" int gis_batch_launch(gis_batch *b, const gis_map_options *opt) {
     if (!ctx->ix.loaded) return fail(ctx, GIS_ERR_STATE, "no index loaded");
     if (b->ws->in_flight) return fail(ctx, GIS_ERR_STATE, IN_FLIGHT_MSG);
     b->pending_opt = opts_or_default(opt);
-    batch_launch(b, run_opts(b, b->pending_opt, 0, STOP_NONE));
+    if (ctx->launched == 0) {  // a burst starts
+        ctx->burst = true;
+        ctx->turn_st = nullptr;
+    }
+    batch_launch(b, run_opts(b, b->pending_opt, 0, STOP_NONE), ctx->burst);
     b->ws->in_flight = b;
+    ctx->launched++;
     return GIS_OK;
     API_END(ctx)
 }
@@ -1241,6 +1286,8 @@ extern "C" int gis_batch_wait(gis_batch *b) {
     if (b->ws->in_flight != b) return fail(ctx, GIS_ERR_STATE, "no launched run of this batch to wait for");
     // released first: after an error the workspace takes runs again
     b->ws->in_flight = nullptr;
+    ctx->launched--;
+    ctx->burst = false;
     batch_complete(b, run_opts(b, b->pending_opt, 0, STOP_NONE));
     return GIS_OK;
     API_END(ctx)

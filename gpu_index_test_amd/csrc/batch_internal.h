@@ -135,7 +135,7 @@ struct gis_batch {
     // captured launch sequences, one per configuration (buffers, mode, cutoffs)
     struct GraphEntry {
         DevBatch key;
-        int cfg[11];
+        int cfg[12];
         uint64_t epoch;  // the index table the graph was captured against
         hipGraph_t graph;
         hipGraphExec_t exec;  // null: met once, not captured yet (lazy_graph)
@@ -161,7 +161,9 @@ struct RunOpts {
     uint32_t rcut, hard;
     int stop;          // STOP_*
     bool graph;        // replay a captured graph
+    int part = 0;      // PART_*: the launches up to the lookup or the fused kernels, the others, or all
 };
+enum { PART_ALL = 0, PART_FRONT = 1, PART_BACK = 2 };
 
 gis_batch *batch_new(gis_ctx *ctx, Workspace *share);  // share = nullptr: a workspace of its own
 gis_batch *batch_new_stream(gis_ctx *ctx);  // a batch with a stream and a workspace of its own
@@ -194,7 +196,7 @@ int batch_upload(gis_batch *b, const char *seqs, const uint64_t *offsets, const 
                  uint32_t n, bool want_sy);
 RunOpts run_opts(const gis_batch *b, const gis_map_options &o, int rescue_mode, int stop);
 // enqueue one run on the batch's stream without waiting
-void batch_launch(gis_batch *b, const RunOpts &r);
+void batch_launch(gis_batch *b, const RunOpts &r, bool in_turn = false);
 // the launched run has finished on the device
 bool batch_ready(const gis_batch *b);
 // wait for the launched run, grow what overflowed and run again until the

@@ -116,6 +116,7 @@ extern "C" void gis_ctx_destroy(gis_ctx *ctx) {
         release(ctx->ix.starts);
         release(ctx->ix.lines);
         release(ctx->build_mem);
+        if (ctx->turn_ev) (void)hipEventDestroy(ctx->turn_ev);
         hostcopy_free(ctx->host_copy);
         ctx->host_copy = nullptr;
         (void)hipStreamDestroy(ctx->stream);

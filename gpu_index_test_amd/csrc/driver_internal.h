@@ -119,6 +119,12 @@ struct gis_ctx {
     std::vector<gis_batch *> lanes;
     // the copy engines those lanes drive directly (stream.cpp), found on first use
     gis::DmaEngines *dma = nullptr;
+    // launched runs not waited for; whether they began as a burst that still lasts;
+    // and the front of the burst's last large run, with its stream (batch_launch)
+    int launched = 0;
+    bool burst = false;
+    hipEvent_t turn_ev = nullptr;
+    hipStream_t turn_st = nullptr;
     gis::HostCopy *host_copy = nullptr;  // pinned chunks of copies of pageable arrays (host_copy.h)
     // concurrent gis_find_nams_qrs calls waiting to be run together
     std::mutex comb_mu;

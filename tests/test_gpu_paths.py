@@ -287,3 +287,34 @@ def test_lookups_of_any_size(ctx, n):
         idx.ctx.check(idx.ctx.L.gis_lookup_batch(idx.ctx.h, k.ctypes.data, n, o.ctypes.data))
         assert np.array_equal(o, exp[at])
     idx.ctx.close()
+
+
+@pytest.mark.parametrize("mode", [G.MODE_PLAIN, G.MODE_FUSED])
+def test_launch_bursts(ctx, mode):
+    """Large and small batches on streams of their own, launched together and
+    again out of step, waited for in any order, against a run alone."""
+    g, lens = G.synth_genome(300_000, n_contigs=2, gc=0.45, repeat_fraction=0.05, n_families=5,
+                             family_len=(300, 1500), copies=(2, 10), seed=5)
+    idx = G.StrobemerIndex(None, G.IndexParameters.from_read_length(150))
+    idx.populate_arrays(g, lens)
+    mappers, exp = [], []
+    for n in (20_000, 16_384, 700, 16_383):
+        s, o, l, _ = G.synth_reads(g, lens, n, lengths=(100, 150), weights=(0.5, 0.5), sub_rate=0.01, seed=n)
+        m = G.Mapper(idx, n, int(l.sum()), own_stream=True)
+        m.upload(s, o, l)
+        m.run(mode=mode)
+        mappers.append(m)
+        exp.append(m.download().nams.tobytes())
+    for order in ([0, 1, 2, 3], [3, 2, 1, 0], [2, 0, 3, 1]):
+        for m in mappers:
+            m.launch(mode=mode)
+        for i in order:
+            mappers[i].wait()
+            assert mappers[i].download().nams.tobytes() == exp[i]
+            mappers[i].launch(mode=mode)
+        for i in order:
+            mappers[i].wait()
+            assert mappers[i].download().nams.tobytes() == exp[i]
+    for m in mappers:
+        m.close()
+    idx.ctx.close()
