@@ -700,10 +700,13 @@ int batch_download(gis_batch *b, gis_nam_out *out) {
         if (out->flags && n) std::memcpy(out->flags, h.flags, n);
         return GIS_OK;
     }
-    if (out->nam_offsets) copy_to_host(ctx, out->nam_offsets, b->ws->nam_off.p, 8ull * (n + 1), st);
+    std::vector<CopyItem> small;
+    if (out->nam_offsets) small.push_back({out->nam_offsets, b->ws->nam_off.p, 8ull * (n + 1)});
+    if (out->nonrepetitive_fraction && n) small.push_back({out->nonrepetitive_fraction, b->ws->frac.p, 4ull * n});
+    if (out->flags && n) small.push_back({out->flags, b->ws->flags.p, n});
+    if (!copy_small_to_host(small, st))
+        for (const CopyItem &c : small) copy_to_host(ctx, c.dst, c.src, c.bytes, st);
     if (b->ws->tot_nams) copy_to_host(ctx, out->nams, b->ws->nams_out.p, sizeof(gis_nam) * b->ws->tot_nams, st);
-    if (out->nonrepetitive_fraction) copy_to_host(ctx, out->nonrepetitive_fraction, b->ws->frac.p, 4ull * n, st);
-    if (out->flags) copy_to_host(ctx, out->flags, b->ws->flags.p, n, st);
     HIP_CHECK(hipStreamSynchronize(st));
     return GIS_OK;
 }

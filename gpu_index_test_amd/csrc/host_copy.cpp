@@ -22,19 +22,47 @@ constexpr int SLOTS = 8;
 // than half the link's rate
 constexpr int THREADS = 3;
 constexpr uint64_t THREADS_MIN = 4;
+// bytes of the arrays that one kernel writes beside a large copy
+constexpr uint64_t SMALL_MAX = 8 << 20;
 // arrays below this go the runtime's way, which copies them through its own pinned
 // memory
 constexpr size_t STAGE_MIN = 512 << 10;
 
 }  // namespace
 
-bool pinned_array(const void *p) {
-    hipPointerAttribute_t a{};
+// the attributes of memory that the runtime knows
+static bool known(const void *p, hipPointerAttribute_t &a) {
+    a = hipPointerAttribute_t{};
     if (hipPointerGetAttributes(&a, p) != hipSuccess) {
         (void)hipGetLastError();
         return false;
     }
     return a.type == hipMemoryTypeHost || a.type == hipMemoryTypeManaged || a.type == hipMemoryTypeDevice;
+}
+
+bool pinned_array(const void *p) {
+    hipPointerAttribute_t a;
+    return known(p, a);
+}
+
+bool copy_small_to_host(const std::vector<CopyItem> &items, hipStream_t st) {
+    CopyList l{};
+    uint64_t bytes = 0;
+    for (const CopyItem &c : items) {
+        hipPointerAttribute_t a;
+        if (l.n == CopyList::MAX || (bytes += c.bytes) > SMALL_MAX) return false;
+        if (!known(c.dst, a) || a.type != hipMemoryTypeHost || !a.devicePointer) return false;
+        if (((uintptr_t)a.devicePointer | (uintptr_t)c.src) % 16) return false;
+        l.src[l.n] = c.src;
+        l.dst[l.n] = a.devicePointer;
+        l.bytes[l.n] = (uint32_t)c.bytes;
+        l.block[l.n + 1] = l.block[l.n] + (uint32_t)((c.bytes + CopyList::BLOCK_BYTES - 1) / CopyList::BLOCK_BYTES);
+        l.n++;
+    }
+    if (l.n == 0) return true;
+    launch_copy_in(l, nullptr, st);
+    HIP_CHECK(hipGetLastError());
+    return true;
 }
 
 struct HostCopy {

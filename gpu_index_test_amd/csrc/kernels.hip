@@ -1279,9 +1279,6 @@ struct WideList {
     uint32_t near_cap;
 };
 
-// a wide list wholly in `p` (LDS or global)
-__device__ __forceinline__ WideList wide_in(WideNam *p) { return WideList{nullptr, p, 0}; }
-
 __device__ __forceinline__ WideNam wget(const WideList &L, uint32_t e) {
     WideNam w;
     if (e < L.near_cap) {

@@ -1,4 +1,6 @@
 """Edges of single kernels and dispatch branches, against the oracle, bit for bit."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -317,4 +319,33 @@ def test_launch_bursts(ctx, mode):
             assert mappers[i].download().nams.tobytes() == exp[i]
     for m in mappers:
         m.close()
+    idx.ctx.close()
+
+
+@pytest.mark.parametrize("at", [0, 16, 4096, 8, 1])
+def test_results_inside_pinned_arrays(ctx, at):
+    """Offsets, fractions and flags downloaded to places inside pinned arrays,
+    aligned and not, with nothing written beside them."""
+    g, lens = G.synth_genome(200_000, seed=3)
+    idx = G.StrobemerIndex(None, G.IndexParameters.from_read_length(150))
+    idx.populate_arrays(g, lens)
+    n = 5001
+    s, o, l, _ = G.synth_reads(g, lens, n, seed=4)
+    m = G.Mapper(idx, n, int(l.sum()))
+    m.upload(s, o, l)
+    m.run()
+    exp = m.download()
+    sizes = {"nam_offsets": 8 * (n + 1), "nonrepetitive_fraction": 4 * n, "flags": n,
+             "nams": len(exp.nams) * G.NAM.itemsize}
+    buf = {k: G.pinned_empty(at + b + 64, np.uint8) for k, b in sizes.items()}
+    for b in buf.values():
+        b[:] = 0xA5
+    out = G._native.NamOut(nam_capacity=len(exp.nams), **{k: b.ctypes.data + at for k, b in buf.items()})
+    idx.ctx.check(idx.ctx.L.gis_batch_download(m.h, ctypes.byref(out)))
+    want = {"nam_offsets": exp.nam_offsets, "nonrepetitive_fraction": exp.nonrepetitive_fraction, "flags": exp.flags,
+            "nams": exp.nams}
+    for k, b in buf.items():
+        assert b[at: at + sizes[k]].tobytes() == np.ascontiguousarray(want[k]).tobytes(), k
+        assert (b[:at] == 0xA5).all() and (b[at + sizes[k]:] == 0xA5).all(), k
+    m.close()
     idx.ctx.close()
