@@ -16,6 +16,7 @@
 #include <vector>
 
 #include "batch_internal.h"
+#include "host_copy.h"
 #include "pairs.h"
 
 using namespace gis;
@@ -137,24 +138,21 @@ static int pairs_download(gis_ctx *ctx, PairWork &w, hipStream_t st, gis_pair_ou
     if (out->joint && out->joint_capacity < w.n_joint)
         return fail(ctx, GIS_ERR_CAPACITY, "joint capacity " + std::to_string(out->joint_capacity) + " < " +
                                                std::to_string(w.n_joint));
-    if (out->nam_offsets)
-        HIP_CHECK(hipMemcpyAsync(out->nam_offsets, w.dev_off, 8ull * (2ull * n + 1), hipMemcpyDeviceToHost, st));
-    if (out->nams && w.n_nams)
-        HIP_CHECK(hipMemcpyAsync(out->nams, w.ord.p, sizeof(gis_nam) * w.n_nams, hipMemcpyDeviceToHost, st));
-    if (out->types && n) HIP_CHECK(hipMemcpyAsync(out->types, w.types.p, n, hipMemcpyDeviceToHost, st));
-    if (out->type_ids && n)
-        HIP_CHECK(hipMemcpyAsync(out->type_ids, w.tids.p, 4ull * n, hipMemcpyDeviceToHost, st));
-    if (out->top_dropoff && n)
-        HIP_CHECK(hipMemcpyAsync(out->top_dropoff, w.drop.p, 8ull * n, hipMemcpyDeviceToHost, st));
-    if (out->mapq && n) HIP_CHECK(hipMemcpyAsync(out->mapq, w.mapq.p, 2ull * n, hipMemcpyDeviceToHost, st));
-    if (out->joint_offsets) {
-        if (w.joint)
-            HIP_CHECK(hipMemcpyAsync(out->joint_offsets, w.joff.p, 8ull * (n + 1ull), hipMemcpyDeviceToHost, st));
-        else std::memset(out->joint_offsets, 0, 8ull * (n + 1ull));
-    }
-    if (out->joint && w.n_joint)
-        HIP_CHECK(hipMemcpyAsync(out->joint, w.jout.p, sizeof(gis_nam_pair) * w.n_joint, hipMemcpyDeviceToHost,
-                                 st));
+    std::vector<CopyItem> small;
+    auto add = [&](void *dst, const void *src, size_t bytes) {
+        if (dst && bytes) small.push_back({dst, src, bytes});
+    };
+    add(out->nam_offsets, w.dev_off, 8ull * (2ull * n + 1));
+    add(out->types, w.types.p, n);
+    add(out->type_ids, w.tids.p, 4ull * n);
+    add(out->top_dropoff, w.drop.p, 8ull * n);
+    add(out->mapq, w.mapq.p, 2ull * n);
+    if (w.joint) add(out->joint_offsets, w.joff.p, 8ull * (n + 1ull));
+    else if (out->joint_offsets) std::memset(out->joint_offsets, 0, 8ull * (n + 1ull));
+    add(out->joint, w.jout.p, sizeof(gis_nam_pair) * w.n_joint);
+    if (!copy_small_to_host(small, st))
+        for (const CopyItem &c : small) copy_to_host(ctx, c.dst, c.src, c.bytes, st);
+    if (out->nams && w.n_nams) copy_to_host(ctx, out->nams, w.ord.p, sizeof(gis_nam) * w.n_nams, st);
     HIP_CHECK(hipStreamSynchronize(st));
     return GIS_OK;
 }
