@@ -592,8 +592,9 @@ static void launch_part(gis_batch *b, const RunOpts &r) {
 // configurations, in two parts each at most.
 //
 // in_turn (a burst: runs launched on streams of their own onto an idle device, none
-// waited for yet): a large batch starts after the front of the one before it, that
-// is its seeding and lookup or its fused kernels. Launched together they would
+// waited for yet): a large plain batch starts after the front of the one before it,
+// its seeding and lookup (fused kernels are nearly the whole run: two batches of
+// 60,000 took 1463 us in turn and 1382 without). Launched together they would
 // share the device from their first kernel and end together, and the first one's
 // copies back could not run beside the others' kernels. (Three batches of 65,536
 // reads of 150 bp and their results: 1797 us, side by side 2046.) Later launches
@@ -627,7 +628,7 @@ void batch_launch(gis_batch *b, const RunOpts &r, bool in_turn) {
             it = b->graphs.erase(it);
         }
     }
-    if (!in_turn || b->n_reads < TURN_READS || st == ctx->stream) {
+    if (!in_turn || b->n_reads < TURN_READS || st == ctx->stream || r.mode == GIS_MODE_FUSED) {
         launch_part(b, r);
         return;
     }

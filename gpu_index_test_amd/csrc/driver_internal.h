@@ -126,6 +126,7 @@ struct gis_ctx {
     hipEvent_t turn_ev = nullptr;
     hipStream_t turn_st = nullptr;
     gis::HostCopy *host_copy = nullptr;  // pinned chunks of copies of pageable arrays (host_copy.h)
+    std::mutex host_copy_mu;             // held for a transfer through them
     // concurrent gis_find_nams_qrs calls waiting to be run together
     std::mutex comb_mu;
     std::condition_variable comb_cv;

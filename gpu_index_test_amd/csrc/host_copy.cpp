@@ -4,6 +4,8 @@
 #include <algorithm>
 #include <atomic>
 #include <cstring>
+#include <mutex>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -107,6 +109,7 @@ static HostCopy *hostcopy_get(gis_ctx *ctx) {
 // longer transfer on threads of its own.
 template <typename Issue, typename Finish>
 static void pipeline(gis_ctx *ctx, hipStream_t st, uint64_t chunks, Issue issue, Finish finish) {
+    std::lock_guard<std::mutex> lock(ctx->host_copy_mu);  // (serving threads copy without the context's lock)
     HostCopy *h = hostcopy_get(ctx);
     const int first = h->next;
     auto slot = [&](uint64_t c) { return (int)((first + c) % SLOTS); };

@@ -998,7 +998,9 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(6))) v
         const float frac = found > 0 ? (float)good / (float)found : 1.0f;
         const bool rescue = rescue_mode == 2 || (rescue_mode == 0 && ((double)frac < 0.7 || hits == 0));
         const bool pooled = !rescue && hits > 0 && (hits > HIT_REGION || !region_ok);
-        if (defer && (rescue || pooled)) {
+        // (a rescued read none of whose seeds is in the table has no hits either way)
+        const bool listed = rescue && found > 0;
+        if (defer && (listed || pooled)) {
             if (lane < n) {
                 b.pos[base + lane] = pos0;
                 b.hcnt[base + lane] = hc0;
@@ -1014,6 +1016,7 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(6))) v
                                    (n == 0 ? GIS_FLAG_NO_RANDSTROBES : 0));
             b.hit_total[r] = rescue ? 0u : hits;  // rescued reads discard these hits
             b.rhit_total[r] = 0;
+            b.rhit_off[r] = 0;
             // hits beyond the read's region: a place in the pool, and k_hits
             // writes them
             uint64_t off = (uint64_t)r * HIT_REGION;
@@ -1022,7 +1025,10 @@ __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(6))) v
                 b.sel_ids[2ull * b.n_reads + atomicAdd(&b.ctl->n_sel[SEL_POOLED], 1u)] = r;
             }
             b.hit_off[r] = off;
-            if (rescue) b.sel_ids[atomicAdd(&b.ctl->n_sel[SEL_RESCUED], 1u)] = r;
+            // (one counter takes an append every ~7 ns: 12 000 reads too short for
+            // any seed, a third of 36 617 of 50 to 101 bp, took 90 us here and 90
+            // more in k_hits)
+            if (listed) b.sel_ids[atomicAdd(&b.ctl->n_sel[SEL_RESCUED], 1u)] = r;
         }
     }
 }
@@ -1126,6 +1132,7 @@ __device__ __forceinline__ void rescued_hits(const DevBatch &b, const DevIndex &
         if (i < n) b.rcnt[base + i] = rh;
         total += wave_sum_dpp(rh);
     }
+    if (total == 0) return;  // (k_lookup has written that)
     unsigned long long off = 0;
     if (lane == 0) {
         off = atomicAdd(&b.ctl->rhit_pool, (unsigned long long)total);
@@ -1137,7 +1144,6 @@ __device__ __forceinline__ void rescued_hits(const DevBatch &b, const DevIndex &
         if (lane == 0) atomicOr(&b.ctl->overflow, OVF_RHITS);
         return;
     }
-    if (total == 0) return;
     wave_sync_mem();
     DevHit *out = b.rhits + off;
     uint32_t carry = 0;
