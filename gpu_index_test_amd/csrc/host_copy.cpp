@@ -1,6 +1,9 @@
 // Copies between HBM and a caller's arrays (host_copy.h).
 #include "host_copy.h"
 
+#include <hsa/hsa.h>
+#include <hsa/hsa_ext_amd.h>
+
 #include <algorithm>
 #include <atomic>
 #include <cstring>
@@ -32,9 +35,8 @@ constexpr size_t STAGE_MIN = 512 << 10;
 
 }  // namespace
 
-// the attributes of memory that the runtime knows
-static bool known(const void *p, hipPointerAttribute_t &a) {
-    a = hipPointerAttribute_t{};
+bool pinned_array(const void *p) {
+    hipPointerAttribute_t a{};
     if (hipPointerGetAttributes(&a, p) != hipSuccess) {
         (void)hipGetLastError();
         return false;
@@ -42,21 +44,27 @@ static bool known(const void *p, hipPointerAttribute_t &a) {
     return a.type == hipMemoryTypeHost || a.type == hipMemoryTypeManaged || a.type == hipMemoryTypeDevice;
 }
 
-bool pinned_array(const void *p) {
-    hipPointerAttribute_t a;
-    return known(p, a);
+bool pinned_range(const void *p, size_t bytes) {
+    hsa_amd_pointer_info_t info{};
+    info.size = sizeof(info);
+    if (hsa_amd_pointer_info(p, &info, nullptr, nullptr, nullptr) != HSA_STATUS_SUCCESS) return false;
+    if (info.type != HSA_EXT_POINTER_TYPE_HSA || !info.hostBaseAddress ||
+        info.agentBaseAddress != info.hostBaseAddress)
+        return false;
+    const char *base = static_cast<const char *>(info.hostBaseAddress), *q = static_cast<const char *>(p);
+    return q >= base && bytes <= info.sizeInBytes && (size_t)(q - base) <= info.sizeInBytes - bytes;
 }
 
 bool copy_small_to_host(const std::vector<CopyItem> &items, hipStream_t st) {
     CopyList l{};
     uint64_t bytes = 0;
     for (const CopyItem &c : items) {
-        hipPointerAttribute_t a;
         if (l.n == CopyList::MAX || (bytes += c.bytes) > SMALL_MAX) return false;
-        if (!known(c.dst, a) || a.type != hipMemoryTypeHost || !a.devicePointer) return false;
-        if (((uintptr_t)a.devicePointer | (uintptr_t)c.src) % 16) return false;
+        // (the kernel writes all of it: a first byte that is pinned is not enough)
+        if (!pinned_range(c.dst, c.bytes)) return false;
+        if (((uintptr_t)c.dst | (uintptr_t)c.src) % 16) return false;
         l.src[l.n] = c.src;
-        l.dst[l.n] = a.devicePointer;
+        l.dst[l.n] = c.dst;
         l.bytes[l.n] = (uint32_t)c.bytes;
         l.block[l.n + 1] = l.block[l.n] + (uint32_t)((c.bytes + CopyList::BLOCK_BYTES - 1) / CopyList::BLOCK_BYTES);
         l.n++;

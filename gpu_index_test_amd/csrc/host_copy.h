@@ -21,8 +21,8 @@ void hostcopy_free(HostCopy *h);
 void copy_to_host(gis_ctx *ctx, void *dst, const void *src, size_t n, hipStream_t st);
 
 // Several arrays of some KB or MB to pinned arrays by one kernel, where a copy each
-// takes ~15 us beside its bytes' time: true if all are pinned and aligned for it,
-// else nothing is done. (Offsets, fractions and flags of 65,536 reads beside their
+// takes ~15 us beside its bytes' time: true if all are pinned to their last byte and
+// aligned for it, else nothing is done. (Offsets, fractions and flags of 65,536 reads beside their
 // NAMs: 25 us, with a copy each 48.)
 bool copy_small_to_host(const std::vector<CopyItem> &items, hipStream_t st);
 
@@ -31,6 +31,11 @@ bool copy_small_to_host(const std::vector<CopyItem> &items, hipStream_t st);
 // filled and emptied on the host (10^6 keys: 790 us with a copy each way, now 440)
 void lookup_through_host(gis_ctx *ctx, const uint64_t *keys, uint64_t n, uint64_t *positions, hipStream_t st);
 
+// p points at memory that the runtime knows: its own copies take such arrays
 bool pinned_array(const void *p);
+
+// [p, p + bytes) lies in one pinned allocation (hipHostMalloc) that the GPU reaches
+// at the same address: a copy engine or a kernel may read or write all of it
+bool pinned_range(const void *p, size_t bytes);
 
 }  // namespace gis

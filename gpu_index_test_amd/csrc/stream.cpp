@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "batch_internal.h"
+#include "host_copy.h"
 
 namespace gis {
 
@@ -117,19 +118,6 @@ DmaEngines *dma_setup(int device) {
     return E;
 }
 
-// [p, p + bytes) lies in one allocation that the GPU reaches at the same
-// address (pinned memory from hipHostMalloc), so an engine can copy it.
-bool engine_reachable(const void *p, size_t bytes) {
-    hsa_amd_pointer_info_t info{};
-    info.size = sizeof(info);
-    if (hsa_amd_pointer_info(p, &info, nullptr, nullptr, nullptr) != HSA_STATUS_SUCCESS) return false;
-    if (info.type != HSA_EXT_POINTER_TYPE_HSA || !info.hostBaseAddress ||
-        info.agentBaseAddress != info.hostBaseAddress)
-        return false;
-    const char *base = static_cast<const char *>(info.hostBaseAddress), *q = static_cast<const char *>(p);
-    return q >= base && bytes <= info.sizeInBytes && (size_t)(q - base) <= info.sizeInBytes - bytes;
-}
-
 // Runs `items`, all in one direction. Those whose host side an engine can
 // reach go to that direction's engine and are waited for on `sig`; the
 // others are enqueued through HIP on `st` (host-to-device copies then
@@ -140,7 +128,7 @@ void run_copies(DmaEngines *E, bool to_device, const std::vector<CopyItem> &item
     std::vector<const CopyItem *> eng, hip;
     for (const CopyItem &c : items) {
         if (!c.bytes) continue;
-        const bool reach = have_sig && E->ok.load() && engine_reachable(to_device ? c.src : c.dst, c.bytes);
+        const bool reach = have_sig && E->ok.load() && pinned_range(to_device ? c.src : c.dst, c.bytes);
         (reach ? eng : hip).push_back(&c);
     }
     size_t issued = 0;
