@@ -225,7 +225,12 @@ void lane_main(StreamJob &J, gis_batch *b, uint32_t lane, uint32_t lanes) {
             if (i < lanes) {
                 std::unique_lock<std::mutex> lk(J.m);
                 J.cv.wait(lk, [&] { return J.failed || J.ran == i; });
-                if (J.failed) break;
+                if (J.failed) {
+                    lk.unlock();
+                    // copies through HIP still read the caller's arrays
+                    HIP_CHECK(hipStreamSynchronize(st));
+                    break;
+                }
             }
             batch_launch(b, r);
             batch_complete(b, r);  // regrowth reruns included
