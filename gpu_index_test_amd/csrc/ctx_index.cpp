@@ -29,27 +29,66 @@ void build_lines(gis_ctx *ctx) {
     HIP_CHECK(hipStreamSynchronize(ctx->stream));
 }
 
+// Loads a table in place of the resident one: load(keep) fills ix and returns false
+// if it refuses the table. The memory of the table before, and of a build before,
+// serves the load where it can, but must not be why one fails: a load that runs out
+// of memory starts again with all of that given back, and keeps none (keep false).
+// A load that fails for good leaves nothing behind.
+template <typename F>
+bool load_table(gis_ctx *ctx, F load) {
+    DevIndexStore &ix = ctx->ix;
+    drop_table(ix);
+    for (bool keep = true;; keep = false) {
+        HipError err{hipSuccess, ""};
+        bool ok = false;
+        struct Undo {
+            gis_ctx *ctx;
+            const bool &ok;
+            ~Undo() {
+                if (ok) return;
+                (void)hipStreamSynchronize(ctx->stream);
+                release_table(ctx->ix);
+                release(ctx->build_mem);
+            }
+        };
+        try {
+            Undo undo{ctx, ok};
+            if (!load(keep)) return false;
+            build_lines(ctx);
+            ok = true;
+        } catch (const HipError &e) {
+            err = e;
+        } catch (const BuildError &e) {
+            err = HipError{e.e, e.what};
+        }
+        if (ok) break;
+        if (err.e != hipErrorOutOfMemory || !keep) throw err;
+        (void)hipGetLastError();
+    }
+    ix.loaded = true;
+    return true;
+}
+
 void upload_index(gis_ctx *ctx, const HostIndex &h) {
     DevIndexStore &ix = ctx->ix;
-    // drop the previous table first so two tables never coexist in HBM
-    drop_table(ix);
-    table_room<gis_ref_randstrobe>(ix.rs, h.rs.size());
-    table_room<uint64_t>(ix.starts, h.starts.size());
-    if (!h.rs.empty())
-        HIP_CHECK(hipMemcpy(ix.rs.p, h.rs.data(), h.rs.size() * sizeof(gis_ref_randstrobe),
-                            hipMemcpyHostToDevice));
-    HIP_CHECK(hipMemcpy(ix.starts.p, h.starts.data(), h.starts.size() * 8, hipMemcpyHostToDevice));
-    ix.n = h.rs.size();
-    ix.bits = h.bits;
-    ix.filter_cutoff = h.filter_cutoff;
-    ix.params = h.params;
-    ix.distinct = h.distinct_strobemers;
-    ix.once = h.tot_occur_once;
-    ix.high = h.tot_high_ab;
-    ix.mid = h.tot_mid_ab;
-    ix.index_cutoff = h.index_cutoff;
-    build_lines(ctx);
-    ix.loaded = true;
+    load_table(ctx, [&](bool) {
+        table_room<gis_ref_randstrobe>(ix.rs, h.rs.size());
+        table_room<uint64_t>(ix.starts, h.starts.size());
+        if (!h.rs.empty())
+            HIP_CHECK(hipMemcpy(ix.rs.p, h.rs.data(), h.rs.size() * sizeof(gis_ref_randstrobe),
+                                hipMemcpyHostToDevice));
+        HIP_CHECK(hipMemcpy(ix.starts.p, h.starts.data(), h.starts.size() * 8, hipMemcpyHostToDevice));
+        ix.n = h.rs.size();
+        ix.bits = h.bits;
+        ix.filter_cutoff = h.filter_cutoff;
+        ix.params = h.params;
+        ix.distinct = h.distinct_strobemers;
+        ix.once = h.tot_occur_once;
+        ix.high = h.tot_high_ab;
+        ix.mid = h.tot_mid_ab;
+        ix.index_cutoff = h.index_cutoff;
+        return true;
+    });
 }
 
 void download_index(gis_ctx *ctx, HostIndex &h) {
@@ -150,41 +189,37 @@ extern "C" int gis_index_build(gis_ctx *ctx, const char *const *seqs, const uint
     if (bits == -1) bits = pick_bits(total, *params);
     if (bits < 8 || bits > 31) return fail(ctx, GIS_ERR_BAD_PARAMETER, "Bits must be between 8 and 31");
     DevIndexStore &ix = ctx->ix;
-    drop_table(ix);
-    uint64_t n = 0;
-    uint64_t hist[RUN_BINS] = {};
-    for (bool again = ix.rs.p != nullptr;; again = false) {
-        try {
-            BuildArena arena(build_estimate(total, *params), ctx->build_mem.p, ctx->build_mem.bytes);
+    load_table(ctx, [&](bool keep) {
+        uint64_t hist[RUN_BINS] = {};
+        uint64_t n = 0;
+        DevBuf once;  // the build's memory if it is not to stay
+        DevBuf &mem = keep ? ctx->build_mem : once;
+        struct Release {
+            DevBuf &b;
+            ~Release() { release(b); }
+        } release_once{once};
+        {
+            BuildArena arena(build_estimate(total, *params), mem.p, mem.bytes);
             const RefSeeds seeds = device_seed_reference(seqs, lens, n_refs, *params, true, arena, ctx->stream);
             n = seeds.n;
             uint4 *rs = table_room<uint4>(ix.rs, n);
             table_room<uint64_t>(ix.starts, (1ull << bits) + 1);
             device_sort_records(seeds, rs, arena, ctx->stream);
             device_finish_index(rs, n, bits, static_cast<uint64_t *>(ix.starts.p), hist, arena, ctx->stream);
-            break;
-        } catch (const BuildError &e) {
-            (void)hipStreamSynchronize(ctx->stream);
-            if (e.e != hipErrorOutOfMemory || !again) throw HipError{e.e, e.what};
-            // once more, without the previous table's memory
-            (void)hipGetLastError();
-            release_table(ix);
-            release(ctx->build_mem);
         }
-    }
-    HostIndex st;
-    filter_stats(hist, f, st);
-    ix.n = n;
-    ix.bits = bits;
-    ix.filter_cutoff = st.filter_cutoff;
-    ix.params = *params;
-    ix.distinct = st.distinct_strobemers;
-    ix.once = st.tot_occur_once;
-    ix.high = st.tot_high_ab;
-    ix.mid = st.tot_mid_ab;
-    ix.index_cutoff = st.index_cutoff;
-    build_lines(ctx);
-    ix.loaded = true;
+        HostIndex st;
+        filter_stats(hist, f, st);
+        ix.n = n;
+        ix.bits = bits;
+        ix.filter_cutoff = st.filter_cutoff;
+        ix.params = *params;
+        ix.distinct = st.distinct_strobemers;
+        ix.once = st.tot_occur_once;
+        ix.high = st.tot_high_ab;
+        ix.mid = st.tot_mid_ab;
+        ix.index_cutoff = st.index_cutoff;
+        return true;
+    });
     return GIS_OK;
     API_END(ctx)
 }
@@ -251,43 +286,35 @@ extern "C" int gis_index_read_sti(gis_ctx *ctx, const char *path, const gis_para
     std::string err;
     const int rc = map_sti(path, expected, m, err);
     if (rc) return fail(ctx, rc, err);
+    const char *why = nullptr;
     try {
         DevIndexStore &ix = ctx->ix;
-        drop_table(ix);
-        table_room<gis_ref_randstrobe>(ix.rs, m.n);
-        table_room<uint64_t>(ix.starts, (1ull << m.bits) + 1);
-        const uint64_t chunk = 256ull << 20;
-        const char *src = reinterpret_cast<const char *>(m.rs);
-        char *dst = static_cast<char *>(ix.rs.p);
-        for (uint64_t o = 0, tot = m.n * sizeof(gis_ref_randstrobe); o < tot; o += chunk)
-            HIP_CHECK(hipMemcpy(dst + o, src + o, std::min(chunk, tot - o), hipMemcpyHostToDevice));
-        HIP_CHECK(hipMemcpy(ix.starts.p, m.starts, ((1ull << m.bits) + 1) * 8, hipMemcpyHostToDevice));
-        // the file's table must be one the lookups can trust
-        const char *why = nullptr;
-        try {
+        load_table(ctx, [&](bool) {
+            table_room<gis_ref_randstrobe>(ix.rs, m.n);
+            table_room<uint64_t>(ix.starts, (1ull << m.bits) + 1);
+            const uint64_t chunk = 256ull << 20;
+            const char *src = reinterpret_cast<const char *>(m.rs);
+            char *dst = static_cast<char *>(ix.rs.p);
+            for (uint64_t o = 0, tot = m.n * sizeof(gis_ref_randstrobe); o < tot; o += chunk)
+                HIP_CHECK(hipMemcpy(dst + o, src + o, std::min(chunk, tot - o), hipMemcpyHostToDevice));
+            HIP_CHECK(hipMemcpy(ix.starts.p, m.starts, ((1ull << m.bits) + 1) * 8, hipMemcpyHostToDevice));
+            // the file's table must be one the lookups can trust
             why = device_validate_index(static_cast<const uint4 *>(ix.rs.p), m.n,
                                         static_cast<const uint64_t *>(ix.starts.p), m.bits, ctx->stream);
-        } catch (const BuildError &e) {
-            throw HipError{e.e, e.what};
-        }
-        if (why) {
-            drop_table(ix);
-            release_table(ix);
-            unmap_sti(m);
-            return fail(ctx, GIS_ERR_INVALID_INDEX, std::string("Index file has incorrect format: ") + why);
-        }
-        ix.n = m.n;
-        ix.bits = m.bits;
-        ix.filter_cutoff = m.filter_cutoff;
-        ix.params = m.params;
-        ix.distinct = ix.once = ix.high = ix.mid = ix.index_cutoff = 0;
-        build_lines(ctx);
-        ix.loaded = true;
+            if (why) return false;
+            ix.n = m.n;
+            ix.bits = m.bits;
+            ix.filter_cutoff = m.filter_cutoff;
+            ix.params = m.params;
+            ix.distinct = ix.once = ix.high = ix.mid = ix.index_cutoff = 0;
+            return true;
+        });
     } catch (...) {
         unmap_sti(m);
         throw;
     }
     unmap_sti(m);
+    if (why) return fail(ctx, GIS_ERR_INVALID_INDEX, std::string("Index file has incorrect format: ") + why);
     return GIS_OK;
     API_END(ctx)
 }

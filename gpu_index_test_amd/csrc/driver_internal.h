@@ -77,12 +77,13 @@ inline void drop_table(DevIndexStore &ix) {
 }
 
 // room for n elements of a table: the memory of the one before, unless that is too
-// small or more than twice as large (an allocation and its release cost ~180 us
-// together, three of them a fifth of a bacterial index's build)
+// small or larger by more than TABLE_SURPLUS (an allocation and its release cost
+// ~180 us together, three of them a fifth of a bacterial index's build)
+constexpr size_t TABLE_SURPLUS = 64u << 20;
 template <typename T>
 T *table_room(DevBuf &b, size_t n) {
     const size_t need = std::max<size_t>(n, 1) * sizeof(T);
-    if (b.bytes < need || b.bytes / 2 > need) release(b);
+    if (b.bytes < need || b.bytes - need > TABLE_SURPLUS) release(b);
     return ensure<T>(b, n);
 }
 

@@ -47,6 +47,9 @@ F real(const char *name) {
 
 std::mutex g_mu;
 bool g_no_room = false;                    // hipMalloc fails, and says so late
+uint64_t g_limit = UINT64_MAX;             // device bytes there are to allocate
+uint64_t g_live = 0, g_peak = 0;           // allocated now, and at most
+std::map<void *, uint64_t> g_blocks;
 std::map<void *, uint64_t> g_copy, g_sync;  // streams: when last copied in on, when last waited for
 uint64_t g_clock = 0;
 
@@ -54,15 +57,33 @@ uint64_t g_clock = 0;
 
 extern "C" int hipMalloc(void **p, size_t n) {
     static const auto f = real<int (*)(void **, size_t)>("hipMalloc");
-    bool fail;
+    std::unique_lock<std::mutex> l(g_mu);
+    if (g_no_room || g_limit - std::min(g_limit, g_live) < n) {
+        const bool late = g_no_room;
+        l.unlock();
+        if (late) std::this_thread::sleep_for(std::chrono::milliseconds(300));
+        *p = nullptr;
+        return 2;
+    }
+    const int e = f(p, n);
+    if (e) return e;
+    g_blocks[*p] = n;
+    g_live += n;
+    g_peak = std::max(g_peak, g_live);
+    return e;
+}
+
+extern "C" int hipFree(void *p) {
+    static const auto f = real<int (*)(void *)>("hipFree");
     {
         std::lock_guard<std::mutex> l(g_mu);
-        fail = g_no_room;
+        const auto b = g_blocks.find(p);
+        if (b != g_blocks.end()) {
+            g_live -= b->second;
+            g_blocks.erase(b);
+        }
     }
-    if (!fail) return f(p, n);
-    std::this_thread::sleep_for(std::chrono::milliseconds(300));
-    *p = nullptr;
-    return 2;
+    return f(p);
 }
 
 extern "C" int hipMemcpyAsync(void *d, const void *s, size_t n, int kind, void *st) {
@@ -209,11 +230,88 @@ static void stream_failure() {
     gis_ctx_destroy(ctx);
 }
 
+// A table that fits an empty device fits one that holds another: replacing it takes
+// no more memory than loading it first does, whatever was kept of the one before.
+// A load that cannot fit leaves nothing allocated, and the next one works.
+static void replace_index() {
+    const Genome small = genome(300000, 2, 5), large = genome(3000000, 2, 6);
+    const std::string path = std::string(std::getenv("TMPDIR") ? std::getenv("TMPDIR") : "/tmp") + "/host_check_" +
+                             std::to_string((long)std::chrono::steady_clock::now().time_since_epoch().count()) + ".sti";
+    const int BITS = 18, BITS_BEFORE = 22;
+    // the table three ways
+    std::vector<gis_ref_randstrobe> rs;
+    std::vector<uint64_t> starts((1ull << BITS) + 1);
+    gis_index_info want{};
+    {
+        gis_ctx *ctx = context();
+        EXPECT(build(ctx, large, BITS) == GIS_OK && gis_index_info_get(ctx, &want) == GIS_OK);
+        rs.resize(want.n_randstrobes);
+        EXPECT(gis_index_download(ctx, rs.data(), starts.data()) == GIS_OK);
+        EXPECT(gis_index_write_sti(ctx, path.c_str()) == GIS_OK);
+        gis_ctx_destroy(ctx);
+    }
+    const auto load = [&](gis_ctx *ctx, int how) {
+        if (how == 0) return build(ctx, large, BITS);
+        if (how == 1)
+            return gis_index_upload(ctx, rs.data(), rs.size(), starts.data(), BITS, want.filter_cutoff, &want.params);
+        return gis_index_read_sti(ctx, path.c_str(), nullptr);
+    };
+    const auto same = [&](gis_ctx *ctx) {
+        std::vector<gis_ref_randstrobe> r(rs.size());
+        std::vector<uint64_t> s(starts.size());
+        gis_index_info i{};
+        EXPECT(gis_index_info_get(ctx, &i) == GIS_OK && i.n_randstrobes == rs.size() && i.bits == BITS);
+        EXPECT(gis_index_download(ctx, r.data(), s.data()) == GIS_OK);
+        EXPECT(!std::memcmp(r.data(), rs.data(), rs.size() * sizeof rs[0]) && s == starts);
+    };
+    for (int how = 0; how < 3; how++) {
+        const uint64_t none = g_live;
+        gis_ctx *ctx = context();
+        g_peak = g_live;
+        EXPECT(load(ctx, how) == GIS_OK);
+        const uint64_t alone = g_peak;
+        gis_ctx_destroy(ctx);
+        EXPECT(g_live == none);
+        for (int before = 0; before < 2; before++) {  // many buckets; many records
+            ctx = context();
+            EXPECT((before ? build(ctx, large, BITS - 2) : build(ctx, small, BITS_BEFORE)) == GIS_OK);
+            g_limit = alone;
+            EXPECT(load(ctx, how) == GIS_OK);
+            same(ctx);
+            EXPECT(g_live <= alone);
+            // too little for more buckets, and then for any load
+            g_limit = none + (1 << 20);
+            EXPECT(build(ctx, large, BITS_BEFORE + 1) == GIS_ERR_HIP);
+            EXPECT(g_live == none);
+            EXPECT(load(ctx, how) == GIS_ERR_HIP);
+            EXPECT(g_live == none);
+            EXPECT(gis_index_info_get(ctx, &want) == GIS_ERR_STATE);
+            g_limit = UINT64_MAX;
+            EXPECT(load(ctx, how) == GIS_OK);
+            same(ctx);
+            gis_ctx_destroy(ctx);
+            EXPECT(g_live == none);
+        }
+    }
+    // a build whose own memory stays with the context when there is room, and goes
+    // before the bucket lines (here most of the table) need it
+    const uint64_t none = g_live;
+    gis_ctx *ctx = context();
+    EXPECT(build(ctx, small, BITS_BEFORE) == GIS_OK && gis_index_info_get(ctx, &want) == GIS_OK);
+    gis_ctx_destroy(ctx);
+    ctx = context();
+    g_limit = none + want.n_randstrobes * 16 + ((1ull << BITS_BEFORE) + 1) * 8 + (128ull << BITS_BEFORE) + (1 << 20);
+    EXPECT(build(ctx, small, BITS_BEFORE) == GIS_OK);
+    gis_ctx_destroy(ctx);
+    g_limit = UINT64_MAX;
+    std::remove(path.c_str());
+}
+
 int main(int argc, char **argv) {
     const struct {
         const char *name;
         void (*run)();
-    } cases[] = {{"pinned_ranges", pinned_ranges}, {"stream_failure", stream_failure}};
+    } cases[] = {{"pinned_ranges", pinned_ranges}, {"stream_failure", stream_failure}, {"replace_index", replace_index}};
     for (const auto &c : cases)
         if (argc == 2 && !std::strcmp(argv[1], c.name)) {
             c.run();
