@@ -380,7 +380,9 @@ extern "C" int gis_index_info_get(gis_ctx *ctx, gis_index_info *out) {
     out->tot_high_ab = ix.high;
     out->tot_mid_ab = ix.mid;
     out->index_cutoff = ix.index_cutoff;
-    out->device_bytes = ix.rs.bytes + ix.starts.bytes + ix.lines.bytes;
+    // (the table's; the arrays may be those of a larger one before it)
+    out->device_bytes = std::max<uint64_t>(ix.n, 1) * sizeof(gis_ref_randstrobe) + ((1ull << ix.bits) + 1) * 8 +
+                        ((uint64_t)BUCKET_LINE * sizeof(uint4) << ix.bits);
     return GIS_OK;
     API_END(ctx)
 }

@@ -307,11 +307,24 @@ static void replace_index() {
     std::remove(path.c_str());
 }
 
+// an index's device bytes are those of its table, whatever was resident before it
+static void index_bytes() {
+    const Genome small = genome(100000, 1, 7), large = genome(1000000, 1, 8);
+    gis_ctx *ctx = context();
+    EXPECT(build(ctx, large, 14) == GIS_OK);
+    for (int bits : {14, 13, 16}) {
+        gis_index_info i{};
+        EXPECT(build(ctx, small, bits) == GIS_OK && gis_index_info_get(ctx, &i) == GIS_OK);
+        EXPECT(i.device_bytes == i.n_randstrobes * 16 + ((1ull << bits) + 1) * 8 + (128ull << bits));
+    }
+    gis_ctx_destroy(ctx);
+}
+
 int main(int argc, char **argv) {
     const struct {
         const char *name;
         void (*run)();
-    } cases[] = {{"pinned_ranges", pinned_ranges}, {"stream_failure", stream_failure}, {"replace_index", replace_index}};
+    } cases[] = {{"pinned_ranges", pinned_ranges}, {"stream_failure", stream_failure}, {"replace_index", replace_index}, {"index_bytes", index_bytes}};
     for (const auto &c : cases)
         if (argc == 2 && !std::strcmp(argv[1], c.name)) {
             c.run();
