@@ -700,16 +700,24 @@ __global__ __launch_bounds__(64 * JOINT_WPB) void k_joint_wave(PairDev P, uint32
         uint32_t size = 0;
         int best = 0;
         const uint64_t cells = (uint64_t)c1 * c2;
-        // this lane's cell, 64 further on each pass
-        uint32_t i = lane / c2, j = lane % c2;
+        // this lane's cell, 64 further on each pass, or, after a row that was left, at
+        // the next row whose first cell does not fail: in lists of hundreds of NAMs
+        // most cells are never reached. (A pair of 1000 x 1000 whose rows end at
+        // their first cell: 10.3 ms with a step for every 64 cells of a row left,
+        // 0.53 ms a row at a time, now 0.09 ms.)
+        const uint32_t i_row = lane / c2, j_row = lane % c2;
+        uint32_t i = i_row, j = j_row;
         const uint32_t di = 64 / c2, dj = 64 % c2;
         uint32_t dead = 0xffffffffu;  // the row left last
-        for (uint64_t q0 = 0; q0 < cells && size < most; q0 += 64) {
+        uint32_t rows = 0;  // lane l's nh_row: the hits of row rows + l
+        int nh_row = nh1;
+        for (uint64_t q0 = 0; q0 < cells && size < most;) {
             const bool valid = lane < cells - q0;
             bool prop = false;
             int joint = 0;
             if (valid) {
-                const CellNam a = in_lds ? ca[i] : cell_nam(A[i]), b = in_lds ? cb[j] : cell_nam(B[j]);
+                const CellNam a = in_lds || i < 64 ? ca[i] : cell_nam(A[i]);
+                const CellNam b = in_lds || j < 64 ? cb[j] : cell_nam(B[j]);
                 joint = a.nh + b.nh;
                 prop = proper_cell(a, b, lim);
             }
@@ -746,6 +754,25 @@ __global__ __launch_bounds__(64 * JOINT_WPB) void k_joint_wave(PairDev P, uint32
                 }
                 dead = readlane_u32(i, (uint32_t)__builtin_ctzll(drop));
                 rem &= ballot(i > dead);
+            }
+            q0 += 64;
+            uint32_t row = dead + 1u;  // (0: no row was left yet)
+            if (q0 < (uint64_t)row * c2) {
+                const int first = __builtin_amdgcn_readfirstlane(nh2);
+                while (row < c1) {
+                    if (row >= rows + 64) {
+                        rows = row;
+                        nh_row = A[min(row + lane, c1 - 1)].n_hits;
+                    }
+                    const uint64_t on = ballot(rows + lane >= c1 || 2 * (nh_row + first) >= best) >> (row - rows);
+                    row = on ? row + (uint32_t)__builtin_ctzll(on) : rows + 64;
+                    if (on) break;
+                }
+                dead = row - 1;
+                q0 = (uint64_t)row * c2;
+                i = row + i_row;
+                j = j_row;
+                continue;
             }
             i += di;
             j += dj;

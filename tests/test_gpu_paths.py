@@ -1,5 +1,6 @@
 """Edges of single kernels and dispatch branches, against the oracle, bit for bit."""
 import ctypes
+import time
 
 import numpy as np
 import pytest
@@ -349,3 +350,57 @@ def test_results_inside_pinned_arrays(ctx, at):
         assert (b[:at] == 0xA5).all() and (b[at + sizes[k]:] == 0xA5).all(), k
     m.close()
     idx.ctx.close()
+
+
+def _long_mates(rng, c1, c2, hits1, hits2, ref=0):
+    """Two lists on one contig, opposite strands, diagonals inside the insert limit
+    or far apart, in any order."""
+    out = []
+    for n, hits, rc, off in ((c1, hits1, 0, 0), (c2, hits2, 1, 300)):
+        x = np.zeros(n, dtype=O.NAM)
+        i = np.arange(n)
+        x["nam_id"], x["query_start"], x["query_end"] = i, i % 50, 100 + i % 50
+        x["ref_start"] = 1000 + rng.integers(0, 3, n) * 100_000 + 40 * i + off
+        x["ref_end"], x["n_hits"], x["score"] = x["ref_start"] + 100, hits, 10.0 * hits
+        x["ref_id"], x["is_rc"] = ref, rc
+        out.append(x[rng.permutation(n)])
+    return out
+
+
+@pytest.mark.parametrize("max_tries", [1, 20, 31])
+@pytest.mark.parametrize("c1,c2", [(1, 200), (200, 1), (63, 64), (64, 65), (65, 63), (70, 70), (130, 129), (300, 90), (90, 700)])
+def test_joint_rows_left_at_any_cell(ctx, c1, c2, max_tries):
+    """The joint scan leaves a row at the first cell whose hits fall below half the
+    best: at its first cell, inside a pass of 64 cells, at its ends, or never."""
+    rng = np.random.default_rng(1000 * c1 + c2)
+    m1, m2 = [], []
+    for kind in range(12):
+        h1, h2 = rng.integers(1, 6, c1), rng.integers(1, 6, c2)
+        if kind % 4 == 1:  # a few rows above the others
+            h1[rng.integers(0, c1, 1 + c1 // 30)] = 200
+            h2[rng.integers(0, c2, 1 + c2 // 2)] = 150
+        elif kind % 4 == 2:  # a best that ends most rows at once, or at a column
+            h1[0], h2[: 1 + int(rng.integers(0, c2))] = 300, 100
+        elif kind % 4 == 3:
+            h1, h2 = rng.integers(1, 400, c1), rng.integers(1, 400, c2)
+        a, b = _long_mates(rng, c1, c2, h1, h2)
+        m1.append(a)
+        m2.append(b)
+    offs, flat = _flatten(m1 + m2)
+    _compare(G.pairs_from_nams(ctx, offs, flat, 12, max_tries=max_tries),
+             O.pairs_batch(offs, flat, 12, max_tries=max_tries), offs)
+
+
+def test_joint_time_of_rows_left(ctx):
+    """A pair of 1000 x 1000 NAMs whose rows end at their first cell: 0.1 ms beside
+    the other steps, where visiting every cell of the rows left took 10 ms."""
+    rng = np.random.default_rng(3)
+    h1, h2 = np.ones(1000, int), np.ones(1000, int)
+    h1[0], h2[:] = 300, 100
+    offs, flat = _flatten(_long_mates(rng, 1000, 1000, h1, h2))
+    best = {}
+    for joint in (True, False) * 4:
+        t = time.perf_counter()
+        G.pairs_from_nams(ctx, offs, flat, 1, joint=joint)
+        best[joint] = min(best.get(joint, 1.0), time.perf_counter() - t)
+    assert best[True] - best[False] < 3e-3, best
