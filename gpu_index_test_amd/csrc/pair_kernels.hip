@@ -4,14 +4,14 @@
 //                 position in the reference order is the number of NAMs of the
 //                 list with a smaller key, counted against the other lanes of
 //                 the row, two NAMs a lane for lists of 17 to 32 (one list in
-//                 eight). A longer list has the whole wave (up to 64:
-//                 against the other lanes; beyond: against 64-key tiles in
-//                 LDS). Keys are unique (each NAM's (is_rc, ref_id,
+//                 eight). Keys are unique (each NAM's (is_rc, ref_id,
 //                 query_start, ref_start) is its own first hit), so counting
 //                 ranks gives the one sorted order the reference's quicksort
-//                 reaches. Lists in canonical order are grouped by (is_rc,
-//                 ref_id), so a 64-NAM chunk only counts against the groups it
-//                 spans.
+//                 reaches.
+//  k_pair_order_long  longer lists, a wave each (up to 64: against the other
+//                 lanes; beyond: against 64-key tiles in LDS). Lists in
+//                 canonical order are grouped by (is_rc, ref_id), so a 64-NAM
+//                 chunk only counts against the groups it spans.
 //  k_pair_type    one lane per pair: type, top_dropoff, MAPQ, per-block type
 //                 counts.
 //  k_type_scatter pair ids grouped by type in id order (the host loop of
@@ -114,7 +114,7 @@ __device__ __forceinline__ void rank_rows(const NamKey &k0, const NamKey &k1, ui
 constexpr int ORDER_WPB = 4;
 
 // a list of more than 32 NAMs, by the whole wave
-__device__ void order_list(const PairDev &P, uint32_t r, NamKey *lk) {
+__device__ __forceinline__ void order_list(const PairDev &P, uint32_t r, NamKey *lk) {
     const uint32_t lane = lane_id();
     const uint64_t o = P.off[r];
     const uint32_t cnt = (uint32_t)(P.off[r + 1] - o);
@@ -198,13 +198,17 @@ __device__ void order_list(const PairDev &P, uint32_t r, NamKey *lk) {
 // gpu_sort_nams, step2/main.cu:3449-3472 (mate 1: step2/main.cu:2275-2286;
 // mate 2: Nam::operator<, step2/my_struct.hpp:54-68). Bound by the latency of a
 // wave's loads, offsets then NAMs: four lists share them. (65 536 lists of 7.8
-// NAMs on average: 37 us, with a wave to a list 100 us.)
+// NAMs on average: 37 us, with a wave to a list 100 us.) Lists of more than 32
+// NAMs go to k_pair_order_long: their time grows with the square of their length,
+// and a wave would take those among its four one after the other. A block appends
+// its sixteen lists' with one atomic.
 __global__ __launch_bounds__(64 * ORDER_WPB) void k_pair_order(PairDev P) {
-    __shared__ NamKey lk[ORDER_WPB][64];
+    __shared__ uint32_t n_long, at_long;
     const uint32_t wid = threadIdx.x >> 6, rl = lane_id() & 15;
     const uint32_t n_lists = 2 * P.n_pairs;
-    for (uint32_t r0 = 4 * wave_index(ORDER_WPB); r0 < n_lists; r0 += 4 * gridDim.x * ORDER_WPB) {
-        const uint32_t r = r0 + lane_id() / 16;
+    constexpr uint32_t PER_BLOCK = 4 * ORDER_WPB;
+    for (uint32_t b0 = PER_BLOCK * blockIdx.x; b0 < n_lists; b0 += PER_BLOCK * gridDim.x) {
+        const uint32_t r = b0 + 4 * wid + lane_id() / 16;
         const bool mate2 = r >= P.n_pairs;
         const uint64_t o = P.off[min(r, n_lists)];
         const uint32_t all = (uint32_t)(P.off[min(r + 1, n_lists)] - o);
@@ -229,9 +233,28 @@ __global__ __launch_bounds__(64 * ORDER_WPB) void k_pair_order(PairDev P) {
         }
         // equal keys have equal ranks
         if ((uint32_t)__popc(row_or(taken)) != cnt && rl == 0) atomicOr(P.err, PAIR_ERR_DUPLICATE);
-        for (uint64_t big = ballot(rl == 0 && all > 32); big; big &= big - 1)
-            order_list(P, r0 + (uint32_t)__builtin_ctzll(big) / 16, lk[wid]);
+        const bool is_long = all > 32 && rl == 0;
+        if (__syncthreads_or(is_long)) {
+            if (threadIdx.x == 0) n_long = 0;
+            __syncthreads();
+            uint32_t at = 0;
+            if (is_long) at = atomicAdd(&n_long, 1u);
+            __syncthreads();
+            if (threadIdx.x == 0) at_long = atomicAdd(P.n_long, n_long);
+            __syncthreads();
+            if (is_long) P.longs[at_long + at] = r;
+            __syncthreads();
+        }
     }
+}
+
+// the lists that k_pair_order appended, a wave each (128 lists of 1000 NAMs and the
+// copies: 3.8 ms, inside k_pair_order 13.4)
+__global__ __launch_bounds__(64 * ORDER_WPB) void k_pair_order_long(PairDev P) {
+    __shared__ NamKey lk[ORDER_WPB][64];
+    const uint32_t n = sload(P.n_long);
+    for (uint32_t w = wave_index(ORDER_WPB); w < n; w += gridDim.x * ORDER_WPB)
+        order_list(P, uni32(P.longs[w]), lk[threadIdx.x >> 6]);
 }
 
 // top_dropoff, step2/main.cu:889-898 (0 for an empty list, which the
@@ -352,7 +375,10 @@ __global__ void k_pair_totals(PairDev P) {
     const uint32_t t = threadIdx.x;
     if (t <= 5) P.totals[t] = P.tpos[(uint64_t)t * P.nblk];
     else if (t == 6) P.totals[t] = P.joint ? P.joff[P.n_pairs] : 0;
-    else if (t == 7) P.totals[t] = *P.err;
+    else if (t == 7) {
+        P.totals[t] = *P.err;
+        *P.err = *P.n_long = 0;  // for the next step
+    }
 }
 
 // where pair p's joint entries are put before their offsets are known: after the
@@ -902,6 +928,8 @@ void launch_pairs_classify(const PairDev &P, uint64_t *scan_tmp, hipStream_t st)
     if (n_lists) {
         const unsigned g = (unsigned)std::min<uint64_t>(((uint64_t)n_lists + 4 * ORDER_WPB - 1) / (4 * ORDER_WPB), 65536);
         hipLaunchKernelGGL(k_pair_order, dim3(g), dim3(64 * ORDER_WPB), 0, st, P);
+        const unsigned gl = (unsigned)std::min<uint64_t>(((uint64_t)n_lists + ORDER_WPB - 1) / ORDER_WPB, 2048);
+        hipLaunchKernelGGL(k_pair_order_long, dim3(gl), dim3(64 * ORDER_WPB), 0, st, P);
     }
     const unsigned nb = (unsigned)pair_blocks(P.n_pairs);
     if (nb) hipLaunchKernelGGL(k_pair_type, dim3(nb), dim3(PAIR_BLOCK), 0, st, P);

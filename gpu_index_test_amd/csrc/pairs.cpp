@@ -33,6 +33,7 @@ struct PairWork {
     uint64_t n_nams = 0, n_joint = 0;
     uint32_t type_counts[5] = {};
     bool joint = false;
+    bool clean = false;  // the words at err are zero: the last step ran to its end
 };
 
 void pairwork_free(PairWork *w) {
@@ -82,7 +83,10 @@ static int pairs_run(gis_ctx *ctx, PairWork &w, hipStream_t st, const uint64_t *
     P.tpos = ensure<uint64_t>(w.tpos, 5 * nb + 1);
     P.tids = ensure<uint32_t>(w.tids, n_pairs);
     P.nblk = (uint32_t)nb;
-    P.err = ensure<unsigned>(w.err, 1);
+    P.err = ensure<unsigned>(w.err, 2);
+    P.n_long = P.err + 1;
+    static_assert(sizeof(*P.longs) == sizeof(*P.drop), "2 n words each");
+    P.longs = reinterpret_cast<uint32_t *>(P.drop);
     P.dropoff = pp.dropoff_threshold;
     P.mu = pp.mu;
     P.sigma = pp.sigma;
@@ -99,12 +103,14 @@ static int pairs_run(gis_ctx *ctx, PairWork &w, hipStream_t st, const uint64_t *
     }
     uint64_t *tmp = ensure<uint64_t>(w.scan_tmp, scan_tmp_words(std::max<uint64_t>(5 * nb, n_pairs)));
     w.owner = nullptr;
-    HIP_CHECK(hipMemsetAsync(P.err, 0, sizeof(unsigned), st));
+    if (!w.clean) HIP_CHECK(hipMemsetAsync(P.err, 0, 2 * sizeof(unsigned), st));
+    w.clean = false;
     launch_pairs_classify(P, tmp, st);
     if (P.joint) launch_pairs_joint(P, tmp, st);
     launch_pairs_totals(P, st);
     HIP_CHECK(hipGetLastError());
     HIP_CHECK(hipStreamSynchronize(st));
+    w.clean = true;
     if (P.joint && h[6] > P.jout_cap) {
         P.jout = ensure<gis_nam_pair>(w.jout, h[6]);
         P.jout_cap = h[6];

@@ -361,7 +361,7 @@ def _long_mates(rng, c1, c2, hits1, hits2, ref=0):
         i = np.arange(n)
         x["nam_id"], x["query_start"], x["query_end"] = i, i % 50, 100 + i % 50
         x["ref_start"] = 1000 + rng.integers(0, 3, n) * 100_000 + 40 * i + off
-        x["ref_end"], x["n_hits"], x["score"] = x["ref_start"] + 100, hits, 10.0 * hits
+        x["ref_end"], x["n_hits"], x["score"] = x["ref_start"] + 100, hits, 10.0 * np.asarray(hits)
         x["ref_id"], x["is_rc"] = ref, rc
         out.append(x[rng.permutation(n)])
     return out
@@ -404,3 +404,24 @@ def test_joint_time_of_rows_left(ctx):
         G.pairs_from_nams(ctx, offs, flat, 1, joint=joint)
         best[joint] = min(best.get(joint, 1.0), time.perf_counter() - t)
     assert best[True] - best[False] < 3e-3, best
+
+
+def test_order_time_of_long_lists(ctx):
+    """128 lists of 1000 NAMs are ordered beside each other, as long as one pair's two
+    lists (four of them one after the other on a wave: 2.3 times that), 33 to 64 and
+    more NAMs beside short ones in their order."""
+    rng = np.random.default_rng(4)
+    ones = np.ones(1000, int)
+    best = {}
+    pairs = [_long_mates(rng, 1000, 1000, ones, ones) for _ in range(64)]
+    for n in (1, 64) * 4:
+        offs, flat = _flatten([a for a, _ in pairs[:n]] + [b for _, b in pairs[:n]])
+        t = time.perf_counter()
+        G.pairs_from_nams(ctx, offs, flat, n, joint=False)
+        best[n] = min(best.get(n, 1.0), time.perf_counter() - t)
+    assert best[64] < 1.6 * best[1], best
+    for n in (1, 7, 8, 9, 40, 300):
+        c = [int(x) for x in rng.choice([0, 1, 16, 31, 32, 33, 63, 64, 65, 128, 129], 2 * n)]
+        lists = [_long_mates(rng, max(x, 1), 1, rng.integers(1, 9, max(x, 1)), [1])[0][:x] for x in c]
+        offs, flat = _flatten(lists)
+        _compare(G.pairs_from_nams(ctx, offs, flat, n, joint=False), O.pairs_batch(offs, flat, n, joint=False), offs)
