@@ -383,9 +383,18 @@ __global__ void k_pair_totals(PairDev P) {
 
 // where pair p's joint entries are put before their offsets are known: after the
 // bounds c1 + c2 + 2 max_tries + 1 of the pairs before it, which needs no scan
-// (and no wait for its total)
+// (and no wait for its total), or after their exact bounds (k_joint_bounds)
 __device__ __forceinline__ uint64_t joint_place(const PairDev &P, uint32_t p, uint64_t o1, uint64_t o2) {
+    if (P.jplace) return P.jplace[p];
     return o1 + (o2 - P.off[P.n_pairs]) + (uint64_t)p * (2 * (uint32_t)P.max_tries + 1);
+}
+
+// exact bounds of the pairs' entries, for joint_place once scanned
+__global__ __launch_bounds__(PAIR_BLOCK) void k_joint_bounds(PairDev P) {
+    const uint32_t p = blockIdx.x * PAIR_BLOCK + threadIdx.x, n = P.n_pairs;
+    if (p >= n) return;
+    P.jcnt[p] = (uint32_t)joint_bound((uint32_t)(P.off[p + 1] - P.off[p]), (uint32_t)(P.off[n + p + 1] - P.off[n + p]),
+                                      P.max_tries);
 }
 
 // an entry's NAM fields that the NamPair comparator reads; an absent NAM is
@@ -935,6 +944,12 @@ void launch_pairs_classify(const PairDev &P, uint64_t *scan_tmp, hipStream_t st)
     if (nb) hipLaunchKernelGGL(k_pair_type, dim3(nb), dim3(PAIR_BLOCK), 0, st, P);
     launch_scan(P.tcnt, const_cast<uint64_t *>(P.tpos), 5ull * nb, scan_tmp, st);
     if (nb) hipLaunchKernelGGL(k_type_scatter, dim3(nb), dim3(PAIR_BLOCK), 0, st, P);
+}
+
+void launch_joint_bounds(const PairDev &P, uint64_t *place, uint64_t *scan_tmp, hipStream_t st) {
+    const unsigned nb = (unsigned)pair_blocks(P.n_pairs);
+    if (nb) hipLaunchKernelGGL(k_joint_bounds, dim3(nb), dim3(PAIR_BLOCK), 0, st, P);
+    launch_scan(P.jcnt, place, P.n_pairs, scan_tmp, st);
 }
 
 void launch_pairs_joint(const PairDev &P, uint64_t *scan_tmp, hipStream_t st) {

@@ -3,7 +3,8 @@
 // A pair step is one sequence of launches on the batch's stream: reference
 // order, pair types, per-type lists and, with GIS_PAIRS_JOINT, the joint NAM
 // pairs. The joint entries are placed by bounds that follow from the list
-// offsets, so nothing is read back in between; the last kernel writes the type
+// offsets, so nothing is read back in between (unless those bounds are large:
+// LOOSE_ENTRIES); the last kernel writes the type
 // counts, the entry total and the error bits to pinned memory, read after one
 // synchronisation. The compacted entries have the room of earlier steps or one
 // NAM's worth of entries; where the total is larger, the compaction alone runs
@@ -25,7 +26,7 @@ namespace gis {
 
 struct PairWork {
     DevBuf in_off, in_nams;  // lists uploaded by gis_pairs_from_nams
-    DevBuf ord, types, drop, mapq, tcnt, tpos, tids, jtmp, jcnt, joff, jout, err, scan_tmp;
+    DevBuf ord, types, drop, mapq, tcnt, tpos, tids, jtmp, jcnt, joff, jout, jplace, err, scan_tmp;
     uint64_t *h = nullptr;  // pinned: [0..5] type starts, [6] joint total, [7] error bits
     const void *owner = nullptr;  // the batch (or context) whose lists the results belong to
     const uint64_t *dev_off = nullptr;
@@ -40,7 +41,7 @@ void pairwork_free(PairWork *w) {
     if (!w) return;
     DevBuf *all[] = {&w->in_off, &w->in_nams, &w->ord,  &w->types, &w->drop, &w->mapq,
                      &w->tcnt,   &w->tpos,    &w->tids, &w->jtmp,  &w->jcnt, &w->joff,
-                     &w->jout,   &w->err,     &w->scan_tmp};
+                     &w->jout,   &w->jplace,  &w->err,  &w->scan_tmp};
     for (DevBuf *x : all) release(*x);
     if (w->h) (void)hipHostFree(w->h);
     delete w;
@@ -65,6 +66,11 @@ static int check_params(gis_ctx *ctx, const gis_pair_params &pp) {
         return fail(ctx, GIS_ERR_BAD_PARAMETER, "pair parameters must be finite");
     return GIS_OK;
 }
+
+// joint entries up to which they are placed by the loose bound (192 MB): each pair
+// has room for 2 max_tries + 1 entries beside its lists, whatever these hold, 6 KB
+// at max_tries = 256. Beyond, their exact bounds are scanned and waited for.
+constexpr uint64_t LOOSE_ENTRIES = 16u << 20;
 
 // the pair step on device lists off[2n+1] / in
 static int pairs_run(gis_ctx *ctx, PairWork &w, hipStream_t st, const uint64_t *off, const gis_nam *in,
@@ -95,7 +101,6 @@ static int pairs_run(gis_ctx *ctx, PairWork &w, hipStream_t st, const uint64_t *
     uint64_t *h = w.h;
     P.totals = h;
     if (P.joint) {
-        P.jtmp = ensure<gis_nam_pair>(w.jtmp, n_nams + (uint64_t)n_pairs * (2ull * P.max_tries + 1));
         P.jcnt = ensure<uint32_t>(w.jcnt, n_pairs);
         P.joff = ensure<uint64_t>(w.joff, n_pairs + 1ull);
         P.jout = ensure<gis_nam_pair>(w.jout, n_nams);
@@ -103,6 +108,19 @@ static int pairs_run(gis_ctx *ctx, PairWork &w, hipStream_t st, const uint64_t *
     }
     uint64_t *tmp = ensure<uint64_t>(w.scan_tmp, scan_tmp_words(std::max<uint64_t>(5 * nb, n_pairs)));
     w.owner = nullptr;
+    if (P.joint) {
+        uint64_t entries = n_nams + (uint64_t)n_pairs * (2ull * P.max_tries + 1);
+        if (entries > LOOSE_ENTRIES) {
+            uint64_t *place = ensure<uint64_t>(w.jplace, n_pairs + 1ull);
+            launch_joint_bounds(P, place, tmp, st);
+            HIP_CHECK(hipGetLastError());
+            HIP_CHECK(hipMemcpyAsync(&h[6], place + n_pairs, 8, hipMemcpyDeviceToHost, st));
+            HIP_CHECK(hipStreamSynchronize(st));
+            entries = h[6];
+            P.jplace = place;
+        }
+        P.jtmp = ensure<gis_nam_pair>(w.jtmp, entries);
+    }
     if (!w.clean) HIP_CHECK(hipMemsetAsync(P.err, 0, 2 * sizeof(unsigned), st));
     w.clean = false;
     launch_pairs_classify(P, tmp, st);

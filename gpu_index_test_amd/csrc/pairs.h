@@ -29,6 +29,7 @@ struct PairDev {
     uint32_t *tids;       // [n] pair ids grouped by type
     uint32_t nblk;
     gis_nam_pair *jtmp;   // entries at joint_place()
+    const uint64_t *jplace; // [n+1] the pairs' places in jtmp (null: by the loose bound)
     uint32_t *jcnt;       // [n]
     const uint64_t *joff; // [n+1]
     gis_nam_pair *jout;   // entries at joff
@@ -49,6 +50,9 @@ constexpr unsigned PAIR_BLOCK = 256;
 size_t pair_blocks(uint32_t n_pairs);
 // reference order, types, dropoff, MAPQ and type lists
 void launch_pairs_classify(const PairDev &P, uint64_t *scan_tmp, hipStream_t st);
+// the pairs' places in jtmp by the exact bounds of their entries, their end in
+// place[n]; jcnt is scratch for it
+void launch_joint_bounds(const PairDev &P, uint64_t *place, uint64_t *scan_tmp, hipStream_t st);
 // joint NAM pairs into jtmp, their counts scanned into joff, compacted into jout
 void launch_pairs_joint(const PairDev &P, uint64_t *scan_tmp, hipStream_t st);
 // the compaction again, with more room at jout

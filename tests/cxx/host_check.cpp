@@ -320,11 +320,47 @@ static void index_bytes() {
     gis_ctx_destroy(ctx);
 }
 
+// the device memory of a pair step follows its lists, not max_tries
+static void pairs_memory() {
+    gis_ctx *ctx = context();
+    const uint32_t n = 100000;
+    std::vector<uint64_t> off(2 * n + 1);
+    std::vector<gis_nam> nams(2 * n);
+    for (uint32_t r = 0; r < 2 * n; r++) {
+        off[r + 1] = r + 1;
+        gis_nam &x = nams[r];
+        x = gis_nam{};
+        x.query_end = 50;
+        x.ref_start = 1000 + r % n + (r < n ? 0 : 200);
+        x.ref_end = x.ref_start + 50;
+        x.n_hits = 3;
+        x.score = 30;
+        x.is_rc = r >= n;
+    }
+    gis_pair_params p;
+    gis_pair_params_default(&p);
+    p.max_tries = 256;
+    p.flags = GIS_PAIRS_JOINT;
+    std::vector<gis_nam_pair> joint(n);
+    std::vector<uint64_t> joff(n + 1);
+    gis_pair_out o{};
+    o.joint = joint.data();
+    o.joint_capacity = n;
+    o.joint_offsets = joff.data();
+    const uint64_t before = g_live;
+    EXPECT(gis_pairs_from_nams(ctx, off.data(), nams.data(), n, &p, &o) == GIS_OK);
+    EXPECT(g_live - before < 100u << 20);
+    EXPECT(o.n_joint == n && joff[n] == n);
+    for (const gis_nam_pair &e : joint) EXPECT(e.score == 6 && e.i1 == 0 && e.i2 == 0);
+    gis_ctx_destroy(ctx);
+}
+
 int main(int argc, char **argv) {
     const struct {
         const char *name;
         void (*run)();
-    } cases[] = {{"pinned_ranges", pinned_ranges}, {"stream_failure", stream_failure}, {"replace_index", replace_index}, {"index_bytes", index_bytes}};
+    } cases[] = {{"pinned_ranges", pinned_ranges}, {"stream_failure", stream_failure}, {"replace_index", replace_index}, {"index_bytes", index_bytes},
+                 {"pairs_memory", pairs_memory}};
     for (const auto &c : cases)
         if (argc == 2 && !std::strcmp(argv[1], c.name)) {
             c.run();

@@ -425,3 +425,19 @@ def test_order_time_of_long_lists(ctx):
         lists = [_long_mates(rng, max(x, 1), 1, rng.integers(1, 9, max(x, 1)), [1])[0][:x] for x in c]
         offs, flat = _flatten(lists)
         _compare(G.pairs_from_nams(ctx, offs, flat, n, joint=False), O.pairs_batch(offs, flat, n, joint=False), offs)
+
+
+@pytest.mark.parametrize("n", [32_000, 32_200])
+def test_joint_entries_placed_by_either_bound(ctx, n):
+    """Around 2^24 entries by the loose bound (513 a pair beside its NAMs) the pairs'
+    places come from their exact bounds."""
+    rng = np.random.default_rng(5)
+    sizes = [0, 1, 2, 5, 17, 33, 70]
+    some = [_long_mates(rng, max(a, 1), max(b, 1), rng.integers(1, 9, max(a, 1)), rng.integers(1, 9, max(b, 1)))
+            for a in sizes for b in sizes]
+    few = [(x[:a], y[:b]) for (x, y), a, b in zip(some, np.repeat(sizes, 7), np.tile(sizes, 7))]
+    few += [few[1]] * 151  # most lists short
+    reps = -(-n // len(few))
+    lists = ([x for x, _ in few] * reps)[:n] + ([y for _, y in few] * reps)[:n]
+    offs, flat = _flatten(lists)
+    _compare(G.pairs_from_nams(ctx, offs, flat, n, max_tries=256), O.pairs_batch(offs, flat, n, max_tries=256), offs)
