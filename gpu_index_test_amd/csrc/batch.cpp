@@ -135,6 +135,10 @@ constexpr size_t SMALL_BYTES = 1u << 20;
 
 static size_t a16(size_t x) { return (x + 15) & ~(size_t)15; }
 
+// NAMs up to which the results of a small call go through h_out (4 MB of them): with
+// more, the copy engines are the faster way
+constexpr uint64_t HOST_NAMS_MAX = (4u << 20) / sizeof(gis_nam);
+
 // the places of a small call's results in h_out
 struct HostOut {
     uint64_t *off;
@@ -149,7 +153,7 @@ static HostOut host_out(gis_batch *b) {
     const size_t n = b->n_reads;
     HostOut h;
     const size_t o_frac = a16(8 * (n + 1)), o_flags = o_frac + a16(4 * n), o_nams = o_flags + a16(n);
-    h.nam_cap = 16 * n + 1024;
+    h.nam_cap = std::max<uint64_t>(16 * n + 1024, b->ws->host_nams);
     h.bytes = o_nams + sizeof(gis_nam) * h.nam_cap;
     uint8_t *p = b->ws->h_out.data();
     h.off = reinterpret_cast<uint64_t *>(p);
@@ -157,6 +161,31 @@ static HostOut host_out(gis_batch *b) {
     h.flags = p + o_flags;
     h.nams = reinterpret_cast<gis_nam *>(p + o_nams);
     return h;
+}
+
+// Whether a small call's results go to h_out: not where the calls before had too many
+// NAMs a read for it. (A call that finds out by itself runs twice.)
+static bool host_out_wanted(gis_batch *b) {
+    if (b->n_reads == 0 || (uint64_t)b->nams_a_read * b->n_reads > HOST_NAMS_MAX) return false;
+    b->ws->h_out.resize(host_out(b).bytes);
+    return true;
+}
+
+// more NAMs than h_out had room for, tot in all: it keeps that room from now on, or
+// they go the large way. True if h_out holds them now.
+static bool host_out_grow(gis_batch *b, uint64_t tot) {
+    const uint64_t need = tot + tot / 8;
+    b->host_out = need <= HOST_NAMS_MAX;
+    if (!b->host_out) return false;
+    b->ws->host_nams = std::max(b->ws->host_nams, need);
+    b->ws->h_out.resize(host_out(b).bytes);
+    return true;
+}
+
+// the NAMs of a finished run, for the calls after it
+static void note_nams(gis_batch *b) {
+    const uint64_t n = b->n_reads, tot = b->ws->tot_nams;
+    if (n) b->nams_a_read = std::max<uint64_t>((tot + n - 1) / n, b->nams_a_read / 2);
 }
 
 // all of `items` through h_in and one launch on the batch's stream (and the
@@ -662,7 +691,7 @@ void batch_complete(gis_batch *b, const RunOpts &r) {
         // not final: grow what overflowed now and size the output next time
         if (ovf & (OVF_HITS | OVF_RHITS | OVF_MERGE)) ovf &= ~(unsigned)OVF_OUT;
         if (ovf & OVF_MERGE) b->ws->merge_scratch = true;
-        if (ovf & OVF_OUT) b->host_out = false;  // more NAMs than h_out holds: the large way
+        if ((ovf & OVF_OUT) && b->host_out && host_out_grow(b, b->ws->tot_nams)) ovf &= ~(unsigned)OVF_OUT;
         ensure_pools(b, (ovf & OVF_HITS) ? b->ws->h_ctl->tot[0] + b->ws->h_ctl->tot[0] / 8 + 4096 : 0,
                      (ovf & OVF_RHITS) ? b->ws->h_ctl->tot[1] + b->ws->h_ctl->tot[1] / 8 + 4096 : 0,
                      (ovf & OVF_OUT) ? b->ws->tot_nams + b->ws->tot_nams / 8 + 1024 : 0);
@@ -673,6 +702,7 @@ void batch_complete(gis_batch *b, const RunOpts &r) {
     b->last_mode = r.mode;
     b->last_graph = r.graph;
     b->ran = r.stop == STOP_NONE;
+    if (b->ran) note_nams(b);
 }
 
 void batch_run(gis_batch *b, const gis_map_options &o, int rescue_mode, int stop) {
@@ -934,8 +964,7 @@ extern "C" int gis_find_nams_batch(gis_ctx *ctx, const char *seqs, const uint64_
     const int rc = batch_stage(b, seqs, offsets, lens, n_reads, false, 0, nullptr, &items, o.mode == GIS_MODE_FUSED);
     if (rc) return rc;
     StreamGuard guard{b->stream};
-    b->host_out = copy_in(b, items) && n_reads > 0;
-    if (b->host_out) b->ws->h_out.resize(host_out(b).bytes);
+    b->host_out = copy_in(b, items) && host_out_wanted(b);
     batch_run(b, o, 0, STOP_NONE);
     guard.armed = false;
     return batch_download(b, out);
@@ -997,8 +1026,8 @@ static int qrs_run(gis_ctx *ctx, const gis_query_randstrobe *qrs, const uint64_t
     b->ran = false;
     ensure_pools(b, (uint64_t)HIT_REGION * n + 16ull * n + 4096, 16ull * n + 4096, 16ull * n + 1024);
     b->tot_rs_cap = total;
-    b->host_out = n > 0 && n <= SMALL_READS && in_bytes <= SMALL_BYTES;
-    if (b->host_out) b->ws->h_out.resize(host_out(b).bytes);
+    const bool small = n > 0 && n <= SMALL_READS && in_bytes <= SMALL_BYTES;
+    b->host_out = small && host_out_wanted(b);
     hipStream_t st = ctx->stream;
     StreamGuard guard{st};
     const CopyItem items[] = {{b->ws->rs_hash.p, hh, 8 * total},
@@ -1006,7 +1035,6 @@ static int qrs_run(gis_ctx *ctx, const gis_query_randstrobe *qrs, const uint64_t
                               {b->ws->rs_cnt.p, cnt, 4ull * n},
                               {b->ws->rs_nfwd.p, nf, 4ull * n},
                               {b->rs_off.p, off, 8ull * (n + 1)}};
-    const bool small = b->host_out;
     if (small) {
         CopyList c{};
         for (const CopyItem &i : items) {
@@ -1041,13 +1069,14 @@ static int qrs_run(gis_ctx *ctx, const gis_query_randstrobe *qrs, const uint64_t
         if (attempt == 5) throw HipError{hipErrorOutOfMemory, "batch arrays still too small after regrowth"};
         if (ovf & (OVF_HITS | OVF_RHITS | OVF_MERGE)) ovf &= ~(unsigned)OVF_OUT;
         if (ovf & OVF_MERGE) b->ws->merge_scratch = true;
-        if (ovf & OVF_OUT) b->host_out = false;
+        if ((ovf & OVF_OUT) && b->host_out && host_out_grow(b, b->ws->tot_nams)) ovf &= ~(unsigned)OVF_OUT;
         ensure_pools(b, (ovf & OVF_HITS) ? b->ws->h_ctl->tot[0] + 4096 : 0,
                      (ovf & OVF_RHITS) ? b->ws->h_ctl->tot[1] + 4096 : 0,
                      (ovf & OVF_OUT) ? b->ws->tot_nams + 1024 : 0);
     }
     guard.armed = false;
     b->ran = true;
+    note_nams(b);
     return batch_download(b, out);
 }
 

@@ -95,6 +95,7 @@ struct Workspace {
     DevCtl *h_ctl_dev = nullptr;
     int refs = 0;
     Pinned<uint8_t> h_out;        // results of small host calls, written by the kernels
+    uint64_t host_nams = 0;       // NAMs it has room for at least, as many as a call had
     PairWork *pairs = nullptr;    // the pair step on this workspace's NAMs (pairs.cpp)
 };
 
@@ -123,6 +124,7 @@ struct gis_batch {
     // run writes its results to the workspace's h_out
     gis::Pinned<uint8_t> h_in;
     bool host_out = false;
+    uint64_t nams_a_read = 0;  // of the runs before, the denser ones forgotten by halves
     // capture a graph only when a launch sequence is met again: calls of ever
     // new sizes would pay a capture each
     bool lazy_graph = false;

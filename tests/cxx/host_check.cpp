@@ -52,6 +52,11 @@ uint64_t g_live = 0, g_peak = 0;           // allocated now, and at most
 std::map<void *, uint64_t> g_blocks;
 std::map<void *, uint64_t> g_copy, g_sync;  // streams: when last copied in on, when last waited for
 uint64_t g_clock = 0;
+std::atomic<uint64_t> g_launches{0};  // kernels and graphs
+
+struct Dim3 {
+    uint32_t x, y, z;
+};
 
 }  // namespace
 
@@ -103,6 +108,18 @@ extern "C" int hipStreamSynchronize(void *st) {
     return e;
 }
 
+extern "C" int hipLaunchKernel(const void *k, Dim3 grid, Dim3 block, void **args, size_t lds, void *st) {
+    static const auto f = real<int (*)(const void *, Dim3, Dim3, void **, size_t, void *)>("hipLaunchKernel");
+    g_launches++;
+    return f(k, grid, block, args, lds, st);
+}
+
+extern "C" int hipGraphLaunch(void *exec, void *st) {
+    static const auto f = real<int (*)(void *, void *)>("hipGraphLaunch");
+    g_launches++;
+    return f(exec, st);
+}
+
 // ---------------- inputs ----------------
 
 struct Genome {
@@ -116,8 +133,14 @@ struct Genome {
     }
 };
 
-static Genome genome(uint64_t n, uint32_t contigs, uint64_t seed) {
+static Genome genome(uint64_t n, uint32_t contigs, uint64_t seed, double repeats = 0) {
     gis_genome_spec s{};
+    s.repeat_fraction = repeats;
+    s.n_families = 4;
+    s.family_min_len = 600;
+    s.family_max_len = 900;
+    s.copies_min = 150;
+    s.copies_max = 250;
     s.total_length = n;
     s.n_contigs = contigs;
     s.gc = 0.45;
@@ -141,13 +164,14 @@ struct Reads {
     }
 };
 
-static Reads reads(const Genome &g, uint32_t n, uint32_t len, uint64_t seed) {
+static Reads reads(const Genome &g, uint32_t n, uint32_t len, uint64_t seed, double errors = 0.005) {
     gis_read_spec s{};
     s.n_reads = n;
     s.lengths[0] = len;
     s.weights[0] = 1;
     s.n_lengths = 1;
-    s.sub_rate = 0.005;
+    s.sub_rate = errors;
+    s.indel_rate = errors / 5;
     s.rc_fraction = 0.5;
     s.seed = seed;
     Reads r;
@@ -355,12 +379,80 @@ static void pairs_memory() {
     gis_ctx_destroy(ctx);
 }
 
+struct Nams {
+    std::vector<uint64_t> off;
+    std::vector<gis_nam> nams;
+    std::vector<float> frac;
+    std::vector<uint8_t> flags;
+    gis_nam_out o{};
+    Nams(uint32_t n, uint64_t cap) : off(n + 1), nams(cap), frac(n), flags(n) {
+        o = gis_nam_out{off.data(), nams.data(), cap, frac.data(), flags.data(), 0};
+    }
+    bool operator==(const Nams &x) const {
+        return o.n_nams == x.o.n_nams && off == x.off && frac == x.frac && flags == x.flags &&
+               !std::memcmp(nams.data(), x.nams.data(), o.n_nams * sizeof(gis_nam));
+    }
+};
+
+// A small call of reads with many NAMs runs once, like any other, when the calls
+// before it were like it: more NAMs than pinned room for them at first (100 reads of
+// 4000 bp), and more than go that way at all (reads of a repeat).
+static void dense_calls() {
+    const Genome quiet = genome(1000000, 1, 9), rich = genome(1000000, 1, 10, 0.5);
+    for (int kind = 0; kind < 3; kind++) {
+        const Genome &g = kind < 2 ? quiet : rich;
+        gis_ctx *ctx = context();
+        EXPECT(build(ctx, g) == GIS_OK);
+        const Reads r = kind == 0 ? reads(g, 100, 150, 11) : kind == 1 ? reads(g, 100, 4000, 11, 0.05) : reads(g, 2500, 300, 11);
+        const uint32_t n = r.n();
+        // by a resident batch
+        gis_batch *b = nullptr;
+        EXPECT(gis_batch_create(ctx, n, r.seqs.size(), &b) == GIS_OK);
+        EXPECT(gis_batch_upload(b, r.seqs.data(), r.offs.data(), r.lens.data(), n) == GIS_OK);
+        EXPECT(gis_batch_run(b, nullptr) == GIS_OK);
+        uint64_t total = 0;
+        EXPECT(gis_batch_nam_count(b, &total) == GIS_OK);
+        Nams want(n, total);
+        EXPECT(gis_batch_download(b, &want.o) == GIS_OK);
+        gis_batch_destroy(b);
+        EXPECT(kind == 0 ? total < 16 * n : kind == 1 ? total > 16 * n + 1024 : total > (4u << 20) / sizeof(gis_nam));
+        // host calls
+        for (int call = 0; call < 5; call++) {
+            Nams got(n, total);
+            const uint64_t before = g_launches;
+            EXPECT(gis_find_nams_batch(ctx, r.seqs.data(), r.offs.data(), r.lens.data(), n, nullptr, &got.o) == GIS_OK);
+            EXPECT(got == want);
+            // the inputs and the run's graph; the NAMs of the last kind come by chunks
+            if (call > 2) EXPECT(g_launches - before == 2 + (kind < 2 ? 0 : (total * sizeof(gis_nam) - 1) / (1 << 20) + 1));
+        }
+        // and per query
+        std::vector<uint64_t> qoff(n + 1);
+        std::vector<gis_query_randstrobe> q(r.seqs.size());
+        uint64_t nq = 0;
+        EXPECT(gis_randstrobes_batch(ctx, r.seqs.data(), r.offs.data(), r.lens.data(), n, qoff.data(), q.data(), q.size(),
+                                     &nq) == GIS_OK);
+        uint64_t first = 0;
+        for (int call = 0; call < 4; call++) {
+            Nams got(n, 2 * total + 1024);
+            const uint64_t before = g_launches;
+            EXPECT(gis_find_nams_qrs(ctx, q.data(), qoff.data(), n, 0, 0, 0, &got.o) == GIS_OK);
+            const uint64_t launches = g_launches - before;
+            if (call == 0) first = got.o.n_nams;
+            EXPECT(got.o.n_nams == first);
+            // (inputs or the reset, lookup, hits, up to four for the merge, two for the output)
+            if (call > 0 && kind < 2) EXPECT(launches <= 9);
+        }
+        gis_ctx_destroy(ctx);
+    }
+}
+
 int main(int argc, char **argv) {
     const struct {
         const char *name;
         void (*run)();
     } cases[] = {{"pinned_ranges", pinned_ranges}, {"stream_failure", stream_failure}, {"replace_index", replace_index}, {"index_bytes", index_bytes},
-                 {"pairs_memory", pairs_memory}};
+                 {"pairs_memory", pairs_memory},
+                 {"dense_calls", dense_calls}};
     for (const auto &c : cases)
         if (argc == 2 && !std::strcmp(argv[1], c.name)) {
             c.run();
