@@ -563,13 +563,17 @@ static void launch_part(gis_batch *b, const RunOpts &r) {
     if (r.graph) {
         bool replay = true;
         const DevBatch key = make_devbatch(b);
+        // (launch arguments beside it; a seeding call may have moved the scan's alone)
+        const void *const args[2] = {b->ws->scan_tmp.p, b->queue.p};
         const gis_fused_config &fc = ctx->fcfg;
         const int cfg[12] = {r.mode, r.rescue_mode, (int)r.rcut, (int)r.hard, r.stop,
                              (b->want_sy ? 1 : 0) | (b->any_long ? 2 : 0), fc.waves_per_block,
                              fc.length_split, fc.chunk, fc.blocks_per_cu, (int)b->n_long, r.part};
         gis_batch::GraphEntry *hit = nullptr;
         for (auto &g : b->graphs)
-            if (std::memcmp(&key, &g.key, sizeof key) == 0 && std::memcmp(cfg, g.cfg, sizeof cfg) == 0) hit = &g;
+            if (std::memcmp(&key, &g.key, sizeof key) == 0 && std::memcmp(args, g.args, sizeof args) == 0 &&
+                std::memcmp(cfg, g.cfg, sizeof cfg) == 0)
+                hit = &g;
         if (!hit) {
             if (b->graphs.size() >= 16) {
                 auto old = b->graphs.begin();
@@ -581,6 +585,7 @@ static void launch_part(gis_batch *b, const RunOpts &r) {
             }
             gis_batch::GraphEntry e{};
             e.key = key;
+            std::memcpy(e.args, args, sizeof args);
             e.epoch = ctx->ix.epoch;
             std::memcpy(e.cfg, cfg, sizeof cfg);
             b->graphs.push_back(e);

@@ -137,6 +137,7 @@ struct gis_batch {
     // captured launch sequences, one per configuration (buffers, mode, cutoffs)
     struct GraphEntry {
         DevBatch key;
+        const void *args[2];  // the launches' other device arrays
         int cfg[12];
         uint64_t epoch;  // the index table the graph was captured against
         hipGraph_t graph;

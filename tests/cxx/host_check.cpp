@@ -52,7 +52,7 @@ uint64_t g_live = 0, g_peak = 0;           // allocated now, and at most
 std::map<void *, uint64_t> g_blocks;
 std::map<void *, uint64_t> g_copy, g_sync;  // streams: when last copied in on, when last waited for
 uint64_t g_clock = 0;
-std::atomic<uint64_t> g_launches{0};  // kernels and graphs
+std::atomic<uint64_t> g_launches{0}, g_graphs{0};  // kernels and graphs, graphs alone
 
 struct Dim3 {
     uint32_t x, y, z;
@@ -117,6 +117,7 @@ extern "C" int hipLaunchKernel(const void *k, Dim3 grid, Dim3 block, void **args
 extern "C" int hipGraphLaunch(void *exec, void *st) {
     static const auto f = real<int (*)(void *, void *)>("hipGraphLaunch");
     g_launches++;
+    g_graphs++;
     return f(exec, st);
 }
 
@@ -446,13 +447,44 @@ static void dense_calls() {
     }
 }
 
+// Captured launches hold the addresses of every array they use. The scan's scratch
+// grows by tiles of 1024 reads beside arrays that grow by reads, so that a seeding
+// call can move it alone: launches captured before are not replayed then.
+static void moved_scratch() {
+    const Genome g = genome(300000, 1, 12);
+    gis_ctx *ctx = context();
+    EXPECT(build(ctx, g) == GIS_OK);
+    const uint32_t n = 16384, more = 20480;
+    const Reads r = reads(g, more, 150, 13);
+    // (every kind of room for more than these reads need, half as much again each time)
+    Nams got(more, 64ull * more), want(more, 64ull * more);
+    const auto call = [&](uint32_t k, Nams &o) {
+        return gis_find_nams_batch(ctx, r.seqs.data(), r.offs.data(), r.lens.data(), k, nullptr, &o.o);
+    };
+    for (uint32_t k : {10240u, 12288u, n, n, n}) EXPECT(call(k, want) == GIS_OK);
+    uint64_t graphs = g_graphs;
+    EXPECT(call(n, want) == GIS_OK && g_graphs == graphs + 1);
+    std::vector<uint64_t> qoff(more + 1);
+    std::vector<gis_query_randstrobe> q(128ull * more);
+    uint64_t nq = 0;
+    EXPECT(gis_randstrobes_batch(ctx, r.seqs.data(), r.offs.data(), r.lens.data(), more, qoff.data(), q.data(), q.size(),
+                                 &nq) == GIS_OK);
+    graphs = g_graphs;
+    EXPECT(call(n, got) == GIS_OK && g_graphs == graphs);
+    EXPECT(got == want);
+    for (int i = 0; i < 2; i++) EXPECT(call(n, got) == GIS_OK && got == want);
+    EXPECT(g_graphs == graphs + 2);
+    gis_ctx_destroy(ctx);
+}
+
 int main(int argc, char **argv) {
     const struct {
         const char *name;
         void (*run)();
     } cases[] = {{"pinned_ranges", pinned_ranges}, {"stream_failure", stream_failure}, {"replace_index", replace_index}, {"index_bytes", index_bytes},
                  {"pairs_memory", pairs_memory},
-                 {"dense_calls", dense_calls}};
+                 {"dense_calls", dense_calls},
+                 {"moved_scratch", moved_scratch}};
     for (const auto &c : cases)
         if (argc == 2 && !std::strcmp(argv[1], c.name)) {
             c.run();
