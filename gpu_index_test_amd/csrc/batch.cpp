@@ -77,10 +77,12 @@ uint64_t batch_device_bytes(gis_batch *b) {
 }
 
 static void graph_drop(gis_batch::GraphEntry &g) {
-    if (g.exec) (void)hipGraphExecDestroy(g.exec);
-    if (g.graph) (void)hipGraphDestroy(g.graph);
-    g.exec = nullptr;
-    g.graph = nullptr;
+    for (int part = 0; part < 3; part++) {
+        if (g.exec[part]) (void)hipGraphExecDestroy(g.exec[part]);
+        if (g.graph[part]) (void)hipGraphDestroy(g.graph[part]);
+        g.exec[part] = nullptr;
+        g.graph[part] = nullptr;
+    }
 }
 
 void batch_trim(gis_batch *b) {
@@ -566,16 +568,16 @@ static void launch_part(gis_batch *b, const RunOpts &r) {
         // (launch arguments beside it; a seeding call may have moved the scan's alone)
         const void *const args[2] = {b->ws->scan_tmp.p, b->queue.p};
         const gis_fused_config &fc = ctx->fcfg;
-        const int cfg[12] = {r.mode, r.rescue_mode, (int)r.rcut, (int)r.hard, r.stop,
+        const int cfg[11] = {r.mode, r.rescue_mode, (int)r.rcut, (int)r.hard, r.stop,
                              (b->want_sy ? 1 : 0) | (b->any_long ? 2 : 0), fc.waves_per_block,
-                             fc.length_split, fc.chunk, fc.blocks_per_cu, (int)b->n_long, r.part};
+                             fc.length_split, fc.chunk, fc.blocks_per_cu, (int)b->n_long};
         gis_batch::GraphEntry *hit = nullptr;
         for (auto &g : b->graphs)
             if (std::memcmp(&key, &g.key, sizeof key) == 0 && std::memcmp(args, g.args, sizeof args) == 0 &&
                 std::memcmp(cfg, g.cfg, sizeof cfg) == 0)
                 hit = &g;
         if (!hit) {
-            if (b->graphs.size() >= 16) {
+            if (b->graphs.size() >= 8) {
                 auto old = b->graphs.begin();
                 for (auto it = b->graphs.begin(); it != b->graphs.end(); ++it)
                     if (it->used < old->used) old = it;
@@ -593,7 +595,7 @@ static void launch_part(gis_batch *b, const RunOpts &r) {
             replay = !b->lazy_graph;
         }
         hit->used = ++b->graph_clock;
-        if (replay && !hit->exec) {
+        if (replay && !hit->exec[r.part]) {
             hipGraph_t g = nullptr;
             HIP_CHECK(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
             try {
@@ -604,15 +606,15 @@ static void launch_part(gis_batch *b, const RunOpts &r) {
                 throw;
             }
             HIP_CHECK(hipStreamEndCapture(st, &g));
-            const hipError_t ie = hipGraphInstantiate(&hit->exec, g, nullptr, nullptr, 0);
+            const hipError_t ie = hipGraphInstantiate(&hit->exec[r.part], g, nullptr, nullptr, 0);
             if (ie != hipSuccess) {
                 (void)hipGraphDestroy(g);
-                hit->exec = nullptr;
+                hit->exec[r.part] = nullptr;
                 throw HipError{ie, "hipGraphInstantiate"};
             }
-            hit->graph = g;
+            hit->graph[r.part] = g;
         }
-        if (replay) HIP_CHECK(hipGraphLaunch(hit->exec, st));
+        if (replay) HIP_CHECK(hipGraphLaunch(hit->exec[r.part], st));
         else enqueue_run(b, r);
     } else {
         enqueue_run(b, r);
@@ -622,8 +624,8 @@ static void launch_part(gis_batch *b, const RunOpts &r) {
 
 // Enqueue one run on the batch's stream. With r.graph the launch sequence is
 // captured once per configuration (buffers, mode, cutoffs, fused launch
-// configuration) and replayed; a batch keeps the graphs of its last 8
-// configurations, in two parts each at most.
+// configuration) and replayed, a run in two parts by graphs of its own; a batch
+// keeps the graphs of its last 8 configurations.
 //
 // in_turn (a burst: runs launched on streams of their own onto an idle device, none
 // waited for yet): a large plain batch starts after the front of the one before it,

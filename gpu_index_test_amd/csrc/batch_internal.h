@@ -134,14 +134,15 @@ struct gis_batch {
     hipEvent_t ev[16] = {};
     int n_ev = 0;
     std::vector<std::string> ev_names;
-    // captured launch sequences, one per configuration (buffers, mode, cutoffs)
+    // captured launch sequences, by configuration (buffers, mode, cutoffs): the whole
+    // run and its two parts (PART_*), each once it is launched
     struct GraphEntry {
         DevBatch key;
         const void *args[2];  // the launches' other device arrays
-        int cfg[12];
-        uint64_t epoch;  // the index table the graph was captured against
-        hipGraph_t graph;
-        hipGraphExec_t exec;  // null: met once, not captured yet (lazy_graph)
+        int cfg[11];
+        uint64_t epoch;  // the index table the graphs were captured against
+        hipGraph_t graph[3];
+        hipGraphExec_t exec[3];  // null: not captured (yet)
         uint64_t used;
     };
     std::vector<GraphEntry> graphs;

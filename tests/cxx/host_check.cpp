@@ -52,7 +52,7 @@ uint64_t g_live = 0, g_peak = 0;           // allocated now, and at most
 std::map<void *, uint64_t> g_blocks;
 std::map<void *, uint64_t> g_copy, g_sync;  // streams: when last copied in on, when last waited for
 uint64_t g_clock = 0;
-std::atomic<uint64_t> g_launches{0}, g_graphs{0};  // kernels and graphs, graphs alone
+std::atomic<uint64_t> g_launches{0}, g_graphs{0}, g_made{0};  // kernels and graphs, graphs alone, graphs made
 
 struct Dim3 {
     uint32_t x, y, z;
@@ -119,6 +119,12 @@ extern "C" int hipGraphLaunch(void *exec, void *st) {
     g_launches++;
     g_graphs++;
     return f(exec, st);
+}
+
+extern "C" int hipGraphInstantiate(void **exec, void *graph, void **node, char *log, size_t n) {
+    static const auto f = real<int (*)(void **, void *, void **, char *, size_t)>("hipGraphInstantiate");
+    g_made++;
+    return f(exec, graph, node, log, n);
 }
 
 // ---------------- inputs ----------------
@@ -477,6 +483,37 @@ static void moved_scratch() {
     gis_ctx_destroy(ctx);
 }
 
+// A batch keeps the graphs of eight configurations, also where runs in a burst are
+// launched in two parts and others whole.
+static void graphs_kept() {
+    const Genome g = genome(300000, 1, 14);
+    gis_ctx *ctx = context();
+    EXPECT(build(ctx, g) == GIS_OK);
+    const Reads r = reads(g, 16384, 100, 15);  // (as many as take turns)
+    gis_batch *b[2];
+    for (gis_batch *&x : b) {
+        EXPECT(gis_batch_create_async(ctx, r.n(), r.seqs.size(), &x) == GIS_OK);
+        EXPECT(gis_batch_upload(x, r.seqs.data(), r.offs.data(), r.lens.data(), r.n()) == GIS_OK);
+        EXPECT(gis_batch_run(x, nullptr) == GIS_OK);  // (its arrays have their size)
+    }
+    uint64_t made[2];
+    for (int pass = 0; pass < 2; pass++) {
+        const uint64_t before = g_made;
+        for (int c = 0; c < 8; c++) {
+            gis_map_options o;
+            gis_map_options_default(&o);
+            o.hard_cutoff = 900 + c;
+            for (gis_batch *x : b) EXPECT(gis_batch_launch(x, &o) == GIS_OK);
+            for (gis_batch *x : b) EXPECT(gis_batch_wait(x) == GIS_OK);
+            for (gis_batch *x : b) EXPECT(gis_batch_run(x, &o) == GIS_OK);
+        }
+        made[pass] = g_made - before;
+    }
+    EXPECT(made[0] == 2 * 8 * 3 && made[1] == 0);
+    for (gis_batch *x : b) gis_batch_destroy(x);
+    gis_ctx_destroy(ctx);
+}
+
 int main(int argc, char **argv) {
     const struct {
         const char *name;
@@ -484,7 +521,8 @@ int main(int argc, char **argv) {
     } cases[] = {{"pinned_ranges", pinned_ranges}, {"stream_failure", stream_failure}, {"replace_index", replace_index}, {"index_bytes", index_bytes},
                  {"pairs_memory", pairs_memory},
                  {"dense_calls", dense_calls},
-                 {"moved_scratch", moved_scratch}};
+                 {"moved_scratch", moved_scratch},
+                 {"graphs_kept", graphs_kept}};
     for (const auto &c : cases)
         if (argc == 2 && !std::strcmp(argv[1], c.name)) {
             c.run();
