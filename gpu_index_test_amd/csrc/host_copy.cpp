@@ -6,6 +6,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cstring>
 #include <mutex>
 #include <system_error>
@@ -132,8 +133,19 @@ static void pipeline(gis_ctx *ctx, hipStream_t st, uint64_t chunks, Issue issue,
         h->busy[slot(c)] = false;  // (its next copy waits for state 2)
         state[c].store(2, std::memory_order_release);
     };
+    // (a chunk is there within some tens of microseconds, unless the GPU is busy with
+    // other work: then the threads leave their cores alone)
     auto wait_for = [&](uint64_t c, uint8_t s) {
-        while (state[c].load(std::memory_order_acquire) < s && !stop) std::this_thread::yield();
+        const auto t0 = std::chrono::steady_clock::now();
+        bool late = false;
+        for (unsigned turn = 1; state[c].load(std::memory_order_acquire) < s && !stop; turn++) {
+            if (late) {
+                std::this_thread::sleep_for(std::chrono::microseconds(50));
+                continue;
+            }
+            std::this_thread::yield();
+            late = turn % 64 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(500);
+        }
         return state[c].load(std::memory_order_acquire) >= s;
     };
     std::vector<std::thread> th;

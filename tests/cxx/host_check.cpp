@@ -5,6 +5,7 @@
 //
 // usage: host_check <case>; exit status 0 if the case holds
 #include <dlfcn.h>
+#include <sys/resource.h>
 
 #include <algorithm>
 #include <atomic>
@@ -53,6 +54,8 @@ std::map<void *, uint64_t> g_blocks;
 std::map<void *, uint64_t> g_copy, g_sync;  // streams: when last copied in on, when last waited for
 uint64_t g_clock = 0;
 std::atomic<uint64_t> g_launches{0}, g_graphs{0}, g_made{0};  // kernels and graphs, graphs alone, graphs made
+
+std::atomic<int> g_stall{0};  // milliseconds that the next wait for an event takes longer
 
 struct Dim3 {
     uint32_t x, y, z;
@@ -125,6 +128,12 @@ extern "C" int hipGraphInstantiate(void **exec, void *graph, void **node, char *
     static const auto f = real<int (*)(void **, void *, void **, char *, size_t)>("hipGraphInstantiate");
     g_made++;
     return f(exec, graph, node, log, n);
+}
+
+extern "C" int hipEventSynchronize(void *ev) {
+    static const auto f = real<int (*)(void *)>("hipEventSynchronize");
+    std::this_thread::sleep_for(std::chrono::milliseconds(g_stall.exchange(0)));
+    return f(ev);
 }
 
 // ---------------- inputs ----------------
@@ -514,6 +523,37 @@ static void graphs_kept() {
     gis_ctx_destroy(ctx);
 }
 
+// threads of a copy that wait for a chunk the GPU is late with use no CPU time
+static void stalled_copy() {
+    const Genome g = genome(300000, 1, 16);
+    gis_ctx *ctx = context();
+    EXPECT(build(ctx, g) == GIS_OK);
+    std::vector<uint64_t> keys(4u << 20), pos(keys.size()), want(keys.size());
+    for (size_t i = 0; i < keys.size(); i++) keys[i] = i * 0x9e3779b97f4a7c15ull;
+    const auto cpu = [&](int stall, std::vector<uint64_t> &out) {
+        rusage a, b;
+        getrusage(RUSAGE_SELF, &a);
+        g_stall = stall;
+        EXPECT(gis_lookup_batch(ctx, keys.data(), keys.size(), out.data()) == GIS_OK);
+        EXPECT(g_stall == 0);
+        getrusage(RUSAGE_SELF, &b);
+        const auto ms = [](const timeval &t) { return 1e3 * t.tv_sec + 1e-3 * t.tv_usec; };
+        return ms(b.ru_utime) + ms(b.ru_stime) - ms(a.ru_utime) - ms(a.ru_stime);
+    };
+    double plain = 1e9, late = 1e9;
+    cpu(0, want);
+    for (int i = 0; i < 3; i++) {
+        plain = std::min(plain, cpu(0, pos));
+        EXPECT(pos == want);
+        std::fill(pos.begin(), pos.end(), 0);
+        late = std::min(late, cpu(100, pos));
+        EXPECT(pos == want);
+    }
+    std::printf("CPU %.1f ms, with a chunk 100 ms late %.1f\n", plain, late);
+    EXPECT(late - plain < 50);
+    gis_ctx_destroy(ctx);
+}
+
 int main(int argc, char **argv) {
     const struct {
         const char *name;
@@ -522,7 +562,7 @@ int main(int argc, char **argv) {
                  {"pairs_memory", pairs_memory},
                  {"dense_calls", dense_calls},
                  {"moved_scratch", moved_scratch},
-                 {"graphs_kept", graphs_kept}};
+                 {"graphs_kept", graphs_kept}, {"stalled_copy", stalled_copy}};
     for (const auto &c : cases)
         if (argc == 2 && !std::strcmp(argv[1], c.name)) {
             c.run();
