@@ -630,7 +630,7 @@ static void launch_part(gis_batch *b, const RunOpts &r) {
 // in_turn (a burst: runs launched on streams of their own onto an idle device, none
 // waited for yet): a large plain batch starts after the front of the one before it,
 // its seeding and lookup (fused kernels are nearly the whole run: two batches of
-// 60,000 took 1463 us in turn and 1382 without). Launched together they would
+// 60,000 took 1463 us in turn and 1370 to 1382 without). Launched together they would
 // share the device from their first kernel and end together, and the first one's
 // copies back could not run beside the others' kernels. (Three batches of 65,536
 // reads of 150 bp and their results: 1797 us, side by side 2046.) Later launches

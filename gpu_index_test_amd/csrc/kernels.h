@@ -162,8 +162,8 @@ constexpr uint32_t HIT_REGION = 128;
 
 constexpr uint32_t BUCKET_LINE = 8;  // uint4 per bucket line
 
-// Up to MAX small blocks of pinned host memory that one launch copies into device
-// arrays (launch_copy_in). Sources and destinations are 16-byte aligned.
+// Up to MAX small arrays that one launch copies between pinned host memory and the
+// device (launch_copy_in), either way. Sources and destinations are 16-byte aligned.
 struct CopyList {
     static constexpr int MAX = 8;
     static constexpr uint32_t BLOCK_BYTES = 16384;  // bytes a thread block copies
@@ -175,7 +175,7 @@ struct CopyList {
 };
 
 // launch wrappers (kernels.hip)
-// copies, and with ctl the control block cleared (ctl may be null)
+// the copies of c, and with ctl the control block cleared (ctl may be null)
 void launch_copy_in(const CopyList &c, DevCtl *ctl, hipStream_t st);
 void launch_bucket_lines(const uint4 *rs, const uint64_t *starts, int bits, uint4 *lines, hipStream_t st);
 void launch_reset_ctl(DevCtl *ctl, hipStream_t st);

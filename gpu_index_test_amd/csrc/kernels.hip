@@ -294,7 +294,7 @@ __device__ __forceinline__ uint32_t seed_syncmers(const char *__restrict__ seq, 
 
 // LDS of a wave that seeds a long read, and the reads it holds: of up to
 // LONG_LDS_BASES bases with up to LONG_LDS_SYNC syncmers (one in k - s + 1 bases on
-// average: 2200 to 3100 bases). Six waves a SIMD fit.
+// average: 2200 to 3100 bases). 6.4 KB, given out as 7.5: 21 waves a CU, five a SIMD.
 constexpr int LONG_LDS_BASES = 4096;
 constexpr uint32_t LONG_LDS_SYNC = 448;
 constexpr int LONG_RING = 128;
@@ -921,9 +921,8 @@ __device__ __forceinline__ void probe_emit(const DevIndex &ix, const Probe &p, i
 //
 // Write traffic is part of this kernel's bound, so a one-pass read (at most
 // 64 randstrobes) keeps its per-randstrobe results (position, kept-hit count)
-// in registers and stores them only when a later kernel reads them: when the
-// read is rescued (k_hits) or its hits go to the pool
-// (k_hits). Longer reads, and the fused kernel's spilled reads, store them
+// in registers and stores them only when k_hits reads them: when the read is
+// rescued or its hits go to the pool. Longer reads, and the fused kernel's spilled reads, store them
 // in every pass. Wave sums and scans use DPP (52 VGPRs).
 __global__ __launch_bounds__(64 * WPB) __attribute__((amdgpu_waves_per_eu(6))) void k_lookup(
     DevBatch b, ReadSet set, DevIndex ix, int rescue_mode, int keep_spill) {
@@ -2858,7 +2857,7 @@ constexpr int SCAN_BLOCK = 256, SCAN_ITEMS = 4, SCAN_TILE = SCAN_BLOCK * SCAN_IT
 constexpr uint32_t COMPACT_SEG = 16;
 constexpr uint32_t COMPACT_SEG_WORDS = 8 * COMPACT_SEG;  // 11 NAMs of 11 words
 
-// totals into the control block's copy for the host: lane i holds word i
+// the control block with its totals to the host's copy, by the first thread
 __device__ __forceinline__ void ctl_store(const DevBatch &b, DevCtl *dst, uint64_t nams, unsigned overflow) {
     if (threadIdx.x == 0) {
         DevCtl c = *b.ctl;
@@ -3134,9 +3133,10 @@ void launch_bucket_lines(const uint4 *rs, const uint64_t *starts, int bits, uint
     hipLaunchKernelGGL(k_bucket_lines, dim3((unsigned)(g < 65536 ? g : 65536)), dim3(256), 0, st, rs, starts, nb, lines);
 }
 
-// The inputs of a small call from one pinned block into their device arrays, read
-// over PCIe by the kernel itself: seven hipMemcpyAsync of a few kilobytes cost
-// 5-10 us each on the host and a blit kernel each on the device.
+// Small arrays between pinned host memory and the device, read or written over PCIe
+// by the kernel itself: the inputs of a small call from one pinned block, where
+// seven hipMemcpyAsync of a few kilobytes cost 5-10 us each on the host and a blit
+// kernel each on the device, and the small arrays of a large result back.
 __global__ __launch_bounds__(256) void k_copy_in(CopyList c, DevCtl *ctl) {
     if (ctl && blockIdx.x == 0) ctl_clear(ctl);
     int i = 0;
@@ -3243,9 +3243,6 @@ bool launch_fused(const DevBatch &b, const DevIndex &ix, const SeedParams &sp, u
     return false;
 }
 
-// The control block to pinned host memory by a thread's stores, so that the
-// end of a run takes no copy engine (the engines carry the batches' reads and
-// NAMs).
 // n bytes of HBM to pinned memory, 16 a lane (both ends 16-byte aligned): a chunk
 // of a large copy starts ~10 us sooner than on the copy engines
 __global__ __launch_bounds__(256) void k_copy_out(const uint4 *__restrict__ src, uint4 *__restrict__ dst, uint64_t n) {
@@ -3260,6 +3257,9 @@ void launch_copy_out(const void *src, void *dst, uint64_t n, hipStream_t st) {
     hipLaunchKernelGGL(k_copy_out, dim3(g), dim3(256), 0, st, static_cast<const uint4 *>(src), static_cast<uint4 *>(dst), n);
 }
 
+// The control block to pinned host memory by a thread's stores, so that the
+// end of a run takes no copy engine (the engines carry the batches' reads and
+// NAMs).
 __global__ void k_ctl_to_host(DevBatch b, DevCtl *dst) { ctl_store(b, dst, 0, 0u); }
 
 void launch_ctl_to_host(const DevBatch &b, DevCtl *dst, hipStream_t st) {

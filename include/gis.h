@@ -99,7 +99,7 @@ typedef struct {
     gis_params params;
     uint64_t distinct_strobemers; /* IndexCreationStatistics, step2/index.hpp:22-35 */
     uint64_t tot_occur_once, tot_high_ab, tot_mid_ab, index_cutoff;
-    uint64_t device_bytes;
+    uint64_t device_bytes; /* of the table and its bucket lines */
 } gis_index_info;
 
 /* Per-read result flags. GIS_FLAG_SPILLED: in GIS_MODE_FUSED the read did not
@@ -131,7 +131,8 @@ typedef struct {
     int32_t flags;         /* GIS_RUN_* */
 } gis_map_options;
 
-/* GIS_MODE_PLAIN: one launch per stage (seed, lookup, hits, rescue, merge).
+/* GIS_MODE_PLAIN: launches per stage (seed, lookup, hits with those of rescued
+ * reads, merge, output).
  * GIS_MODE_FUSED: one wave-per-read kernel for the whole path; reads beyond
  * its LDS budget go through the per-stage kernels. Same NAMs either way. */
 enum { GIS_MODE_PLAIN = 0, GIS_MODE_FUSED = 1 };
@@ -183,7 +184,9 @@ int gis_device_count(int *count);
  * (gis_reference_randstrobes); the records are sorted, bucketed and counted
  * on the GPU, and the index is left resident in HBM. n_threads is the
  * reference's argument and is not needed: no host thread seeds. Each contig
- * must be shorter than 2^32 bases, and there are fewer than 2^24 of them. */
+ * must be shorter than 2^32 bases, and there are fewer than 2^24 of them. Up to
+ * 512 MB of a build's device memory stays with the context for its next build,
+ * unless a load needs it. */
 int gis_index_build(gis_ctx *ctx, const char *const *seqs, const uint64_t *lens,
                     uint32_t n_refs, const gis_params *params, int bits, float f,
                     int n_threads);
@@ -464,7 +467,9 @@ typedef struct {
 } gis_pair_out;
 
 /* Run the pair step on the NAMs of the batch's last run (2 n reads, mates laid
- * out as above); results stay on the device until downloaded. */
+ * out as above); results stay on the device until downloaded. With
+ * GIS_PAIRS_JOINT it holds 12 bytes per NAM and 24 max_tries + 12 per pair for
+ * the entries, or beyond 192 MB in all what the lists' own lengths allow. */
 int gis_batch_pairs(gis_batch *b, const gis_pair_params *pp);
 /* Copy the pair step's results out. GIS_ERR_CAPACITY (with n_nams / n_joint
  * set) if nam_capacity or joint_capacity is too small. */
