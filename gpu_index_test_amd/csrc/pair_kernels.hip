@@ -4,14 +4,13 @@
 //                 position in the reference order is the number of NAMs of the
 //                 list with a smaller key, counted against the other lanes of
 //                 the row, two NAMs a lane for lists of 17 to 32 (one list in
-//                 eight). Keys are unique (each NAM's (is_rc, ref_id,
-//                 query_start, ref_start) is its own first hit), so counting
-//                 ranks gives the one sorted order the reference's quicksort
-//                 reaches.
-//  k_pair_order_long  longer lists, a wave each (up to 64: against the other
-//                 lanes; beyond: against 64-key tiles in LDS). Lists in
-//                 canonical order are grouped by (is_rc, ref_id), so a 64-NAM
-//                 chunk only counts against the groups it spans.
+//                 eight), one a lane of the whole wave for lists of up to 64.
+//                 Keys are unique (each NAM's (is_rc, ref_id, query_start,
+//                 ref_start) is its own first hit), so counting ranks gives the
+//                 one sorted order the reference's quicksort reaches.
+//  k_pair_order_long  longer lists, a wave each, against 64-key tiles in LDS.
+//                 Lists in canonical order are grouped by (is_rc, ref_id), so a
+//                 64-NAM chunk only counts against the groups it spans.
 //  k_pair_type    one lane per pair: type, top_dropoff, MAPQ, per-block type
 //                 counts.
 //  k_type_scatter pair ids grouped by type in id order (the host loop of
@@ -58,10 +57,6 @@ __device__ __forceinline__ bool key_less(const NamKey &a, const NamKey &b) {
     if (a.dn != b.dn) return a.dn < b.dn;
     if (a.q != b.q) return a.q < b.q;
     return a.r < b.r;
-}
-
-__device__ __forceinline__ bool key_eq(const NamKey &a, const NamKey &b) {
-    return a.g == b.g && a.dn == b.dn && a.q == b.q && a.r == b.r;
 }
 
 // rank += 1 where the key a of the lane q of the row is less than b: the words as
@@ -113,7 +108,35 @@ __device__ __forceinline__ void rank_rows(const NamKey &k0, const NamKey &k1, ui
 
 constexpr int ORDER_WPB = 4;
 
-// a list of more than 32 NAMs, by the whole wave
+// the places of cnt NAMs add up to 0 + 1 + .. + cnt - 1, less one for each two equal
+// keys (those have equal places)
+__device__ __forceinline__ void places_check(const PairDev &P, uint32_t cnt, uint64_t sum) {
+    if (sum != (uint64_t)cnt * (cnt - 1) / 2 && lane_id() == 0) atomicOr(P.err, PAIR_ERR_DUPLICATE);
+}
+
+// a list of 33 to 64 NAMs in the lanes of a wave: each lane ranks its NAM against
+// every other one read straight from the lanes
+__device__ __forceinline__ void order_lanes(const PairDev &P, uint32_t r) {
+    const uint32_t lane = lane_id();
+    const uint64_t o = P.off[r];
+    const uint32_t cnt = (uint32_t)(P.off[r + 1] - o);
+    const bool valid = lane < cnt;
+    gis_nam mine{};
+    NamKey ki{};
+    if (valid) {
+        mine = P.in[o + lane];
+        ki = nam_key(mine, r >= P.n_pairs);
+    }
+    uint32_t rank = 0;
+    for (uint32_t q = 0; q < cnt; q++) {
+        const NamKey kj{readlane_u64(ki.g, q), readlane_u64(ki.dn, q), readlane_u64(ki.q, q), readlane_u64(ki.r, q)};
+        rank += key_less(kj, ki) ? 1u : 0u;
+    }
+    if (valid) P.ord[o + rank] = mine;
+    places_check(P, cnt, wave_sum_dpp(valid ? rank : 0u));
+}
+
+// a longer list by a wave
 __device__ __forceinline__ void order_list(const PairDev &P, uint32_t r, NamKey *lk) {
     const uint32_t lane = lane_id();
     const uint64_t o = P.off[r];
@@ -121,28 +144,7 @@ __device__ __forceinline__ void order_list(const PairDev &P, uint32_t r, NamKey 
     const bool mate2 = r >= P.n_pairs;
     const gis_nam *in = P.in + o;
     gis_nam *out = P.ord + o;
-    if (cnt <= 64) {
-        // the whole list in the lanes: each lane ranks its NAM against
-        // every other one read straight from the lanes
-        const bool valid = lane < cnt;
-        gis_nam mine{};
-        NamKey ki{};
-        if (valid) {
-            mine = in[lane];
-            ki = nam_key(mine, mate2);
-        }
-        uint32_t rank = 0;
-        bool dup = false;
-        for (uint32_t q = 0; q < cnt; q++) {
-            const NamKey kj{readlane_u64(ki.g, q), readlane_u64(ki.dn, q), readlane_u64(ki.q, q),
-                            readlane_u64(ki.r, q)};
-            rank += key_less(kj, ki) ? 1u : 0u;
-            dup |= q != lane && key_eq(kj, ki);
-        }
-        if (valid) out[rank] = mine;
-        if (ballot(valid && dup) != 0 && lane == 0) atomicOr(P.err, PAIR_ERR_DUPLICATE);
-        return;
-    }
+    uint64_t places = 0;
     for (uint32_t i0 = 0; i0 < cnt; i0 += 64) {
         const uint32_t i = i0 + lane;
         const bool valid = i < cnt;
@@ -175,7 +177,6 @@ __device__ __forceinline__ void order_list(const PairDev &P, uint32_t r, NamKey 
             u1 = lo;
         }
         uint32_t rank = 0;
-        bool dup = false;
         for (uint32_t t = u0; t < u1; t += 64) {
             const uint32_t j = t + lane;
             if (j < u1) lk[lane] = nam_key(in[j], mate2);
@@ -185,26 +186,29 @@ __device__ __forceinline__ void order_list(const PairDev &P, uint32_t r, NamKey 
                 for (uint32_t q = 0; q < m; q++) {
                     const NamKey kj = lk[q];
                     rank += key_less(kj, ki) ? 1u : 0u;
-                    dup |= (t + q != i) && key_eq(kj, ki);
                 }
             }
             wave_sync();
         }
-        if (valid) out[u0 + rank] = mine;
-        if (dup) atomicOr(P.err, PAIR_ERR_DUPLICATE);
+        if (valid) {
+            out[u0 + rank] = mine;
+            places += u0 + rank;
+        }
     }
+    for (int d = 32; d >= 1; d >>= 1) places += __shfl_xor(places, d, 64);
+    places_check(P, cnt, places);
 }
 
 // gpu_sort_nams, step2/main.cu:3449-3472 (mate 1: step2/main.cu:2275-2286;
 // mate 2: Nam::operator<, step2/my_struct.hpp:54-68). Bound by the latency of a
 // wave's loads, offsets then NAMs: four lists share them. (65 536 lists of 7.8
-// NAMs on average: 37 us, with a wave to a list 100 us.) Lists of more than 32
-// NAMs go to k_pair_order_long: their time grows with the square of their length,
-// and a wave would take those among its four one after the other. A block appends
-// its sixteen lists' with one atomic.
+// NAMs on average: 37 us, with a wave to a list 100 us.) A list of 33 to 64 NAMs has
+// the whole wave for some microseconds. Longer ones go to k_pair_order_long: their
+// time grows with the square of their length, and a wave would take those among its
+// four one after the other. A block appends its sixteen lists' with one atomic.
 __global__ __launch_bounds__(64 * ORDER_WPB) void k_pair_order(PairDev P) {
     __shared__ uint32_t n_long, at_long;
-    const uint32_t wid = threadIdx.x >> 6, rl = lane_id() & 15;
+    const uint32_t wid = uni32(threadIdx.x >> 6), rl = lane_id() & 15;
     const uint32_t n_lists = 2 * P.n_pairs;
     constexpr uint32_t PER_BLOCK = 4 * ORDER_WPB;
     for (uint32_t b0 = PER_BLOCK * blockIdx.x; b0 < n_lists; b0 += PER_BLOCK * gridDim.x) {
@@ -233,7 +237,9 @@ __global__ __launch_bounds__(64 * ORDER_WPB) void k_pair_order(PairDev P) {
         }
         // equal keys have equal ranks
         if ((uint32_t)__popc(row_or(taken)) != cnt && rl == 0) atomicOr(P.err, PAIR_ERR_DUPLICATE);
-        const bool is_long = all > 32 && rl == 0;
+        for (uint64_t big = ballot(rl == 0 && all > 32 && all <= 64); big; big &= big - 1)
+            order_lanes(P, b0 + 4 * wid + (uint32_t)__builtin_ctzll(big) / 16);
+        const bool is_long = all > 64 && rl == 0;
         if (__syncthreads_or(is_long)) {
             if (threadIdx.x == 0) n_long = 0;
             __syncthreads();
@@ -249,7 +255,7 @@ __global__ __launch_bounds__(64 * ORDER_WPB) void k_pair_order(PairDev P) {
 }
 
 // the lists that k_pair_order appended, a wave each (128 lists of 1000 NAMs and the
-// copies: 3.8 ms, inside k_pair_order 13.4)
+// copies: 3.5 ms, inside k_pair_order 13.4)
 __global__ __launch_bounds__(64 * ORDER_WPB) void k_pair_order_long(PairDev P) {
     __shared__ NamKey lk[ORDER_WPB][64];
     const uint32_t n = sload(P.n_long);

@@ -37,7 +37,7 @@ struct PairDev {
     uint64_t *totals;     // [8], pinned host words: type starts in tids and their total, joint total, err
     unsigned *err;        // PAIR_ERR_* bits
     uint32_t *n_long;     // lists in longs; 0 between steps, like err
-    uint32_t *longs;      // [2n] lists of more than 32 NAMs, in drop's memory before drop is written
+    uint32_t *longs;      // [2n] lists of more than 64 NAMs, in drop's memory before drop is written
     float dropoff, mu, sigma;
     int max_tries;
     int joint;

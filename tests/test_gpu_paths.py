@@ -441,3 +441,20 @@ def test_joint_entries_placed_by_either_bound(ctx, n):
     lists = ([x for x, _ in few] * reps)[:n] + ([y for _, y in few] * reps)[:n]
     offs, flat = _flatten(lists)
     _compare(G.pairs_from_nams(ctx, offs, flat, n, max_tries=256), O.pairs_batch(offs, flat, n, max_tries=256), offs)
+
+
+@pytest.mark.parametrize("n", [2, 16, 17, 32, 33, 64, 65, 128, 129, 300])
+def test_equal_nams_are_refused_in_lists_of_any_length(ctx, n):
+    rng = np.random.default_rng(n)
+    a, b = _long_mates(rng, n, 3, rng.integers(1, 9, n), rng.integers(1, 9, 3))
+    for i, j in {(0, 1), (0, n - 1), (n // 2, n // 2 - 1)}:
+        x = a.copy()
+        x[i] = x[j]
+        if i == j:
+            continue
+        for lists in ([x, b], [b, x]):
+            offs, flat = _flatten(lists)
+            with pytest.raises(G.GisError):
+                G.pairs_from_nams(ctx, offs, flat, 1, joint=False)
+        offs, flat = _flatten([a, b])
+        _compare(G.pairs_from_nams(ctx, offs, flat, 1, joint=False), O.pairs_batch(offs, flat, 1, joint=False), offs)
