@@ -568,8 +568,8 @@ __global__ __launch_bounds__(PAIR_BLOCK) void k_joint(PairDev P) {
 // The reference's scan over (i, j) is sequential: at each j of a row i it
 // leaves the row when the joint hits fall below half the best pushed so far,
 // ends when more than 2 max_tries entries are pushed, and else pushes (i, j) if
-// the NAMs form a proper pair. Here the cells of all rows are taken in order,
-// 64 at once. The running best and count change at proper cells only, and few
+// the NAMs form a proper pair. Here, in rows of fewer than 64 cells, the cells of
+// all rows are taken in order, 64 at once (longer rows: joint_rows). The running best and count change at proper cells only, and few
 // cells are proper: one step per proper cell tests the cells of its row up to
 // it that were not tested before against the running best and then pushes it
 // or, if one of them fails, drops the row. (A row at a time, 64 columns each,
@@ -689,6 +689,65 @@ struct JointLds {
     }
 };
 
+// The reference's scan a row at a time, 64 columns each: for rows of 64 cells or more.
+// In lists of hundreds of NAMs most cells are never reached: a row is left at the
+// first cell whose hits fall below half the best, and rows that fail at their first
+// cell are passed over together. a0, b0: the lists' first 64 NAMs in the lanes.
+// (100 pairs of a repeat-rich genome, lists of up to 458 NAMs: 0.6 ms, by cells of
+// all rows in order 1.5 ms. A pair of 1000 x 1000 NAMs whose rows end at
+// their first cell: 0.1 ms, by cells 10.3 ms.)
+__device__ __forceinline__ void joint_rows(const gis_nam *A, const gis_nam *B, uint32_t c1, uint32_t c2, int mt,
+                                           float lim, CellNam a0, const CellNam &b0, gis_nam_pair *E, uint32_t *f1,
+                                           uint32_t *f2, uint32_t &size, int &best) {
+    const uint32_t lane = lane_id(), most = 2 * (uint32_t)mt + 1;
+    const int first = __builtin_amdgcn_readfirstlane(b0.nh);
+    uint32_t rows = 0;  // a0: NAMs rows .. rows + 63 of the first list
+    for (uint32_t i = 0; i < c1 && size < most; i++) {
+        if (i == rows + 64) {
+            rows = i;
+            a0 = cell_nam(A[min(i + lane, c1 - 1)]);
+        }
+        // on to the next row whose first cell does not fail (joint < 0.5 * best in
+        // double is 2 joint < best in integers)
+        const uint64_t on = ballot(2 * (a0.nh + first) >= best) >> (i - rows);
+        i = on ? i + (uint32_t)__builtin_ctzll(on) : rows + 64;
+        if (i >= c1) break;
+        if (!on) {  // none of these 64
+            i--;
+            continue;
+        }
+        const uint32_t l = i - rows;
+        const CellNam a{__builtin_amdgcn_readlane(a0.ref_id, (int)l), __builtin_amdgcn_readlane(a0.diag, (int)l),
+                        __builtin_amdgcn_readlane(a0.nh, (int)l), readlane_u32(a0.is_rc, l)};
+        bool left = false;
+        for (uint32_t jc = 0; jc < c2 && !left && size < most; jc += 64) {
+            const uint32_t j = jc + lane;
+            const bool valid = j < c2;
+            CellNam b = b0;
+            if (jc && valid) b = cell_nam(B[j]);
+            const int joint = a.nh + b.nh;
+            uint64_t prop = ballot(valid && proper_cell(a, b, lim)), fail = ballot(valid && 2 * joint < best);
+            // the proper cells before the first that fails, one after the other
+            for (; prop; prop &= prop - 1) {
+                const uint64_t me = prop & (0 - prop);
+                if (fail & (me | (me - 1)) || size == most) break;
+                if (lane_bit(me)) {
+                    E[size] = gis_nam_pair{joint, (int)i, (int)j};
+                    if (i < (uint32_t)mt) f1[i >> 5] |= 1u << (i & 31);
+                    if (j < (uint32_t)mt) f2[j >> 5] |= 1u << (j & 31);
+                }
+                size++;
+                const int jh = __builtin_amdgcn_readlane(joint, __builtin_ctzll(me));
+                if (jh > best) {
+                    best = jh;
+                    fail = ballot(valid && 2 * joint < best) & ~(me | (me - 1));
+                }
+            }
+            left = fail != 0;
+        }
+    }
+}
+
 // the ranks of a list's c < 64 NAMs and of the absent NAM (at c) under the
 // comparator's NAM part; true if a score is a NaN
 __device__ __forceinline__ bool rank_nams(const gis_nam *L, uint32_t c, uint8_t *ranks) {
@@ -722,43 +781,29 @@ __global__ __launch_bounds__(64 * JOINT_WPB) void k_joint_wave(PairDev P, uint32
         }
         const gis_nam *A = P.ord + o1, *B = P.ord + o2;
         gis_nam_pair *out = P.jtmp + joint_place(P, p, o1, o2);
-        // hits of the first 64 NAMs of each list (lane i: NAM i)
-        int nh1 = 0, nh2 = 0;
-        if (lane < c1) {
-            const CellNam c = cell_nam(A[lane]);
-            ca[lane] = c;
-            nh1 = c.nh;
-        }
-        if (lane < c2) {
-            const CellNam c = cell_nam(B[lane]);
-            cb[lane] = c;
-            nh2 = c.nh;
-        }
+        // the first 64 NAMs of each list (lane i: NAM i)
+        CellNam a0{}, b0{};
+        if (lane < c1) ca[lane] = a0 = cell_nam(A[lane]);
+        if (lane < c2) cb[lane] = b0 = cell_nam(B[lane]);
+        const int nh1 = a0.nh, nh2 = b0.nh;
         if (lane < 2 * FLAG_WORDS) f1[lane] = 0;
         wave_sync();
-        const bool in_lds = c1 <= 64 && c2 <= 64;
         const uint32_t most = 2 * (uint32_t)mt + 1;
         uint32_t size = 0;
         int best = 0;
         const uint64_t cells = (uint64_t)c1 * c2;
-        // this lane's cell, 64 further on each pass, or, after a row that was left, at
-        // the next row whose first cell does not fail: in lists of hundreds of NAMs
-        // most cells are never reached. (A pair of 1000 x 1000 whose rows end at
-        // their first cell: 10.3 ms with a step for every 64 cells of a row left,
-        // 0.53 ms a row at a time, now 0.09 ms.)
-        const uint32_t i_row = lane / c2, j_row = lane % c2;
-        uint32_t i = i_row, j = j_row;
+        // rows of 64 cells or more fill the lanes by themselves
+        if (c2 >= 64) joint_rows(A, B, c1, c2, mt, lim, a0, b0, E, f1, f2, size, best);
+        // this lane's cell, 64 further on each pass
+        uint32_t i = lane / c2, j = lane % c2;
         const uint32_t di = 64 / c2, dj = 64 % c2;
         uint32_t dead = 0xffffffffu;  // the row left last
-        uint32_t rows = 0;  // lane l's nh_row: the hits of row rows + l
-        int nh_row = nh1;
-        for (uint64_t q0 = 0; q0 < cells && size < most;) {
+        for (uint64_t q0 = 0; c2 < 64 && q0 < cells && size < most; q0 += 64) {
             const bool valid = lane < cells - q0;
             bool prop = false;
             int joint = 0;
             if (valid) {
-                const CellNam a = in_lds || i < 64 ? ca[i] : cell_nam(A[i]);
-                const CellNam b = in_lds || j < 64 ? cb[j] : cell_nam(B[j]);
+                const CellNam a = i < 64 ? ca[i] : cell_nam(A[i]), b = cb[j];
                 joint = a.nh + b.nh;
                 prop = proper_cell(a, b, lim);
             }
@@ -795,25 +840,6 @@ __global__ __launch_bounds__(64 * JOINT_WPB) void k_joint_wave(PairDev P, uint32
                 }
                 dead = readlane_u32(i, (uint32_t)__builtin_ctzll(drop));
                 rem &= ballot(i > dead);
-            }
-            q0 += 64;
-            uint32_t row = dead + 1u;  // (0: no row was left yet)
-            if (q0 < (uint64_t)row * c2) {
-                const int first = __builtin_amdgcn_readfirstlane(nh2);
-                while (row < c1) {
-                    if (row >= rows + 64) {
-                        rows = row;
-                        nh_row = A[min(row + lane, c1 - 1)].n_hits;
-                    }
-                    const uint64_t on = ballot(rows + lane >= c1 || 2 * (nh_row + first) >= best) >> (row - rows);
-                    row = on ? row + (uint32_t)__builtin_ctzll(on) : rows + 64;
-                    if (on) break;
-                }
-                dead = row - 1;
-                q0 = (uint64_t)row * c2;
-                i = row + i_row;
-                j = j_row;
-                continue;
             }
             i += di;
             j += dj;
