@@ -387,12 +387,14 @@ __global__ void k_pair_totals(PairDev P) {
     }
 }
 
-// where pair p's joint entries are put before their offsets are known: after the
-// bounds c1 + c2 + 2 max_tries + 1 of the pairs before it, which needs no scan
-// (and no wait for its total), or after their exact bounds (k_joint_bounds)
+// where pair p's joint entries are put before their offsets are known: after bounds
+// of those of the pairs before it that are linear in their lists' lengths (PairDev),
+// which needs no scan and no wait for its total, or after their exact bounds
+// (k_joint_bounds)
 __device__ __forceinline__ uint64_t joint_place(const PairDev &P, uint32_t p, uint64_t o1, uint64_t o2) {
     if (P.jplace) return P.jplace[p];
-    return o1 + (o2 - P.off[P.n_pairs]) + (uint64_t)p * (2 * (uint32_t)P.max_tries + 1);
+    const uint64_t s = o1 + (o2 - P.off[P.n_pairs]);
+    return s + (s * P.jmul >> 16) + (uint64_t)p * P.jadd;
 }
 
 // exact bounds of the pairs' entries, for joint_place once scanned
@@ -569,11 +571,11 @@ __global__ __launch_bounds__(PAIR_BLOCK) void k_joint(PairDev P) {
 // leaves the row when the joint hits fall below half the best pushed so far,
 // ends when more than 2 max_tries entries are pushed, and else pushes (i, j) if
 // the NAMs form a proper pair. Here, in rows of fewer than 64 cells, the cells of
-// all rows are taken in order, 64 at once (longer rows: joint_rows). The running best and count change at proper cells only, and few
-// cells are proper: one step per proper cell tests the cells of its row up to
-// it that were not tested before against the running best and then pushes it
-// or, if one of them fails, drops the row. (A row at a time, 64 columns each,
-// left most lanes idle: lists are of 7.8 NAMs on average.)
+// all rows are taken in order, 64 at once (longer rows: joint_rows). The running
+// best and count change at proper cells only, and few cells are proper: one step
+// per proper cell tests the cells of its row up to it that were not tested before
+// against the running best and then pushes it or, if one of them fails, drops the
+// row. (A row at a time left most lanes idle: lists are of 7.8 NAMs on average.)
 // The entries are then sorted by counting smaller ones. For that each list's NAMs
 // get their rank under the comparator's NAM part, ties sharing one, so that an
 // entry is one word: score, rank, rank. Without equal entries the sorted order is

@@ -4,7 +4,7 @@
 // order, pair types, per-type lists and, with GIS_PAIRS_JOINT, the joint NAM
 // pairs. The joint entries are placed by bounds that follow from the list
 // offsets, so nothing is read back in between (unless those bounds are large:
-// LOOSE_ENTRIES); the last kernel writes the type
+// LINEAR_ENTRIES); the last kernel writes the type
 // counts, the entry total and the error bits to pinned memory, read after one
 // synchronisation. The compacted entries have the room of earlier steps or one
 // NAM's worth of entries; where the total is larger, the compaction alone runs
@@ -67,10 +67,11 @@ static int check_params(gis_ctx *ctx, const gis_pair_params &pp) {
     return GIS_OK;
 }
 
-// joint entries up to which they are placed by the loose bound (192 MB): each pair
-// has room for 2 max_tries + 1 entries beside its lists, whatever these hold, 6 KB
-// at max_tries = 256. Beyond, their exact bounds are scanned and waited for.
-constexpr uint64_t LOOSE_ENTRIES = 16u << 20;
+// Joint entries up to which they are placed by a linear bound (400 MB), the smaller of
+// the two: room for 2 max_tries + 1 of a pair beside its lists (41 at 20 tries; at
+// 256 tries 6 KB a pair whatever its lists hold), or for 3.2 (20 tries) to 11.3 (256)
+// beside each NAM. Beyond, their exact bounds are scanned and waited for.
+constexpr uint64_t LINEAR_ENTRIES = 32u << 20;
 
 // the pair step on device lists off[2n+1] / in
 static int pairs_run(gis_ctx *ctx, PairWork &w, hipStream_t st, const uint64_t *off, const gis_nam *in,
@@ -109,8 +110,15 @@ static int pairs_run(gis_ctx *ctx, PairWork &w, hipStream_t st, const uint64_t *
     uint64_t *tmp = ensure<uint64_t>(w.scan_tmp, scan_tmp_words(std::max<uint64_t>(5 * nb, n_pairs)));
     w.owner = nullptr;
     if (P.joint) {
-        uint64_t entries = n_nams + (uint64_t)n_pairs * (2ull * P.max_tries + 1);
-        if (entries > LOOSE_ENTRIES) {
+        const uint64_t most = 2ull * P.max_tries + 1;
+        P.jmul = (uint64_t)std::ceil(std::sqrt((double)most) * 32768.0);
+        uint64_t entries = n_nams + (n_nams * P.jmul >> 16);
+        if (n_nams + n_pairs * most < entries) {
+            P.jmul = 0;
+            P.jadd = most;
+            entries = n_nams + n_pairs * most;
+        }
+        if (entries > LINEAR_ENTRIES) {
             uint64_t *place = ensure<uint64_t>(w.jplace, n_pairs + 1ull);
             launch_joint_bounds(P, place, tmp, st);
             HIP_CHECK(hipGetLastError());

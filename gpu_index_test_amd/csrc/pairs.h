@@ -29,7 +29,12 @@ struct PairDev {
     uint32_t *tids;       // [n] pair ids grouped by type
     uint32_t nblk;
     gis_nam_pair *jtmp;   // entries at joint_place()
-    const uint64_t *jplace; // [n+1] the pairs' places in jtmp (null: by the loose bound)
+    const uint64_t *jplace; // [n+1] the pairs' places in jtmp (null: by a linear bound)
+    // A pair of lists of c1 and c2 NAMs, M = 2 max_tries + 1, has at most
+    // min(c1 c2, M) + c1 + c2 entries: at most c1 + c2 + jadd with jadd = M, and at
+    // most c1 + c2 + (c1 + c2) jmul / 2^16 with jmul / 2^16 >= sqrt(M) / 2 (c1 c2 is at
+    // most x^2, x = (c1 + c2) / 2, and min(x^2, M) at most x sqrt(M)). One of the two.
+    uint64_t jmul, jadd;
     uint32_t *jcnt;       // [n]
     const uint64_t *joff; // [n+1]
     gis_nam_pair *jout;   // entries at joff

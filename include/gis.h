@@ -468,8 +468,9 @@ typedef struct {
 
 /* Run the pair step on the NAMs of the batch's last run (2 n reads, mates laid
  * out as above); results stay on the device until downloaded. With
- * GIS_PAIRS_JOINT it holds 12 bytes per NAM and 24 max_tries + 12 per pair for
- * the entries, or beyond 192 MB in all what the lists' own lengths allow. */
+ * GIS_PAIRS_JOINT it also holds room for the entries: 12 bytes per NAM and the
+ * smaller of 24 max_tries + 12 per pair and 6 sqrt(2 max_tries + 1) per NAM, or
+ * beyond 400 MB in all what the single lists' lengths allow. */
 int gis_batch_pairs(gis_batch *b, const gis_pair_params *pp);
 /* Copy the pair step's results out. GIS_ERR_CAPACITY (with n_nams / n_joint
  * set) if nam_capacity or joint_capacity is too small. */

@@ -427,20 +427,25 @@ def test_order_time_of_long_lists(ctx):
         _compare(G.pairs_from_nams(ctx, offs, flat, n, joint=False), O.pairs_batch(offs, flat, n, joint=False), offs)
 
 
-@pytest.mark.parametrize("n", [32_000, 32_200])
-def test_joint_entries_placed_by_either_bound(ctx, n):
-    """Around 2^24 entries by the loose bound (513 a pair beside its NAMs) the pairs'
-    places come from their exact bounds."""
+@pytest.mark.parametrize("n,max_tries", [(1, 256), (3000, 1), (3000, 40), (3000, 256), (72_500, 256), (75_000, 256)])
+def test_joint_entries_placed_by_any_bound(ctx, n, max_tries):
+    """The pairs' places come from the smaller of two bounds linear in their lists'
+    lengths, and from their exact bounds where that is more than 2^25 entries (the
+    last case; the one before it just is not)."""
     rng = np.random.default_rng(5)
     sizes = [0, 1, 2, 5, 17, 33, 70]
     some = [_long_mates(rng, max(a, 1), max(b, 1), rng.integers(1, 9, max(a, 1)), rng.integers(1, 9, max(b, 1)))
             for a in sizes for b in sizes]
-    few = [(x[:a], y[:b]) for (x, y), a, b in zip(some, np.repeat(sizes, 7), np.tile(sizes, 7))]
-    few += [few[1]] * 151  # most lists short
-    reps = -(-n // len(few))
-    lists = ([x for x, _ in few] * reps)[:n] + ([y for _, y in few] * reps)[:n]
+    some = [(x[:a], y[:b]) for (x, y), a, b in zip(some, np.repeat(sizes, 7), np.tile(sizes, 7))]
+    if n == 3000:  # mostly short lists
+        some += [some[8]] * 100
+    reps = -(-n // len(some))
+    lists = ([x for x, _ in some] * reps)[:n] + ([y for _, y in some] * reps)[:n]
     offs, flat = _flatten(lists)
-    _compare(G.pairs_from_nams(ctx, offs, flat, n, max_tries=256), O.pairs_batch(offs, flat, n, max_tries=256), offs)
+    linear = len(flat) + min(int(len(flat) * np.sqrt(2 * max_tries + 1) / 2), n * (2 * max_tries + 1))
+    assert (linear > 2 ** 25) == (n == 75_000) and (n < 72_500 or abs(linear / 2 ** 25 - 1) < 0.03)
+    _compare(G.pairs_from_nams(ctx, offs, flat, n, max_tries=max_tries), O.pairs_batch(offs, flat, n, max_tries=max_tries),
+             offs)
 
 
 @pytest.mark.parametrize("n", [2, 16, 17, 32, 33, 64, 65, 128, 129, 300])
