@@ -31,8 +31,8 @@ constexpr uint64_t THREADS_MIN = 4;
 // bytes of the arrays that one kernel writes beside a large copy
 constexpr uint64_t SMALL_MAX = 8 << 20;
 // arrays below this go the runtime's way, which copies them through its own pinned
-// memory
-constexpr size_t STAGE_MIN = 512 << 10;
+// memory (0.79 MB: 51 us, in chunks 56; 1.4 MB: 93 and 89)
+constexpr size_t STAGE_MIN = 1 << 20;
 
 }  // namespace
 
