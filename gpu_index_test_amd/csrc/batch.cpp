@@ -412,6 +412,7 @@ int batch_stage(gis_batch *b, const char *seqs, const uint64_t *offsets, const u
         b->h_long_off[r + 1] = long_at;
     }
     b->n_reads = n;
+    b->staged++;
     b->host_out = false;
     b->want_sy = want_sy;
     b->n_long = n_long;
@@ -642,9 +643,11 @@ constexpr uint32_t TURN_READS = 16384;
 void batch_launch(gis_batch *b, const RunOpts &r, bool in_turn) {
     gis_ctx *ctx = b->ctx;
     hipStream_t st = b->stream;
-    prepare_workspace(b);
+    // (first: arrays of the workspace may move, also where a later one finds no memory)
     b->ws->owner = b;
     b->ran = false;
+    b->last_run = RunId{b->staged, ctx->ix.epoch, r.rcut, r.hard};
+    prepare_workspace(b);
     if (r.mode == GIS_MODE_FUSED && r.stop == STOP_NONE) {
         if (!b->queue_ok) throw HipError{hipErrorInvalidValue, "fused run of reads staged without the work queue"};
         ensure<gis_nam>(b->ws->nam_slots, (size_t)b->n_reads * F_NAMCAP);
@@ -709,7 +712,9 @@ void batch_complete(gis_batch *b, const RunOpts &r) {
     b->last_mode = r.mode;
     b->last_graph = r.graph;
     b->ran = r.stop == STOP_NONE;
-    if (b->ran) note_nams(b);
+    if (!b->ran) return;
+    b->last_run.over = true;
+    note_nams(b);
 }
 
 void batch_run(gis_batch *b, const gis_map_options &o, int rescue_mode, int stop) {

@@ -99,6 +99,16 @@ struct Workspace {
     PairWork *pairs = nullptr;    // the pair step on this workspace's NAMs (pairs.cpp)
 };
 
+// what the NAMs of a run depend on: runs of a batch that agree in it have the same
+struct RunId {
+    uint64_t staged = 0, epoch = 0;
+    uint32_t rcut = 0, hard = 0;
+    bool over = false;
+    bool same(const RunId &o) const {
+        return over && o.over && staged == o.staged && epoch == o.epoch && rcut == o.rcut && hard == o.hard;
+    }
+};
+
 }  // namespace gis
 
 struct gis_batch {
@@ -130,6 +140,8 @@ struct gis_batch {
     bool lazy_graph = false;
     int last_mode = GIS_MODE_PLAIN;
     bool last_graph = false;
+    uint64_t staged = 0;      // how often reads were staged
+    gis::RunId last_run;      // of the run launched last
     bool ran = false;
     hipEvent_t ev[16] = {};
     int n_ev = 0;

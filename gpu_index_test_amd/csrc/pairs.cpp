@@ -29,7 +29,7 @@ struct PairWork {
     DevBuf ord, types, drop, mapq, tcnt, tpos, tids, jtmp, jcnt, joff, jout, jplace, err, scan_tmp;
     uint64_t *h = nullptr;  // pinned: [0..5] type starts, [6] joint total, [7] error bits
     const void *owner = nullptr;  // the batch (or context) whose lists the results belong to
-    const uint64_t *dev_off = nullptr;
+    RunId run;                    // and the batch's run that made the lists
     uint32_t n_pairs = 0;
     uint64_t n_nams = 0, n_joint = 0;
     uint32_t type_counts[5] = {};
@@ -154,11 +154,11 @@ static int pairs_run(gis_ctx *ctx, PairWork &w, hipStream_t st, const uint64_t *
     w.n_nams = n_nams;
     w.n_joint = h[6];
     w.joint = P.joint != 0;
-    w.dev_off = off;
     return GIS_OK;
 }
 
-static int pairs_download(gis_ctx *ctx, PairWork &w, hipStream_t st, gis_pair_out *out) {
+// off: the lists' offsets (not kept from the step: the batch's arrays may have moved)
+static int pairs_download(gis_ctx *ctx, PairWork &w, const uint64_t *off, hipStream_t st, gis_pair_out *out) {
     if (!out) return fail(ctx, GIS_ERR_BAD_PARAMETER, "null output");
     const uint32_t n = w.n_pairs;
     out->n_nams = w.n_nams;
@@ -174,7 +174,7 @@ static int pairs_download(gis_ctx *ctx, PairWork &w, hipStream_t st, gis_pair_ou
     auto add = [&](void *dst, const void *src, size_t bytes) {
         if (dst && bytes) small.push_back({dst, src, bytes});
     };
-    add(out->nam_offsets, w.dev_off, 8ull * (2ull * n + 1));
+    add(out->nam_offsets, off, 8ull * (2ull * n + 1));
     add(out->types, w.types.p, n);
     add(out->type_ids, w.tids.p, 4ull * n);
     add(out->top_dropoff, w.drop.p, 8ull * n);
@@ -217,8 +217,10 @@ extern "C" int gis_batch_pairs(gis_batch *b, const gis_pair_params *pp) {
     PairWork *w = pairwork_get(b->ws->pairs);
     int rc = pairs_run(ctx, *w, b->stream, static_cast<const uint64_t *>(b->ws->nam_off.p),
                        static_cast<const gis_nam *>(b->ws->nams_out.p), b->ws->tot_nams, b->n_reads / 2, 1, p);
-    if (rc == GIS_OK) w->owner = b;
-    return rc;
+    if (rc) return rc;
+    w->owner = b;
+    w->run = b->last_run;
+    return GIS_OK;
     API_END(ctx)
 }
 
@@ -227,9 +229,9 @@ extern "C" int gis_batch_pairs_download(gis_batch *b, gis_pair_out *out) {
     gis_ctx *ctx = b->ctx;
     API_BEGIN(ctx)
     PairWork *w = b->ws->pairs;
-    if (!w || w->owner != b || b->ws->owner != b)
+    if (!w || w->owner != b || b->ws->owner != b || !w->run.same(b->last_run))
         return fail(ctx, GIS_ERR_STATE, "no pair step of this batch's last run");
-    return pairs_download(ctx, *w, b->stream, out);
+    return pairs_download(ctx, *w, static_cast<const uint64_t *>(b->ws->nam_off.p), b->stream, out);
     API_END(ctx)
 }
 
@@ -256,6 +258,6 @@ extern "C" int gis_pairs_from_nams(gis_ctx *ctx, const uint64_t *nam_offsets, co
     int rc = pairs_run(ctx, *w, ctx->stream, doff, dn, total, n_pairs, 0, p);
     if (rc) return rc;
     w->owner = ctx;
-    return pairs_download(ctx, *w, ctx->stream, out);
+    return pairs_download(ctx, *w, doff, ctx->stream, out);
     API_END(ctx)
 }

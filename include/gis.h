@@ -473,7 +473,8 @@ typedef struct {
  * beyond 400 MB in all what the single lists' lengths allow. */
 int gis_batch_pairs(gis_batch *b, const gis_pair_params *pp);
 /* Copy the pair step's results out. GIS_ERR_CAPACITY (with n_nams / n_joint
- * set) if nam_capacity or joint_capacity is too small. */
+ * set) if nam_capacity or joint_capacity is too small; GIS_ERR_STATE if the batch
+ * has been run again since, unless with the same reads, index and cutoffs. */
 int gis_batch_pairs_download(gis_batch *b, gis_pair_out *out);
 /* The pair step on NAM lists from host memory (any order within a list;
  * NAMs of one list must differ in (is_rc, ref_id, query_start, ref_start)). */

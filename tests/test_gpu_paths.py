@@ -463,3 +463,46 @@ def test_equal_nams_are_refused_in_lists_of_any_length(ctx, n):
                 G.pairs_from_nams(ctx, offs, flat, 1, joint=False)
         offs, flat = _flatten([a, b])
         _compare(G.pairs_from_nams(ctx, offs, flat, 1, joint=False), O.pairs_batch(offs, flat, 1, joint=False), offs)
+
+
+def test_pair_results_are_of_the_last_run(ctx):
+    """A pair step's results can be read until other reads are run, or the same ones with
+    other cutoffs; reads run again as they were have the same NAMs."""
+    g, lens = G.synth_genome(200_000, n_contigs=2, gc=0.45, repeat_fraction=0.5, n_families=12,
+                             family_len=(400, 1500), copies=(2, 40), divergence=(0.0, 0.005), seed=3)
+    idx = G.StrobemerIndex(None, G.IndexParameters.from_read_length(150))
+    idx.populate_arrays(g, lens)
+    s, o, l, _ = G.synth_reads(g, lens, 3000, lengths=(100, 150), weights=(1, 1), sub_rate=0.01, seed=4)
+    m = G.Mapper(idx, 20, 20 * 150)
+    m.upload(s, o[:20], l[:20])
+    m.run()
+    want = m.pairs()
+    m.run()
+    m.run(mode=G.MODE_FUSED)
+    again = m.pairs_download()
+    assert again.nams.tobytes() == want.nams.tobytes() and np.array_equal(again.nam_offsets, want.nam_offsets)
+    m.run(rescue_level=100, hard_cutoff=5)
+    with pytest.raises(G.GisError):
+        m.pairs_download()
+    m.run()
+    assert m.pairs_download().nams.tobytes() == want.nams.tobytes()
+    m2 = G.Mapper(idx, 20, 20 * 150, share=m)
+    m.upload(s, o, l)  # (the batch's arrays grow with the run)
+    m.run()
+    with pytest.raises(G.GisError):
+        m.pairs_download()
+    assert len(m.pairs().types) == 1500
+    # another batch of the workspace between
+    m2.upload(s, o[:20], l[:20])
+    m2.run()
+    with pytest.raises(G.GisError):
+        m.pairs_download()
+    assert m2.pairs().nams.tobytes() == want.nams.tobytes()
+    m.run()
+    with pytest.raises(G.GisError):
+        m2.pairs_download()
+    m2.run()
+    assert m2.pairs_download().nams.tobytes() == want.nams.tobytes()
+    for x in (m2, m):
+        x.close()
+    idx.ctx.close()
