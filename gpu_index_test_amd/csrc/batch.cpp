@@ -224,16 +224,6 @@ static bool copy_in(gis_batch *b, const std::vector<CopyItem> &items) {
     return small;
 }
 
-// waits for the stream when a call leaves it early, so that the pinned blocks and
-// the caller's arrays are free
-struct StreamGuard {
-    hipStream_t st;
-    bool armed = true;
-    ~StreamGuard() {
-        if (armed) (void)hipStreamSynchronize(st);
-    }
-};
-
 DevBatch make_devbatch(gis_batch *b) {
     DevBatch d{};
     d.seqs = static_cast<const char *>(b->seqs.p);

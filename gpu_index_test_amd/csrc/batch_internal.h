@@ -99,6 +99,16 @@ struct Workspace {
     PairWork *pairs = nullptr;    // the pair step on this workspace's NAMs (pairs.cpp)
 };
 
+// waits for the stream when a call leaves it early, so that the pinned blocks and
+// the caller's arrays are free
+struct StreamGuard {
+    hipStream_t st;
+    bool armed = true;
+    ~StreamGuard() {
+        if (armed) (void)hipStreamSynchronize(st);
+    }
+};
+
 // what the NAMs of a run depend on: runs of a batch that agree in it have the same
 struct RunId {
     uint64_t staged = 0, epoch = 0;

@@ -253,9 +253,11 @@ extern "C" int gis_pairs_from_nams(gis_ctx *ctx, const uint64_t *nam_offsets, co
     PairWork *w = pairwork_get(ctx->pairs);
     uint64_t *doff = ensure<uint64_t>(w->in_off, n_lists + 1);
     gis_nam *dn = ensure<gis_nam>(w->in_nams, total);
+    StreamGuard guard{ctx->stream};
     HIP_CHECK(hipMemcpyAsync(doff, nam_offsets, 8 * (n_lists + 1), hipMemcpyHostToDevice, ctx->stream));
     if (total) HIP_CHECK(hipMemcpyAsync(dn, nams, sizeof(gis_nam) * total, hipMemcpyHostToDevice, ctx->stream));
     int rc = pairs_run(ctx, *w, ctx->stream, doff, dn, total, n_pairs, 0, p);
+    guard.armed = false;
     if (rc) return rc;
     w->owner = ctx;
     return pairs_download(ctx, *w, doff, ctx->stream, out);

@@ -395,6 +395,50 @@ static void pairs_memory() {
     gis_ctx_destroy(ctx);
 }
 
+// A call on NAM lists that finds no memory once their copies are in flight waits for
+// them before it returns the caller's arrays.
+static void pairs_failure() {
+    const uint32_t n = 2000, each = 20;
+    std::vector<uint64_t> off(2 * n + 1);
+    std::vector<gis_nam> nams(2 * n * each);
+    for (uint32_t r = 0; r < 2 * n; r++) {
+        off[r + 1] = (r + 1ull) * each;
+        for (uint32_t i = 0; i < each; i++) {
+            gis_nam &x = nams[(size_t)r * each + i];
+            x = gis_nam{};
+            x.query_end = 50;
+            x.ref_start = 1000 + 100 * (int)i + (r < n ? 0 : 200);
+            x.ref_end = x.ref_start + 50;
+            x.n_hits = 3;
+            x.score = 30;
+            x.is_rc = r >= n;
+        }
+    }
+    gis_pair_params p;
+    gis_pair_params_default(&p);
+    std::vector<uint8_t> types(n), want(n);
+    gis_pair_out o{};
+    o.types = want.data();
+    gis_ctx *ctx = context();
+    EXPECT(gis_pairs_from_nams(ctx, off.data(), nams.data(), n, &p, &o) == GIS_OK);
+    gis_ctx_destroy(ctx);
+    ctx = context();
+    o.types = types.data();
+    int failed = 0, rc = GIS_ERR_HIP;
+    const uint64_t lists = off.size() * 8 + nams.size() * sizeof(gis_nam);
+    for (g_limit = g_live + lists; rc; g_limit += lists / 4) {
+        g_copy.clear();
+        g_sync.clear();
+        rc = gis_pairs_from_nams(ctx, off.data(), nams.data(), n, &p, &o);
+        EXPECT(rc == GIS_OK || rc == GIS_ERR_HIP);
+        if (rc && !g_copy.empty()) failed++;
+        for (const auto &c : g_copy) EXPECT(g_sync.count(c.first) && g_sync[c.first] > c.second);
+    }
+    EXPECT(failed > 0 && types == want);
+    g_limit = ~0ull;
+    gis_ctx_destroy(ctx);
+}
+
 struct Nams {
     std::vector<uint64_t> off;
     std::vector<gis_nam> nams;
@@ -560,6 +604,7 @@ int main(int argc, char **argv) {
         void (*run)();
     } cases[] = {{"pinned_ranges", pinned_ranges}, {"stream_failure", stream_failure}, {"replace_index", replace_index}, {"index_bytes", index_bytes},
                  {"pairs_memory", pairs_memory},
+                 {"pairs_failure", pairs_failure},
                  {"dense_calls", dense_calls},
                  {"moved_scratch", moved_scratch},
                  {"graphs_kept", graphs_kept}, {"stalled_copy", stalled_copy}};
