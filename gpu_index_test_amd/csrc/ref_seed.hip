@@ -340,7 +340,8 @@ RefSeeds device_seed_reference(const char *const *seqs, const uint64_t *lens, ui
     RefSeeds out;
     const SeedParams P = make_seed_params(gp);
     // contig c at cstart[c], one 'N' after each; cstart[n_refs] = T
-    std::vector<uint64_t> cstart(n_refs + 1);
+    std::vector<uint64_t> cstart(n_refs + 1), sy_start(n_refs + 1), rs_start(n_refs + 1);
+    std::vector<uint8_t> is_short(std::max<uint32_t>(n_refs, 1), 0);
     uint64_t T = 0, longest = 0;
     for (uint32_t c = 0; c < n_refs; c++) {
         cstart[c] = T;
@@ -407,10 +408,8 @@ RefSeeds device_seed_reference(const char *const *seqs, const uint64_t *lens, ui
     hipLaunchKernelGGL(k_ref_contig_syncmers, dim3(grid(n_refs + 1, 256)), dim3(256), 0, st, pos, nsy, cs, n_refs,
                        sys);
     check(hipGetLastError(), "k_ref_contig_syncmers");
-    std::vector<uint64_t> sy_start(n_refs + 1), rs_start(n_refs + 1);
     check(hipMemcpyAsync(sy_start.data(), sys, 8ull * (n_refs + 1), hipMemcpyDeviceToHost, st), "syncmer ranges");
     check(hipStreamSynchronize(st), "syncmer ranges");
-    std::vector<uint8_t> is_short(std::max<uint32_t>(n_refs, 1), 0);
     uint64_t total = 0;
     for (uint32_t c = 0; c < n_refs; c++) {
         rs_start[c] = total;

@@ -61,7 +61,29 @@ struct Dim3 {
     uint32_t x, y, z;
 };
 
+// host arrays of copies in to the device that their streams were not waited for since
+struct Src {
+    const char *p;
+    size_t n;
+    void *st;
+};
+constexpr int MAX_SRC = 4096;
+Src g_src[MAX_SRC];
+int g_n_src = 0;
+std::mutex g_src_mu;             // (not g_mu, under which memory is freed)
+std::atomic<int> g_freed{0};     // those freed all the same
+
 }  // namespace
+
+void operator delete(void *p) noexcept {
+    const char *c = static_cast<const char *>(p);
+    if (c) {
+        std::lock_guard<std::mutex> l(g_src_mu);
+        for (int i = 0; i < g_n_src; i++) g_freed += g_src[i].p == c;
+    }
+    std::free(p);
+}
+void operator delete(void *p, size_t) noexcept { operator delete(p); }
 
 extern "C" int hipMalloc(void **p, size_t n) {
     static const auto f = real<int (*)(void **, size_t)>("hipMalloc");
@@ -100,12 +122,20 @@ extern "C" int hipMemcpyAsync(void *d, const void *s, size_t n, int kind, void *
         std::lock_guard<std::mutex> l(g_mu);
         if (kind == 1) g_copy[st] = ++g_clock;
     }
+    if (kind == 1) {
+        std::lock_guard<std::mutex> l(g_src_mu);
+        if (g_n_src < MAX_SRC) g_src[g_n_src++] = {static_cast<const char *>(s), n, st};
+    }
     return f(d, s, n, kind, st);
 }
 
 extern "C" int hipStreamSynchronize(void *st) {
     static const auto f = real<int (*)(void *)>("hipStreamSynchronize");
     const int e = f(st);
+    {
+        std::lock_guard<std::mutex> l(g_src_mu);
+        g_n_src = (int)(std::remove_if(g_src, g_src + g_n_src, [&](const Src &x) { return x.st == st; }) - g_src);
+    }
     std::lock_guard<std::mutex> l(g_mu);
     g_sync[st] = ++g_clock;
     return e;
@@ -347,6 +377,30 @@ static void replace_index() {
     std::remove(path.c_str());
 }
 
+// Seeding a reference that finds no memory, at any of its arrays, frees no host array
+// that a copy to the device may still read.
+static void build_failure() {
+    const Genome g = genome(3000000, 40, 12);
+    uint64_t total = 0, n = 0;
+    for (uint64_t x : g.lens) total += x;
+    const gis_params p = params(150);
+    gis_ctx *ctx = context();
+    const auto at = g.at();
+    int failed = 0, rc = GIS_ERR_HIP;
+    std::vector<gis_ref_randstrobe> out(total);
+    for (g_limit = g_live + (1 << 16); rc; g_limit += 1 << 19) {
+        g_freed = 0;
+        rc = gis_reference_randstrobes(ctx, at.data(), g.lens.data(), (uint32_t)g.lens.size(), &p, out.data(), total,
+                                       &n);
+        EXPECT(rc == GIS_OK || rc == GIS_ERR_HIP);
+        EXPECT(g_freed == 0);
+        failed += rc != GIS_OK;
+    }
+    EXPECT(failed > 8 && n > 0);
+    g_limit = UINT64_MAX;
+    gis_ctx_destroy(ctx);
+}
+
 // an index's device bytes are those of its table, whatever was resident before it
 static void index_bytes() {
     const Genome small = genome(100000, 1, 7), large = genome(1000000, 1, 8);
@@ -435,7 +489,7 @@ static void pairs_failure() {
         for (const auto &c : g_copy) EXPECT(g_sync.count(c.first) && g_sync[c.first] > c.second);
     }
     EXPECT(failed > 0 && types == want);
-    g_limit = ~0ull;
+    g_limit = UINT64_MAX;
     gis_ctx_destroy(ctx);
 }
 
@@ -603,6 +657,7 @@ int main(int argc, char **argv) {
         const char *name;
         void (*run)();
     } cases[] = {{"pinned_ranges", pinned_ranges}, {"stream_failure", stream_failure}, {"replace_index", replace_index}, {"index_bytes", index_bytes},
+                 {"build_failure", build_failure},
                  {"pairs_memory", pairs_memory},
                  {"pairs_failure", pairs_failure},
                  {"dense_calls", dense_calls},
