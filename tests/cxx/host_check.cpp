@@ -621,6 +621,35 @@ static void graphs_kept() {
     gis_ctx_destroy(ctx);
 }
 
+// files of uneven reads mapped in turn: 16 configurations of one lane
+static void stream_graphs() {
+    const Genome g = genome(300000, 1, 16);
+    gis_ctx *ctx = context();
+    EXPECT(build(ctx, g) == GIS_OK);
+    const uint32_t FILES = 4, PER = 1000, BATCHES = 4;
+    std::vector<Reads> files;
+    for (uint32_t f = 0; f < FILES; f++) {
+        Reads r;
+        for (uint32_t i = 0; i < BATCHES; i++) {
+            const uint32_t longer = 100 + 50 * (f * BATCHES + i);
+            r.add(reads(g, PER - longer, 100, 17 + f));
+            r.add(reads(g, longer, 300, 18 + f));
+        }
+        files.push_back(std::move(r));
+    }
+    Nams out(PER * BATCHES, 400000);
+    uint64_t made = 0;
+    for (int pass = 0; pass < 4; pass++) {  // (the arrays have their size after the first)
+        const uint64_t before = g_made;
+        for (const Reads &r : files)
+            EXPECT(gis_find_nams_stream(ctx, r.seqs.data(), r.offs.data(), r.lens.data(), r.n(), PER, 1, nullptr, &out.o,
+                                        nullptr) == GIS_OK);
+        made = g_made - before;
+    }
+    EXPECT(made == 0);
+    gis_ctx_destroy(ctx);
+}
+
 // threads of a copy that wait for a chunk the GPU is late with use no CPU time
 static void stalled_copy() {
     const Genome g = genome(300000, 1, 16);
@@ -662,7 +691,7 @@ int main(int argc, char **argv) {
                  {"pairs_failure", pairs_failure},
                  {"dense_calls", dense_calls},
                  {"moved_scratch", moved_scratch},
-                 {"graphs_kept", graphs_kept}, {"stalled_copy", stalled_copy}};
+                 {"graphs_kept", graphs_kept}, {"stream_graphs", stream_graphs}, {"stalled_copy", stalled_copy}};
     for (const auto &c : cases)
         if (argc == 2 && !std::strcmp(argv[1], c.name)) {
             c.run();
